@@ -1,0 +1,761 @@
+// K4 for shapes the tuned kernels do not take: fp32 q, k, v; any head dim up to 128; any
+// group size; block sizes 16 .. 256; dense attention of those types and head dims.
+//
+// Reference: pisa_pg_fwd_kernel, svg/kernels/triton/group_pisa_attention.py:135-262; any float
+// dtype (:380), any group size (:312) and any power-of-two block size (:311).  Rounding: for
+// 16-bit inputs kc, vc and Hbar are rounded to the input type at their use, P and P-bar before
+// their products, and the output at its store, as the reference does; fp32 inputs are not
+// rounded anywhere.
+//
+// Every product runs on the 16x16 MFMAs: 16x16x32 for bf16 and fp16, 16x16x4 (fp32 operands,
+// fp32 accumulation) for fp32.  Both leave element i of lane l = row 4 (l / 16) + i, column
+// l % 16 of the result, so one kernel serves the three types: S^T[key][q] = K Q^T,
+// O^T[e][q] += V^T P^T and O^T += Hbar^T Q^T f, a lane holding query l % 16 of each 16-row
+// query tile throughout (the softmax of a row stays in its four lanes, and P never moves
+// between lanes).
+//   16 bits: a k-step of 32 takes slots {4g .. 4g + 3, 16 + 4g .. 16 + 4g + 3} (g = l / 16),
+//     the slots the transposing LDS reads deliver for V^T and Hbar^T and the ones a lane's
+//     scores already are; K rows are staged with their features in that order, so a K operand
+//     is one 16-byte read.
+//   fp32: a step of 4 takes slots {4g + i}, so one 16-byte read of a K row feeds four steps and
+//     the scores are P's operands as they stand; V and Hbar operands are 4-byte reads.
+//
+// Work split.  A workgroup is four waves of RW query rows.  BT >= 64 (TEAM = 4): the waves share
+// a 64-row (RW 16) or 128-row (RW 32) tile of one query block, its selected blocks and the K/V
+// chunks staged in LDS.  BT < 64 (TEAM = 1): each wave owns a 16- or 32-row query block (fp32: 16
+// rows of one) and walks its own selected blocks through chunks of its own in LDS, with no
+// workgroup barrier; so all 64 lanes work at any block size, and the four waves share the
+// operands of phase 2, which every query block reads in full.  The next chunk's rows load into registers while one is multiplied.
+//
+// What bounds it: in fp32 the MFMA pipe (153 TFLOP/s in a large fp32 matrix product here; 12 heads
+// x 7,800 rows, D 128, block 64: 75 GFLOP in 0.84 ms, where one FMA per lane took 2.07 ms); in 16
+// bits the latency of the staged loads and the LDS operand reads (16 heads x 8,610 rows, D 96,
+// block 32, groups of 16: 149 GFLOP in 0.66 ms, where one FMA per lane took 9.7 ms with half its
+// lanes idle).
+//
+// fp32 sums are taken in short chains (16 features, a chunk of keys, 32 features of Hbar) that
+// are then added, because the MFMA rounds after every product: the error against 64 bits is
+// 3.4e-7 (7.3e-7 for the one-FMA-per-lane form) at the fp32 shape above.
+#include <initializer_list>
+#include <type_traits>
+
+#include "common.h"
+#include "kernels.h"
+
+namespace pasa {
+
+namespace {
+
+template <typename M_>
+struct Any16 {
+  using M = M_;
+  static constexpr int ES = 2;
+  using frag = typename M::vec8;
+};
+struct Any32 {
+  static constexpr int ES = 4;
+  using frag = f32x4_t;
+};
+
+constexpr int pow2_at_least(int x) {
+  int p = 1;
+  while (p < x) p *= 2;
+  return p;
+}
+
+// DP: the head dim padded to 64, 96 or 128 (zeros in LDS and registers).
+template <typename E, int DP, int TEAM, int RW>
+struct AnyCfg {
+  static constexpr int ES = E::ES;
+  static constexpr bool F32 = ES == 4;
+  static constexpr int QT = RW / 16;       // 16-row query tiles per wave
+  static constexpr int ROWS = 4 * RW;      // query rows per workgroup (TEAM = 4)
+  static constexpr int NF = DP * ES / 64;  // 64-byte feature steps per row: one fragment each
+  static constexpr int DT = DP / 16;       // 16-feature tiles of O
+  // Keys per chunk: about 16 KB of K and of V per team (8 KB where each wave stages its own).
+  static constexpr int KC = TEAM == 1 ? (F32 ? 16 : 32) : (F32 && DP > 64 ? 32 : 64);
+  // Row strides.  K: an odd number of 16-byte chunks, so that 16 rows read at one chunk touch 16
+  // distinct bank groups.  V in 16 bits: twice an odd number of chunks, so that the 8 rows x 32
+  // bytes half a wave transposes do; in fp32 4 rows x 64 bytes, four rows apart, already do.
+  static constexpr int KROW = DP * ES + 16;
+  static constexpr int VROW = DP * ES + (F32 ? 16 : 32);
+  static constexpr int SLAB = KC * (KROW + VROW);
+  static constexpr int KZ = 32;                  // blocks per zero-order chunk
+  static constexpr int HR = F32 ? 32 : DP;       // rows of Hbar staged at a time
+  static constexpr int Z_BYTES = KZ * (KROW + VROW);
+  static constexpr int P1 = (4 / TEAM) * SLAB;
+  static constexpr int P2 = Z_BYTES + HR * VROW;
+  static constexpr int LDS = P1 > P2 ? P1 : P2;
+  static constexpr int CH = DP * ES / 16;        // 16-byte chunks per row
+  static constexpr int CHP = pow2_at_least(CH);  // lanes per staged row
+  static constexpr int TT = 64 * TEAM;
+  static constexpr int RPP = TT / CHP;           // rows per staging pass
+  static constexpr int PASSES = KC / RPP;
+  static constexpr int C4 = DP / 4;              // 4-feature pieces of a statistics row
+  static constexpr int C4P = pow2_at_least(C4);
+  static constexpr int RPP4 = 256 / C4P;
+  static_assert(PASSES * RPP == KC && KZ % RPP4 == 0 && HR % RPP4 == 0, "staging split");
+};
+
+// 16 bytes of a row from element c * 16 / ES on; elements past D read as zero.  Rows that are not
+// whole 16-byte chunks, or not aligned to them, go element by element.
+template <int ES>
+__device__ __forceinline__ uint4 load_chunk(const unsigned char* row, int c, int D, bool vec) {
+  if (vec) return *reinterpret_cast<const uint4*>(row + c * 16);
+  uint32_t w[4] = {0u, 0u, 0u, 0u};
+  if constexpr (ES == 2) {
+#pragma unroll
+    for (int i = 0; i < 8; ++i)
+      if (8 * c + i < D) w[i >> 1] |= (uint32_t)reinterpret_cast<const uint16_t*>(row)[8 * c + i] << (16 * (i & 1));
+  } else {
+#pragma unroll
+    for (int i = 0; i < 4; ++i)
+      if (4 * c + i < D) w[i] = reinterpret_cast<const uint32_t*>(row)[4 * c + i];
+  }
+  return make_uint4(w[0], w[1], w[2], w[3]);
+}
+
+// Four floats of a statistics row from 4 c on, zero past D.
+__device__ __forceinline__ float4 load_stat4(const float* row, int c, int D, bool vec) {
+  if (vec) return *reinterpret_cast<const float4*>(row + 4 * c);
+  float f[4] = {0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+  for (int i = 0; i < 4; ++i)
+    if (4 * c + i < D) f[i] = row[4 * c + i];
+  return make_float4(f[0], f[1], f[2], f[3]);
+}
+
+}  // namespace
+
+// vec: q, k, v and o rows are whole aligned 16-byte chunks; vec_stats: kc, vc and hgroup rows are.
+// all: dense (every key of the segment, no selection, no correction; BT is then ROWS).
+// video: query blocks are computed (0: the text rows alone, where the blocks run with TEAM = 1).
+template <typename E, int DP, int TEAM, int RW>
+__global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2))) void k4_any_mfma(
+    const unsigned char* __restrict__ q, const unsigned char* __restrict__ k, const unsigned char* __restrict__ v,
+    const float* __restrict__ kc, const float* __restrict__ vc, const float* __restrict__ hgroup,
+    const uint32_t* __restrict__ selmask, unsigned char* __restrict__ o, float scale, float c, int T, int text,
+    int text_valid, int D, int BT, int NT, int G, int NG, int NW, int gamma_literal, int all, int nvt, int ntiles,
+    int vec_, int vec_stats_) {
+  using C = AnyCfg<E, DP, TEAM, RW>;
+  using frag = typename E::frag;
+  constexpr int ES = C::ES, QT = C::QT, NF = C::NF, DT = C::DT, KC = C::KC;
+  constexpr int KROW = C::KROW, VROW = C::VROW;
+  constexpr bool F32 = C::F32;
+  __shared__ __attribute__((aligned(16))) unsigned char lds[C::LDS];
+
+  const int tid = threadIdx.x;
+  const int lane = tid & 63;
+  const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+  const int l16 = lane & 15;
+  const int g4 = lane >> 4;
+  const bool vec = vec_ != 0, vec_stats = vec_stats_ != 0;
+  const int bh = blockIdx.y;
+  // Consecutive workgroups go to consecutive XCDs; each takes a contiguous run of a slice's tiles.
+  const int tile = (int)(blockIdx.x & 7) * (int)(gridDim.x >> 3) + (int)(blockIdx.x >> 3);
+  if (tile >= ntiles) return;
+
+  const int Ttot = T + text;
+  const int seg = T + text_valid;
+  // This wave's rows [row0, row_end), its query block I (video tiles of a sparse call) and the
+  // run of keys [cur, cend) that follows its selected blocks.
+  int I = -1, row0, row_end, cur, cend;
+  const int upb = TEAM == 1 ? BT / RW : 1;  // TEAM = 1: waves per query block
+  if (TEAM == 1) {
+    const int u = tile * 4 + wave;  // RW rows of a block; a wave past the last block repeats it and stores nothing
+    I = min(u / upb, NT - 1);
+    row0 = I * BT + (u - u / upb * upb) * RW;
+    row_end = u < NT * upb ? min(T, row0 + RW) : row0;
+    cur = T;
+    cend = seg;
+  } else if (tile < nvt) {
+    const int tpb = (BT + C::ROWS - 1) / C::ROWS;
+    I = tile / tpb;
+    const int r0 = I * BT + (tile - I * tpb) * C::ROWS;
+    row_end = min(T, min(r0 + C::ROWS, (I + 1) * BT));
+    if (r0 >= row_end) return;  // a tile past the last block's rows
+    row0 = r0 + wave * RW;
+    cur = all ? 0 : T;
+    cend = seg;
+    if (all) I = -1;
+  } else {
+    const int t = tile - nvt;
+    const int ptiles = (text_valid + C::ROWS - 1) / C::ROWS;
+    row0 = (t < ptiles ? T + t * C::ROWS : seg + (t - ptiles) * C::ROWS) + wave * RW;
+    row_end = t < ptiles ? seg : Ttot;
+    cur = t < ptiles ? 0 : seg;
+    cend = row_end;
+  }
+  const int64_t row_bytes = (int64_t)D * ES;
+  const int64_t slice = (int64_t)bh * Ttot * row_bytes;
+  const unsigned char* ksl = k + slice;
+  const unsigned char* vsl = v + slice;
+
+  // Q as B operands: fragment f of query tile qt holds the slots of feature step f.
+  frag qf[QT][NF];
+#pragma unroll
+  for (int qt = 0; qt < QT; ++qt) {
+    const int r = row0 + 16 * qt + l16;
+    const unsigned char* qrow = q + slice + (int64_t)r * row_bytes;
+#pragma unroll
+    for (int f = 0; f < NF; ++f) {
+      uint32_t w[4] = {0u, 0u, 0u, 0u};
+      if (r < row_end) {
+        if constexpr (F32) {
+          const int d = 16 * f + 4 * g4;
+          if (d < D) {
+            const uint4 x = load_chunk<4>(qrow, d / 4, D, vec);
+            w[0] = x.x; w[1] = x.y; w[2] = x.z; w[3] = x.w;
+          }
+        } else {
+#pragma unroll
+          for (int h = 0; h < 2; ++h) {
+            const int d = 32 * f + 16 * h + 4 * g4;
+            if (vec) {
+              if (d < D) {
+                const uint2 x = *reinterpret_cast<const uint2*>(qrow + d * 2);
+                w[2 * h] = x.x;
+                w[2 * h + 1] = x.y;
+              }
+            } else {
+#pragma unroll
+              for (int i = 0; i < 4; ++i)
+                if (d + i < D)
+                  w[2 * h + (i >> 1)] |= (uint32_t)reinterpret_cast<const uint16_t*>(qrow)[d + i] << (16 * (i & 1));
+            }
+          }
+        }
+      }
+      qf[qt][f] = __builtin_bit_cast(frag, (u32x4_t){w[0], w[1], w[2], w[3]});
+    }
+  }
+
+  f32x4_t oacc[DT][QT];
+  float l_run[QT], g_run[QT], m_run[QT];  // m: on all four lanes of a row; l, Gamma: this lane's keys
+#pragma unroll
+  for (int qt = 0; qt < QT; ++qt) {
+    m_run[qt] = -INFINITY;
+    l_run[qt] = g_run[qt] = 0.f;
+#pragma unroll
+    for (int dt = 0; dt < DT; ++dt) oacc[dt][qt] = (f32x4_t){0.f, 0.f, 0.f, 0.f};
+  }
+
+  // A operands of O^T from `rows` (V, V^ or Hbar rows in LDS): feature tile dt, row step s.
+  auto vt16 = [&](const unsigned char* rows, int s, int dt) {
+    const unsigned char* p = rows + (32 * s + 4 * g4 + (l16 >> 2)) * VROW + dt * 32 + (l16 & 3) * 8;
+    const uint2 lo = lds_read_tr16(p, 0);
+    const uint2 hi = lds_read_tr16(p, 16 * VROW);
+    return __builtin_bit_cast(frag, (u32x4_t){lo.x, lo.y, hi.x, hi.y});
+  };
+  auto vt32 = [&](const unsigned char* rows, int r, int dt) {
+    return lds_ld<float>(rows, (r + 4 * g4) * VROW + dt * 64 + l16 * 4);
+  };
+
+  // One online-softmax step over the 16 KTN rows at Kb / Vb.  mask(s) drops scores (to -inf),
+  // on_rescale(qt, alpha) sees a rise of the running max, add(qt, key, p) every weight.
+  auto step = [&](const unsigned char* Kb, const unsigned char* Vb, auto ktn, auto mask, auto on_rescale,
+                  auto add) __attribute__((always_inline)) {
+    constexpr int KTN = decltype(ktn)::value;
+    f32x4_t s[KTN][QT];
+#pragma unroll
+    for (int f = 0; f < NF; ++f)
+#pragma unroll
+      for (int kt = 0; kt < KTN; ++kt) {
+        const frag a = lds_ld<frag>(Kb, (kt * 16 + l16) * KROW + f * 64 + g4 * 16);
+#pragma unroll
+        for (int qt = 0; qt < QT; ++qt) {
+          if constexpr (F32) {  // 16-feature chains, added: shorter fp32 chains round less
+            f32x4_t t = {0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+            for (int i = 0; i < 4; ++i) t = __builtin_amdgcn_mfma_f32_16x16x4f32(a[i], qf[qt][f][i], t, 0, 0, 0);
+            s[kt][qt] = f == 0 ? t : s[kt][qt] + t;
+          } else {
+            if (f == 0) s[kt][qt] = (f32x4_t){0.f, 0.f, 0.f, 0.f};
+            s[kt][qt] = E::M::mfma16(a, qf[qt][f], s[kt][qt]);
+          }
+        }
+      }
+    mask(s);
+#pragma unroll
+    for (int qt = 0; qt < QT; ++qt) {
+      float mx = -INFINITY;
+#pragma unroll
+      for (int kt = 0; kt < KTN; ++kt)
+#pragma unroll
+        for (int i = 0; i < 4; ++i) mx = fmaxf(mx, s[kt][qt][i]);
+      const float mxc = quad16_max(mx) * c;
+      if (__any(mxc > m_run[qt])) {
+        const float m_new = fmaxf(m_run[qt], mxc);
+        const float alpha = fast_exp2(m_run[qt] - m_new);  // 0 on the first step
+        m_run[qt] = m_new;
+        l_run[qt] *= alpha;
+        on_rescale(qt, alpha);
+#pragma unroll
+        for (int dt = 0; dt < DT; ++dt)
+#pragma unroll
+          for (int i = 0; i < 4; ++i) oacc[dt][qt][i] *= alpha;
+      }
+#pragma unroll
+      for (int kt = 0; kt < KTN; ++kt)
+#pragma unroll
+        for (int i = 0; i < 4; ++i) {
+          const float p = fast_exp2(fmaf(s[kt][qt][i], c, -m_run[qt]));
+          add(qt, 16 * kt + i, p);
+          s[kt][qt][i] = p;
+        }
+    }
+    if constexpr (F32) {
+      // Each chunk's products are summed by themselves and added to o once (shorter fp32 chains).
+#pragma unroll
+      for (int d2 = 0; d2 < DT; d2 += 2) {
+        f32x4_t t[2][QT];
+#pragma unroll
+        for (int j = 0; j < 2; ++j)
+#pragma unroll
+          for (int qt = 0; qt < QT; ++qt) t[j][qt] = (f32x4_t){0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+        for (int kt = 0; kt < KTN; ++kt)
+#pragma unroll
+          for (int i = 0; i < 4; ++i)
+#pragma unroll
+            for (int j = 0; j < 2; ++j) {
+              const float a = vt32(Vb, 16 * kt + i, d2 + j);
+#pragma unroll
+              for (int qt = 0; qt < QT; ++qt)
+                t[j][qt] = __builtin_amdgcn_mfma_f32_16x16x4f32(a, s[kt][qt][i], t[j][qt], 0, 0, 0);
+            }
+#pragma unroll
+        for (int j = 0; j < 2; ++j)
+#pragma unroll
+          for (int qt = 0; qt < QT; ++qt) oacc[d2 + j][qt] += t[j][qt];
+      }
+    } else {
+#pragma unroll
+      for (int s2 = 0; s2 < KTN / 2; ++s2) {
+        frag pf[QT];
+#pragma unroll
+        for (int qt = 0; qt < QT; ++qt) {
+          const f32x4_t &a = s[2 * s2][qt], &b = s[2 * s2 + 1][qt];
+          pf[qt] = __builtin_bit_cast(frag, (u32x4_t){E::M::pack2(a[0], a[1]), E::M::pack2(a[2], a[3]),
+                                                      E::M::pack2(b[0], b[1]), E::M::pack2(b[2], b[3])});
+        }
+#pragma unroll
+        for (int dt = 0; dt < DT; ++dt) {
+          const frag a = vt16(Vb, s2, dt);
+#pragma unroll
+          for (int qt = 0; qt < QT; ++qt) oacc[dt][qt] = E::M::mfma16(a, pf[qt], oacc[dt][qt]);
+        }
+      }
+    }
+  };
+
+  // ---------------- Phase 1: the selected blocks, then the run [cur, cend) --------
+  typedef const __attribute__((address_space(4))) uint32_t* const const_u32_ptr;
+  const const_u32_ptr mrow = (const_u32_ptr)(selmask + ((int64_t)bh * NT + (I < 0 ? 0 : I)) * NW);
+  {
+    unsigned char* Kb = lds + (TEAM == 1 ? wave : 0) * C::SLAB;
+    unsigned char* Vb = Kb + KC * KROW;
+    const int tt = tid & (C::TT - 1);
+    const int sc = tt % C::CHP;   // this thread's 16-byte chunk of a staged row
+    const int sr = tt / C::CHP;   // its row in each pass
+    const bool in_row = sc * (16 / ES) < D;
+    auto sync = [&]() {
+      if (TEAM == 1) {  // LDS operations of a wave complete in order: only its own writes need waiting for
+        __builtin_amdgcn_s_waitcnt(0xC07F);
+        asm volatile("" ::: "memory");
+      } else {
+        __syncthreads();
+      }
+    };
+    int w = 0, j0 = 0, j1 = 0;  // the selected block being walked: rows [j0, j1)
+    uint32_t bits = I >= 0 && NW > 0 ? mrow[0] : 0u;
+    auto next_block = [&]() -> bool {
+      if (I < 0) return false;
+      while (bits == 0u) {
+        if (++w >= NW) return false;
+        bits = mrow[w];
+      }
+      const int j = 32 * w + __builtin_ctz(bits);
+      bits &= bits - 1u;
+      j0 = j * BT;
+      j1 = min(T, j0 + BT);
+      return true;
+    };
+    // The next chunk: rows ra .. (16 rows from ra, then from rb, where a chunk holds two 16-row
+    // blocks); returns its number of rows, 0 at the end.
+    bool tail = false;
+    auto next_chunk = [&](int& ra, int& rb) -> int {
+      if (j0 >= j1 && !tail && !next_block()) {
+        tail = true;
+        j0 = cur;
+        j1 = cend;
+      }
+      if (j0 >= j1) return 0;
+      ra = j0;
+      int n = min(KC, j1 - j0);
+      j0 += n;
+      rb = ra + 16;
+      if (TEAM == 1 && KC == 32 && BT == 16 && !tail && n == 16 && next_block()) {
+        rb = j0;
+        n += j1 - j0;
+        j0 = j1;
+      }
+      return n;
+    };
+    uint4 kreg[C::PASSES], vreg[C::PASSES];
+    auto fetch = [&](int ra, int rb, int n) {
+#pragma unroll
+      for (int p = 0; p < C::PASSES; ++p) {
+        const int r = p * C::RPP + sr;
+        kreg[p] = vreg[p] = make_uint4(0u, 0u, 0u, 0u);
+        if (r < n && in_row) {
+          const int64_t off = (int64_t)((TEAM == 1 && r >= 16) ? rb + (r - 16) : ra + r) * row_bytes;
+          kreg[p] = load_chunk<ES>(ksl + off, sc, D, vec);
+          vreg[p] = load_chunk<ES>(vsl + off, sc, D, vec);
+        }
+      }
+    };
+    auto stash = [&]() {
+      if (sc >= C::CH) return;
+#pragma unroll
+      for (int p = 0; p < C::PASSES; ++p) {
+        const int r = p * C::RPP + sr;
+        if constexpr (F32) {
+          lds_st(Kb, r * KROW + sc * 16, kreg[p]);
+        } else {  // features in slot order: 8 sc .. + 3 and + 4 .. + 7 are halves of two slots
+          const int b = r * KROW + (sc >> 2) * 64 + (sc & 1) * 32 + ((sc >> 1) & 1) * 8;
+          lds_st(Kb, b, make_uint2(kreg[p].x, kreg[p].y));
+          lds_st(Kb, b + 16, make_uint2(kreg[p].z, kreg[p].w));
+        }
+        lds_st(Vb, r * VROW + sc * 16, vreg[p]);
+      }
+    };
+    int ra = 0, rb = 0;
+    int n = next_chunk(ra, rb);
+    if (n > 0) fetch(ra, rb, n);
+    while (n > 0) {
+      const int n2 = next_chunk(ra, rb);
+      sync();  // the previous chunk has been read
+      stash();
+      sync();
+      if (n2 > 0) fetch(ra, rb, n2);
+      step(Kb, Vb, std::integral_constant<int, KC / 16>{},
+           [&](auto& s) {
+             if (n < KC) {
+               const int lim = n - 4 * g4;  // key 16 kt + 4 g4 + i is past the chunk iff 16 kt + i >= lim
+#pragma unroll
+               for (int kt = 0; kt < KC / 16; ++kt)
+#pragma unroll
+                 for (int qt = 0; qt < QT; ++qt)
+#pragma unroll
+                   for (int i = 0; i < 4; ++i)
+                     if (16 * kt + i >= lim) s[kt][qt][i] = -INFINITY;
+             }
+           },
+           [](int, float) {}, [&](int qt, int, float p) { l_run[qt] += p; });
+      n = n2;
+    }
+  }
+
+  // ---------------- Phase 2: zero- and first-order correction per group -----------
+  if (I >= 0) {
+    const int last_len = T - (NT - 1) * BT;
+    const float* kcb = kc + (int64_t)bh * NT * D;
+    const float* vcb = vc + (int64_t)bh * NT * D;
+    unsigned char* Kz = lds;
+    unsigned char* Vz = lds + C::KZ * KROW;
+    unsigned char* Hs = lds + C::Z_BYTES;
+    const int c4 = tid % C::C4P, r4 = tid / C::C4P;
+    // Blocks [a, b) of one mask word that some wave of the workgroup does not select.
+    auto word_unselected = [&](int wd) -> uint32_t {
+      if (TEAM != 1) return ~mrow[wd];
+      uint32_t m = 0xffffffffu;
+#pragma unroll
+      for (int i = 0; i < 4; ++i)
+        m &= ((const_u32_ptr)(selmask + ((int64_t)bh * NT + min((tile * 4 + i) / upb, NT - 1)) * NW))[wd];
+      return ~m;
+    };
+    auto any_unselected = [&](int a, int b) -> bool {
+      for (int wd = a >> 5; wd <= (b - 1) >> 5; ++wd) {
+        uint32_t m = word_unselected(wd);
+        if (wd == a >> 5) m &= 0xffffffffu << (a & 31);
+        if (wd == (b - 1) >> 5) m &= 0xffffffffu >> (31 - ((b - 1) & 31));
+        if (m) return true;
+      }
+      return false;
+    };
+    // Bit t: block jc + t (t < cn <= 32) is approximated for this wave's query block.
+    auto approx_bits = [&](int jc, int cn) -> uint32_t {
+      const int wd = jc >> 5, sh = jc & 31;
+      uint32_t sel = mrow[wd] >> sh;
+      if (sh != 0 && wd + 1 < NW) sel |= mrow[wd + 1] << (32 - sh);
+      return ~sel & (cn >= 32 ? 0xffffffffu : (1u << cn) - 1u);
+    };
+    // Four floats to LDS as four elements of the input type.
+    auto st4 = [&](unsigned char* base, int off16, int off32, const float4& x) {
+      if constexpr (F32)
+        lds_st(base, off32, x);
+      else
+        lds_st(base, off16, make_uint2(E::M::pack2(x.x, x.y), E::M::pack2(x.z, x.w)));
+    };
+    const float4 zero4 = make_float4(0.f, 0.f, 0.f, 0.f);
+    const bool in4 = 4 * c4 < D;
+    auto stage_z = [&](int jc, int cn) {
+#pragma unroll
+      for (int p = 0; p < C::KZ / C::RPP4; ++p) {
+        const int r = p * C::RPP4 + r4;
+        float4 xk = zero4, xv = zero4;
+        if (r < cn && in4) {
+          xk = load_stat4(kcb + (int64_t)(jc + r) * D, c4, D, vec_stats);
+          xv = load_stat4(vcb + (int64_t)(jc + r) * D, c4, D, vec_stats);
+        }
+        if (c4 < C::C4) {
+          st4(Kz, r * KROW + (c4 >> 3) * 64 + (c4 & 3) * 16 + ((c4 >> 2) & 1) * 8, r * KROW + c4 * 16, xk);
+          st4(Vz, r * VROW + c4 * 8, r * VROW + c4 * 16, xv);
+        }
+      }
+    };
+    auto stage_h = [&](const float* hg, int d0) {
+#pragma unroll 8
+      for (int p = 0; p < C::HR / C::RPP4; ++p) {
+        const int r = p * C::RPP4 + r4;
+        float4 x = zero4;
+        if (d0 + r < D && in4) x = load_stat4(hg + (int64_t)(d0 + r) * D, c4, D, vec_stats);
+        if (c4 < C::C4) st4(Hs, r * VROW + c4 * 8, r * VROW + c4 * 16, x);
+      }
+    };
+    for (int g = 0; g < NG; ++g) {
+      const int ja = g * G;
+      const int jb = min((int64_t)NT, (int64_t)ja + G);
+      if (!any_unselected(ja, jb)) continue;  // nothing approximated: no contribution
+      const float* hg = hgroup + ((int64_t)bh * NG + g) * D * D;
+      // Zero order, 32 blocks at a time: o += p V^, and per row the sums of p and of p times the
+      // block's length, kept relative to the running max until the group ends (Gamma itself is
+      // rescaled only in the consistent form, :231-235).
+      float psum[QT], gsum[QT];
+#pragma unroll
+      for (int qt = 0; qt < QT; ++qt) psum[qt] = gsum[qt] = 0.f;
+      bool h_staged = false;
+      for (int jc = ja; jc < jb; jc += C::KZ) {
+        const int cn = min(C::KZ, jb - jc);
+        if (!any_unselected(jc, jc + cn)) continue;
+        __syncthreads();  // the previous operands have been read
+        stage_z(jc, cn);
+        if (!h_staged) stage_h(hg, 0);
+        h_staged = true;
+        __syncthreads();
+        const uint32_t ub = approx_bits(jc, cn) >> (4 * g4);
+        const int last = NT - 1 - jc - 4 * g4;  // this lane's key index of the last block
+        step(Kz, Vz, std::integral_constant<int, C::KZ / 16>{},
+             [&](auto& s) {
+#pragma unroll
+               for (int kt = 0; kt < C::KZ / 16; ++kt)
+#pragma unroll
+                 for (int qt = 0; qt < QT; ++qt)
+#pragma unroll
+                   for (int i = 0; i < 4; ++i)
+                     if (!((ub >> (16 * kt + i)) & 1u)) s[kt][qt][i] = -INFINITY;
+             },
+             [&](int qt, float alpha) {
+               psum[qt] *= alpha;
+               gsum[qt] *= alpha;
+               if (!gamma_literal) g_run[qt] *= alpha;
+             },
+             [&](int qt, int key, float p) {
+               psum[qt] += p;
+               gsum[qt] += p * (float)(key == last ? last_len : BT);
+             });
+      }
+      // First order: o += scale * (sum of p) * (q . Hbar).
+      float f[QT];
+#pragma unroll
+      for (int qt = 0; qt < QT; ++qt) {
+        g_run[qt] += gsum[qt];
+        f[qt] = quad16_sum(psum[qt]) * scale;
+      }
+#pragma unroll
+      for (int hs = 0; hs < DP / C::HR; ++hs) {
+        if (hs > 0) {
+          if (hs * C::HR >= D) break;
+          __syncthreads();
+          stage_h(hg, hs * C::HR);
+          __syncthreads();
+        }
+        if constexpr (F32) {
+#pragma unroll
+          for (int d2 = 0; d2 < DT; d2 += 2) {
+            f32x4_t r[2][QT];
+#pragma unroll
+            for (int j = 0; j < 2; ++j)
+#pragma unroll
+              for (int qt = 0; qt < QT; ++qt) r[j][qt] = (f32x4_t){0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+            for (int cc = 0; cc < C::HR / 16; ++cc)
+#pragma unroll
+              for (int i = 0; i < 4; ++i)
+#pragma unroll
+                for (int j = 0; j < 2; ++j) {
+                  const float a = vt32(Hs, 16 * cc + i, d2 + j);
+#pragma unroll
+                  for (int qt = 0; qt < QT; ++qt)
+                    r[j][qt] = __builtin_amdgcn_mfma_f32_16x16x4f32(a, qf[qt][hs * (C::HR / 16) + cc][i], r[j][qt], 0,
+                                                                    0, 0);
+                }
+#pragma unroll
+            for (int j = 0; j < 2; ++j)
+#pragma unroll
+              for (int qt = 0; qt < QT; ++qt)
+#pragma unroll
+                for (int i = 0; i < 4; ++i) oacc[d2 + j][qt][i] = fmaf(r[j][qt][i], f[qt], oacc[d2 + j][qt][i]);
+          }
+        } else {
+#pragma unroll
+          for (int dt = 0; dt < DT; ++dt) {
+            f32x4_t r[QT];
+#pragma unroll
+            for (int qt = 0; qt < QT; ++qt) r[qt] = (f32x4_t){0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+            for (int s2 = 0; s2 < NF; ++s2) {
+              const frag a = vt16(Hs, s2, dt);
+#pragma unroll
+              for (int qt = 0; qt < QT; ++qt) r[qt] = E::M::mfma16(a, qf[qt][s2], r[qt]);
+            }
+#pragma unroll
+            for (int qt = 0; qt < QT; ++qt)
+#pragma unroll
+              for (int i = 0; i < 4; ++i) oacc[dt][qt][i] = fmaf(r[qt][i], f[qt], oacc[dt][qt][i]);
+          }
+        }
+      }
+    }
+  }
+
+  // o = A / (L + Gamma) (:258-259), stored in the input type (:262).
+#pragma unroll
+  for (int qt = 0; qt < QT; ++qt) {
+    const int r = row0 + 16 * qt + l16;
+    const float den = quad16_sum(l_run[qt]) + quad16_sum(g_run[qt]);
+    if (r < row_end) {
+      unsigned char* orow = o + slice + (int64_t)r * row_bytes;
+#pragma unroll
+      for (int dt = 0; dt < DT; ++dt) {
+        const int e = 16 * dt + 4 * g4;
+        const float x[4] = {oacc[dt][qt][0] / den, oacc[dt][qt][1] / den, oacc[dt][qt][2] / den,
+                            oacc[dt][qt][3] / den};
+        if (vec && e < D) {
+          if constexpr (F32)
+            *reinterpret_cast<float4*>(orow + e * 4) = make_float4(x[0], x[1], x[2], x[3]);
+          else
+            *reinterpret_cast<uint2*>(orow + e * 2) = make_uint2(E::M::pack2(x[0], x[1]), E::M::pack2(x[2], x[3]));
+        } else {
+#pragma unroll
+          for (int i = 0; i < 4; ++i)
+            if (e + i < D) {
+              if constexpr (F32)
+                reinterpret_cast<float*>(orow)[e + i] = x[i];
+              else
+                reinterpret_cast<uint16_t*>(orow)[e + i] = (uint16_t)E::M::bits(x[i]);
+            }
+        }
+      }
+    }
+  }
+}
+
+namespace {
+
+struct AnyCall {
+  const void *q, *k, *v;
+  const float *kc, *vc, *hgroup;
+  const uint32_t* selmask;
+  void* o;
+  float scale;
+  int bh, T, text, text_valid, D, BT, G, gamma_literal, all;
+  hipStream_t stream;
+};
+
+bool aligned16(std::initializer_list<const void*> ps) {
+  uintptr_t x = 0;
+  for (const void* p : ps) x |= (uintptr_t)p;
+  return (x & 15u) == 0;
+}
+
+int text_tiles(const AnyCall& a, int rows) {
+  return (a.text_valid + rows - 1) / rows + (a.text - a.text_valid + rows - 1) / rows;
+}
+
+template <typename E, int DP, int TEAM, int RW>
+hipError_t launch_any(const AnyCall& a, int BT, int nvt, int ntiles) {
+  const int NT = (a.T + BT - 1) / BT;
+  const bool vec = (a.D * E::ES) % 16 == 0 && aligned16({a.q, a.k, a.v, a.o});
+  const bool vec_stats = a.D % 4 == 0 && aligned16({a.kc, a.vc, a.hgroup});
+  const dim3 grid((unsigned)((ntiles + 7) / 8 * 8), (unsigned)a.bh);
+  hipLaunchKernelGGL((k4_any_mfma<E, DP, TEAM, RW>), grid, dim3(256), 0, a.stream, (const unsigned char*)a.q,
+                     (const unsigned char*)a.k, (const unsigned char*)a.v, a.kc, a.vc, a.hgroup, a.selmask,
+                     (unsigned char*)a.o, a.scale, a.scale * kLog2e, a.T, a.text, a.text_valid, a.D, BT, NT, a.G,
+                     (NT + a.G - 1) / a.G, (NT + 31) / 32, a.gamma_literal, a.all, nvt, ntiles, (int)vec,
+                     (int)vec_stats);
+  return hipGetLastError();
+}
+
+// The workgroup tile of TEAM = 4: 128 rows when the blocks are that long and such tiles fill the
+// 256 CUs, else 64.
+bool wide_tiles(const AnyCall& a, int BT) {
+  return BT >= 128 && (int64_t)a.bh * ((a.T + 127) / 128) >= 256;
+}
+
+template <typename E, int DP>
+hipError_t launch_dp(const AnyCall& a) {
+  constexpr bool F32 = E::ES == 4;  // 16 rows per wave: its MFMAs outlast their LDS reads, and 32 rows spill
+  if (!a.all && a.BT < 64) {
+    const int NT = (a.T + a.BT - 1) / a.BT;
+    hipError_t e;
+    if (F32 || a.BT == 16) {
+      const int ntiles = (NT * (a.BT / 16) + 3) / 4;
+      e = launch_any<E, DP, 1, 16>(a, a.BT, ntiles, ntiles);
+    } else {
+      const int ntiles = (NT + 3) / 4;
+      e = launch_any<E, DP, 1, F32 ? 16 : 32>(a, a.BT, ntiles, ntiles);
+    }
+    if (e != hipSuccess || a.text == 0) return e;
+    return launch_any<E, DP, 4, 16>(a, a.BT, 0, text_tiles(a, 64));  // the text rows
+  }
+  const bool wide = !F32 && wide_tiles(a, a.all ? 128 : a.BT);
+  const int rows = wide ? 128 : 64;
+  const int BT = a.all ? rows : a.BT;
+  const int nvt = (a.T + BT - 1) / BT * ((BT + rows - 1) / rows);
+  const int ntiles = nvt + text_tiles(a, rows);
+  return wide ? launch_any<E, DP, 4, F32 ? 16 : 32>(a, BT, nvt, ntiles) : launch_any<E, DP, 4, 16>(a, BT, nvt, ntiles);
+}
+
+template <typename E>
+hipError_t launch_type(const AnyCall& a) {
+  return a.D <= 64 ? launch_dp<E, 64>(a) : (a.D <= 96 ? launch_dp<E, 96>(a) : launch_dp<E, 128>(a));
+}
+
+}  // namespace
+
+int64_t sparse_attn_any_tiles(int T, int text, int text_valid, int BT) {
+  const int64_t NT = (T + BT - 1) / BT;
+  const int64_t tpb = (BT + 63) / 64;
+  return NT * tpb + (text_valid + 63) / 64 + (text - text_valid + 63) / 64;
+}
+
+hipError_t launch_sparse_attn_any(const void* q, const void* k, const void* v, const float* kc, const float* vc,
+                                  const float* hgroup, const uint32_t* selmask, void* o, float scale, int bh, int T,
+                                  int text, int text_valid, int D, int BT, int G, int gamma_literal, int all,
+                                  int dtype, hipStream_t stream) {
+  if (D < 1 || D > 128 || BT < 16 || BT > 256 || (BT & (BT - 1)) || G < 1 || text_valid < 0 || text_valid > text)
+    return hipErrorInvalidValue;
+  if (!all && (kc == nullptr || vc == nullptr || hgroup == nullptr || selmask == nullptr)) return hipErrorInvalidValue;
+  const AnyCall a{q, k, v, kc, vc, hgroup, selmask, o, scale, bh, T, text, text_valid, D, BT, G, gamma_literal, all,
+                  stream};
+  switch (dtype) {
+    case kAnyF32: return launch_type<Any32>(a);
+    case kAnyBf16: return launch_type<Any16<Bf16>>(a);
+    case kAnyF16: return launch_type<Any16<F16>>(a);
+    default: return hipErrorInvalidValue;
+  }
+}
+
+}  // namespace pasa

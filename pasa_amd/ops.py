@@ -79,8 +79,7 @@ def tuned_shape(dtype: torch.dtype, head_dim: int, block_size: int, group_size: 
     at head_dim 128), head_dim 64 or 128, block size 64 or 128, group size 32, and a text
     segment only at head_dim 128.  Every other shape the library takes (fp32 inputs, head dims
     1 .. 128, block sizes 16 .. 256 that are powers of two, any group size) runs on the
-    any-shape kernels: the same mathematics with plain VALU arithmetic, for completeness
-    rather than speed."""
+    any-shape kernels: the same mathematics without the tuned kernels' fixed tiles."""
     return (head_dim in (64, 128) and block_size in (64, 128) and group_size == GROUP_SIZE
             and (dtype == torch.bfloat16 or (dtype == torch.float16 and head_dim == 128))
             and (text_tokens == 0 or head_dim == 128))

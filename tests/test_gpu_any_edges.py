@@ -1,0 +1,97 @@
+"""The any-shape kernels at the edges of their tiles: head dims that are not whole 16-byte chunks
+(the element-wise loads), tensors whose data is not 16-byte aligned, block counts that leave a
+workgroup's last waves without a block, 16-row blocks two to a chunk (odd counts of them), groups
+longer than one zero-order chunk, and the smallest sizes of each.
+
+The attention stage runs on the GPU's own statistics and selection and is held to the oracle's
+attention stage on that selection: fp32 to a relative 2-norm of 4e-6 (the longest fp32 chain here
+has a few hundred terms of rounding 2^-24: sqrt(300) * 6e-8 = 1e-6 in the scores, which the
+softmax passes on about once, and as much again in the products with V), 16 bits to 1.5 times the
+error of the oracle run with the reference's own roundings, plus one ulp."""
+import pytest
+import torch
+
+from oracle import pisa_oracle as O
+from pasa_amd import ops
+
+pytestmark = pytest.mark.gpu
+
+B16, F16, F32 = torch.bfloat16, torch.float16, torch.float32
+
+
+def make(heads, T, D, dtype, seed, shift=0):
+    """q, k, v [1, heads, T, D] whose data starts ``shift`` elements into its storage."""
+    g = torch.Generator().manual_seed(seed)
+    out = []
+    for _ in range(3):
+        buf = torch.randn(heads * T * D + shift, generator=g).to(dtype)
+        out.append(buf[shift:].view(1, heads, T, D))
+    return out
+
+
+def to_dev(t, device, shift):
+    buf = torch.empty(t.numel() + shift, dtype=t.dtype, device=device)
+    view = buf[shift:].view(t.shape)
+    view.copy_(t)
+    assert view.is_contiguous()
+    return view
+
+
+# heads, T, D, BT, G, density, dtype, gamma, text, valid, shift
+CASES = [
+    (1, 16, 16, 16, 1, 1.0, F32, "literal", 0, 0, 0),          # one block, nothing approximated
+    (2, 17, 1, 16, 32, 0.5, F32, "literal", 0, 0, 0),          # one feature, a block of one row
+    (1, 700, 37, 64, 7, 0.2, F32, "consistent", 0, 0, 0),      # odd head dim, fp32
+    (1, 700, 37, 32, 7, 0.2, B16, "literal", 0, 0, 0),         # odd head dim, 16 bits
+    (2, 530, 96, 32, 16, 0.2, B16, "literal", 0, 0, 3),        # misaligned data
+    (1, 530, 128, 64, 32, 0.2, F32, "literal", 0, 0, 1),       # misaligned data, fp32
+    (1, 1111, 40, 16, 5, 0.11, F16, "literal", 0, 0, 0),       # 70 blocks of 16: 7 selected, an odd count
+    (1, 1111, 100, 16, 64, 0.03, F32, "literal", 33, 5, 0),    # 16-row blocks in fp32, text and padding
+    (1, 2079, 72, 16, 100, 0.05, B16, "consistent", 31, 31, 0),  # groups of 100: several zero-order chunks
+    (2, 993, 64, 32, 64, 0.3, F32, "literal", 0, 0, 0),        # two waves per 32-row block
+    (1, 1250, 112, 256, 2, 0.5, F16, "literal", 130, 70, 0),   # two tiles per block, text
+    (3, 129, 128, 128, 8, 0.5, B16, "literal", 0, 0, 0),       # a last block of one row
+    (1, 33000, 64, 128, 16, 0.02, B16, "literal", 0, 0, 0),    # enough blocks for 128-row tiles
+]
+
+
+@pytest.mark.parametrize("case", CASES, ids=lambda c: "-".join(str(x).replace("torch.", "") for x in c))
+def test_attention_edges(device, case):
+    heads, T, D, BT, G, density, dtype, gamma, text, valid, shift = case
+    q, k, v = make(heads, T, D, dtype, T + D + BT)
+    assert not ops.tuned_shape(dtype, D, BT, G, text)
+    qd, kd, vd = (to_dev(t, device, shift) for t in (q, k, v))
+    scale = D ** -0.5
+    st = ops.block_stats(qd, kd, vd, BT, G, text_tokens=text)
+    sel = ops.select_blocks(st, density, scale)
+    out = to_dev(torch.zeros_like(v), device, shift)
+    o = ops.sparse_attn(qd, kd, vd, st, sel, scale, BT, gamma, out=out, text_tokens=text, text_valid=valid,
+                        group_size=G).cpu()
+    kw = dict(gamma=gamma, indices=sel.idx.cpu(), text_tokens=text, text_valid=valid)
+    ref = O.pisa_pg_attention(q, k, v, density, BT, G, scale, dtype=torch.float64, **kw)
+    err = (o.double() - ref).norm() / ref.norm()
+    print(f"[edges] {case}: rel {err:.2e}", flush=True)
+    if dtype == F32:
+        assert err <= 4e-6
+        return
+    rp = O.pisa_pg_attention(q, k, v, density, BT, G, scale, ref_precision=dtype, **kw).double()
+    ulp = float(O.ulp(ref.abs().max(), dtype))
+    assert float((o.double() - ref).abs().max()) <= 1.5 * float((rp - ref).abs().max()) + ulp
+    assert err <= 1.5 * float((rp - ref).norm() / ref.norm())
+
+
+@pytest.mark.parametrize("T,D,dtype,text,valid,shift", [(1, 5, F32, 0, 0, 0), (333, 72, B16, 0, 0, 1),
+                                                       (200, 64, F32, 70, 1, 0), (33000, 96, F16, 0, 0, 0)])
+def test_dense_edges(device, T, D, dtype, text, valid, shift):
+    q, k, v = make(1, T, D, dtype, T + D)
+    qd, kd, vd = (to_dev(t, device, shift) for t in (q, k, v))
+    o = ops.dense_attention(qd, kd, vd, text_tokens=text, text_valid=valid).double().cpu()
+    seg, es = T - text + valid, O.effective_scale(D ** -0.5)
+    rows = torch.cat([torch.arange(0, min(seg, 100)), torch.arange(max(0, seg - 100), T)]).unique()
+    a, b = rows[rows < seg], rows[rows >= seg]
+    ref = torch.cat([O.dense_attention(q[..., r, :].double(), k[..., s, :].double(), v[..., s, :].double(), es)
+                     for r, s in ((a, slice(0, seg)), (b, slice(seg, T))) if len(r)], dim=2)
+    err = float((o[..., rows, :] - ref).norm() / ref.norm())
+    print(f"[edges] dense T={T} D={D} {dtype}: rel {err:.2e}", flush=True)
+    # 16 bits: P and o rounded once each to 8 (bf16) or 11 (fp16) bits
+    assert err <= {F32: 4e-6, B16: 6e-3, F16: 1e-3}[dtype]
