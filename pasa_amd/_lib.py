@@ -61,6 +61,7 @@ SIGNATURES = {
     "pasa_block_stats_ws": (_int, [_vp, _vp, _vp, _vp, _vp, _vp, _vp, _vp, _i64, _i64, _i64, _i64, _i64,
                                    _i64, _int, _vp, _sz, _vp]),
     "pasa_block_stats_workspace_bytes": (_sz, [_i64, _i64, _i64, _i64, _i64, _i64]),
+    "pasa_block_stats_workspace_bytes_dtype": (_sz, [_i64, _i64, _i64, _i64, _i64, _i64, _int]),
     "pasa_select": (_int, [_vp, _vp, _vp, _vp, _dbl, _dbl, _int, _vp, _vp, _vp, _vp, _sz, _i64, _i64,
                            _i64, _vp]),
     "pasa_select_workspace_bytes": (_sz, [_i64, _i64]),

@@ -1,6 +1,6 @@
 // Statistics and selection scores for shapes the tuned kernels do not take: fp32 q, k, v; any
 // head dim up to 128; any group size; block sizes 16 .. 256 (the attention stage of the same
-// shapes is any_attn.hip).  Plain VALU arithmetic, one workgroup per (slice, group).
+// shapes is any_attn.hip).
 //
 // Reference: svg/kernels/triton/group_pisa_attention.py
 //   k2_block_stats_any   fused_chunk_reduce_kernel :66-129 (+ sqrt :287) and
@@ -16,144 +16,274 @@ namespace pasa {
 
 namespace {
 
-// Element access for the three input types.
+// The three input types: a 16-byte chunk as fp32, and element i of a chunk's four words taken from
+// a row that is not whole aligned chunks.
 struct F32E {
-  __device__ static float load(const void* p, int64_t i) { return ((const float*)p)[i]; }
-};
-struct Bf16E {
-  __device__ static float load(const void* p, int64_t i) {
-    return bf16_bits_to_f32(((const uint16_t*)p)[i]);
+  static constexpr int ES = 4;
+  __device__ static void put(uint32_t (&w)[4], int i, const unsigned char* row, int d) {
+    w[i] = reinterpret_cast<const uint32_t*>(row)[d];
+  }
+  __device__ static void widen(const uint4& c, float (&f)[4]) {
+    f[0] = __uint_as_float(c.x);
+    f[1] = __uint_as_float(c.y);
+    f[2] = __uint_as_float(c.z);
+    f[3] = __uint_as_float(c.w);
   }
 };
-struct F16E {
-  __device__ static float load(const void* p, int64_t i) { return (float)((const _Float16*)p)[i]; }
+template <typename M>
+struct E16 {
+  static constexpr int ES = 2;
+  __device__ static void put(uint32_t (&w)[4], int i, const unsigned char* row, int d) {
+    w[i >> 1] |= (uint32_t)reinterpret_cast<const uint16_t*>(row)[d] << (16 * (i & 1));
+  }
+  __device__ static void widen(const uint4& c, float (&f)[8]) { M::widen8(c, f); }
 };
+using Bf16E = E16<Bf16>;
+using F16E = E16<F16>;
 
-constexpr int kAnyChunk = 32;   // rows of a staged K/V chunk
-constexpr int kAnyLd = 132;     // LDS row stride (floats) of staged rows: 16-byte aligned, so
-                                // row pieces are ds_read_b128
+constexpr int kAnyChunk = 32;  // rows of a staged K/V chunk
 
 }  // namespace
 
 // ---- block statistics ---------------------------------------------------------
-// One workgroup (256 threads) per (group of G key blocks, slice); the group's blocks in
-// ascending order, each in 32-row chunks of k and v staged in LDS as fp32 (132-float rows,
-// feature columns D .. 127 zero).  Thread t owns an 8 x 8 tile of the D x D moment, rows
-// d = 8 (t >> 4) .. + 7 and columns e = 8 (t & 15) .. + 7: per staged row, four 16-byte
-// reads feed 64 FMAs.  H_j[d][e] = sum_t k_t[d] v_t[e] - kbar_j[d] V^_j[e] (:106-107), the
-// sum over the block's rows in order; entries past D stay zero and are not stored.  Threads
-// t < D own column t of the block sums of q, k and v.  The group sum adds H_j in block order,
-// then / G.
-template <typename EL>
-__global__ __launch_bounds__(256) void k2_block_stats_any(const void* __restrict__ q, const void* __restrict__ k,
-                                                          const void* __restrict__ v, float* __restrict__ qc,
-                                                          float* __restrict__ kc, float* __restrict__ vc,
-                                                          float* __restrict__ hnorm, float* __restrict__ hgroup,
-                                                          int T, int Tslice, int D, int BT, int NT, int G) {
-  constexpr int CH = kAnyChunk, LD = kAnyLd;
-  __shared__ __attribute__((aligned(16))) float ks[CH * LD];
-  __shared__ __attribute__((aligned(16))) float vs[CH * LD];
-  __shared__ float qsm[CH * 128];  // the chunk's q rows (only their column sums are needed)
-  __shared__ float kbar[128];
-  __shared__ float vhat[128];
+// One workgroup (four waves) per part of a group of G key blocks; the part's blocks in ascending
+// order, each in chunks of up to 32 rows of q, k and v staged in LDS as fp32 (feature columns D ..
+// DP - 1 zero), the next chunk's rows in registers meanwhile.
+//
+// H_j = K^T V - kbar_j V^_j^T (:106-107) runs on the 16x16x4 fp32 MFMA for every input type, each
+// wave on a quarter of the D x D moment, rows in ascending order: that MFMA is a chain of fused
+// multiply-adds in k order, bit for bit, so kc, qc, ||H_j|| and the selection made from them do not
+// depend on how the work is split.  ||H_j||^2 is summed in 8 x 8 tiles (H_j through LDS), then over
+// the wave, then over the waves; column sums run down a block's rows in order, one column per
+// thread.  The group sum stays in registers; with split > 1 each part writes its own to `partials`
+// and k2_any_reduce adds the parts in order.
+//
+// Bound: the fp32 MFMA (2 D^2 FLOP per row) against three rows read; a block of 64 rows at D 128 is
+// 3.4 us of MFMA issue.  One workgroup per group left most of the 256 CUs idle and its FMAs waited
+// on four LDS reads per row: 12 heads x 7,800 fp32 rows of D 128 took 847 us (now 73 + 12 for the
+// reduction), 2 heads x 1,024 of D 64 291 us (now 11 + 6), 16 x 8,610 bf16 of D 96 248 us (65 + 7).
+template <typename EL, int DP>
+struct StatsCfg {
+  static constexpr int CH = kAnyChunk;
+  static constexpr int LD = DP + 16;   // four consecutive rows start 16 banks apart
+  static constexpr int HLD = DP + 4;   // rows four apart do, and 16-byte rows
+  static constexpr int KV_FLOATS = 3 * CH * LD;
+  static constexpr int H_FLOATS = DP * HLD;
+  static constexpr int LDS_FLOATS = KV_FLOATS > H_FLOATS ? KV_FLOATS : H_FLOATS;  // one after the other
+  static constexpr int EPC = 16 / EL::ES;             // elements per 16-byte chunk
+  static constexpr int NCH = DP / EPC;                // chunks per row
+  static constexpr int NCHP = NCH <= 8 ? 8 : (NCH <= 16 ? 16 : 32);
+  static constexpr int RPP = 256 / NCHP;              // rows per staging pass
+  static constexpr int PASSES = CH / RPP;
+  static constexpr int TL = DP / 32;                  // 16 x 16 tiles per side of a wave's quarter
+};
+
+template <typename EL, int DP>
+__global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2))) void k2_block_stats_any(
+    const unsigned char* __restrict__ q, const unsigned char* __restrict__ k, const unsigned char* __restrict__ v,
+    float* __restrict__ qc, float* __restrict__ kc, float* __restrict__ vc, float* __restrict__ hnorm,
+    float* __restrict__ hgroup, float* __restrict__ partials, int T, int Tslice, int D, int BT, int NT, int G,
+    int split, int vec) {
+  using C = StatsCfg<EL, DP>;
+  constexpr int CH = C::CH, LD = C::LD, HLD = C::HLD, TL = C::TL, EPC = C::EPC;
+  __shared__ __attribute__((aligned(16))) float buf[C::LDS_FLOATS];  // K, V and Q chunk; then H_j
+  __shared__ __attribute__((aligned(16))) float kbar[DP];
+  __shared__ float vhat[DP];
   __shared__ float red[4];
-  const int g = blockIdx.x;
+  float* ks = buf;
+  float* vs = buf + CH * LD;
+  float* qsm = buf + 2 * CH * LD;
+  const int g = blockIdx.x / split;
+  const int part = blockIdx.x - g * split;
   const int bh = blockIdx.y;
   const int tid = threadIdx.x;
+  const int lane = tid & 63;
+  const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+  const int l16 = lane & 15;
+  const int g4 = lane >> 4;
+  const int dq = (wave >> 1) * (DP / 2);
+  const int eq = (wave & 1) * (DP / 2);
   const int NG = (NT + G - 1) / G;
-  const int64_t base = (int64_t)bh * Tslice * D;
-  const int d0 = 8 * (tid >> 4);
-  const int e0 = 8 * (tid & 15);
-  const bool owns = d0 < D && e0 < D;  // the tile holds at least one entry of the moment
-  for (int i = tid; i < CH * LD; i += 256) {
-    ks[i] = 0.f;
-    vs[i] = 0.f;
-  }
-  if (tid < 128) {
-    kbar[tid] = 0.f;
-    vhat[tid] = 0.f;
-  }
-  float gacc[64];
+  const int nblk = min(G, NT - g * G);
+  const int per = (nblk + split - 1) / split;
+  const int j0 = g * G + min(part * per, nblk);
+  const int j1 = g * G + min((part + 1) * per, nblk);
+  const int64_t row_bytes = (int64_t)D * EL::ES;
+  const int64_t slice = (int64_t)bh * Tslice * row_bytes;
+
+  if (tid < DP) kbar[tid] = vhat[tid] = 0.f;  // columns past D stay zero
+
+  // Staging: thread (sr, sc) moves chunk sc of rows sr, sr + RPP, ...
+  const int sc = tid % C::NCHP;
+  const int sr = tid / C::NCHP;
+  // Column sums: threads 0 .. 127 column tid of k and q, threads 128 .. 255 column tid - 128 of v.
+  const int col = tid & 127;
+  const bool kq_side = tid < 128;
+  uint4 kreg[C::PASSES], vreg[C::PASSES], qreg[C::PASSES];
+  auto load = [&](const unsigned char* base, int row) -> uint4 {
+    const unsigned char* p = base + slice + (int64_t)row * row_bytes;
+    if (vec) return *reinterpret_cast<const uint4*>(p + sc * 16);
+    uint32_t w[4] = {0u, 0u, 0u, 0u};
 #pragma unroll
-  for (int m = 0; m < 64; ++m) gacc[m] = 0.f;
-  const int j1 = min(NT, (g + 1) * G);
-  for (int j = g * G; j < j1; ++j) {
+    for (int i = 0; i < EPC; ++i)
+      if (sc * EPC + i < D) EL::put(w, i, p, sc * EPC + i);
+    return make_uint4(w[0], w[1], w[2], w[3]);
+  };
+  // Rows [r0, r0 + n) into registers, zero past n and past D.
+  auto fetch = [&](int r0, int n) {
+#pragma unroll
+    for (int p = 0; p < C::PASSES; ++p) {
+      const int r = p * C::RPP + sr;
+      kreg[p] = vreg[p] = qreg[p] = make_uint4(0u, 0u, 0u, 0u);
+      if (r < n && sc * EPC < D) {
+        kreg[p] = load(k, r0 + r);
+        vreg[p] = load(v, r0 + r);
+        qreg[p] = load(q, r0 + r);
+      }
+    }
+  };
+  auto stash1 = [&](float* dst, const uint4& x) {
+    float f[EPC];
+    EL::widen(x, f);
+#pragma unroll
+    for (int i = 0; i < EPC; i += 4) *reinterpret_cast<float4*>(dst + i) = make_float4(f[i], f[i + 1], f[i + 2], f[i + 3]);
+  };
+  auto stash = [&]() {
+    if (sc >= C::NCH) return;
+#pragma unroll
+    for (int p = 0; p < C::PASSES; ++p) {
+      const int o = (p * C::RPP + sr) * LD + sc * EPC;
+      stash1(ks + o, kreg[p]);
+      stash1(vs + o, vreg[p]);
+      stash1(qsm + o, qreg[p]);
+    }
+  };
+
+  f32x4_t gacc[TL][TL];
+#pragma unroll
+  for (int a = 0; a < TL; ++a)
+#pragma unroll
+    for (int b = 0; b < TL; ++b) gacc[a][b] = (f32x4_t){0.f, 0.f, 0.f, 0.f};
+  if (j0 < j1) fetch(j0 * BT, min(CH, min(BT, T - j0 * BT)));
+  for (int j = j0; j < j1; ++j) {
     const int r0 = j * BT;
     const int n = min(BT, T - r0);
-    float hacc[64];
+    f32x4_t acc[TL][TL];
 #pragma unroll
-    for (int m = 0; m < 64; ++m) hacc[m] = 0.f;
-    float qs = 0.f, ksum = 0.f, vsum = 0.f;
+    for (int a = 0; a < TL; ++a)
+#pragma unroll
+      for (int b = 0; b < TL; ++b) acc[a][b] = (f32x4_t){0.f, 0.f, 0.f, 0.f};
+    float ksum = 0.f, qs = 0.f;  // ksum: of v on the upper threads
     for (int c0 = 0; c0 < n; c0 += CH) {
       const int cn = min(CH, n - c0);
-      __syncthreads();  // the previous chunk's reads are done (and the zero fill landed)
-      for (int i = tid; i < cn * D; i += 256) {
-        const int t = i / D;
-        const int d = i - t * D;
-        const int64_t off = base + (int64_t)(r0 + c0 + t) * D + d;
-        ks[t * LD + d] = EL::load(k, off);
-        vs[t * LD + d] = EL::load(v, off);
-        qsm[t * 128 + d] = EL::load(q, off);
-      }
+      __syncthreads();  // the buffers have been read
+      stash();
       __syncthreads();
-      if (tid < D) {
-        for (int t = 0; t < cn; ++t) {
-          ksum += ks[t * LD + tid];
-          vsum += vs[t * LD + tid];
-          qs += qsm[t * 128 + tid];
+      if (c0 + CH < n)
+        fetch(r0 + c0 + CH, min(CH, n - c0 - CH));
+      else if (j + 1 < j1)
+        fetch(r0 + BT, min(CH, min(BT, T - r0 - BT)));
+      if (col < D) {  // rows past cn are zero, and adding them changes no bit
+        const float* p = (kq_side ? ks : vs) + col;
+#pragma unroll 8
+        for (int t = 0; t < CH; ++t) ksum += p[t * LD];
+        if (kq_side) {
+#pragma unroll 8
+          for (int t = 0; t < CH; ++t) qs += qsm[t * LD + col];
         }
       }
-      if (owns) {
-        for (int t = 0; t < cn; ++t) {
-          const float4 k0 = *reinterpret_cast<const float4*>(ks + t * LD + d0);
-          const float4 k1 = *reinterpret_cast<const float4*>(ks + t * LD + d0 + 4);
-          const float4 v0 = *reinterpret_cast<const float4*>(vs + t * LD + e0);
-          const float4 v1 = *reinterpret_cast<const float4*>(vs + t * LD + e0 + 4);
-          const float kk[8] = {k0.x, k0.y, k0.z, k0.w, k1.x, k1.y, k1.z, k1.w};
-          const float vv[8] = {v0.x, v0.y, v0.z, v0.w, v1.x, v1.y, v1.z, v1.w};
+      const float* ka = ks + g4 * LD + dq + l16;
+      const float* va = vs + g4 * LD + eq + l16;
+      for (int t0 = 0; t0 < cn; t0 += 16) {  // 16 rows (rows past cn are zero), four per MFMA
 #pragma unroll
-          for (int a = 0; a < 8; ++a)
+        for (int s = 0; s < 4; ++s) {
+          float a[TL], b[TL];
 #pragma unroll
-            for (int b = 0; b < 8; ++b) hacc[8 * a + b] = fmaf(kk[a], vv[b], hacc[8 * a + b]);
+          for (int t = 0; t < TL; ++t) {
+            a[t] = ka[(t0 + 4 * s) * LD + 16 * t];
+            b[t] = va[(t0 + 4 * s) * LD + 16 * t];
+          }
+#pragma unroll
+          for (int x = 0; x < TL; ++x)
+#pragma unroll
+            for (int y = 0; y < TL; ++y)
+              acc[x][y] = __builtin_amdgcn_mfma_f32_16x16x4f32(a[x], b[y], acc[x][y], 0, 0, 0);
         }
       }
     }
-    __syncthreads();
-    if (tid < D) {
-      const float kb = ksum / (float)n;
-      kbar[tid] = kb;
-      vhat[tid] = vsum;
-      const int64_t so = ((int64_t)bh * NT + j) * D + tid;
-      qc[so] = qs / (float)n;  // :101
-      kc[so] = kb;             // :102
-      vc[so] = vsum;           // :103 (a sum, not a mean)
+    if (col < D) {
+      const int64_t so = ((int64_t)bh * NT + j) * D + col;
+      if (kq_side) {
+        const float kb = ksum / (float)n;
+        kbar[col] = kb;
+        qc[so] = qs / (float)n;  // :101
+        kc[so] = kb;             // :102
+      } else {
+        vhat[col] = ksum;
+        vc[so] = ksum;           // :103 (a sum, not a mean)
+      }
+    }
+    __syncthreads();  // the sums are in place, and the K/V chunk has been read
+#pragma unroll
+    for (int x = 0; x < TL; ++x) {
+      const float4 kb = *reinterpret_cast<const float4*>(kbar + dq + 16 * x + 4 * g4);
+      const float kbv[4] = {kb.x, kb.y, kb.z, kb.w};
+#pragma unroll
+      for (int y = 0; y < TL; ++y) {
+        const float vh = vhat[eq + 16 * y + l16];
+#pragma unroll
+        for (int i = 0; i < 4; ++i) {
+          const float h = fmaf(-kbv[i], vh, acc[x][y][i]);  // :107 (zero past D)
+          gacc[x][y][i] += h;
+          buf[(dq + 16 * x + 4 * g4 + i) * HLD + eq + 16 * y + l16] = h;
+        }
+      }
     }
     __syncthreads();
     float nsq = 0.f;
-    if (owns) {
+    const int d0 = 8 * (tid >> 4);
+    const int e0 = 8 * (tid & 15);
+    if (d0 < D && e0 < D) {
 #pragma unroll
-      for (int a = 0; a < 8; ++a)
+      for (int a = 0; a < 8; ++a) {
+        const float4 h0 = *reinterpret_cast<const float4*>(buf + (d0 + a) * HLD + e0);
+        const float4 h1 = *reinterpret_cast<const float4*>(buf + (d0 + a) * HLD + e0 + 4);
+        const float h[8] = {h0.x, h0.y, h0.z, h0.w, h1.x, h1.y, h1.z, h1.w};
 #pragma unroll
-        for (int b = 0; b < 8; ++b) {
-          const float h = hacc[8 * a + b] - kbar[d0 + a] * vhat[e0 + b];  // :107 (zero past D)
-          nsq = fmaf(h, h, nsq);
-          gacc[8 * a + b] += h;
-        }
+        for (int b = 0; b < 8; ++b) nsq = fmaf(h[b], h[b], nsq);
+      }
     }
-    nsq = wave_sum(nsq);
-    if ((tid & 63) == 0) red[tid >> 6] = nsq;
+    nsq = wave_sum_xor(nsq);
+    if (lane == 0) red[wave] = nsq;
     __syncthreads();
     if (tid == 0) hnorm[(int64_t)bh * NT + j] = sqrt_rn((red[0] + red[1]) + (red[2] + red[3]));  // :110, :287
   }
   // hbar_g = (1/G) sum over the group, the missing blocks of the last group counting as zeros (:294-299).
-  if (owns) {
-    float* hg = hgroup + ((int64_t)bh * NG + g) * D * D;
+  float* hg = split == 1 ? hgroup + ((int64_t)bh * NG + g) * D * D
+                         : partials + (((int64_t)bh * NG + g) * split + part) * D * D;
+  const float Gf = split == 1 ? (float)G : 1.f;
 #pragma unroll
-    for (int a = 0; a < 8; ++a)
+  for (int x = 0; x < TL; ++x)
 #pragma unroll
-      for (int b = 0; b < 8; ++b)
-        if (d0 + a < D && e0 + b < D) hg[(d0 + a) * D + e0 + b] = gacc[8 * a + b] / (float)G;
-  }
+    for (int y = 0; y < TL; ++y)
+#pragma unroll
+      for (int i = 0; i < 4; ++i) {
+        const int d = dq + 16 * x + 4 * g4 + i;
+        const int e = eq + 16 * y + l16;
+        if (d < D && e < D) hg[d * D + e] = gacc[x][y][i] / Gf;
+      }
+}
+
+// hgroup[g] = (sum over the parts of partials[g], in part order) / G; one entry per thread.
+__global__ __launch_bounds__(256) void k2_any_reduce(const float* __restrict__ partials, float* __restrict__ hgroup,
+                                                     int split, int G, int dd) {
+  const int i = blockIdx.x * 256 + threadIdx.x;
+  if (i >= dd) return;
+  const int64_t grp = (int64_t)blockIdx.z * gridDim.y + blockIdx.y;
+  const float* src = partials + grp * split * dd + i;
+  float a = src[0];
+  for (int p = 1; p < split; ++p) a += src[(int64_t)p * dd];
+  hgroup[grp * dd + i] = a / (float)G;
 }
 
 // ---- selection scores -----------------------------------------------------------
@@ -194,17 +324,42 @@ hipError_t by_dtype(int dtype, F&& f) {
 
 }  // namespace
 
+// Parts per group: about two workgroups per CU (256 CUs), at least one block each.
+int block_stats_any_split(int bh, int T, int BT, int G) {
+  const int NT = (T + BT - 1) / BT;
+  const int64_t groups = (int64_t)((NT + G - 1) / G) * bh;
+  const int nblk = min(G, NT);
+  int split = 1;
+  while (groups * split < 512 && 2 * split <= nblk) split *= 2;
+  return split;
+}
+
 hipError_t launch_block_stats_any(const void* q, const void* k, const void* v, float* qc, float* kc, float* vc,
-                                  float* hnorm, float* hgroup, int bh, int T, int Tslice, int D, int BT, int G,
-                                  int dtype, hipStream_t stream) {
-  if (D < 1 || D > 128 || BT < 1 || G < 1) return hipErrorInvalidValue;
+                                  float* hnorm, float* hgroup, float* partials, int split, int bh, int T, int Tslice,
+                                  int D, int BT, int G, int dtype, hipStream_t stream) {
+  if (D < 1 || D > 128 || BT < 1 || G < 1 || split < 1 || (split > 1 && partials == nullptr)) return hipErrorInvalidValue;
   const int NT = (T + BT - 1) / BT;
   const int NG = (NT + G - 1) / G;
-  const dim3 grid(NG, bh);
-  return by_dtype(dtype, [&](auto el) {
-    hipLaunchKernelGGL(k2_block_stats_any<decltype(el)>, grid, dim3(256), 0, stream, q, k, v, qc, kc, vc, hnorm,
-                       hgroup, T, Tslice, D, BT, NT, G);
+  const dim3 grid(NG * split, bh);
+  const hipError_t e = by_dtype(dtype, [&](auto el) {
+    using EL = decltype(el);
+    const int vec = (D * EL::ES) % 16 == 0 && (((uintptr_t)q | (uintptr_t)k | (uintptr_t)v) & 15u) == 0;
+    auto go = [&](auto kern) {
+      hipLaunchKernelGGL(kern, grid, dim3(256), 0, stream, (const unsigned char*)q, (const unsigned char*)k,
+                         (const unsigned char*)v, qc, kc, vc, hnorm, hgroup, partials, T, Tslice, D, BT, NT, G, split,
+                         vec);
+    };
+    if (D <= 64)
+      go(k2_block_stats_any<EL, 64>);
+    else if (D <= 96)
+      go(k2_block_stats_any<EL, 96>);
+    else
+      go(k2_block_stats_any<EL, 128>);
   });
+  if (e != hipSuccess || split == 1) return e;
+  hipLaunchKernelGGL(k2_any_reduce, dim3((D * D + 255) / 256, NG, bh), dim3(256), 0, stream, (const float*)partials,
+                     hgroup, split, G, D * D);
+  return hipGetLastError();
 }
 
 hipError_t launch_scores_any(const float* qc, const float* kc, const float* hnorm, const float* noise, float scale,

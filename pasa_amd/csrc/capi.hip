@@ -218,8 +218,16 @@ static int block_stats_impl(const void* q, const void* k, const void* v, float* 
       return rc;
     const int64_t ng = cdiv(cdiv(seq_len - text_len, block_size), group_size);
     if (ng > 65535 * 1024LL) return fail(PASA_ERR_OVERFLOW, "pasa_block_stats: too many groups");
-    return launch_status(pasa::launch_block_stats_any(q, k, v, qc, kc, vc, hnorm, hgroup, (int)bh,
-                                                      (int)(seq_len - text_len), (int)seq_len, (int)head_dim,
+    // Any workspace is accepted: the groups split over as many workgroups as its partial sums allow
+    // (the reduction's grid holds 65,535 groups per slice).
+    int split = 1;
+    if (workspace != nullptr && ((uintptr_t)workspace & 3u) == 0 && ng <= 65535) {
+      const size_t per_part = (size_t)bh * (size_t)ng * (size_t)(head_dim * head_dim) * sizeof(float);
+      split = pasa::block_stats_any_split((int)bh, (int)(seq_len - text_len), (int)block_size, (int)group_size);
+      while (split > 1 && workspace_bytes / per_part < (size_t)split) split /= 2;
+    }
+    return launch_status(pasa::launch_block_stats_any(q, k, v, qc, kc, vc, hnorm, hgroup, (float*)workspace, split,
+                                                      (int)bh, (int)(seq_len - text_len), (int)seq_len, (int)head_dim,
                                                       (int)block_size, (int)group_size, dtype, (hipStream_t)stream),
                          "pasa_block_stats");
   }
@@ -256,6 +264,19 @@ size_t pasa_block_stats_workspace_bytes(int64_t bh, int64_t seq_len, int64_t tex
     return 0;
   const int split = pasa::block_stats_split((int)bh, (int)(seq_len - text_len), (int)head_dim, (int)block_size,
                                             (int)group_size);
+  if (split == 1) return 0;
+  const int64_t ng = cdiv(cdiv(seq_len - text_len, block_size), group_size);
+  return (size_t)bh * (size_t)ng * (size_t)split * (size_t)(head_dim * head_dim) * sizeof(float);
+}
+
+size_t pasa_block_stats_workspace_bytes_dtype(int64_t bh, int64_t seq_len, int64_t text_len, int64_t head_dim,
+                                              int64_t block_size, int64_t group_size, int dtype) {
+  if (tuned_shape(dtype, head_dim, block_size) && (text_len == 0 || head_dim == 128))
+    return pasa_block_stats_workspace_bytes(bh, seq_len, text_len, head_dim, block_size, group_size);
+  if (check_any_dtype(dtype, "pasa_block_stats") ||
+      check_any_shape(bh, seq_len, text_len, head_dim, block_size, group_size, "pasa_block_stats"))
+    return 0;
+  const int split = pasa::block_stats_any_split((int)bh, (int)(seq_len - text_len), (int)block_size, (int)group_size);
   if (split == 1) return 0;
   const int64_t ng = cdiv(cdiv(seq_len - text_len, block_size), group_size);
   return (size_t)bh * (size_t)ng * (size_t)split * (size_t)(head_dim * head_dim) * sizeof(float);

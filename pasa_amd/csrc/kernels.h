@@ -64,9 +64,12 @@ hipError_t launch_dense_attn(const void* q, const void* k, const void* v, void* 
 constexpr int kAnyBf16 = 0;
 constexpr int kAnyF16 = 1;
 constexpr int kAnyF32 = 2;
+// split > 1: as launch_block_stats (partials: [bh, NG, split, D, D] fp32); statistics and selection
+// do not depend on it.
 hipError_t launch_block_stats_any(const void* q, const void* k, const void* v, float* qc, float* kc, float* vc,
-                                  float* hnorm, float* hgroup, int bh, int T, int Tslice, int D, int BT, int G,
-                                  int dtype, hipStream_t stream);
+                                  float* hnorm, float* hgroup, float* partials, int split, int bh, int T, int Tslice,
+                                  int D, int BT, int G, int dtype, hipStream_t stream);
+int block_stats_any_split(int bh, int T, int BT, int G);
 hipError_t launch_scores_any(const float* qc, const float* kc, const float* hnorm, const float* noise, float scale,
                              int use_cov_bias, float* scores, int bh, int NT, int D, hipStream_t stream);
 // all: dense (every key block exact, no correction; kc, vc, hgroup, selmask unused).

@@ -160,8 +160,9 @@ def block_stats(q: torch.Tensor, k: torch.Tensor, v: torch.Tensor, block_size: i
     hgroup = torch.empty(B, H, NG, D, D, **f32)
     args = (q.data_ptr(), k.data_ptr(), v.data_ptr(), qc.data_ptr(), kc.data_ptr(), vc.data_ptr(),
             hnorm.data_ptr(), hgroup.data_ptr(), B * H, T, int(text_tokens), D, block_size, group_size)
-    ws_bytes = _lib.load().pasa_block_stats_workspace_bytes(B * H, T, int(text_tokens), D, block_size,
-                                                            group_size) if split else 0
+    dt = _DTYPES.get(q.dtype, -1)
+    ws_bytes = _lib.load().pasa_block_stats_workspace_bytes_dtype(B * H, T, int(text_tokens), D, block_size,
+                                                                  group_size, dt) if split else 0
     ws = torch.empty(ws_bytes, device=q.device, dtype=torch.uint8) if ws_bytes > 0 else None
     ws_ptr = None if ws is None else ws.data_ptr()
     if placement is None and ws is not None:

@@ -95,3 +95,34 @@ def test_dense_edges(device, T, D, dtype, text, valid, shift):
     print(f"[edges] dense T={T} D={D} {dtype}: rel {err:.2e}", flush=True)
     # 16 bits: P and o rounded once each to 8 (bf16) or 11 (fp16) bits
     assert err <= {F32: 4e-6, B16: 6e-3, F16: 1e-3}[dtype]
+
+
+@pytest.mark.parametrize("heads,T,D,BT,G,dtype", [(2, 1024, 64, 64, 32, F32), (1, 777, 37, 16, 50, F16),
+                                                  (3, 1000, 96, 32, 16, B16), (1, 300, 128, 256, 2, F32)])
+def test_block_stats_split_any(device, heads, T, D, BT, G, dtype):
+    """A group split over several workgroups: the per-block statistics are the unsplit call's bit for
+    bit, and the group moment differs by the order of at most G sums (G 2^-24 of the sum of their
+    magnitudes).  A workspace smaller than asked for is used as far as it reaches."""
+    from pasa_amd import _lib
+    q, k, v = (t.to(device) for t in make(heads, T, D, dtype, T + D))
+    lib = _lib.load()
+    need = lib.pasa_block_stats_workspace_bytes_dtype(heads, T, 0, D, BT, G, ops._DTYPES[dtype])
+    assert need > 0
+    one = ops.block_stats(q, k, v, BT, G, split=False)
+    runs = [ops.block_stats(q, k, v, BT, G)]
+    for nbytes in (need // 2, 4):
+        st = ops.BlockStats(*(torch.full_like(getattr(one, n), float("nan"))
+                              for n in ("qc", "kc", "vc", "hnorm", "hgroup")))
+        ws = torch.empty(need, dtype=torch.uint8, device=device)
+        _lib.call("pasa_block_stats_ws", q.data_ptr(), k.data_ptr(), v.data_ptr(), st.qc.data_ptr(), st.kc.data_ptr(),
+                  st.vc.data_ptr(), st.hnorm.data_ptr(), st.hgroup.data_ptr(), heads, T, 0, D, BT, G,
+                  ops._DTYPES[dtype], ws.data_ptr(), nbytes, ops._stream(q))
+        torch.cuda.synchronize()
+        runs.append(st)
+    ref = O.block_stats(*(t.cpu().reshape(heads, T, D) for t in (q, k, v)), BT, dtype=torch.float64)
+    bound = G * 2.0 ** -24 * O.group_moment(ref.hc.abs(), G) + 1e-6
+    for st in runs:
+        for n in ("qc", "kc", "vc", "hnorm"):
+            assert torch.equal(getattr(st, n), getattr(one, n)), n
+        diff = (st.hgroup - one.hgroup).abs().double().cpu().reshape(bound.shape)
+        assert bool((diff <= bound).all())
