@@ -126,3 +126,20 @@ def test_block_stats_split_any(device, heads, T, D, BT, G, dtype):
             assert torch.equal(getattr(st, n), getattr(one, n)), n
         diff = (st.hgroup - one.hgroup).abs().double().cpu().reshape(bound.shape)
         assert bool((diff <= bound).all())
+
+
+@pytest.mark.parametrize("heads,NT,D", [(1, 1, 1), (2, 63, 127), (1, 65, 96), (2, 130, 38), (1, 64, 100)])
+def test_scores_any(device, heads, NT, D):
+    """Selection scores at the edges of the 64 x 64 tile and at head dims that are not whole 16-byte
+    pieces, against 64 bits: a chain of D fused multiply-adds, each rounding at most 2^-24 of the
+    running sum's bound sum |q k|, and the log and the two additions about as much again."""
+    g = torch.Generator().manual_seed(NT + D)
+    qc, kc = (torch.randn(1, heads, NT, D, generator=g) for _ in range(2))
+    hn = torch.rand(1, heads, NT, generator=g) + 0.5
+    st = ops.BlockStats(qc.to(device), kc.to(device), torch.empty(0), hn.to(device), torch.empty(0))
+    sel = ops.select_blocks(st, 0.3, 0.37, return_scores=True)
+    ref = O.select_scores(qc.double(), kc.double(), hn.double(), 0.37)
+    mag = O.select_scores(qc.double().abs(), kc.double().abs(), hn.double(), 0.37, use_cov_bias=False)
+    assert bool(((sel.scores.cpu().double() - ref).abs() <= (D + 8) * 2.0 ** -24 * (mag + 1)).all())
+    idx = O.topk_indices(sel.scores.cpu(), sel.ns)
+    assert torch.equal(idx.reshape(sel.idx.shape), sel.idx.cpu())
