@@ -28,9 +28,9 @@
 // operands of phase 2, which every query block reads in full.  The next chunk's rows load into registers while one is multiplied.
 //
 // What bounds it: in fp32 the MFMA pipe (153 TFLOP/s in a large fp32 matrix product here; 12 heads
-// x 7,800 rows, D 128, block 64: 75 GFLOP in 0.84 ms, where one FMA per lane took 2.07 ms); in 16
+// x 7,800 rows, D 128, block 64: 75 GFLOP in 0.76 ms, where one FMA per lane took 2.07 ms); in 16
 // bits the latency of the staged loads and the LDS operand reads (16 heads x 8,610 rows, D 96,
-// block 32, groups of 16: 149 GFLOP in 0.66 ms, where one FMA per lane took 9.7 ms with half its
+// block 32, groups of 16: 149 GFLOP in 0.42 ms, where one FMA per lane took 9.7 ms with half its
 // lanes idle).
 //
 // fp32 sums are taken in short chains (16 features, a chunk of keys, 32 features of Hbar) that
@@ -97,11 +97,10 @@ struct AnyCfg {
   static_assert(PASSES * RPP == KC && KZ % RPP4 == 0 && HR % RPP4 == 0, "staging split");
 };
 
-// 16 bytes of a row from element c * 16 / ES on; elements past D read as zero.  Rows that are not
-// whole 16-byte chunks, or not aligned to them, go element by element.
+// Element-wise forms, for rows that are not whole 16-byte chunks or not aligned to them: 16 bytes of
+// a row from chunk c on, and four floats of a statistics row; elements past D are zero.
 template <int ES>
-__device__ __forceinline__ uint4 load_chunk(const unsigned char* row, int c, int D, bool vec) {
-  if (vec) return *reinterpret_cast<const uint4*>(row + c * 16);
+__device__ __forceinline__ uint4 load_elems(const unsigned char* row, int c, int D) {
   uint32_t w[4] = {0u, 0u, 0u, 0u};
   if constexpr (ES == 2) {
 #pragma unroll
@@ -115,28 +114,23 @@ __device__ __forceinline__ uint4 load_chunk(const unsigned char* row, int c, int
   return make_uint4(w[0], w[1], w[2], w[3]);
 }
 
-// Four floats of a statistics row from 4 c on, zero past D.
-__device__ __forceinline__ float4 load_stat4(const float* row, int c, int D, bool vec) {
-  if (vec) return *reinterpret_cast<const float4*>(row + 4 * c);
-  float f[4] = {0.f, 0.f, 0.f, 0.f};
-#pragma unroll
-  for (int i = 0; i < 4; ++i)
-    if (4 * c + i < D) f[i] = row[4 * c + i];
-  return make_float4(f[0], f[1], f[2], f[3]);
-}
+constexpr uint32_t kOutside = 0x80000000u;  // a buffer offset past every chunk: the load gives zeros
 
 }  // namespace
 
-// vec: q, k, v and o rows are whole aligned 16-byte chunks; vec_stats: kc, vc and hgroup rows are.
+// VEC: the rows of q, k, v, o, kc, vc and hgroup are whole aligned 16-byte chunks.  They are then
+// loaded through buffer resources over just the rows wanted, so rows past them read as zero with
+// no branch around any load (a branch per load makes the compiler wait for each by itself: the
+// bf16 call above took 0.67 ms, now 0.42, with a run-time test of the alignment in its load loop).
 // all: dense (every key of the segment, no selection, no correction; BT is then ROWS).
 // video: query blocks are computed (0: the text rows alone, where the blocks run with TEAM = 1).
-template <typename E, int DP, int TEAM, int RW>
+template <typename E, int DP, int TEAM, int RW, bool VEC>
 __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2))) void k4_any_mfma(
     const unsigned char* __restrict__ q, const unsigned char* __restrict__ k, const unsigned char* __restrict__ v,
     const float* __restrict__ kc, const float* __restrict__ vc, const float* __restrict__ hgroup,
     const uint32_t* __restrict__ selmask, unsigned char* __restrict__ o, float scale, float c, int T, int text,
-    int text_valid, int D, int BT, int NT, int G, int NG, int NW, int gamma_literal, int all, int nvt, int ntiles,
-    int vec_, int vec_stats_) {
+    int text_valid, int D, int BT, int NT, int G, int NG, int NW, int gamma_literal, int all, int nvt,
+    int ntiles) {
   using C = AnyCfg<E, DP, TEAM, RW>;
   using frag = typename E::frag;
   constexpr int ES = C::ES, QT = C::QT, NF = C::NF, DT = C::DT, KC = C::KC;
@@ -149,7 +143,6 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2))) void k
   const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
   const int l16 = lane & 15;
   const int g4 = lane >> 4;
-  const bool vec = vec_ != 0, vec_stats = vec_stats_ != 0;
   const int bh = blockIdx.y;
   // Consecutive workgroups go to consecutive XCDs; each takes a contiguous run of a slice's tiles.
   const int tile = (int)(blockIdx.x & 7) * (int)(gridDim.x >> 3) + (int)(blockIdx.x >> 3);
@@ -193,40 +186,41 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2))) void k
 
   // Q as B operands: fragment f of query tile qt holds the slots of feature step f.
   frag qf[QT][NF];
+  const rsrc_t qrs = make_rsrc(q + slice + (int64_t)row0 * row_bytes,
+                               (uint32_t)(min(RW, max(0, row_end - row0)) * (int)row_bytes));
 #pragma unroll
   for (int qt = 0; qt < QT; ++qt) {
-    const int r = row0 + 16 * qt + l16;
-    const unsigned char* qrow = q + slice + (int64_t)r * row_bytes;
+    const int r = 16 * qt + l16;
+    const unsigned char* qrow = q + slice + (int64_t)(row0 + r) * row_bytes;
 #pragma unroll
     for (int f = 0; f < NF; ++f) {
-      uint32_t w[4] = {0u, 0u, 0u, 0u};
-      if (r < row_end) {
-        if constexpr (F32) {
-          const int d = 16 * f + 4 * g4;
-          if (d < D) {
-            const uint4 x = load_chunk<4>(qrow, d / 4, D, vec);
-            w[0] = x.x; w[1] = x.y; w[2] = x.z; w[3] = x.w;
-          }
-        } else {
+      u32x4_t w = {0u, 0u, 0u, 0u};
+      if constexpr (F32) {
+        const int d = 16 * f + 4 * g4;
+        if constexpr (VEC) {
+          w = __builtin_amdgcn_raw_buffer_load_b128(qrs, d < D ? (uint32_t)(r * (int)row_bytes + d * 4) : kOutside, 0, 0);
+        } else if (row0 + r < row_end) {
+          const uint4 x = load_elems<4>(qrow, d / 4, D);
+          w = (u32x4_t){x.x, x.y, x.z, x.w};
+        }
+      } else {
 #pragma unroll
-          for (int h = 0; h < 2; ++h) {
-            const int d = 32 * f + 16 * h + 4 * g4;
-            if (vec) {
-              if (d < D) {
-                const uint2 x = *reinterpret_cast<const uint2*>(qrow + d * 2);
-                w[2 * h] = x.x;
-                w[2 * h + 1] = x.y;
-              }
-            } else {
+        for (int h = 0; h < 2; ++h) {
+          const int d = 32 * f + 16 * h + 4 * g4;
+          if constexpr (VEC) {
+            const auto x = __builtin_amdgcn_raw_buffer_load_b64(
+                qrs, d < D ? (uint32_t)(r * (int)row_bytes + d * 2) : kOutside, 0, 0);
+            w[2 * h] = x[0];
+            w[2 * h + 1] = x[1];
+          } else if (row0 + r < row_end) {
 #pragma unroll
-              for (int i = 0; i < 4; ++i)
-                if (d + i < D)
-                  w[2 * h + (i >> 1)] |= (uint32_t)reinterpret_cast<const uint16_t*>(qrow)[d + i] << (16 * (i & 1));
-            }
+            for (int i = 0; i < 4; ++i)
+              if (d + i < D)
+                w[2 * h + (i >> 1)] |= (uint32_t)reinterpret_cast<const uint16_t*>(qrow)[d + i] << (16 * (i & 1));
           }
         }
       }
-      qf[qt][f] = __builtin_bit_cast(frag, (u32x4_t){w[0], w[1], w[2], w[3]});
+      qf[qt][f] = __builtin_bit_cast(frag, w);
     }
   }
 
@@ -403,15 +397,31 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2))) void k
       return n;
     };
     uint4 kreg[C::PASSES], vreg[C::PASSES];
+    // Rows r of a chunk: ra + r, and rb + r - 16 from row 16 on where each wave stages its own.
+    const uint32_t lane_off = in_row ? (uint32_t)(sr * (int)row_bytes + sc * 16) : kOutside;
     auto fetch = [&](int ra, int rb, int n) {
+      constexpr int SPLIT = TEAM == 1 && KC == 32 ? 16 : KC;
+      const int na = min(n, SPLIT), nb = n - na;
+      const unsigned char* base_k[2] = {ksl + (int64_t)ra * row_bytes, ksl + (int64_t)rb * row_bytes};
+      const unsigned char* base_v[2] = {vsl + (int64_t)ra * row_bytes, vsl + (int64_t)rb * row_bytes};
+      const rsrc_t rk[2] = {make_rsrc(base_k[0], (uint32_t)(na * (int)row_bytes)),
+                            make_rsrc(base_k[1], (uint32_t)(nb * (int)row_bytes))};
+      const rsrc_t rv[2] = {make_rsrc(base_v[0], (uint32_t)(na * (int)row_bytes)),
+                            make_rsrc(base_v[1], (uint32_t)(nb * (int)row_bytes))};
 #pragma unroll
       for (int p = 0; p < C::PASSES; ++p) {
-        const int r = p * C::RPP + sr;
-        kreg[p] = vreg[p] = make_uint4(0u, 0u, 0u, 0u);
-        if (r < n && in_row) {
-          const int64_t off = (int64_t)((TEAM == 1 && r >= 16) ? rb + (r - 16) : ra + r) * row_bytes;
-          kreg[p] = load_chunk<ES>(ksl + off, sc, D, vec);
-          vreg[p] = load_chunk<ES>(vsl + off, sc, D, vec);
+        const int h = p * C::RPP >= SPLIT ? 1 : 0;
+        const int r0 = p * C::RPP - h * SPLIT;  // of the pass, within its run
+        if constexpr (VEC) {
+          const uint32_t off = lane_off + (uint32_t)(r0 * (int)row_bytes);
+          kreg[p] = buf_load16(rk[h], off);
+          vreg[p] = buf_load16(rv[h], off);
+        } else {
+          kreg[p] = vreg[p] = make_uint4(0u, 0u, 0u, 0u);
+          if (r0 + sr < (h ? nb : na) && in_row) {
+            kreg[p] = load_elems<ES>(base_k[h] + (int64_t)(r0 + sr) * row_bytes, sc, D);
+            vreg[p] = load_elems<ES>(base_v[h] + (int64_t)(r0 + sr) * row_bytes, sc, D);
+          }
         }
       }
     };
@@ -498,30 +508,55 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2))) void k
       else
         lds_st(base, off16, make_uint2(E::M::pack2(x.x, x.y), E::M::pack2(x.z, x.w)));
     };
-    const float4 zero4 = make_float4(0.f, 0.f, 0.f, 0.f);
     const bool in4 = 4 * c4 < D;
+    const uint32_t off4 = in4 ? (uint32_t)(r4 * D + 4 * c4) * 4u : kOutside;
+    // Piece c4 of row r0 + r4 of the statistics rows at base, of which n are wanted.
+    auto load4 = [&](const float* base, const rsrc_t& rs, int r0, int n) -> float4 {
+      if constexpr (VEC) {
+        const uint4 x = buf_load16(rs, off4 + (uint32_t)(r0 * D) * 4u);
+        return make_float4(__uint_as_float(x.x), __uint_as_float(x.y), __uint_as_float(x.z), __uint_as_float(x.w));
+      } else {
+        uint4 x = make_uint4(0u, 0u, 0u, 0u);
+        if (r0 + r4 < n) x = load_elems<4>((const unsigned char*)(base + (int64_t)(r0 + r4) * D), c4, D);
+        return make_float4(__uint_as_float(x.x), __uint_as_float(x.y), __uint_as_float(x.z), __uint_as_float(x.w));
+      }
+    };
     auto stage_z = [&](int jc, int cn) {
+      const float* kb = kcb + (int64_t)jc * D;
+      const float* vb = vcb + (int64_t)jc * D;
+      const rsrc_t rk = make_rsrc(kb, (uint32_t)(cn * D * 4)), rv = make_rsrc(vb, (uint32_t)(cn * D * 4));
+      float4 xk[C::KZ / C::RPP4], xv[C::KZ / C::RPP4];
 #pragma unroll
       for (int p = 0; p < C::KZ / C::RPP4; ++p) {
-        const int r = p * C::RPP4 + r4;
-        float4 xk = zero4, xv = zero4;
-        if (r < cn && in4) {
-          xk = load_stat4(kcb + (int64_t)(jc + r) * D, c4, D, vec_stats);
-          xv = load_stat4(vcb + (int64_t)(jc + r) * D, c4, D, vec_stats);
-        }
-        if (c4 < C::C4) {
-          st4(Kz, r * KROW + (c4 >> 3) * 64 + (c4 & 3) * 16 + ((c4 >> 2) & 1) * 8, r * KROW + c4 * 16, xk);
-          st4(Vz, r * VROW + c4 * 8, r * VROW + c4 * 16, xv);
+        xk[p] = load4(kb, rk, p * C::RPP4, cn);
+        xv[p] = load4(vb, rv, p * C::RPP4, cn);
+      }
+      if (c4 < C::C4) {
+#pragma unroll
+        for (int p = 0; p < C::KZ / C::RPP4; ++p) {
+          const int r = p * C::RPP4 + r4;
+          st4(Kz, r * KROW + (c4 >> 3) * 64 + (c4 & 3) * 16 + ((c4 >> 2) & 1) * 8, r * KROW + c4 * 16, xk[p]);
+          st4(Vz, r * VROW + c4 * 8, r * VROW + c4 * 16, xv[p]);
         }
       }
     };
     auto stage_h = [&](const float* hg, int d0) {
-#pragma unroll 8
-      for (int p = 0; p < C::HR / C::RPP4; ++p) {
-        const int r = p * C::RPP4 + r4;
-        float4 x = zero4;
-        if (d0 + r < D && in4) x = load_stat4(hg + (int64_t)(d0 + r) * D, c4, D, vec_stats);
-        if (c4 < C::C4) st4(Hs, r * VROW + c4 * 8, r * VROW + c4 * 16, x);
+      const int n = min(C::HR, D - d0);
+      const float* hb = hg + (int64_t)d0 * D;
+      const rsrc_t rh = make_rsrc(hb, (uint32_t)(n * D * 4));
+      constexpr int HP = C::HR / C::RPP4, HB = HP < 8 ? HP : 8;  // passes, and passes in flight
+#pragma unroll
+      for (int p0 = 0; p0 < HP; p0 += HB) {
+        float4 x[HB];
+#pragma unroll
+        for (int p = 0; p < HB; ++p) x[p] = load4(hb, rh, (p0 + p) * C::RPP4, n);
+        if (c4 < C::C4) {
+#pragma unroll
+          for (int p = 0; p < HB; ++p) {
+            const int r = (p0 + p) * C::RPP4 + r4;
+            st4(Hs, r * VROW + c4 * 8, r * VROW + c4 * 16, x[p]);
+          }
+        }
       }
     };
     for (int g = 0; g < NG; ++g) {
@@ -642,7 +677,7 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2))) void k
         const int e = 16 * dt + 4 * g4;
         const float x[4] = {oacc[dt][qt][0] / den, oacc[dt][qt][1] / den, oacc[dt][qt][2] / den,
                             oacc[dt][qt][3] / den};
-        if (vec && e < D) {
+        if (VEC && e < D) {
           if constexpr (F32)
             *reinterpret_cast<float4*>(orow + e * 4) = make_float4(x[0], x[1], x[2], x[3]);
           else
@@ -684,17 +719,14 @@ int text_tiles(const AnyCall& a, int rows) {
   return (a.text_valid + rows - 1) / rows + (a.text - a.text_valid + rows - 1) / rows;
 }
 
-template <typename E, int DP, int TEAM, int RW>
+template <typename E, int DP, int TEAM, int RW, bool VEC>
 hipError_t launch_any(const AnyCall& a, int BT, int nvt, int ntiles) {
   const int NT = (a.T + BT - 1) / BT;
-  const bool vec = (a.D * E::ES) % 16 == 0 && aligned16({a.q, a.k, a.v, a.o});
-  const bool vec_stats = a.D % 4 == 0 && aligned16({a.kc, a.vc, a.hgroup});
   const dim3 grid((unsigned)((ntiles + 7) / 8 * 8), (unsigned)a.bh);
-  hipLaunchKernelGGL((k4_any_mfma<E, DP, TEAM, RW>), grid, dim3(256), 0, a.stream, (const unsigned char*)a.q,
+  hipLaunchKernelGGL((k4_any_mfma<E, DP, TEAM, RW, VEC>), grid, dim3(256), 0, a.stream, (const unsigned char*)a.q,
                      (const unsigned char*)a.k, (const unsigned char*)a.v, a.kc, a.vc, a.hgroup, a.selmask,
                      (unsigned char*)a.o, a.scale, a.scale * kLog2e, a.T, a.text, a.text_valid, a.D, BT, NT, a.G,
-                     (NT + a.G - 1) / a.G, (NT + 31) / 32, a.gamma_literal, a.all, nvt, ntiles, (int)vec,
-                     (int)vec_stats);
+                     (NT + a.G - 1) / a.G, (NT + 31) / 32, a.gamma_literal, a.all, nvt, ntiles);
   return hipGetLastError();
 }
 
@@ -704,33 +736,39 @@ bool wide_tiles(const AnyCall& a, int BT) {
   return BT >= 128 && (int64_t)a.bh * ((a.T + 127) / 128) >= 256;
 }
 
-template <typename E, int DP>
+// WIDE: 32 rows per wave where the blocks are long enough (not in fp32: its MFMAs outlast their
+// LDS reads with 16 rows already, and 32 spill).
+template <typename E, int DP, bool VEC, bool WIDE>
 hipError_t launch_dp(const AnyCall& a) {
-  constexpr bool F32 = E::ES == 4;  // 16 rows per wave: its MFMAs outlast their LDS reads, and 32 rows spill
   if (!a.all && a.BT < 64) {
     const int NT = (a.T + a.BT - 1) / a.BT;
     hipError_t e;
-    if (F32 || a.BT == 16) {
-      const int ntiles = (NT * (a.BT / 16) + 3) / 4;
-      e = launch_any<E, DP, 1, 16>(a, a.BT, ntiles, ntiles);
+    if (!WIDE || a.BT == 16) {
+      const int ntiles = (int)(((int64_t)NT * (a.BT / 16) + 3) / 4);
+      e = launch_any<E, DP, 1, 16, VEC>(a, a.BT, ntiles, ntiles);
     } else {
       const int ntiles = (NT + 3) / 4;
-      e = launch_any<E, DP, 1, F32 ? 16 : 32>(a, a.BT, ntiles, ntiles);
+      e = launch_any<E, DP, 1, WIDE ? 32 : 16, VEC>(a, a.BT, ntiles, ntiles);
     }
     if (e != hipSuccess || a.text == 0) return e;
-    return launch_any<E, DP, 4, 16>(a, a.BT, 0, text_tiles(a, 64));  // the text rows
+    return launch_any<E, DP, 4, 16, VEC>(a, a.BT, 0, text_tiles(a, 64));  // the text rows
   }
-  const bool wide = !F32 && wide_tiles(a, a.all ? 128 : a.BT);
+  const bool wide = WIDE && wide_tiles(a, a.all ? 128 : a.BT);
   const int rows = wide ? 128 : 64;
   const int BT = a.all ? rows : a.BT;
   const int nvt = (a.T + BT - 1) / BT * ((BT + rows - 1) / rows);
   const int ntiles = nvt + text_tiles(a, rows);
-  return wide ? launch_any<E, DP, 4, F32 ? 16 : 32>(a, BT, nvt, ntiles) : launch_any<E, DP, 4, 16>(a, BT, nvt, ntiles);
+  return wide ? launch_any<E, DP, 4, WIDE ? 32 : 16, VEC>(a, BT, nvt, ntiles)
+              : launch_any<E, DP, 4, 16, VEC>(a, BT, nvt, ntiles);
 }
 
 template <typename E>
 hipError_t launch_type(const AnyCall& a) {
-  return a.D <= 64 ? launch_dp<E, 64>(a) : (a.D <= 96 ? launch_dp<E, 96>(a) : launch_dp<E, 128>(a));
+  constexpr bool WIDE = E::ES == 2;
+  const bool vec = (a.D * E::ES) % 16 == 0 && a.D % 4 == 0 && aligned16({a.q, a.k, a.v, a.o, a.kc, a.vc, a.hgroup});
+  if (!vec) return launch_dp<E, 128, false, false>(a);
+  return a.D <= 64 ? launch_dp<E, 64, true, WIDE>(a)
+                   : (a.D <= 96 ? launch_dp<E, 96, true, WIDE>(a) : launch_dp<E, 128, true, WIDE>(a));
 }
 
 }  // namespace
