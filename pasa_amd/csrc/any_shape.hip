@@ -78,12 +78,14 @@ struct StatsCfg {
   static constexpr int TL = DP / 32;                  // 16 x 16 tiles per side of a wave's quarter
 };
 
-template <typename EL, int DP>
+// VEC: rows are whole aligned 16-byte chunks, loaded through a buffer resource over the rows wanted
+// (rows past them read as zero, with no branch around a load); else element by element.
+template <typename EL, int DP, bool VEC>
 __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2))) void k2_block_stats_any(
     const unsigned char* __restrict__ q, const unsigned char* __restrict__ k, const unsigned char* __restrict__ v,
     float* __restrict__ qc, float* __restrict__ kc, float* __restrict__ vc, float* __restrict__ hnorm,
     float* __restrict__ hgroup, float* __restrict__ partials, int T, int Tslice, int D, int BT, int NT, int G,
-    int split, int vec) {
+    int split) {
   using C = StatsCfg<EL, DP>;
   constexpr int CH = C::CH, LD = C::LD, HLD = C::HLD, TL = C::TL, EPC = C::EPC;
   __shared__ __attribute__((aligned(16))) float buf[C::LDS_FLOATS];  // K, V and Q chunk; then H_j
@@ -120,27 +122,30 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2))) void k
   const int col = tid & 127;
   const bool kq_side = tid < 128;
   uint4 kreg[C::PASSES], vreg[C::PASSES], qreg[C::PASSES];
-  auto load = [&](const unsigned char* base, int row) -> uint4 {
-    const unsigned char* p = base + slice + (int64_t)row * row_bytes;
-    if (vec) return *reinterpret_cast<const uint4*>(p + sc * 16);
-    uint32_t w[4] = {0u, 0u, 0u, 0u};
-#pragma unroll
-    for (int i = 0; i < EPC; ++i)
-      if (sc * EPC + i < D) EL::put(w, i, p, sc * EPC + i);
-    return make_uint4(w[0], w[1], w[2], w[3]);
-  };
-  // Rows [r0, r0 + n) into registers, zero past n and past D.
-  auto fetch = [&](int r0, int n) {
+  const uint32_t lane_off = sc * EPC < D ? (uint32_t)(sr * (int)row_bytes + sc * 16) : 0x80000000u;
+  // Chunk sc of the rows r0 + p RPP + sr, zero past the n rows from r0.
+  auto load = [&](const unsigned char* base, int r0, int n, uint4 (&dst)[C::PASSES]) {
+    const unsigned char* p0 = base + slice + (int64_t)r0 * row_bytes;
+    const rsrc_t rs = make_rsrc(p0, (uint32_t)(n * (int)row_bytes));
 #pragma unroll
     for (int p = 0; p < C::PASSES; ++p) {
-      const int r = p * C::RPP + sr;
-      kreg[p] = vreg[p] = qreg[p] = make_uint4(0u, 0u, 0u, 0u);
-      if (r < n && sc * EPC < D) {
-        kreg[p] = load(k, r0 + r);
-        vreg[p] = load(v, r0 + r);
-        qreg[p] = load(q, r0 + r);
+      if constexpr (VEC) {
+        dst[p] = buf_load16(rs, lane_off + (uint32_t)(p * C::RPP * (int)row_bytes));
+      } else {
+        uint32_t w[4] = {0u, 0u, 0u, 0u};
+        if (p * C::RPP + sr < n) {
+#pragma unroll
+          for (int i = 0; i < EPC; ++i)
+            if (sc * EPC + i < D) EL::put(w, i, p0 + (int64_t)(p * C::RPP + sr) * row_bytes, sc * EPC + i);
+        }
+        dst[p] = make_uint4(w[0], w[1], w[2], w[3]);
       }
     }
+  };
+  auto fetch = [&](int r0, int n) {
+    load(k, r0, n, kreg);
+    load(v, r0, n, vreg);
+    load(q, r0, n, qreg);
   };
   auto stash1 = [&](float* dst, const uint4& x) {
     float f[EPC];
@@ -410,18 +415,19 @@ hipError_t launch_block_stats_any(const void* q, const void* k, const void* v, f
   const dim3 grid(NG * split, bh);
   const hipError_t e = by_dtype(dtype, [&](auto el) {
     using EL = decltype(el);
-    const int vec = (D * EL::ES) % 16 == 0 && (((uintptr_t)q | (uintptr_t)k | (uintptr_t)v) & 15u) == 0;
+    const bool vec = (D * EL::ES) % 16 == 0 && (((uintptr_t)q | (uintptr_t)k | (uintptr_t)v) & 15u) == 0;
     auto go = [&](auto kern) {
       hipLaunchKernelGGL(kern, grid, dim3(256), 0, stream, (const unsigned char*)q, (const unsigned char*)k,
-                         (const unsigned char*)v, qc, kc, vc, hnorm, hgroup, partials, T, Tslice, D, BT, NT, G, split,
-                         vec);
+                         (const unsigned char*)v, qc, kc, vc, hnorm, hgroup, partials, T, Tslice, D, BT, NT, G, split);
     };
-    if (D <= 64)
-      go(k2_block_stats_any<EL, 64>);
+    if (!vec)
+      go(k2_block_stats_any<EL, 128, false>);
+    else if (D <= 64)
+      go(k2_block_stats_any<EL, 64, true>);
     else if (D <= 96)
-      go(k2_block_stats_any<EL, 96>);
+      go(k2_block_stats_any<EL, 96, true>);
     else
-      go(k2_block_stats_any<EL, 128>);
+      go(k2_block_stats_any<EL, 128, true>);
   });
   if (e != hipSuccess || split == 1) return e;
   hipLaunchKernelGGL(k2_any_reduce, dim3((D * D + 255) / 256, NG, bh), dim3(256), 0, stream, (const float*)partials,
