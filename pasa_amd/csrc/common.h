@@ -169,14 +169,6 @@ struct PadTile {
   static constexpr int bytes(int rows) { return rows * ROW_BYTES; }
 };
 
-// Token permutation inside each 16-token group: swap bits 2 and 3.  Applied to
-// the token axis of transposed tiles ([feature][token]) so that the 8 tokens a
-// lane feeds to one 32x32x16 MFMA as its A-operand slots (tokens
-// 16s + 4h + {0..3} and 16s + 8 + 4h + {0..3}) form one 16-byte chunk.
-__host__ __device__ __forceinline__ constexpr int tok_perm(int t) {
-  return (t & ~12) | ((t & 4) << 1) | ((t & 8) >> 1);
-}
-
 template <typename T>
 __device__ __forceinline__ T lds_ld(const unsigned char* base, int byte_off) {
   return *reinterpret_cast<const T*>(base + byte_off);

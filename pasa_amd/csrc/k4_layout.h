@@ -1,5 +1,5 @@
-// LDS images shared by the D = 128 K4 kernel (k4_sparse_attn_dma) and the pack kernel
-// that writes its phase-2 operands.
+// LDS images shared by the K4 kernels (head_dim 128 and 64) and the pack kernel that writes
+// their phase-2 operands.
 #pragma once
 
 #include "common.h"
@@ -18,26 +18,34 @@ __host__ __device__ __forceinline__ constexpr int vt_block_of(int chunk, int i) 
   return ((i & 4) << 2) | (chunk << 2) | (i & 3);
 }
 
-// Phase-2 pack image for the D = 128 direct-load kernels, split between their two
-// LDS tile buffers: [Hbar^T: 128 rows x 256 B, XOR layout of a K tile] -> K buffer;
-// [kbar: 32 rows x 256 B, XOR layout][V^ transposed: 128 rows x kVtRow] -> V buffer.
-// Both parts are whole multiples of 4 KB, so the waves of a workgroup (four, or two)
-// split their 1 KB direct loads evenly.
-template <int BT>
-struct K4DPack {
-  static constexpr int HT_BYTES = 128 * 256;
+// Tiles of D-feature rows, 16-byte chunk c of row r stored at c ^ kx(r) (K, kbar, Hbar^T: the
+// reads of 16 rows at one chunk touch 16 distinct 16-byte bank groups) or c ^ vx(r) (V: the
+// transposing reads of 8 rows x 2 chunks do).  At D = 64 two rows share a 256-byte bank line, so
+// the swizzle takes the row's bits from the second on.  Both depend on r mod 16 only.
+template <int D>
+struct K4Tile {
+  static_assert(D == 128 || D == 64, "head dims of the tuned kernels");
+  static constexpr int ROWB = 2 * D;
+  __host__ __device__ static constexpr int kx(int r) { return D == 128 ? (r & 15) : ((r >> 1) & 7); }
+  __host__ __device__ static constexpr int vx(int r) { return D == 128 ? 2 * (r & 7) : 2 * ((r >> 1) & 3); }
+  __host__ __device__ static constexpr int k_byte(int row, int col) {
+    return row * ROWB + (((col >> 3) ^ kx(row)) << 4) + (col & 7) * 2;
+  }
+};
+
+// Phase-2 pack image, split between the two LDS tile buffers: [Hbar^T: D rows in the K layout] ->
+// K buffer; [kbar: 32 rows in the K layout][V^ transposed: D rows x kVtRow] -> V buffer.
+// Both parts are whole multiples of 4 KB, so the four waves of a workgroup split their 1 KB
+// direct loads evenly.
+template <int D>
+struct K4Pack {
+  static constexpr int HT_BYTES = D * 2 * D;
   static constexpr int KB_OFF = 0;                       // within the V-buffer part
-  static constexpr int VT_OFF = 32 * 256;
-  static constexpr int RAW2 = VT_OFF + 128 * kVtRow;
+  static constexpr int VT_OFF = 32 * 2 * D;
+  static constexpr int RAW2 = VT_OFF + D * kVtRow;
   static constexpr int PART2 = (RAW2 + 4095) / 4096 * 4096;
   static constexpr int BYTES = HT_BYTES + PART2;
   static_assert(HT_BYTES % 4096 == 0, "pack split");
 };
-
-// Byte offset of element (row, col) in a 256-byte-row tile whose 16-byte chunk c
-// of row r is stored at c ^ (r & 15).
-__host__ __device__ __forceinline__ constexpr int xor_tile_byte(int row, int col) {
-  return row * 256 + ((((col >> 3) ^ row) & 15) << 4) + (col & 7) * 2;
-}
 
 }  // namespace pasa

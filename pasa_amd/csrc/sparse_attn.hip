@@ -55,81 +55,20 @@
 
 namespace pasa {
 
-template <int D, int BT>
-struct K4Cfg {
-  static constexpr int WAVES = BT / 32;
-  static constexpr int THREADS = WAVES * 64;
-  static constexpr int CH = D / 8;
-  using KT = PadTile<D>;       // K tile:        BT rows x D
-  // V tile: BT rows x D, natural chunk order, row stride 2D + 64 bytes, which
-  // makes the transposing reads of 32 lanes (4 rows x 2 chunks per 16-lane
-  // group, two groups side by side) hit 64 distinct banks.
-  static constexpr int VROW = 2 * D + 64;
-  using PKB = PadTile<D>;      // kbar:          32 rows x D
-  using PVT = PadTile<kGroup>; // V^ transposed: D rows x 32 means (tok_perm order)
-  using PHT = PadTile<D>;      // Hbar^T:        D rows (e) x D (d)
-  static constexpr int KS_BYTES = KT::bytes(BT);
-  static constexpr int P1_BYTES = KS_BYTES + BT * VROW;
-  static constexpr int PK_VT_OFF = PKB::bytes(kGroup);
-  static constexpr int PK_HT_OFF = PK_VT_OFF + PVT::bytes(D);
-  static constexpr int PK_RAW = PK_HT_OFF + PHT::bytes(D);
-  static constexpr int PK_BYTES = (PK_RAW + 16 * THREADS - 1) / (16 * THREADS) * (16 * THREADS);
-  static constexpr int LDS_BYTES = P1_BYTES > PK_BYTES ? P1_BYTES : PK_BYTES;
-  static constexpr int K_LOADS = (BT * D / 8) / THREADS;   // 16-byte K chunks per thread
-  static constexpr int V_LOADS = K_LOADS;                  // 16-byte V chunks per thread
-  static constexpr int PK_LOADS = PK_BYTES / 16 / THREADS;
-  static_assert(K_LOADS * THREADS * 8 == BT * D, "K tile split");
-  static_assert(THREADS % CH == 0, "K rows per pass");
-};
-
-
 // ---- phase-2 operand pack ---------------------------------------------------
-
-template <int D, int BT>
-__global__ __launch_bounds__(256) void k4_pack(const float* __restrict__ kc,
-                                               const float* __restrict__ vc,
-                                               const float* __restrict__ hgroup,
-                                               unsigned char* __restrict__ pack, int NT, int NG) {
-  using C = K4Cfg<D, BT>;
-  const int g = blockIdx.x;
-  const int bh = blockIdx.y;
-  unsigned char* out = pack + ((int64_t)bh * NG + g) * C::PK_BYTES;
-  const float* kb = kc + (int64_t)bh * NT * D;
-  const float* vb = vc + (int64_t)bh * NT * D;
-  const float* hb = hgroup + ((int64_t)bh * NG + g) * D * D;
-  for (int u = threadIdx.x; u < kGroup * D; u += 256) {
-    const int m = u / D;
-    const int d = u - m * D;
-    const int jj = g * kGroup + m;
-    const float x = jj < NT ? kb[(int64_t)jj * D + d] : 0.f;
-    *(uint16_t*)(out + C::PKB::elem_byte(m, d)) = (uint16_t)f32_to_bf16_bits(x);
-  }
-  for (int u = threadIdx.x; u < D * kGroup; u += 256) {
-    const int m = u % kGroup;
-    const int e = u / kGroup;
-    const int jj = g * kGroup + m;
-    const float x = jj < NT ? vb[(int64_t)jj * D + e] : 0.f;
-    *(uint16_t*)(out + C::PK_VT_OFF + C::PVT::elem_byte(e, tok_perm(m))) =
-        (uint16_t)f32_to_bf16_bits(x);
-  }
-  for (int u = threadIdx.x; u < D * D; u += 256) {
-    const int d = u / D;  // Hbar[d][e] row-major in, Hbar^T[e][d] out
-    const int e = u - d * D;
-    *(uint16_t*)(out + C::PK_HT_OFF + C::PHT::elem_byte(e, d)) = (uint16_t)f32_to_bf16_bits(hb[u]);
-  }
-}
 
 // One workgroup per (group, slice).  Every output element is written once, as part of
 // a 16-byte chunk: Hbar^T goes through LDS (coalesced fp32 reads of Hbar rows, column
 // reads from a padded tile), kbar rows are read as 32-byte runs, V^T columns with the
 // token index fastest across lanes.  Rounding is round-to-nearest-even, as everywhere.
-template <int BT, typename E = Bf16>
+template <int D, typename E = Bf16>
 __global__ __launch_bounds__(256) void k4_pack_xor(const float* __restrict__ kc,
                                                    const float* __restrict__ vc,
                                                    const float* __restrict__ hgroup,
                                                    unsigned char* __restrict__ pack, int NT, int NG) {
-  using P = K4DPack<BT>;
-  constexpr int D = 128;
+  using P = K4Pack<D>;
+  using TL = K4Tile<D>;
+  constexpr int CH = D / 8;   // 16-byte chunks per row
   constexpr int HS = D + 1;  // padded row of the fp32 Hbar tile
   __shared__ float hs[D * HS];
   const int g = blockIdx.x;
@@ -142,21 +81,21 @@ __global__ __launch_bounds__(256) void k4_pack_xor(const float* __restrict__ kc,
 #pragma unroll 4
   for (int it = 0; it < D * D / 4 / 256; ++it) {
     const int idx = it * 256 + tid;
-    const int d = idx >> 5;
-    const int e4 = (idx & 31) * 4;
+    const int d = idx / (D / 4);
+    const int e4 = (idx % (D / 4)) * 4;
     const float4 x = *(const float4*)(hb + d * D + e4);
     hs[d * HS + e4 + 0] = x.x;
     hs[d * HS + e4 + 1] = x.y;
     hs[d * HS + e4 + 2] = x.z;
     hs[d * HS + e4 + 3] = x.w;
   }
-  // kbar: rows m (block of the group) x 16 chunks of 8 features, XOR layout.
+  // kbar: rows m (block of the group) x D / 8 chunks of 8 features, K layout.
   unsigned char* part2 = out + P::HT_BYTES;
 #pragma unroll
   for (int it = 0; it < kGroup * D / 8 / 256; ++it) {
     const int qi = it * 256 + tid;
-    const int m = qi >> 4;
-    const int cc = qi & 15;
+    const int m = qi / CH;
+    const int cc = qi % CH;
     const int jj = g * kGroup + m;
     float f[8];
     if (jj < NT) {
@@ -169,14 +108,14 @@ __global__ __launch_bounds__(256) void k4_pack_xor(const float* __restrict__ kc,
       for (int i = 0; i < 8; ++i) f[i] = 0.f;
     }
     const uint4 w = make_uint4(E::pack2(f[0], f[1]), E::pack2(f[2], f[3]), E::pack2(f[4], f[5]), E::pack2(f[6], f[7]));
-    *(uint4*)(part2 + P::KB_OFF + xor_tile_byte(m, cc * 8)) = w;
+    *(uint4*)(part2 + P::KB_OFF + TL::k_byte(m, cc * 8)) = w;
   }
   // V^T: feature rows e x 4 chunks of 8 blocks (vt_block_of order), kVtRow bytes per row.
 #pragma unroll
   for (int it = 0; it < D * kGroup / 8 / 256; ++it) {
     const int qi = it * 256 + tid;
     const int e = qi & (D - 1);
-    const int cc = qi >> 7;
+    const int cc = qi / D;
     float f[8];
 #pragma unroll
     for (int i = 0; i < 8; ++i) {
@@ -191,307 +130,13 @@ __global__ __launch_bounds__(256) void k4_pack_xor(const float* __restrict__ kc,
 #pragma unroll 2
   for (int it = 0; it < D * D / 8 / 256; ++it) {
     const int qi = it * 256 + tid;
-    const int e = qi >> 4;
-    const int cc = qi & 15;
+    const int e = qi / CH;
+    const int cc = qi % CH;
     float f[8];
 #pragma unroll
     for (int i = 0; i < 8; ++i) f[i] = hs[(cc * 8 + i) * HS + e];
     const uint4 w = make_uint4(E::pack2(f[0], f[1]), E::pack2(f[2], f[3]), E::pack2(f[4], f[5]), E::pack2(f[6], f[7]));
-    *(uint4*)(out + xor_tile_byte(e, cc * 8)) = w;
-  }
-}
-
-// ---- main kernel ------------------------------------------------------------
-
-template <int D, int BT>
-__global__ __attribute__((amdgpu_flat_work_group_size(1, 256), amdgpu_waves_per_eu(2, 2)))
-void k4_sparse_attn(const uint16_t* __restrict__ q, const uint16_t* __restrict__ k,
-                    const uint16_t* __restrict__ v, const unsigned char* __restrict__ pack,
-                    const uint32_t* __restrict__ selmask, uint16_t* __restrict__ o, float scale,
-                    float c, int T, int NT, int NG, int NW, int xcd_chunk, int gamma_literal) {
-  using C = K4Cfg<D, BT>;
-  using KT = typename C::KT;
-  __shared__ __attribute__((aligned(16))) unsigned char lds[C::LDS_BYTES];
-  unsigned char* Ks = lds;
-  unsigned char* Vs = lds + C::KS_BYTES;
-
-  // XCD-aware workgroup -> (slice, query block) map: consecutive workgroup ids
-  // go to consecutive XCDs, so slot = wg / 8 indexes within one XCD's run.
-  const int wg = blockIdx.x;
-  const int xcd = wg & 7;
-  const int slot = wg >> 3;
-  const int bh = slot / xcd_chunk;
-  const int qb = xcd * xcd_chunk + (slot - bh * xcd_chunk);
-  if (qb >= NT) return;
-
-  const int tid = threadIdx.x;
-  const int lane = tid & 63;
-  const int wave = tid >> 6;
-  const int h = lane >> 5;
-  const int l32 = lane & 31;
-  const int64_t slice = (int64_t)bh * T * D;
-  const int qrow = qb * BT + wave * 32 + l32;  // the query this lane owns
-
-  const uint32_t slice_bytes = (uint32_t)T * D * 2u;
-  const rsrc_t qr = make_rsrc(q + slice, slice_bytes);
-  const rsrc_t kr = make_rsrc(k + slice, slice_bytes);
-  const rsrc_t vr = make_rsrc(v + slice, slice_bytes);
-
-  // Q fragments (B operand of S^T and of r^T): lane holds Q[qrow][16ks + 8h .. +7].
-  bf16x8_t qf[D / 16];
-#pragma unroll
-  for (int ks = 0; ks < D / 16; ++ks)
-    qf[ks] = as_bf16x8(buf_load16(qr, ((uint32_t)qrow * D + ks * 16 + h * 8) * 2u));
-
-  f32x16_t oacc[D / 32];
-#pragma unroll
-  for (int et = 0; et < D / 32; ++et)
-#pragma unroll
-    for (int r = 0; r < 16; ++r) oacc[et][r] = 0.f;
-  float l_run = 0.f;
-  float g_run = 0.f;
-
-  const uint32_t* mrow = selmask + ((int64_t)bh * NT + qb) * NW;
-
-  // Lane-constant parts of the tile load / store / read addresses.
-  constexpr int KROWS = C::THREADS / C::CH;  // rows covered per load pass
-  const uint32_t goff = (uint32_t)((tid / C::CH) * D + (tid % C::CH) * 8) * 2u;
-  const int k_soff = KT::chunk_byte(tid / C::CH, tid % C::CH);
-  const int v_soff = (tid / C::CH) * C::VROW + (tid % C::CH) * 16;
-  const int ka_base = KT::frag_base(l32, h);
-  // Transposing V reads: group g = lane / 16 covers keys +4*(g/2) and columns
-  // +16*(g%2); lane i of the group addresses row i/4, columns 4*(i%4) .. +3.
-  const int g16 = lane >> 4;
-  const int i16 = lane & 15;
-  const int vtr_base = (4 * (g16 >> 1) + (i16 >> 2)) * C::VROW + (16 * (g16 & 1) + 4 * (i16 & 3)) * 2;
-
-  // ---------------- Phase 1: exact attention over the selected blocks --------
-  uint4 kreg[C::K_LOADS];
-  uint4 vreg[C::V_LOADS];
-  auto fetch = [&](int blk) {
-    const uint32_t base = (uint32_t)blk * BT * D * 2u + goff;
-#pragma unroll
-    for (int it = 0; it < C::K_LOADS; ++it) kreg[it] = buf_load16(kr, base + it * KROWS * D * 2);
-#pragma unroll
-    for (int it = 0; it < C::V_LOADS; ++it) vreg[it] = buf_load16(vr, base + it * KROWS * D * 2);
-  };
-  auto stash = [&]() {
-#pragma unroll
-    for (int it = 0; it < C::K_LOADS; ++it) lds_st(Ks, k_soff + it * KROWS * KT::ROW_BYTES, kreg[it]);
-#pragma unroll
-    for (int it = 0; it < C::V_LOADS; ++it) lds_st(Vs, v_soff + it * KROWS * C::VROW, vreg[it]);
-  };
-
-  // Selected blocks in ascending order, from the selection bitmask (uniform).
-  int wsel = 0;
-  uint32_t bits = NW > 0 ? mrow[0] : 0u;
-  auto next_selected = [&]() -> int {
-    while (bits == 0u) {
-      if (++wsel >= NW) return -1;
-      bits = mrow[wsel];
-    }
-    const int j = 32 * wsel + __builtin_ctz(bits);
-    bits &= bits - 1u;
-    return j;
-  };
-
-  float m_run = -INFINITY;  // exact running max of the scores (log2 units)
-  int blk = next_selected();
-  if (blk >= 0) fetch(blk);
-  while (blk >= 0) {
-    const int nxt = next_selected();
-    __syncthreads();
-    stash();
-    __syncthreads();
-    if (nxt >= 0) fetch(nxt);
-
-    const int nvalid = min(BT, T - blk * BT);
-#pragma unroll
-    for (int kh = 0; kh < BT / 64; ++kh) {
-      if (kh * 64 >= nvalid) break;  // fully masked half (ragged last block)
-      f32x16_t sacc[2];
-#pragma unroll
-      for (int mt = 0; mt < 2; ++mt)
-#pragma unroll
-        for (int r = 0; r < 16; ++r) sacc[mt][r] = 0.f;
-#pragma unroll
-      for (int ks = 0; ks < D / 16; ++ks)
-#pragma unroll
-        for (int mt = 0; mt < 2; ++mt) {
-          const bf16x8_t a = as_bf16x8(
-              lds_ld<uint4>(Ks, ka_base + (kh * 64 + mt * 32) * KT::ROW_BYTES + ks * 16));
-          sacc[mt] = mfma32(a, qf[ks], sacc[mt]);
-        }
-      if (nvalid < (kh + 1) * 64) {
-#pragma unroll
-        for (int mt = 0; mt < 2; ++mt)
-#pragma unroll
-          for (int r = 0; r < 16; ++r)
-            if (kh * 64 + mt * 32 + mfma32_row(r, h) >= nvalid) sacc[mt][r] = -INFINITY;
-      }
-      float mx = -INFINITY;
-#pragma unroll
-      for (int mt = 0; mt < 2; ++mt)
-#pragma unroll
-        for (int r = 0; r < 16; ++r) mx = fmaxf(mx, sacc[mt][r]);
-      const float mxc = halves_max(mx) * c;
-      if (__any(mxc > m_run)) {
-        const float m_new = fmaxf(m_run, mxc);
-        const float alpha = fast_exp2(m_run - m_new);  // 0 on the first step
-        m_run = m_new;
-        l_run *= alpha;
-#pragma unroll
-        for (int et = 0; et < D / 32; ++et)
-#pragma unroll
-          for (int r = 0; r < 16; ++r) oacc[et][r] *= alpha;
-      }
-      bf16x8_t pf[4];
-      float lsum[4] = {0.f, 0.f, 0.f, 0.f};  // fp32 row sum of p, as gpa.py:182-184
-#pragma unroll
-      for (int s4 = 0; s4 < 4; ++s4) {
-        uint32_t w[4];
-#pragma unroll
-        for (int i = 0; i < 4; ++i) {
-          const float p0 = fast_exp2(fmaf(sacc[s4 >> 1][8 * (s4 & 1) + 2 * i], c, -m_run));
-          const float p1 = fast_exp2(fmaf(sacc[s4 >> 1][8 * (s4 & 1) + 2 * i + 1], c, -m_run));
-          w[i] = pack_bf16x2(p0, p1);
-          lsum[i] += p0 + p1;
-        }
-        pf[s4] = __builtin_bit_cast(bf16x8_t, (u32x4_t){w[0], w[1], w[2], w[3]});
-      }
-      l_run += (lsum[0] + lsum[1]) + (lsum[2] + lsum[3]);
-#pragma unroll
-      for (int s4 = 0; s4 < 4; ++s4) {
-        const int rowk = 16 * (kh * 4 + s4);
-#pragma unroll
-        for (int et = 0; et < D / 32; ++et) {
-          const int off = vtr_base + rowk * C::VROW + et * 64;
-          const uint2 lo = lds_read_tr16(Vs, off);
-          const uint2 hi = lds_read_tr16(Vs, off + 8 * C::VROW);
-          const bf16x8_t a = __builtin_bit_cast(bf16x8_t, (u32x4_t){lo.x, lo.y, hi.x, hi.y});
-          oacc[et] = mfma32(a, pf[s4], oacc[et]);
-        }
-      }
-    }
-    blk = nxt;
-  }
-
-  // ---------------- Phase 2: zero- + first-order correction per group --------
-  using PKB = typename C::PKB;
-  using PVT = typename C::PVT;
-  using PHT = typename C::PHT;
-  const unsigned char* Pkb = lds;
-  const unsigned char* Pvt = lds + C::PK_VT_OFF;
-  const unsigned char* Pht = lds + C::PK_HT_OFF;
-  const int kb_base = PKB::frag_base(l32, h);
-  const int pv_base = PVT::frag_base(l32, h);
-  const int ph_base = PHT::frag_base(l32, h);
-  const int last_len = T - (NT - 1) * BT;
-  for (int g = 0; g < NG; ++g) {
-    // Blocks of this group that take the approximation (uniform over the workgroup).
-    const int nin = min(kGroup, NT - g * kGroup);
-    const uint32_t inrange = nin >= 32 ? 0xffffffffu : ((1u << nin) - 1u);
-    const uint32_t approx = inrange & ~mrow[g];
-    if (approx == 0u) continue;  // every block exact or absent: no contribution
-
-    __syncthreads();
-    {
-      const uint4* src = (const uint4*)(pack + ((int64_t)bh * NG + g) * C::PK_BYTES);
-      uint4 preg[C::PK_LOADS];
-#pragma unroll
-      for (int i = 0; i < C::PK_LOADS; ++i) preg[i] = src[i * C::THREADS + tid];
-#pragma unroll
-      for (int i = 0; i < C::PK_LOADS; ++i) ((uint4*)lds)[i * C::THREADS + tid] = preg[i];
-    }
-    __syncthreads();
-
-    f32x16_t sb;
-#pragma unroll
-    for (int r = 0; r < 16; ++r) sb[r] = 0.f;
-#pragma unroll
-    for (int ks = 0; ks < D / 16; ++ks) {
-      const bf16x8_t a = as_bf16x8(lds_ld<uint4>(Pkb, kb_base + ks * 16));
-      sb = mfma32(a, qf[ks], sb);
-    }
-    float gmx = -INFINITY;
-#pragma unroll
-    for (int r = 0; r < 16; ++r) {
-      const int mm = mfma32_row(r, h);
-      if (!((approx >> mm) & 1u)) sb[r] = -INFINITY;
-      gmx = fmaxf(gmx, sb[r]);
-    }
-    const float m_new = fmaxf(m_run, halves_max(gmx) * c);
-    const float alpha = fast_exp2(m_run - m_new);
-    m_run = m_new;
-    l_run *= alpha;
-    if (!gamma_literal) g_run *= alpha;
-    if (__any(alpha != 1.f)) {
-#pragma unroll
-      for (int et = 0; et < D / 32; ++et)
-#pragma unroll
-        for (int r = 0; r < 16; ++r) oacc[et][r] *= alpha;
-    }
-    float psum = 0.f;
-    float gsum = 0.f;
-    bf16x8_t pbf[2];
-#pragma unroll
-    for (int s = 0; s < 2; ++s) {
-      uint32_t w[4];
-#pragma unroll
-      for (int i = 0; i < 4; ++i) {
-        const int r0 = 8 * s + 2 * i;
-        const float p0 = fast_exp2(fmaf(sb[r0], c, -m_new));
-        const float p1 = fast_exp2(fmaf(sb[r0 + 1], c, -m_new));
-        const int j0 = g * kGroup + mfma32_row(r0, h);
-        const int j1 = g * kGroup + mfma32_row(r0 + 1, h);
-        psum += p0 + p1;
-        gsum += p0 * (float)(j0 == NT - 1 ? last_len : BT) + p1 * (float)(j1 == NT - 1 ? last_len : BT);
-        w[i] = pack_bf16x2(p0, p1);
-      }
-      pbf[s] = __builtin_bit_cast(bf16x8_t, (u32x4_t){w[0], w[1], w[2], w[3]});
-    }
-    g_run += gsum;
-    psum = halves_sum(psum);
-#pragma unroll
-    for (int s = 0; s < 2; ++s)
-#pragma unroll
-      for (int et = 0; et < D / 32; ++et) {
-        const bf16x8_t a = as_bf16x8(lds_ld<uint4>(Pvt, pv_base + et * 32 * PVT::ROW_BYTES + s * 16));
-        oacc[et] = mfma32(a, pbf[s], oacc[et]);
-      }
-    f32x16_t racc[D / 32];
-#pragma unroll
-    for (int et = 0; et < D / 32; ++et)
-#pragma unroll
-      for (int r = 0; r < 16; ++r) racc[et][r] = 0.f;
-#pragma unroll
-    for (int ks = 0; ks < D / 16; ++ks)
-#pragma unroll
-      for (int et = 0; et < D / 32; ++et) {
-        const bf16x8_t a = as_bf16x8(lds_ld<uint4>(Pht, ph_base + et * 32 * PHT::ROW_BYTES + ks * 16));
-        racc[et] = mfma32(a, qf[ks], racc[et]);
-      }
-    const float f = psum * scale;
-#pragma unroll
-    for (int et = 0; et < D / 32; ++et)
-#pragma unroll
-      for (int r = 0; r < 16; ++r) oacc[et][r] = fmaf(racc[et][r], f, oacc[et][r]);
-  }
-
-  // ---------------- Finalize ---------------------------------------------------
-  const float denom = halves_sum(l_run) + halves_sum(g_run);
-  if (qrow < T) {
-    uint16_t* orow = o + slice + (int64_t)qrow * D;
-#pragma unroll
-    for (int et = 0; et < D / 32; ++et)
-#pragma unroll
-      for (int rq = 0; rq < 4; ++rq) {
-        const int e0 = et * 32 + 8 * rq + 4 * h;
-        uint2 w;
-        w.x = pack_bf16x2(oacc[et][4 * rq + 0] / denom, oacc[et][4 * rq + 1] / denom);
-        w.y = pack_bf16x2(oacc[et][4 * rq + 2] / denom, oacc[et][4 * rq + 3] / denom);
-        *(uint2*)(orow + e0) = w;
-      }
+    *(uint4*)(out + TL::k_byte(e, cc * 8)) = w;
   }
 }
 
@@ -524,23 +169,27 @@ void k4_sparse_attn(const uint16_t* __restrict__ q, const uint16_t* __restrict__
 
 // PAIR: two query blocks per workgroup, one wave group (QWAVES waves) each, with
 // their K/V tiles side by side in the K and V buffers.
-template <int BT, bool PAIR = false>
+template <int D_, int BT, bool PAIR = false>
 struct K4D {
-  static constexpr int D = 128;
+  static constexpr int D = D_;
+  static constexpr int ROWB = 2 * D;                       // bytes of a tile row
   static constexpr int QWAVES = BT / 32;                   // waves of one query block
   static constexpr int QBLOCKS = PAIR ? 2 : 1;             // query blocks per workgroup
   static constexpr int WAVES = QWAVES * QBLOCKS;
   static constexpr int THREADS = WAVES * 64;
-  static constexpr int TILE = BT * 256;                    // bytes of one K or V tile
-  static constexpr int VW = 4 / QWAVES;                    // 4-row load slots per wave per 16 rows
-  static constexpr int TILE_LOADS = TILE / 1024 / QWAVES;  // 1 KB direct loads per wave per tile
+  static constexpr int TILE = BT * ROWB;                   // bytes of one K or V tile
+  // A 1 KB direct load covers RPL rows; a query block's waves cover SPAN rows (a multiple of 16,
+  // the period of the swizzles) in VW loads each.
+  static constexpr int RPL = 1024 / ROWB;
+  static constexpr int SPAN = RPL * QWAVES > 16 ? RPL * QWAVES : 16;
+  static constexpr int VW = SPAN / (RPL * QWAVES);
   static constexpr int KT = BT / 16;                       // 16-key tiles of S per block
   static constexpr int KS = D / 32;                        // 32-feature k-steps
   static constexpr int DT = D / 16;                        // 16-feature tiles of O
-  using PK = K4DPack<BT>;
+  using PK = K4Pack<D>;
   static constexpr int KBUF = QBLOCKS * TILE > PK::HT_BYTES ? QBLOCKS * TILE : PK::HT_BYTES;
   static constexpr int VBUF = QBLOCKS * TILE > PK::PART2 ? QBLOCKS * TILE : PK::PART2;
-  static_assert(TILE_LOADS == 8, "load schedule");
+  static_assert(BT % SPAN == 0, "load schedule");
   static_assert(WAVES == 4, "four-wave workgroups (BT = 128, or BT = 64 in pairs)");
   static_assert(PK::PART2 % (1024 * WAVES) == 0 && PK::HT_BYTES % (1024 * WAVES) == 0, "pack split");
 };
@@ -548,11 +197,12 @@ struct K4D {
 // Byte offset in a V tile of the 8 bytes lane `lane` reads with ds_read_b64_tr_b16 for
 // 16-feature tile dt and key rows row0 + 4 (lane / 16) + {0..3}: row row0 + 4 (lane / 16)
 // + (lane % 16) / 4, features 16 dt + 4 (lane % 4) .. + 3 (chunk 2 dt + (lane % 4) / 2,
-// half lane % 2), the chunk stored at c ^ 2 (row & 7).  row0 is a multiple of 16.
+// half lane % 2).  row0 is a multiple of 16.
+template <int D>
 __device__ __forceinline__ int vtile_tr_byte(int row0, int dt, int lane) {
   const int r = row0 + 4 * (lane >> 4) + ((lane & 15) >> 2);
   const int c = 2 * dt + ((lane & 3) >> 1);
-  return r * 256 + ((c ^ (2 * (r & 7))) << 4) + 8 * (lane & 1);
+  return r * K4Tile<D>::ROWB + ((c ^ K4Tile<D>::vx(r)) << 4) + 8 * (lane & 1);
 }
 
 // Instruction-group masks of __builtin_amdgcn_sched_group_barrier.
@@ -572,19 +222,19 @@ constexpr int kSchedDsRead = 0x100;
 // either block approximates; a group the other block approximates and this one
 // does not adds exact zeros here (p = 0, alpha = 1), so each block's result is the
 // one the unpaired kernel computes.
-template <int BT, bool ALL, bool PERM, bool PAIR = false, typename E = Bf16>
-__global__ __attribute__((amdgpu_flat_work_group_size(1, 256), amdgpu_waves_per_eu(2, 2)))
-void k4_sparse_attn_dma(const uint16_t* __restrict__ q, const uint16_t* __restrict__ k,
-                        const uint16_t* __restrict__ v, const unsigned char* __restrict__ pack,
-                        const uint32_t* __restrict__ selmask, uint16_t* __restrict__ o,
-                        float scale, float c, int T, int NT, int NG, int NW, int xcd_chunk,
-                        int gamma_literal, int text, int text_valid, int n_text_wg, int nbh, RowMap rm) {
+template <int D, int BT, bool ALL, bool PERM, bool PAIR, typename E>
+__device__ __forceinline__ void k4_body(const uint16_t* __restrict__ q, const uint16_t* __restrict__ k,
+                                        const uint16_t* __restrict__ v, const unsigned char* __restrict__ pack,
+                                        const uint32_t* __restrict__ selmask, uint16_t* __restrict__ o, float scale,
+                                        float c, int T, int NT, int NG, int NW, int xcd_chunk, int gamma_literal,
+                                        int text, int text_valid, int n_text_wg, int nbh, const RowMap& rm) {
   static_assert(!PAIR || (!ALL && !PERM), "pairs run selected video blocks only");
   constexpr bool all_tiles = ALL;
-  using C = K4D<BT, PAIR>;
+  using C = K4D<D, BT, PAIR>;
+  using TL = K4Tile<D>;
   using PK = typename C::PK;
   using vec8 = typename E::vec8;
-  constexpr int D = 128;
+  constexpr int ROWB = C::ROWB;
   constexpr int KT = C::KT, KS = C::KS, DT = C::DT;
   // Two distinct LDS objects, so the compiler can tell loads into one from reads of the other.
   __shared__ __attribute__((aligned(1024))) unsigned char Ks[C::KBUF];
@@ -693,17 +343,18 @@ void k4_sparse_attn_dma(const uint16_t* __restrict__ q, const uint16_t* __restri
   const const_u32_ptr mrow0 = (const_u32_ptr)(selmask + ((int64_t)bh * NT + qb) * NW);
   const const_u32_ptr mrow1 = (const_u32_ptr)(selmask + ((int64_t)bh * NT + min(qb + 1, NT - 1)) * NW);
 
-  // Direct-load lane constants.  Load (vw, n) of this wave covers tile rows
-  // 16n + 4*(qw + QWAVES*vw) + lane/16 of its query block's tile; the lane's 16 bytes
-  // land at chunk lane % 16, so it fetches the logical chunk stored there.
-  const int lrow = lane >> 4;
-  const int lch = lane & 15;
+  // Direct-load lane constants.  Load (vw, n) of this wave covers RPL tile rows from
+  // SPAN n + RPL (qw + QWAVES vw) of its query block's tile; lane l's 16 bytes land at chunk
+  // l % CPR of row l / CPR (CPR chunks per row), so it fetches the logical chunk stored there.
+  constexpr int RPL = C::RPL, SPAN = C::SPAN, CPR = ROWB / 16;
+  const int lrow = lane / CPR;
+  const int lch = lane % CPR;
   uint32_t k_lane[C::VW], v_lane[C::VW];
 #pragma unroll
   for (int vw = 0; vw < C::VW; ++vw) {
-    const int r = 4 * (qw + C::QWAVES * vw) + lrow;  // row mod 16
-    k_lane[vw] = (uint32_t)(r * 256 + ((lch ^ r) << 4));
-    v_lane[vw] = (uint32_t)(r * 256 + ((lch ^ (2 * (r & 7))) << 4));
+    const int r = RPL * (qw + C::QWAVES * vw) + lrow;  // row mod SPAN
+    k_lane[vw] = (uint32_t)(r * ROWB + ((lch ^ TL::kx(r)) << 4));
+    v_lane[vw] = (uint32_t)(r * ROWB + ((lch ^ TL::vx(r)) << 4));
   }
 
   const u32x4_t kd = make_rsrc_words(k + slice, slice_bytes);
@@ -716,31 +367,31 @@ void k4_sparse_attn_dma(const uint16_t* __restrict__ q, const uint16_t* __restri
   const uint32_t vt_lds = vs_lds + tile_off;
   // A tile is BT key rows starting at row `row0` of the slice (rows past the slice read as zero).
   auto load_k = [&](int row0) {
-    const uint32_t soff = (uint32_t)row0 * 256u;
+    const uint32_t soff = (uint32_t)row0 * (uint32_t)ROWB;
 #pragma unroll
     for (int vw = 0; vw < C::VW; ++vw)
 #pragma unroll
-      for (int n = 0; n < BT / 16; ++n)
-        dma_load16_lds(kd, kt_lds + (16 * n + 4 * (qw + C::QWAVES * vw)) * 256, k_lane[vw] + 16 * n * 256, soff);
+      for (int n = 0; n < BT / SPAN; ++n)
+        dma_load16_lds(kd, kt_lds + (SPAN * n + RPL * (qw + C::QWAVES * vw)) * ROWB, k_lane[vw] + SPAN * n * ROWB, soff);
   };
   auto load_v = [&](int row0) {
-    const uint32_t soff = (uint32_t)row0 * 256u;
+    const uint32_t soff = (uint32_t)row0 * (uint32_t)ROWB;
 #pragma unroll
     for (int vw = 0; vw < C::VW; ++vw)
 #pragma unroll
-      for (int n = 0; n < BT / 16; ++n)
-        dma_load16_lds(vd, vt_lds + (16 * n + 4 * (qw + C::QWAVES * vw)) * 256, v_lane[vw] + 16 * n * 256, soff);
+      for (int n = 0; n < BT / SPAN; ++n)
+        dma_load16_lds(vd, vt_lds + (SPAN * n + RPL * (qw + C::QWAVES * vw)) * ROWB, v_lane[vw] + SPAN * n * ROWB, soff);
   };
 
   // MFMA A-operand offsets of K-layout tiles (K, Hbar^T, kbar): row l16 of a 16-row tile,
-  // chunk 4 ks + g4 (features 32 ks + 8 g4 .. + 7), stored at chunk ^ l16.
+  // chunk 4 ks + g4 (features 32 ks + 8 g4 .. + 7).
   int kofs[KS];
 #pragma unroll
-  for (int ks = 0; ks < KS; ++ks) kofs[ks] = l16 * 256 + (((4 * ks + g4) ^ l16) << 4);
+  for (int ks = 0; ks < KS; ++ks) kofs[ks] = l16 * ROWB + (((4 * ks + g4) ^ TL::kx(l16)) << 4);
   // The transposing V reads of 32-key step s: keys 32 s + 16 h2 + 4 g4 + {0..3} (h2 = 0, 1).
   int vofs[DT];
 #pragma unroll
-  for (int dt = 0; dt < DT; ++dt) vofs[dt] = vtile_tr_byte(0, dt, lane);
+  for (int dt = 0; dt < DT; ++dt) vofs[dt] = vtile_tr_byte<D>(0, dt, lane);
 
   int wsel = 0;
   int jall = 0;
@@ -811,7 +462,7 @@ void k4_sparse_attn_dma(const uint16_t* __restrict__ q, const uint16_t* __restri
     for (int ks = 0; ks < KS; ++ks)
 #pragma unroll
       for (int kt = 0; kt < KT; ++kt) {
-        const vec8 a = as_vec8<E>(lds_ld<uint4>(Ks + tile_off, kofs[ks] + kt * 16 * 256));
+        const vec8 a = as_vec8<E>(lds_ld<uint4>(Ks + tile_off, kofs[ks] + kt * 16 * ROWB));
 #pragma unroll
         for (int qt = 0; qt < 2; ++qt) sacc[kt][qt] = E::mfma16(a, qf[qt][ks], sacc[kt][qt]);
       }
@@ -898,8 +549,8 @@ void k4_sparse_attn_dma(const uint16_t* __restrict__ q, const uint16_t* __restri
     for (int s = 0; s < KT / 2; ++s)
 #pragma unroll
       for (int dt = 0; dt < DT; ++dt) {
-        const uint2 lo = lds_read_tr16(Vs + tile_off, vofs[dt] + s * 32 * 256);
-        const uint2 hi = lds_read_tr16(Vs + tile_off, vofs[dt] + s * 32 * 256 + 16 * 256);
+        const uint2 lo = lds_read_tr16(Vs + tile_off, vofs[dt] + s * 32 * ROWB);
+        const uint2 hi = lds_read_tr16(Vs + tile_off, vofs[dt] + s * 32 * ROWB + 16 * ROWB);
         const vec8 a = as_vec8<E>((u32x4_t){lo.x, lo.y, hi.x, hi.y});
 #pragma unroll
         for (int qt = 0; qt < 2; ++qt) oacc[dt][qt] = E::mfma16(a, pf[s][qt], oacc[dt][qt]);
@@ -995,7 +646,7 @@ void k4_sparse_attn_dma(const uint16_t* __restrict__ q, const uint16_t* __restri
     for (int ks = 0; ks < KS; ++ks)
 #pragma unroll
       for (int bt = 0; bt < 2; ++bt) {
-        const vec8 a = as_vec8<E>(lds_ld<uint4>(Vs, PK::KB_OFF + kofs[ks] + bt * 16 * 256));
+        const vec8 a = as_vec8<E>(lds_ld<uint4>(Vs, PK::KB_OFF + kofs[ks] + bt * 16 * ROWB));
 #pragma unroll
         for (int qt = 0; qt < 2; ++qt) sb[bt][qt] = E::mfma16(a, qf[qt][ks], sb[bt][qt]);
       }
@@ -1089,7 +740,7 @@ void k4_sparse_attn_dma(const uint16_t* __restrict__ q, const uint16_t* __restri
     for (int ks = 0; ks < KS; ++ks)
 #pragma unroll
       for (int dt = 0; dt < DT; ++dt) {
-        const vec8 a = as_vec8<E>(lds_ld<uint4>(Ks, kofs[ks] + dt * 16 * 256));
+        const vec8 a = as_vec8<E>(lds_ld<uint4>(Ks, kofs[ks] + dt * 16 * ROWB));
 #pragma unroll
         for (int qt = 0; qt < 2; ++qt) racc[dt][qt] = E::mfma16(a, qf[qt][ks], racc[dt][qt]);
       }
@@ -1124,12 +775,34 @@ void k4_sparse_attn_dma(const uint16_t* __restrict__ q, const uint16_t* __restri
   }
 }
 
+#define PASA_K4_PARAMS                                                                                         \
+  const uint16_t *__restrict__ q, const uint16_t *__restrict__ k, const uint16_t *__restrict__ v,              \
+      const unsigned char *__restrict__ pack, const uint32_t *__restrict__ selmask, uint16_t *__restrict__ o,  \
+      float scale, float c, int T, int NT, int NG, int NW, int xcd_chunk, int gamma_literal, int text,         \
+      int text_valid, int n_text_wg, int nbh, RowMap rm
+#define PASA_K4_ARGS                                                                                        \
+  q, k, v, pack, selmask, o, scale, c, T, NT, NG, NW, xcd_chunk, gamma_literal, text, text_valid, n_text_wg, \
+      nbh, rm
+
+// D = 128: two waves per SIMD (256 VGPRs each), two workgroups of 64 KB of LDS per CU.
+template <int BT, bool ALL, bool PERM, bool PAIR = false, typename E = Bf16>
+__global__ __attribute__((amdgpu_flat_work_group_size(1, 256), amdgpu_waves_per_eu(2, 2)))
+void k4_sparse_attn_dma(PASA_K4_PARAMS) {
+  k4_body<128, BT, ALL, PERM, PAIR, E>(PASA_K4_ARGS);
+}
+
+// D = 64: half the accumulators, operands and tile bytes.
+template <int D, int BT>
+__global__ __attribute__((amdgpu_flat_work_group_size(1, 256), amdgpu_waves_per_eu(2)))
+void k4_sparse_attn(PASA_K4_PARAMS) {
+  k4_body<D, BT, false, false, BT == 64, Bf16>(PASA_K4_ARGS);
+}
+#undef PASA_K4_PARAMS
+#undef PASA_K4_ARGS
+
 size_t k4_pack_bytes(int D, int BT) {
-  if (D == 128 && BT == 128) return K4DPack<128>::BYTES;
-  if (D == 128 && BT == 64) return K4DPack<64>::BYTES;
-  if (D == 64 && BT == 128) return K4Cfg<64, 128>::PK_BYTES;
-  if (D == 64 && BT == 64) return K4Cfg<64, 64>::PK_BYTES;
-  return 0;
+  if (BT != 64 && BT != 128) return 0;
+  return D == 128 ? K4Pack<128>::BYTES : (D == 64 ? K4Pack<64>::BYTES : 0);
 }
 
 hipError_t launch_pack_phase2(const float* kc, const float* vc, const float* hgroup, void* pack,
@@ -1137,25 +810,13 @@ hipError_t launch_pack_phase2(const float* kc, const float* vc, const float* hgr
   const int NT = (T + BT - 1) / BT;
   const int NG = (NT + kGroup - 1) / kGroup;
   dim3 grid(NG, bh);
-  auto out = (unsigned char*)pack;
-  if (f16 && D != 128) return hipErrorInvalidValue;
-  if (D == 128 && BT == 128) {
-    if (f16)
-      hipLaunchKernelGGL((k4_pack_xor<128, F16>), grid, dim3(256), 0, stream, kc, vc, hgroup, out, NT, NG);
-    else
-      hipLaunchKernelGGL((k4_pack_xor<128, Bf16>), grid, dim3(256), 0, stream, kc, vc, hgroup, out, NT, NG);
-  } else if (D == 128 && BT == 64) {
-    if (f16)
-      hipLaunchKernelGGL((k4_pack_xor<64, F16>), grid, dim3(256), 0, stream, kc, vc, hgroup, out, NT, NG);
-    else
-      hipLaunchKernelGGL((k4_pack_xor<64, Bf16>), grid, dim3(256), 0, stream, kc, vc, hgroup, out, NT, NG);
-  } else if (D == 64 && BT == 128)
-    hipLaunchKernelGGL((k4_pack<64, 128>), grid, dim3(256), 0, stream, kc, vc, hgroup, out, NT, NG);
-  else if (D == 64 && BT == 64)
-    hipLaunchKernelGGL((k4_pack<64, 64>), grid, dim3(256), 0, stream, kc, vc, hgroup, out, NT, NG);
-  else
-    return hipErrorInvalidValue;
-  return hipGetLastError();
+  auto go = [&](auto kern) {
+    hipLaunchKernelGGL(kern, grid, dim3(256), 0, stream, kc, vc, hgroup, (unsigned char*)pack, NT, NG);
+    return hipGetLastError();
+  };
+  if ((BT != 64 && BT != 128) || (D != 64 && D != 128) || (f16 && D != 128)) return hipErrorInvalidValue;
+  if (f16) return go(k4_pack_xor<128, F16>);
+  return D == 128 ? go(k4_pack_xor<128, Bf16>) : go(k4_pack_xor<64, Bf16>);
 }
 
 hipError_t launch_sparse_attn(const void* q, const void* k, const void* v, const void* pack,
@@ -1172,22 +833,24 @@ hipError_t launch_sparse_attn(const void* q, const void* k, const void* v, const
   const int text_qtiles = (text_valid + BT - 1) / BT + (text - text_valid + BT - 1) / BT;
   const int n_text_wg = (bh * text_qtiles + 7) / 8 * 8;
   dim3 grid(n_text_wg + 8 * bh * xcd_chunk);
-  dim3 grid_video(8 * bh * xcd_chunk);
   const float c = scale * kLog2e;
   auto a = (const uint16_t*)q;
   auto b = (const uint16_t*)k;
   auto cc = (const uint16_t*)v;
   auto pk = (const unsigned char*)pack;
   auto oo = (uint16_t*)o;
-  // The D = 128 kernels, for either element type.
   auto dma = [&](auto kern, dim3 g, int chunk, int n_text, const RowMap& map) {
     hipLaunchKernelGGL(kern, g, dim3(256), 0, stream, a, b, cc, pk, selmask, oo, scale, c, T, NT, NG, NW, chunk,
                        gamma_literal, text, text_valid, n_text, bh, map);
   };
-  static_assert(K4D<128>::THREADS == 256 && K4D<64, true>::THREADS == 256, "four-wave workgroups");
-#define PASA_K4_LAUNCH(DD, BB)                                                                   \
-  hipLaunchKernelGGL((k4_sparse_attn<DD, BB>), grid_video, dim3(K4Cfg<DD, BB>::THREADS), 0, stream, a, \
-                     b, cc, pk, selmask, oo, scale, c, T, NT, NG, NW, xcd_chunk, gamma_literal)
+  static_assert(K4D<128, 128>::THREADS == 256 && K4D<128, 64, true>::THREADS == 256 &&
+                    K4D<64, 128>::THREADS == 256 && K4D<64, 64, true>::THREADS == 256,
+                "four-wave workgroups");
+  // Query blocks (and text tiles) in pairs at block size 64: each XCD takes a contiguous run of a
+  // slice's pairs.
+  const int pair_chunk = ((NT + 1) / 2 + 7) / 8;
+  const int n_text_pairs = (bh * ((text_qtiles + 1) / 2) + 7) / 8 * 8;
+  const dim3 grid_pairs(n_text_pairs + 8 * bh * pair_chunk);
   if (rm != nullptr) {  // token-major view of frame-major slices: D = 128, BT = 128 only
     if (D != 128 || BT != 128) return hipErrorInvalidValue;
     if (f16)
@@ -1200,23 +863,17 @@ hipError_t launch_sparse_attn(const void* q, const void* k, const void* v, const
     else
       dma(k4_sparse_attn_dma<128, false, false, false, Bf16>, grid, xcd_chunk, n_text_wg, RowMap{});
   } else if (D == 128 && BT == 64) {
-    // Query blocks (and text tiles) in pairs: each XCD takes a contiguous run of a
-    // slice's pairs.
-    const int pair_chunk = ((NT + 1) / 2 + 7) / 8;
-    const int n_text_pairs = (bh * ((text_qtiles + 1) / 2) + 7) / 8 * 8;
-    const dim3 gp(n_text_pairs + 8 * bh * pair_chunk);
     if (f16)
-      dma(k4_sparse_attn_dma<64, false, false, true, F16>, gp, pair_chunk, n_text_pairs, RowMap{});
+      dma(k4_sparse_attn_dma<64, false, false, true, F16>, grid_pairs, pair_chunk, n_text_pairs, RowMap{});
     else
-      dma(k4_sparse_attn_dma<64, false, false, true, Bf16>, gp, pair_chunk, n_text_pairs, RowMap{});
-  }
-  else if (D == 64 && BT == 128)
-    PASA_K4_LAUNCH(64, 128);
-  else if (D == 64 && BT == 64)
-    PASA_K4_LAUNCH(64, 64);
-  else
+      dma(k4_sparse_attn_dma<64, false, false, true, Bf16>, grid_pairs, pair_chunk, n_text_pairs, RowMap{});
+  } else if (D == 64 && BT == 128) {
+    dma(k4_sparse_attn<64, 128>, grid, xcd_chunk, 0, RowMap{});
+  } else if (D == 64 && BT == 64) {
+    dma(k4_sparse_attn<64, 64>, grid_pairs, pair_chunk, 0, RowMap{});
+  } else {
     return hipErrorInvalidValue;
-#undef PASA_K4_LAUNCH
+  }
   return hipGetLastError();
 }
 
@@ -1230,7 +887,7 @@ hipError_t launch_dense_attn(const void* q, const void* k, const void* v, void* 
   const int n_text_wg = (bh * text_qtiles + 7) / 8 * 8;
   dim3 grid(n_text_wg + 8 * bh * xcd_chunk);
   auto launch = [&](auto kern) {
-    hipLaunchKernelGGL(kern, grid, dim3(K4D<BT>::THREADS), 0, stream, (const uint16_t*)q, (const uint16_t*)k,
+    hipLaunchKernelGGL(kern, grid, dim3(K4D<128, BT>::THREADS), 0, stream, (const uint16_t*)q, (const uint16_t*)k,
                        (const uint16_t*)v, nullptr, nullptr, (uint16_t*)o, scale, scale * kLog2e, T, NT, 0, 0,
                        xcd_chunk, 1, text, text_valid, n_text_wg, bh, RowMap{});
   };
