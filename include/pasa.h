@@ -144,9 +144,10 @@ size_t pasa_block_stats_workspace_bytes(int64_t bh, int64_t seq_len, int64_t tex
                                         int64_t head_dim, int64_t block_size, int64_t group_size);
 
 /* The workspace of a pasa_block_stats_ws call for inputs of this dtype: the size above where the
- * tuned kernels run, and for the any-shape kernels (which the size above does not cover) the
- * partial sums of every group that splits.  Those kernels take a workspace of any size, NULL
- * included, and split only as far as it reaches; qc, kc, vc and hnorm do not depend on it. */
+ * tuned head_dim 128 kernels run, and elsewhere (head_dim 64 and the any-shape kernels, which the
+ * size above does not cover) the partial sums of every group that splits.  Those kernels take a
+ * workspace of any size, NULL included, and split only as far as it reaches; qc, kc, vc and hnorm
+ * do not depend on it. */
 size_t pasa_block_stats_workspace_bytes_dtype(int64_t bh, int64_t seq_len, int64_t text_len,
                                               int64_t head_dim, int64_t block_size,
                                               int64_t group_size, int dtype);

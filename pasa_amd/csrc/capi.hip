@@ -240,13 +240,16 @@ static int block_stats_impl(const void* q, const void* k, const void* v, float* 
   if (group_size <= 0 || group_size > 1 << 20) return fail(PASA_ERR_GROUP_SIZE, "group_size %lld must be in [1, 2^20]", (long long)group_size);
   int split = 1;
   if (workspace != nullptr) {
-    split = pasa::block_stats_split((int)bh, (int)(seq_len - text_len), (int)head_dim, (int)block_size,
-                                    (int)group_size);
+    split = pasa::block_stats_split((int)bh, (int)(seq_len - text_len), (int)block_size, (int)group_size);
     const size_t need = pasa_block_stats_workspace_bytes(bh, seq_len, text_len, head_dim, block_size, group_size);
     if (workspace_bytes < need)
       return fail(PASA_ERR_WORKSPACE, "pasa_block_stats_ws: workspace %zu bytes < %zu", workspace_bytes, need);
     if (((uintptr_t)workspace | (uintptr_t)hgroup) & 15u)
       return fail(PASA_ERR_BAD_ARG, "pasa_block_stats_ws: workspace and hgroup must be 16-byte aligned");
+    // Where that size is 0 (head_dim 64) the split goes as far as the workspace reaches.
+    const int64_t ng = cdiv(cdiv(seq_len - text_len, block_size), group_size);
+    const size_t per_part = (size_t)bh * (size_t)ng * (size_t)(head_dim * head_dim) * sizeof(float);
+    while (split > 1 && workspace_bytes / per_part < (size_t)split) split /= 2;
   }
   return launch_status(pasa::launch_block_stats(q, k, v, qc, kc, vc, hnorm, hgroup, (int)bh,
                                                 (int)(seq_len - text_len), (int)seq_len, (int)head_dim,
@@ -262,8 +265,8 @@ size_t pasa_block_stats_workspace_bytes(int64_t bh, int64_t seq_len, int64_t tex
       (head_dim != 64 && head_dim != 128) || (block_size != 64 && block_size != 128) || group_size <= 0 ||
       group_size > 1 << 20)
     return 0;
-  const int split = pasa::block_stats_split((int)bh, (int)(seq_len - text_len), (int)head_dim, (int)block_size,
-                                            (int)group_size);
+  if (head_dim != 128) return 0;
+  const int split = pasa::block_stats_split((int)bh, (int)(seq_len - text_len), (int)block_size, (int)group_size);
   if (split == 1) return 0;
   const int64_t ng = cdiv(cdiv(seq_len - text_len, block_size), group_size);
   return (size_t)bh * (size_t)ng * (size_t)split * (size_t)(head_dim * head_dim) * sizeof(float);
@@ -271,12 +274,15 @@ size_t pasa_block_stats_workspace_bytes(int64_t bh, int64_t seq_len, int64_t tex
 
 size_t pasa_block_stats_workspace_bytes_dtype(int64_t bh, int64_t seq_len, int64_t text_len, int64_t head_dim,
                                               int64_t block_size, int64_t group_size, int dtype) {
-  if (tuned_shape(dtype, head_dim, block_size) && (text_len == 0 || head_dim == 128))
+  const bool tuned = tuned_shape(dtype, head_dim, block_size) && (text_len == 0 || head_dim == 128);
+  if (tuned && head_dim == 128)
     return pasa_block_stats_workspace_bytes(bh, seq_len, text_len, head_dim, block_size, group_size);
   if (check_any_dtype(dtype, "pasa_block_stats") ||
       check_any_shape(bh, seq_len, text_len, head_dim, block_size, group_size, "pasa_block_stats"))
     return 0;
-  const int split = pasa::block_stats_any_split((int)bh, (int)(seq_len - text_len), (int)block_size, (int)group_size);
+  const int split = tuned ? pasa::block_stats_split((int)bh, (int)(seq_len - text_len), (int)block_size, (int)group_size)
+                          : pasa::block_stats_any_split((int)bh, (int)(seq_len - text_len), (int)block_size,
+                                                        (int)group_size);
   if (split == 1) return 0;
   const int64_t ng = cdiv(cdiv(seq_len - text_len, block_size), group_size);
   return (size_t)bh * (size_t)ng * (size_t)split * (size_t)(head_dim * head_dim) * sizeof(float);

@@ -98,9 +98,10 @@ def test_dense_edges(device, T, D, dtype, text, valid, shift):
 
 
 @pytest.mark.parametrize("heads,T,D,BT,G,dtype", [(2, 1024, 64, 64, 32, F32), (1, 777, 37, 16, 50, F16),
-                                                  (3, 1000, 96, 32, 16, B16), (1, 300, 128, 256, 2, F32)])
+                                                  (3, 1000, 96, 32, 16, B16), (1, 300, 128, 256, 2, F32),
+                                                  (2, 3001, 64, 64, 32, B16), (1, 4099, 64, 128, 32, B16)])
 def test_block_stats_split_any(device, heads, T, D, BT, G, dtype):
-    """A group split over several workgroups: the per-block statistics are the unsplit call's bit for
+    """A group split over several workgroups (any-shape kernels and the head_dim 64 ones): the per-block statistics are the unsplit call's bit for
     bit, and the group moment differs by the order of at most G sums (G 2^-24 of the sum of their
     magnitudes).  A workspace smaller than asked for is used as far as it reaches."""
     from pasa_amd import _lib
