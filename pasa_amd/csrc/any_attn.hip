@@ -28,14 +28,15 @@
 // operands of phase 2, which every query block reads in full.  The next chunk's rows load into registers while one is multiplied.
 //
 // What bounds it: in fp32 the MFMA pipe (153 TFLOP/s in a large fp32 matrix product here; 12 heads
-// x 7,800 rows, D 128, block 64: 75 GFLOP in 0.76 ms, where one FMA per lane took 2.07 ms); in 16
-// bits the latency of the staged loads and the LDS operand reads (16 heads x 8,610 rows, D 96,
-// block 32, groups of 16: 149 GFLOP in 0.42 ms, where one FMA per lane took 9.7 ms with half its
-// lanes idle).
+// x 7,800 rows, D 128, block 64: 75 GFLOP in 0.71 ms, each further selected block at 118 TFLOP/s,
+// where one FMA per lane took 2.07 ms); in 16 bits the latency of the staged loads and, in phase 2,
+// of Hbar (16 heads x 8,610 rows, D 96, block 32, groups of 16: 149 GFLOP in 0.35 ms, half of it
+// phase 2, where one FMA per lane took 9.7 ms with half its lanes idle).
 //
-// fp32 sums are taken in short chains (16 features, a chunk of keys, 32 features of Hbar) that
+// fp32 sums are taken in short chains (half the features, a chunk of keys, 32 rows of Hbar) that
 // are then added, because the MFMA rounds after every product: the error against 64 bits is
-// 3.4e-7 (7.3e-7 for the one-FMA-per-lane form) at the fp32 shape above.
+// 5.0e-7 (7.3e-7 for the one-FMA-per-lane form) at the fp32 shape above.  Chains of 16 features
+// give 3.4e-7 and are 8% slower (their additions wait for the MFMA).
 #include <initializer_list>
 #include <type_traits>
 
@@ -73,7 +74,7 @@ struct AnyCfg {
   static constexpr int NF = DP * ES / 64;  // 64-byte feature steps per row: one fragment each
   static constexpr int DT = DP / 16;       // 16-feature tiles of O
   // Keys per chunk: about 16 KB of K and of V per team (8 KB where each wave stages its own).
-  static constexpr int KC = TEAM == 1 ? (F32 ? 16 : 32) : (F32 && DP > 64 ? 32 : 64);
+  static constexpr int KC = TEAM == 1 ? (F32 ? 16 : 32) : 64;
   // Row strides.  K: an odd number of 16-byte chunks, so that 16 rows read at one chunk touch 16
   // distinct bank groups.  V in 16 bits: twice an odd number of chunks, so that the 8 rows x 32
   // bytes half a wave transposes do; in fp32 4 rows x 64 bytes, four rows apart, already do.
@@ -250,7 +251,7 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2))) void k
   auto step = [&](const unsigned char* Kb, const unsigned char* Vb, auto ktn, auto mask, auto on_rescale,
                   auto add) __attribute__((always_inline)) {
     constexpr int KTN = decltype(ktn)::value;
-    f32x4_t s[KTN][QT];
+    f32x4_t s[KTN][QT], sb[F32 ? KTN : 1][QT];
 #pragma unroll
     for (int f = 0; f < NF; ++f)
 #pragma unroll
@@ -258,11 +259,12 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2))) void k
         const frag a = lds_ld<frag>(Kb, (kt * 16 + l16) * KROW + f * 64 + g4 * 16);
 #pragma unroll
         for (int qt = 0; qt < QT; ++qt) {
-          if constexpr (F32) {  // 16-feature chains, added: shorter fp32 chains round less
-            f32x4_t t = {0.f, 0.f, 0.f, 0.f};
+          if constexpr (F32) {  // chains of half the features, added: shorter fp32 chains round less
+            f32x4_t& t = f < NF / 2 ? s[kt][qt] : sb[kt][qt];
+            if (f == 0 || f == NF / 2) t = (f32x4_t){0.f, 0.f, 0.f, 0.f};
 #pragma unroll
             for (int i = 0; i < 4; ++i) t = __builtin_amdgcn_mfma_f32_16x16x4f32(a[i], qf[qt][f][i], t, 0, 0, 0);
-            s[kt][qt] = f == 0 ? t : s[kt][qt] + t;
+            if (f == NF - 1) s[kt][qt] += t;
           } else {
             if (f == 0) s[kt][qt] = (f32x4_t){0.f, 0.f, 0.f, 0.f};
             s[kt][qt] = E::M::mfma16(a, qf[qt][f], s[kt][qt]);
@@ -389,7 +391,7 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2))) void k
       int n = min(KC, j1 - j0);
       j0 += n;
       rb = ra + 16;
-      if (TEAM == 1 && KC == 32 && BT == 16 && !tail && n == 16 && next_block()) {
+      if (TEAM == 1 && KC == 32 && RW == 16 && BT == 16 && !tail && n == 16 && next_block()) {
         rb = j0;
         n += j1 - j0;
         j0 = j1;
@@ -400,7 +402,7 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2))) void k
     // Rows r of a chunk: ra + r, and rb + r - 16 from row 16 on where each wave stages its own.
     const uint32_t lane_off = in_row ? (uint32_t)(sr * (int)row_bytes + sc * 16) : kOutside;
     auto fetch = [&](int ra, int rb, int n) {
-      constexpr int SPLIT = TEAM == 1 && KC == 32 ? 16 : KC;
+      constexpr int SPLIT = TEAM == 1 && KC == 32 && RW == 16 ? 16 : KC;  // 32-row blocks (RW 32) fill a chunk
       const int na = min(n, SPLIT), nb = n - na;
       const unsigned char* base_k[2] = {ksl + (int64_t)ra * row_bytes, ksl + (int64_t)rb * row_bytes};
       const unsigned char* base_v[2] = {vsl + (int64_t)ra * row_bytes, vsl + (int64_t)rb * row_bytes};
@@ -521,65 +523,103 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2))) void k
         return make_float4(__uint_as_float(x.x), __uint_as_float(x.y), __uint_as_float(x.z), __uint_as_float(x.w));
       }
     };
-    auto stage_z = [&](int jc, int cn) {
+    // Work items in order: a group's zero-order chunks of 32 blocks (the first one brings Hbar's
+    // first HR rows along), then the rest of its Hbar HR rows at a time.  In 16 bits the next item's
+    // rows load into registers while one is computed (430 -> 391 us at the bf16 shape above); fp32,
+    // bound by its MFMAs, is 2% slower with that.
+    int ig = -1, ijc = 0, ihs = 0;
+    auto group_end = [&](int g) -> int { return (int)min((int64_t)NT, (int64_t)(g + 1) * G); };
+    auto chunk_from = [&](int g, int jc) -> bool {  // the group's first chunk at or after jc with work
+      for (const int jb = group_end(g); jc < jb; jc += C::KZ)
+        if (any_unselected(jc, min(jc + C::KZ, jb))) {
+          ijc = jc;
+          return true;
+        }
+      return false;
+    };
+    auto next_item = [&]() -> bool {
+      if (ig >= 0) {
+        if (ihs == 0 && chunk_from(ig, ijc + C::KZ)) return true;
+        if ((ihs + 1) * C::HR < D) {
+          ++ihs;
+          return true;
+        }
+      }
+      ihs = 0;
+      while (++ig < NG)
+        if (chunk_from(ig, ig * G)) return true;
+      return false;
+    };
+    constexpr int ZP = C::KZ / C::RPP4, HP = C::HR / C::RPP4;
+    float4 zk[ZP], zv[ZP], hx[HP];
+    auto fetch_h = [&](int g, int hs) {
+      const int n = min(C::HR, D - hs * C::HR);
+      const float* hb = hgroup + ((int64_t)bh * NG + g) * D * D + (int64_t)hs * C::HR * D;
+      const rsrc_t rh = make_rsrc(hb, (uint32_t)(n * D * 4));
+#pragma unroll
+      for (int p = 0; p < HP; ++p) hx[p] = load4(hb, rh, p * C::RPP4, n);
+    };
+    auto fetch_z = [&](int jc, int cn) {
       const float* kb = kcb + (int64_t)jc * D;
       const float* vb = vcb + (int64_t)jc * D;
       const rsrc_t rk = make_rsrc(kb, (uint32_t)(cn * D * 4)), rv = make_rsrc(vb, (uint32_t)(cn * D * 4));
-      float4 xk[C::KZ / C::RPP4], xv[C::KZ / C::RPP4];
 #pragma unroll
-      for (int p = 0; p < C::KZ / C::RPP4; ++p) {
-        xk[p] = load4(kb, rk, p * C::RPP4, cn);
-        xv[p] = load4(vb, rv, p * C::RPP4, cn);
-      }
-      if (c4 < C::C4) {
-#pragma unroll
-        for (int p = 0; p < C::KZ / C::RPP4; ++p) {
-          const int r = p * C::RPP4 + r4;
-          st4(Kz, r * KROW + (c4 >> 3) * 64 + (c4 & 3) * 16 + ((c4 >> 2) & 1) * 8, r * KROW + c4 * 16, xk[p]);
-          st4(Vz, r * VROW + c4 * 8, r * VROW + c4 * 16, xv[p]);
-        }
+      for (int p = 0; p < ZP; ++p) {
+        zk[p] = load4(kb, rk, p * C::RPP4, cn);
+        zv[p] = load4(vb, rv, p * C::RPP4, cn);
       }
     };
-    auto stage_h = [&](const float* hg, int d0) {
-      const int n = min(C::HR, D - d0);
-      const float* hb = hg + (int64_t)d0 * D;
-      const rsrc_t rh = make_rsrc(hb, (uint32_t)(n * D * 4));
-      constexpr int HP = C::HR / C::RPP4, HB = HP < 8 ? HP : 8;  // passes, and passes in flight
+    auto stash_h = [&]() {
+      if (c4 >= C::C4) return;
 #pragma unroll
-      for (int p0 = 0; p0 < HP; p0 += HB) {
-        float4 x[HB];
-#pragma unroll
-        for (int p = 0; p < HB; ++p) x[p] = load4(hb, rh, (p0 + p) * C::RPP4, n);
-        if (c4 < C::C4) {
-#pragma unroll
-          for (int p = 0; p < HB; ++p) {
-            const int r = (p0 + p) * C::RPP4 + r4;
-            st4(Hs, r * VROW + c4 * 8, r * VROW + c4 * 16, x[p]);
-          }
-        }
+      for (int p = 0; p < HP; ++p) {
+        const int r = p * C::RPP4 + r4;
+        st4(Hs, r * VROW + c4 * 8, r * VROW + c4 * 16, hx[p]);
       }
     };
-    for (int g = 0; g < NG; ++g) {
-      const int ja = g * G;
-      const int jb = min((int64_t)NT, (int64_t)ja + G);
-      if (!any_unselected(ja, jb)) continue;  // nothing approximated: no contribution
-      const float* hg = hgroup + ((int64_t)bh * NG + g) * D * D;
-      // Zero order, 32 blocks at a time: o += p V^, and per row the sums of p and of p times the
-      // block's length, kept relative to the running max until the group ends (Gamma itself is
-      // rescaled only in the consistent form, :231-235).
-      float psum[QT], gsum[QT];
+    auto stash_z = [&]() {
+      if (c4 >= C::C4) return;
 #pragma unroll
-      for (int qt = 0; qt < QT; ++qt) psum[qt] = gsum[qt] = 0.f;
-      bool h_staged = false;
-      for (int jc = ja; jc < jb; jc += C::KZ) {
-        const int cn = min(C::KZ, jb - jc);
-        if (!any_unselected(jc, jc + cn)) continue;
-        __syncthreads();  // the previous operands have been read
-        stage_z(jc, cn);
-        if (!h_staged) stage_h(hg, 0);
-        h_staged = true;
-        __syncthreads();
-        const uint32_t ub = approx_bits(jc, cn) >> (4 * g4);
+      for (int p = 0; p < ZP; ++p) {
+        const int r = p * C::RPP4 + r4;
+        st4(Kz, r * KROW + (c4 >> 3) * 64 + (c4 & 3) * 16 + ((c4 >> 2) & 1) * 8, r * KROW + c4 * 16, zk[p]);
+        st4(Vz, r * VROW + c4 * 8, r * VROW + c4 * 16, zv[p]);
+      }
+    };
+    // Per row, of the current group: the sums of p and of p times the block's length, relative to
+    // the running max until the group ends (Gamma itself is rescaled only in the consistent form,
+    // :231-235), then f = scale * (sum of p).
+    float psum[QT], gsum[QT], f[QT];
+    int pg = -1;  // the group of the previous item
+    bool more = next_item();
+    if (more && !F32) {
+      fetch_z(ijc, min(C::KZ, group_end(ig) - ijc));
+      fetch_h(ig, 0);
+    }
+    while (more) {
+      const int g = ig, jc = ijc, hs = ihs;
+      const bool first = g != pg;
+      pg = g;
+      __syncthreads();  // the previous item's rows have been read
+      if (F32) {
+        if (hs == 0) fetch_z(jc, min(C::KZ, group_end(g) - jc));
+        if (hs > 0 || first) fetch_h(g, hs);
+      }
+      if (hs == 0) stash_z();
+      if (hs > 0 || first) stash_h();
+      __syncthreads();
+      more = next_item();
+      if (more && !F32) {
+        if (ihs == 0) fetch_z(ijc, min(C::KZ, group_end(ig) - ijc));
+        if (ihs > 0 || ig != g) fetch_h(ig, ihs);
+      }
+      if (hs == 0) {
+        if (first) {
+#pragma unroll
+          for (int qt = 0; qt < QT; ++qt) psum[qt] = gsum[qt] = 0.f;
+        }
+        // Zero order: o += p V^.
+        const uint32_t ub = approx_bits(jc, min(C::KZ, group_end(g) - jc)) >> (4 * g4);
         const int last = NT - 1 - jc - 4 * g4;  // this lane's key index of the last block
         step(Kz, Vz, std::integral_constant<int, C::KZ / 16>{},
              [&](auto& s) {
@@ -600,23 +640,18 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2))) void k
                psum[qt] += p;
                gsum[qt] += p * (float)(key == last ? last_len : BT);
              });
-      }
-      // First order: o += scale * (sum of p) * (q . Hbar).
-      float f[QT];
+        if (more && ig == g && ihs == 0) continue;  // another chunk of this group
 #pragma unroll
-      for (int qt = 0; qt < QT; ++qt) {
-        g_run[qt] += gsum[qt];
-        f[qt] = quad16_sum(psum[qt]) * scale;
-      }
-#pragma unroll
-      for (int hs = 0; hs < DP / C::HR; ++hs) {
-        if (hs > 0) {
-          if (hs * C::HR >= D) break;
-          __syncthreads();
-          stage_h(hg, hs * C::HR);
-          __syncthreads();
+        for (int qt = 0; qt < QT; ++qt) {
+          g_run[qt] += gsum[qt];
+          f[qt] = quad16_sum(psum[qt]) * scale;
         }
-        if constexpr (F32) {
+      }
+      // First order: o += f (q . Hbar), over this item's rows of Hbar.
+      if constexpr (F32) {
+#pragma unroll
+        for (int h = 0; h < DP / C::HR; ++h) {
+          if (h != hs) continue;
 #pragma unroll
           for (int d2 = 0; d2 < DT; d2 += 2) {
             f32x4_t r[2][QT];
@@ -633,7 +668,7 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2))) void k
                   const float a = vt32(Hs, 16 * cc + i, d2 + j);
 #pragma unroll
                   for (int qt = 0; qt < QT; ++qt)
-                    r[j][qt] = __builtin_amdgcn_mfma_f32_16x16x4f32(a, qf[qt][hs * (C::HR / 16) + cc][i], r[j][qt], 0,
+                    r[j][qt] = __builtin_amdgcn_mfma_f32_16x16x4f32(a, qf[qt][h * (C::HR / 16) + cc][i], r[j][qt], 0,
                                                                     0, 0);
                 }
 #pragma unroll
@@ -643,23 +678,23 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2))) void k
 #pragma unroll
                 for (int i = 0; i < 4; ++i) oacc[d2 + j][qt][i] = fmaf(r[j][qt][i], f[qt], oacc[d2 + j][qt][i]);
           }
-        } else {
+        }
+      } else {
 #pragma unroll
-          for (int dt = 0; dt < DT; ++dt) {
-            f32x4_t r[QT];
+        for (int dt = 0; dt < DT; ++dt) {
+          f32x4_t r[QT];
 #pragma unroll
-            for (int qt = 0; qt < QT; ++qt) r[qt] = (f32x4_t){0.f, 0.f, 0.f, 0.f};
+          for (int qt = 0; qt < QT; ++qt) r[qt] = (f32x4_t){0.f, 0.f, 0.f, 0.f};
 #pragma unroll
-            for (int s2 = 0; s2 < NF; ++s2) {
-              const frag a = vt16(Hs, s2, dt);
+          for (int s2 = 0; s2 < NF; ++s2) {
+            const frag a = vt16(Hs, s2, dt);
 #pragma unroll
-              for (int qt = 0; qt < QT; ++qt) r[qt] = E::M::mfma16(a, qf[qt][s2], r[qt]);
-            }
-#pragma unroll
-            for (int qt = 0; qt < QT; ++qt)
-#pragma unroll
-              for (int i = 0; i < 4; ++i) oacc[dt][qt][i] = fmaf(r[qt][i], f[qt], oacc[dt][qt][i]);
+            for (int qt = 0; qt < QT; ++qt) r[qt] = E::M::mfma16(a, qf[qt][s2], r[qt]);
           }
+#pragma unroll
+          for (int qt = 0; qt < QT; ++qt)
+#pragma unroll
+            for (int i = 0; i < 4; ++i) oacc[dt][qt][i] = fmaf(r[qt][i], f[qt], oacc[dt][qt][i]);
         }
       }
     }
