@@ -318,6 +318,14 @@ int pasa_dense_attn(const void* q, const void* k, const void* v, void* o, double
                     int64_t bh, int64_t seq_len, int64_t text_len, int64_t text_valid,
                     int64_t head_dim, int dtype, void* stream);
 
+/* Dense attention of q [BH, q_len, D] to k, v [BH, kv_len, D] with o token-major,
+ * [BH / heads, q_len, heads, D]; bf16 or fp16 at head_dim 128.  q_len == kv_len: pasa_dense_attn
+ * (text segment included); else every query row attends to all kv_len keys (the text
+ * cross-attention of svg/models/wan/attention.py:218-221) and text_len must be 0. */
+int pasa_dense_attn_bshd(const void* q, const void* k, const void* v, void* o, double scale, int64_t bh,
+                         int64_t heads, int64_t q_len, int64_t kv_len, int64_t text_len, int64_t text_valid,
+                         int64_t head_dim, int dtype, void* stream);
+
 /* ---- Processor prologue (K5) ------------------------------------------------ */
 
 typedef enum {

@@ -78,6 +78,7 @@ SIGNATURES = {
                                        _i64, _i64, _i64, _pl, _int, _vp, _sz, _vp]),
     "pasa_sparse_attn_packed_placed": (_int, [_vp, _vp, _vp, _vp, _sz, _vp, _vp, _vp, _dbl, _i64, _i64, _i64,
                                               _i64, _i64, _i64, _i64, _i64, _int, _pl, _int, _vp]),
+    "pasa_dense_attn_bshd": (_int, [_vp, _vp, _vp, _vp, _dbl, _i64, _i64, _i64, _i64, _i64, _i64, _i64, _int, _vp]),
     "pasa_dense_attn": (_int, [_vp, _vp, _vp, _vp, _dbl, _i64, _i64, _i64, _i64, _i64, _int, _vp]),
     "pasa_qkv_prologue": (_int, [_vp, _vp, _vp, _vp, _vp, _vp, _vp, _vp, _i64, _i64, _i64, _i64, _int, _int,
                                  _i64, _i64, _int, _int, _dbl, _vp, _vp, _int, _i64, _int, _vp]),

@@ -521,6 +521,12 @@ static int sparse_attn_packed_impl(const void* q, const void* k, const void* v, 
                        "pasa_sparse_attn");
 }
 
+static int check_o_heads(int64_t heads, int64_t bh) {
+  if (heads < 1 || bh < 1 || bh % heads != 0)
+    return fail(PASA_ERR_BAD_SHAPE, "heads=%lld must divide bh=%lld", (long long)heads, (long long)bh);
+  return PASA_OK;
+}
+
 int pasa_sparse_attn_packed(const void* q, const void* k, const void* v, const void* pack, size_t pack_bytes,
                             const int32_t* idx, const uint32_t* selmask, void* o, double scale, int64_t bh,
                             int64_t seq_len, int64_t text_len, int64_t text_valid, int64_t head_dim,
@@ -687,9 +693,40 @@ int pasa_dense_attn(const void* q, const void* k, const void* v, void* o, double
   const int64_t grid = 8 * bh * cdiv(cdiv(seq_len - text_len, 128), 8) + 8 * cdiv(bh * (cdiv(text_len, 128) + 1), 8);
   if (grid > kMaxI32) return fail(PASA_ERR_OVERFLOW, "grid too large");
   return launch_status(pasa::launch_dense_attn(q, k, v, o, (float)scale, (int)bh, (int)(seq_len - text_len),
-                                               (int)text_len, (int)text_valid, dtype == PASA_DTYPE_F16,
+                                               (int)text_len, (int)text_valid, 0, dtype == PASA_DTYPE_F16,
                                                (hipStream_t)stream),
                        "pasa_dense_attn");
+}
+
+int pasa_dense_attn_bshd(const void* q, const void* k, const void* v, void* o, double scale, int64_t bh,
+                         int64_t heads, int64_t q_len, int64_t kv_len, int64_t text_len, int64_t text_valid,
+                         int64_t head_dim, int dtype, void* stream) {
+  if (!q || !k || !v || !o) return fail(PASA_ERR_NULL_POINTER, "pasa_dense_attn_bshd: NULL pointer");
+  int rc;
+  if (head_dim != 128) return fail(PASA_ERR_HEAD_DIM, "pasa_dense_attn_bshd: head_dim %lld is not 128", (long long)head_dim);
+  if ((rc = check_attn_dtype(dtype, head_dim, "pasa_dense_attn_bshd"))) return rc;
+  if ((rc = check_o_heads(heads, bh))) return rc;
+  if ((rc = check_bh_seq(bh, q_len, head_dim)) || (rc = check_bh_seq(bh, kv_len, head_dim))) return rc;
+  if ((rc = check_slice_bytes(q_len, head_dim, 2)) || (rc = check_slice_bytes(kv_len, head_dim, 2))) return rc;
+  if (!std::isfinite(scale) || !(scale > 0.0)) return fail(PASA_ERR_BAD_ARG, "scale must be finite and > 0");
+  const bool f16 = dtype == PASA_DTYPE_F16;
+  if (q_len != kv_len) {
+    if (text_len != 0 || text_valid != 0)
+      return fail(PASA_ERR_TEXT_SEGMENT, "a text segment needs q_len == kv_len");
+    if (8 * bh * cdiv(cdiv(q_len, 128), 8) > kMaxI32) return fail(PASA_ERR_OVERFLOW, "grid too large");
+    return launch_status(pasa::launch_cross_attn(q, k, v, o, (float)scale, (int)bh, (int)q_len, (int)kv_len,
+                                                 (int)heads, f16, (hipStream_t)stream),
+                         "pasa_dense_attn_bshd");
+  }
+  if ((rc = check_text(q_len, text_len, head_dim))) return rc;
+  if (text_valid < 0 || text_valid > text_len)
+    return fail(PASA_ERR_TEXT_SEGMENT, "text_valid=%lld must be in [0, text_len=%lld]", (long long)text_valid,
+                (long long)text_len);
+  const int64_t grid = 8 * bh * cdiv(cdiv(q_len - text_len, 128), 8) + 8 * cdiv(bh * (cdiv(text_len, 128) + 1), 8);
+  if (grid > kMaxI32) return fail(PASA_ERR_OVERFLOW, "grid too large");
+  return launch_status(pasa::launch_dense_attn(q, k, v, o, (float)scale, (int)bh, (int)(q_len - text_len),
+                                               (int)text_len, (int)text_valid, (int)heads, f16, (hipStream_t)stream),
+                       "pasa_dense_attn_bshd");
 }
 
 int pasa_qkv_prologue(const void* xq, const void* xk, const void* xv, void* q, void* k, void* v,

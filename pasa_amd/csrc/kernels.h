@@ -53,9 +53,12 @@ hipError_t launch_sparse_attn(const void* q, const void* k, const void* v, const
 // Dense softmax attention with K4's phase-1 machinery (every key block exact, no
 // selection, no correction), D = 128.  T video rows, then `text` rows of which the
 // first text_valid are the prompt: rows attend within [0, T + text_valid) or within
-// the padding [T + text_valid, T + text).
+// the padding [T + text_valid, T + text).  o_heads: 0, or o is token-major, [batch, row, o_heads, D].
 hipError_t launch_dense_attn(const void* q, const void* k, const void* v, void* o, float scale, int bh,
-                             int T, int text, int text_valid, bool f16, hipStream_t stream);
+                             int T, int text, int text_valid, int o_heads, bool f16, hipStream_t stream);
+// ... of q_len query rows to kv_len key rows per slice.
+hipError_t launch_cross_attn(const void* q, const void* k, const void* v, void* o, float scale, int bh, int q_len,
+                             int kv_len, int o_heads, bool f16, hipStream_t stream);
 
 // ---- any-shape path (any_shape.hip) ----------------------------------------------
 // fp32, bf16 or fp16 q, k, v (dtype: kAnyBf16 / kAnyF16 / kAnyF32, the pasa_dtype_t

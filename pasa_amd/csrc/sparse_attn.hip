@@ -222,12 +222,18 @@ constexpr int kSchedDsRead = 0x100;
 // either block approximates; a group the other block approximates and this one
 // does not adds exact zeros here (p = 0, alpha = 1), so each block's result is the
 // one the unpaired kernel computes.
-template <int D, int BT, bool ALL, bool PERM, bool PAIR, typename E>
+// CROSS (with ALL): the slices of q and o have q_len rows, those of k and v T; the query tiles
+// cover q's rows and each visits all of k's.
+// o_heads: 0, o is [slice, row, D] as q; else o is [batch, row, head, D] with o_heads heads, the
+// layout the projection after the attention reads.
+template <int D, int BT, bool ALL, bool PERM, bool PAIR, typename E, bool CROSS = false>
 __device__ __forceinline__ void k4_body(const uint16_t* __restrict__ q, const uint16_t* __restrict__ k,
                                         const uint16_t* __restrict__ v, const unsigned char* __restrict__ pack,
                                         const uint32_t* __restrict__ selmask, uint16_t* __restrict__ o, float scale,
                                         float c, int T, int NT, int NG, int NW, int xcd_chunk, int gamma_literal,
-                                        int text, int text_valid, int n_text_wg, int nbh, const RowMap& rm) {
+                                        int text, int text_valid, int n_text_wg, int nbh, int o_heads, int q_len,
+                                        const RowMap& rm) {
+  static_assert(!CROSS || (ALL && !PERM), "separate key rows: dense attention only");
   static_assert(!PAIR || (!ALL && !PERM), "pairs run selected video blocks only");
   constexpr bool all_tiles = ALL;
   using C = K4D<D, BT, PAIR>;
@@ -287,11 +293,12 @@ __device__ __forceinline__ void k4_body(const uint16_t* __restrict__ q, const ui
     const int slot = w >> 3;
     bh = slot / xcd_chunk;
     qb = (xcd * xcd_chunk + (slot - bh * xcd_chunk)) * C::QBLOCKS;
-    if (qb >= NT) return;
-    store_rows = qb + half < NT;
+    const int nq = CROSS ? (q_len + BT - 1) / BT : NT;
+    if (qb >= nq) return;
+    store_rows = qb + half < nq;
     qbw = qb + (store_rows ? half : 0);
     qrow0 = qbw * BT;
-    row_limit = T;
+    row_limit = CROSS ? q_len : T;
   }
 
   const int l16 = lane & 15;  // query row within a 16-row query tile; A-operand row
@@ -309,7 +316,8 @@ __device__ __forceinline__ void k4_body(const uint16_t* __restrict__ q, const ui
   }
 
   const uint32_t slice_bytes = (uint32_t)Ttot * D * 2u;
-  const rsrc_t qr = make_rsrc(q + slice, slice_bytes);
+  const int q_rows = CROSS ? q_len : Ttot;
+  const rsrc_t qr = make_rsrc(q + (int64_t)bh * q_rows * D, (uint32_t)q_rows * D * 2u);
   // Q as B operands: qf[qt][ks] holds features 32 ks + 8 g4 .. + 7 of row qrow[qt].
   vec8 qf[2][KS];
 #pragma unroll
@@ -758,12 +766,16 @@ __device__ __forceinline__ void k4_body(const uint16_t* __restrict__ q, const ui
     g = gn;
   }
 
+  const int ob = o_heads > 0 ? bh / o_heads : bh;  // o's rows are o_heads (or one) rows of D apart
+  const int on = o_heads > 0 ? o_heads : 1;
+  uint16_t* const oslice = o + ((int64_t)ob * q_rows * on + (bh - ob * on)) * D;
+  const int ostride = on * D;
   // O = A / (L + Gamma): one correctly rounded reciprocal per row, then products.
 #pragma unroll
   for (int qt = 0; qt < 2; ++qt) {
     const float inv = 1.f / (quad16_sum(l_run[qt]) + quad16_sum(g_run[qt]));
     if (store_rows && qrow[qt] < row_limit) {
-      uint16_t* orow = o + slice + (int64_t)qrow_st[qt] * D;
+      uint16_t* orow = oslice + (int64_t)qrow_st[qt] * ostride;
 #pragma unroll
       for (int dt = 0; dt < DT; ++dt) {
         uint2 w;
@@ -779,16 +791,24 @@ __device__ __forceinline__ void k4_body(const uint16_t* __restrict__ q, const ui
   const uint16_t *__restrict__ q, const uint16_t *__restrict__ k, const uint16_t *__restrict__ v,              \
       const unsigned char *__restrict__ pack, const uint32_t *__restrict__ selmask, uint16_t *__restrict__ o,  \
       float scale, float c, int T, int NT, int NG, int NW, int xcd_chunk, int gamma_literal, int text,         \
-      int text_valid, int n_text_wg, int nbh, RowMap rm
+      int text_valid, int n_text_wg, int nbh, int o_heads, int q_len, RowMap rm
 #define PASA_K4_ARGS                                                                                        \
   q, k, v, pack, selmask, o, scale, c, T, NT, NG, NW, xcd_chunk, gamma_literal, text, text_valid, n_text_wg, \
-      nbh, rm
+      nbh, o_heads, q_len, rm
 
 // D = 128: two waves per SIMD (256 VGPRs each), two workgroups of 64 KB of LDS per CU.
 template <int BT, bool ALL, bool PERM, bool PAIR = false, typename E = Bf16>
 __global__ __attribute__((amdgpu_flat_work_group_size(1, 256), amdgpu_waves_per_eu(2, 2)))
 void k4_sparse_attn_dma(PASA_K4_PARAMS) {
   k4_body<128, BT, ALL, PERM, PAIR, E>(PASA_K4_ARGS);
+}
+
+// Dense attention of q_len query rows to T key rows per slice (the text cross-attention of a DiT
+// block).  32,760 x 512 at 12 heads: 128 us, where PyTorch's SDPA takes 244.
+template <typename E>
+__global__ __attribute__((amdgpu_flat_work_group_size(1, 256), amdgpu_waves_per_eu(2, 2)))
+void k4_cross_attn(PASA_K4_PARAMS) {
+  k4_body<128, 128, true, false, false, E, true>(PASA_K4_ARGS);
 }
 
 // D = 64: half the accumulators, operands and tile bytes.
@@ -841,7 +861,7 @@ hipError_t launch_sparse_attn(const void* q, const void* k, const void* v, const
   auto oo = (uint16_t*)o;
   auto dma = [&](auto kern, dim3 g, int chunk, int n_text, const RowMap& map) {
     hipLaunchKernelGGL(kern, g, dim3(256), 0, stream, a, b, cc, pk, selmask, oo, scale, c, T, NT, NG, NW, chunk,
-                       gamma_literal, text, text_valid, n_text, bh, map);
+                       gamma_literal, text, text_valid, n_text, bh, 0, 0, map);
   };
   static_assert(K4D<128, 128>::THREADS == 256 && K4D<128, 64, true>::THREADS == 256 &&
                     K4D<64, 128>::THREADS == 256 && K4D<64, 64, true>::THREADS == 256,
@@ -878,7 +898,7 @@ hipError_t launch_sparse_attn(const void* q, const void* k, const void* v, const
 }
 
 hipError_t launch_dense_attn(const void* q, const void* k, const void* v, void* o, float scale, int bh,
-                             int T, int text, int text_valid, bool f16, hipStream_t stream) {
+                             int T, int text, int text_valid, int o_heads, bool f16, hipStream_t stream) {
   constexpr int BT = 128;
   if (T < 1 || text < 0 || text_valid < 0 || text_valid > text) return hipErrorInvalidValue;
   const int NT = (T + BT - 1) / BT;
@@ -889,12 +909,29 @@ hipError_t launch_dense_attn(const void* q, const void* k, const void* v, void* 
   auto launch = [&](auto kern) {
     hipLaunchKernelGGL(kern, grid, dim3(K4D<128, BT>::THREADS), 0, stream, (const uint16_t*)q, (const uint16_t*)k,
                        (const uint16_t*)v, nullptr, nullptr, (uint16_t*)o, scale, scale * kLog2e, T, NT, 0, 0,
-                       xcd_chunk, 1, text, text_valid, n_text_wg, bh, RowMap{});
+                       xcd_chunk, 1, text, text_valid, n_text_wg, bh, o_heads, 0, RowMap{});
   };
   if (f16)
     launch(k4_sparse_attn_dma<BT, true, false, false, F16>);
   else
     launch(k4_sparse_attn_dma<BT, true, false, false, Bf16>);
+  return hipGetLastError();
+}
+
+hipError_t launch_cross_attn(const void* q, const void* k, const void* v, void* o, float scale, int bh, int q_len,
+                             int kv_len, int o_heads, bool f16, hipStream_t stream) {
+  constexpr int BT = 128;
+  if (q_len < 1 || kv_len < 1) return hipErrorInvalidValue;
+  const int xcd_chunk = ((q_len + BT - 1) / BT + 7) / 8;
+  auto launch = [&](auto kern) {
+    hipLaunchKernelGGL(kern, dim3(8 * bh * xcd_chunk), dim3(K4D<128, BT>::THREADS), 0, stream, (const uint16_t*)q,
+                       (const uint16_t*)k, (const uint16_t*)v, nullptr, nullptr, (uint16_t*)o, scale, scale * kLog2e,
+                       kv_len, (kv_len + BT - 1) / BT, 0, 0, xcd_chunk, 1, 0, 0, 0, bh, o_heads, q_len, RowMap{});
+  };
+  if (f16)
+    launch(k4_cross_attn<F16>);
+  else
+    launch(k4_cross_attn<Bf16>);
   return hipGetLastError();
 }
 

@@ -251,6 +251,14 @@ def pack_phase2(q: torch.Tensor, stats: BlockStats, block_size: int = 64, text_t
     return pack
 
 
+def _token_major(q: torch.Tensor, out: Optional[torch.Tensor]) -> torch.Tensor:
+    """A new [B, H, T, D] output whose memory is [B, T, H, D] (the kernels' token-major store)."""
+    if out is not None:
+        raise ValueError("token_major_out allocates its output: out must be None")
+    B, H, T, D = q.shape
+    return torch.empty(B, T, H, D, device=q.device, dtype=q.dtype).transpose(1, 2)
+
+
 def _check_out(v: torch.Tensor, out: Optional[torch.Tensor]) -> torch.Tensor:
     """The output buffer: a new tensor like ``v``, or ``out`` if it matches ``v`` exactly
     (the kernels store every row of it without bounds checks)."""
@@ -374,20 +382,43 @@ def sparse_attn_noalloc(q: torch.Tensor, k: torch.Tensor, v: torch.Tensor, stats
 
 def dense_attention(q: torch.Tensor, k: torch.Tensor, v: torch.Tensor, scale: Optional[float] = None,
                     text_tokens: int = 0, text_valid: Optional[int] = None,
-                    out: Optional[torch.Tensor] = None) -> torch.Tensor:
+                    out: Optional[torch.Tensor] = None, token_major_out: bool = False) -> torch.Tensor:
     """Dense softmax attention on K4's exact-tile path (bf16 or fp16 at head_dim 128; fp32 and
     other head dims up to 128 on the any-shape kernel), for the processors' warm-up layers (reference flash_attention, svg/models/wan/attention.py:299-301,
     svg/models/hyvideo/attention.py:459-476).  With ``text_tokens`` / ``text_valid``
     the attention is block-diagonal over [0, T - text_tokens + text_valid) and the
-    rest (the dense HunyuanVideo path's cu_seqlens).  q, k, v: [B, H, T, D]."""
+    rest (the dense HunyuanVideo path's cu_seqlens).  q, k, v: [B, H, T, D].
+    ``token_major_out``: the output's memory is [B, T, H, D] (bf16 or fp16 at head_dim 128), so
+    that o.transpose(1, 2).flatten(2, 3), the output projection's input, is a view."""
     _check_qkv(q, k, v)
     _check_device(q, k, v)
     B, H, T, D = q.shape
     scale = D ** -0.5 if scale is None else scale
-    o = _check_out(v, out)
     tv = text_tokens if text_valid is None else text_valid
+    if token_major_out and D == 128 and q.dtype in (torch.bfloat16, torch.float16):
+        o = _token_major(q, out)
+        _lib.call("pasa_dense_attn_bshd", q.data_ptr(), k.data_ptr(), v.data_ptr(), o.data_ptr(), float(scale), B * H,
+                  H, T, T, int(text_tokens), int(tv), D, _DTYPES[q.dtype], _stream(q))
+        return o
+    o = _check_out(v, out)
     _lib.call("pasa_dense_attn", q.data_ptr(), k.data_ptr(), v.data_ptr(), o.data_ptr(), float(scale), B * H, T,
               int(text_tokens), int(tv), D, _DTYPES.get(q.dtype, -1), _stream(q))
+    return o
+
+
+def cross_attention(q: torch.Tensor, k: torch.Tensor, v: torch.Tensor, scale: Optional[float] = None) -> torch.Tensor:
+    """Dense softmax attention of q [B, H, S, D] to k, v [B, H, L, D] (bf16 or fp16, D = 128): a DiT
+    block's attention to its text tokens.  Returns [B, H, S, D] over [B, S, H, D] memory."""
+    _check_qkv(k, k, v)
+    _check_device(q, k, v)
+    if q.dim() != 4 or q.shape[:2] != k.shape[:2] or q.shape[3] != k.shape[3] or q.dtype != k.dtype:
+        raise ValueError(f"q must be [B, H, S, D] with k's batch, heads, head dim and dtype, got {tuple(q.shape)} "
+                         f"{q.dtype} for k {tuple(k.shape)} {k.dtype}")
+    B, H, S, D = q.shape
+    o = _token_major(q, None)
+    _lib.call("pasa_dense_attn_bshd", q.data_ptr(), k.data_ptr(), v.data_ptr(), o.data_ptr(),
+              float(D ** -0.5 if scale is None else scale), B * H, H, S, k.shape[2], 0, 0, D,
+              _DTYPES.get(q.dtype, -1), _stream(q))
     return o
 
 

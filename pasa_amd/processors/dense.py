@@ -24,14 +24,15 @@ def kernel_ok(query: torch.Tensor, key: torch.Tensor, value: torch.Tensor) -> bo
 
 
 def attention(query: torch.Tensor, key: torch.Tensor, value: torch.Tensor,
-              valid: Optional[int] = None) -> torch.Tensor:
-    """softmax attention of [B, H, N, D] tensors; with ``valid`` < N, block-diagonal over
+              valid: Optional[int] = None, token_major_out: bool = False) -> torch.Tensor:
+    """softmax attention of [B, H, N, D] tensors (``token_major_out``: the kernel's result over
+    [B, N, H, D] memory, for the output projection); with ``valid`` < N, block-diagonal over
     [0, valid) and [valid, N) (cu_seqlens [0, valid, N])."""
     N = query.shape[2]
     valid = N if valid is None else int(valid)
     if kernel_ok(query, key, value) and 1 <= valid <= N:
         return ops.dense_attention(query.contiguous(), key.contiguous(), value.contiguous(),
-                                   text_tokens=N - valid, text_valid=0)
+                                   text_tokens=N - valid, text_valid=0, token_major_out=token_major_out)
     if valid >= N:
         return F.scaled_dot_product_attention(query, key, value, dropout_p=0.0, is_causal=False)
     out = torch.empty_like(query)

@@ -42,7 +42,7 @@ from ..ops import pisa_pg_attention
 from ..placement import hunyuan_hidden_states_placement, hunyuan_sparse_head_placement
 from ..prologue import qkv_prologue, rope_tables_cossin
 from . import dense as _dense
-from .qknorm import fusable, module_rounding, norm_eps
+from .qknorm import fusable, merge_heads, module_rounding, norm_eps
 from .rope import apply_rotary_emb_cos_sin
 from .timestep_hook import current_timestep, install_hunyuan
 
@@ -54,7 +54,7 @@ def _split_heads(attn, x):
 def block_diagonal_attention(query, key, value, valid: int):
     """softmax attention restricted to [0, valid) x [0, valid) and [valid, N) x [valid, N)
     (the HIP dense path for bf16 device tensors, see ``processors.dense``)."""
-    return _dense.attention(query, key, value, valid)
+    return _dense.attention(query, key, value, valid, token_major_out=True)
 
 
 def _valid_length(attention_mask, n: int) -> int:
@@ -289,7 +289,7 @@ class Hunyuan_SVGAttn_Processor2_0:
             timestep = current_timestep()      # set by the installed forward hook
         cu_max_seqlens = self.get_cu_max_seqlen(attention_mask, query.device)
         hidden_states = self.attention_core_logic(query, key, value, timestep, self.layer_idx, cu_max_seqlens)
-        hidden_states = hidden_states.transpose(1, 2).flatten(2, 3).to(query.dtype)
+        hidden_states = merge_heads(hidden_states).to(query.dtype)
         return self.get_o(attn, hidden_states, encoder_hidden_states)
 
     def flash_attention(self, query, key, value, cu_max_seqlens):

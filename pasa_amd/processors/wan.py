@@ -27,7 +27,7 @@ from .. import density as _density
 from ..ops import pisa_pg_attention
 from ..prologue import qkv_prologue, rope_tables_complex
 from . import dense as _dense
-from .qknorm import fusable, is_rmsnorm, norm_eps, rms_norm_once
+from .qknorm import fusable, is_rmsnorm, merge_heads, norm_eps, rms_norm_once
 from .rope import apply_rotary_emb_complex
 from .timestep_hook import current_timestep, install_wan
 
@@ -117,7 +117,7 @@ class WanAttn_SVGAttn_Processor2_0:
         return query, key
 
     def get_o(self, attn, query, hidden_states, hidden_states_img):
-        hidden_states = hidden_states.transpose(1, 2).flatten(2, 3)
+        hidden_states = merge_heads(hidden_states)
         hidden_states = hidden_states.type_as(query)
         if hidden_states_img is not None:
             hidden_states = hidden_states + hidden_states_img
@@ -170,7 +170,7 @@ class WanAttn_SVGAttn_Processor2_0:
     def flash_attention(self, query, key, value):
         """Dense attention (reference :299-301): the HIP exact-tile path for bf16 device
         tensors with head_dim 128, else PyTorch SDPA (``processors.dense``)."""
-        return _dense.attention(query, key, value)
+        return _dense.attention(query, key, value, token_major_out=True)
 
     def attention_core_logic(self, query, key, value, timestep):  # pragma: no cover - abstract
         raise NotImplementedError

@@ -1,0 +1,64 @@
+"""Dense attention with its output token-major (and to a different number of keys), and the head
+merge of the processors, at the edges of the 128-row tiles.
+
+Reference: softmax(scale q k^T) v in 64 bits.  P and the output are rounded once each to 8 (bf16)
+or 11 (fp16) bits, so the relative error stays within twice half an ulp, 2^-8 or 2^-11, in the
+2-norm."""
+import pytest
+import torch
+
+from oracle import pisa_oracle as O
+from pasa_amd import ops
+from pasa_amd.processors.qknorm import merge_heads
+
+pytestmark = pytest.mark.gpu
+
+TOL = {torch.bfloat16: 2.0 ** -8, torch.float16: 2.0 ** -11}
+
+
+def make(B, H, S, L, dtype, seed):
+    g = torch.Generator().manual_seed(seed)
+    q = torch.randn(B, H, S, 128, generator=g).to(dtype)
+    k, v = (torch.randn(B, H, L, 128, generator=g).to(dtype) for _ in range(2))
+    return q, k, v
+
+
+@pytest.mark.parametrize("B,H,S,L,dtype", [(1, 1, 1, 1, torch.bfloat16), (2, 3, 129, 512, torch.bfloat16),
+                                           (1, 2, 1000, 77, torch.float16), (1, 5, 127, 257, torch.bfloat16),
+                                           (1, 1, 2048, 128, torch.float16), (1, 2, 300, 300, torch.bfloat16)])
+def test_cross_attention(device, B, H, S, L, dtype):
+    q, k, v = make(B, H, S, L, dtype, S + L)
+    o = ops.cross_attention(q.to(device), k.to(device), v.to(device))
+    assert o.shape == q.shape and o.transpose(1, 2).is_contiguous()
+    ref = O.dense_attention(q, k, v, O.effective_scale(128 ** -0.5))
+    err = float((o.cpu().double() - ref).norm() / ref.norm())
+    print(f"[cross] B={B} H={H} S={S} L={L} {dtype}: rel {err:.2e}", flush=True)
+    assert err <= TOL[dtype]
+
+
+@pytest.mark.parametrize("B,H,T,text,valid,dtype", [(1, 3, 700, 0, None, torch.bfloat16),
+                                                    (2, 2, 513, 100, 37, torch.float16)])
+def test_dense_token_major_is_the_same(device, B, H, T, text, valid, dtype):
+    q, k, v = (t.to(device) for t in make(B, H, T, T, dtype, T))
+    a = ops.dense_attention(q, k, v, text_tokens=text, text_valid=valid)
+    b = ops.dense_attention(q, k, v, text_tokens=text, text_valid=valid, token_major_out=True)
+    assert b.transpose(1, 2).is_contiguous() and torch.equal(a, b)
+
+
+@pytest.mark.parametrize("B,H,S,D", [(1, 12, 1000, 128), (2, 3, 5, 64), (1, 1, 7, 128), (1, 70, 9, 128)])
+def test_merge_heads(device, B, H, S, D):
+    x = torch.randn(B, H, S, D, device=device, dtype=torch.bfloat16)
+    want = x.transpose(1, 2).flatten(2, 3)
+    assert torch.equal(merge_heads(x), want)
+    view = x.transpose(1, 2).contiguous().transpose(1, 2)   # token-major memory: a view suffices
+    assert torch.equal(merge_heads(view), want) and merge_heads(view).data_ptr() == view.data_ptr()
+
+
+def test_rejected_arguments(device):
+    q, k, v = (t.to(device) for t in make(1, 2, 16, 8, torch.bfloat16, 0))
+    with pytest.raises(ValueError):
+        ops.cross_attention(q[:, :1].contiguous(), k, v)
+    with pytest.raises(ValueError):
+        ops.cross_attention(q.float(), k, v)
+    with pytest.raises(ops._lib.PasaError):
+        ops.cross_attention(q[..., :64].contiguous(), k[..., :64].contiguous(), v[..., :64].contiguous())
