@@ -99,3 +99,25 @@ def test_rope_survives_dtype_cast():
     m = W.WanDiT(tiny_cfg(1)).to(torch.bfloat16)
     f = m.rope(torch.zeros(1, 16, 3, 4, 6))
     assert f.dtype == torch.complex128 and f.imag.abs().max() > 0.5
+
+
+def test_fused_paths_leave_replaced_and_hooked_modules_alone():
+    """The block's fused feed-forward and cross-attention step aside for anything that a module call
+    would run and they would not: subclasses (adapters), hooks, another activation or processor."""
+    cfg = W.WanDiTConfig(num_layers=1, num_attention_heads=2, ffn_dim=64, text_dim=32, freq_dim=16)
+    blk = W.WanBlock(cfg)
+
+    class Adapter(torch.nn.Linear):
+        pass
+
+    assert W._plain(blk.ffn, torch.nn.Sequential) and W._plain(blk.ffn[0], torch.nn.Linear)
+    assert not W._plain(Adapter(4, 4), torch.nn.Linear)
+    handle = blk.attn2.register_forward_hook(lambda m, a, o: o)
+    assert not W._plain(blk.attn2, W.WanAttention)
+    handle.remove()
+    assert W._plain(blk.attn2, W.WanAttention)
+    x, text = torch.randn(1, 3, 256), torch.randn(1, 5, 256)
+    assert not W._cross_fusable(blk.attn2, x, text)          # host tensors
+    blk.ffn[1] = torch.nn.GELU()                             # the erf form has no fused counterpart
+    with torch.no_grad():
+        torch.testing.assert_close(blk._ffn_fused(x), blk.ffn(x))
