@@ -25,18 +25,27 @@
 // chunks staged in LDS.  BT < 64 (TEAM = 1): each wave owns a 16- or 32-row query block (fp32: 16
 // rows of one) and walks its own selected blocks through chunks of its own in LDS, with no
 // workgroup barrier; so all 64 lanes work at any block size, and the four waves share the
-// operands of phase 2, which every query block reads in full.  The next chunk's rows load into registers while one is multiplied.
+// operands of phase 2, which every query block reads in full.  The next chunk's rows load into
+// registers while one is multiplied.
 //
-// What bounds it: in fp32 the MFMA pipe (153 TFLOP/s in a large fp32 matrix product here; 12 heads
-// x 7,800 rows, D 128, block 64: 75 GFLOP in 0.71 ms, each further selected block at 118 TFLOP/s,
-// where one FMA per lane took 2.07 ms); in 16 bits the latency of the staged loads and, in phase 2,
-// of Hbar (16 heads x 8,610 rows, D 96, block 32, groups of 16: 149 GFLOP in 0.35 ms, half of it
-// phase 2, where one FMA per lane took 9.7 ms with half its lanes idle).
+// fp32 with TEAM = 4 (Split32) runs on the bf16 MFMA: every operand is split into three bf16 planes,
+// x = x1 + x2 + x3 to its last bit (q in registers, K/V/V^/Hbar as they are staged, P after its
+// exponential), and a product is six MFMAs: x1 y1 into one sum, the smaller five into another, so
+// that they round at their own size.  Six bf16 MFMAs take 3/8 of the fp32 MFMA's time for the same
+// product, and round less: one addition per 32 terms where the fp32 MFMA rounds after every product.
+// Error against 64 bits at 12 heads x 7,800 rows, D 128, block 64: 7.3e-7 with one FMA per lane,
+// 5.0e-7 on the fp32 MFMA, 4.0e-7 so (with q and k of mean 1 and 3, where the scores cancel, 2.3e-6
+// and 2.1e-6 at 3,000 rows; with one sum over all 128 features 2.4e-6); K4 there 2.07 ms, 0.66 and
+// 0.45.
+// TEAM = 1 stays on the fp32 MFMA (Any32): a wave would split its own K/V rows for 16 queries.
+// Its fp32 sums are taken in short chains (half the features, a chunk of keys, 32 rows of Hbar) that
+// are then added; chains of 16 features round less and are 8% slower.
 //
-// fp32 sums are taken in short chains (half the features, a chunk of keys, 32 rows of Hbar) that
-// are then added, because the MFMA rounds after every product: the error against 64 bits is
-// 5.0e-7 (7.3e-7 for the one-FMA-per-lane form) at the fp32 shape above.  Chains of 16 features
-// give 3.4e-7 and are 8% slower (their additions wait for the MFMA).
+// What bounds it: Split32, the MFMA pipe (75 GFLOP of fp32, so 450 of bf16, in 0.45 ms, where a
+// large bf16 product takes 0.34), with a third as many VALU instructions for the splits;
+// Any32, the fp32 MFMA (153 TFLOP/s in a large product); 16 bits, the latency of the staged loads
+// and, in phase 2, of Hbar (16 heads x 8,610 rows, D 96, block 32, groups of 16: 149 GFLOP in
+// 0.35 ms, half of it phase 2, where one FMA per lane took 9.7 ms with half its lanes idle).
 #include <initializer_list>
 #include <type_traits>
 
@@ -47,15 +56,25 @@ namespace pasa {
 
 namespace {
 
+struct Split32 {  // fp32 rows, three bf16 planes of each in LDS
+  using M = Bf16;
+  static constexpr int ES = 4;
+  static constexpr bool SPLIT = true;
+  using frag = bf16x8_t;
+};
+struct Any32 {  // fp32 rows in LDS, fp32 MFMA
+  static constexpr int ES = 4;
+  static constexpr bool SPLIT = false;
+  using frag = f32x4_t;
+  using Team4 = Split32;
+};
 template <typename M_>
 struct Any16 {
   using M = M_;
   static constexpr int ES = 2;
+  static constexpr bool SPLIT = false;
   using frag = typename M::vec8;
-};
-struct Any32 {
-  static constexpr int ES = 4;
-  using frag = f32x4_t;
+  using Team4 = Any16;
 };
 
 constexpr int pow2_at_least(int x) {
@@ -68,24 +87,29 @@ constexpr int pow2_at_least(int x) {
 template <typename E, int DP, int TEAM, int RW>
 struct AnyCfg {
   static constexpr int ES = E::ES;
-  static constexpr bool F32 = ES == 4;
-  static constexpr int QT = RW / 16;       // 16-row query tiles per wave
-  static constexpr int ROWS = 4 * RW;      // query rows per workgroup (TEAM = 4)
-  static constexpr int NF = DP * ES / 64;  // 64-byte feature steps per row: one fragment each
+  static constexpr bool SPLIT = E::SPLIT;
+  static constexpr bool F32 = ES == 4 && !SPLIT;
+  static constexpr int LE = F32 ? 4 : 2;         // bytes of an element in LDS
+  static constexpr int NPL = SPLIT ? 3 : 1;      // planes of every row in LDS
+  static constexpr int QT = RW / 16;             // 16-row query tiles per wave
+  static constexpr int ROWS = 4 * RW;            // query rows per workgroup (TEAM = 4)
+  static constexpr int NF = DP * LE / 64;  // 64-byte feature steps per row: one fragment each
   static constexpr int DT = DP / 16;       // 16-feature tiles of O
-  // Keys per chunk: about 16 KB of K and of V per team (8 KB where each wave stages its own).
-  static constexpr int KC = TEAM == 1 ? (F32 ? 16 : 32) : 64;
+  // Keys per chunk: what two workgroups per CU leave room for (fp32 planes: 27 KB each of K and V).
+  static constexpr int KC = TEAM == 1 ? (F32 ? 16 : 32) : (SPLIT ? 32 : 64);
   // Row strides.  K: an odd number of 16-byte chunks, so that 16 rows read at one chunk touch 16
   // distinct bank groups.  V in 16 bits: twice an odd number of chunks, so that the 8 rows x 32
   // bytes half a wave transposes do; in fp32 4 rows x 64 bytes, four rows apart, already do.
-  static constexpr int KROW = DP * ES + 16;
-  static constexpr int VROW = DP * ES + (F32 ? 16 : 32);
-  static constexpr int SLAB = KC * (KROW + VROW);
+  static constexpr int KROW = DP * LE + 16;
+  static constexpr int VROW = DP * LE + (F32 ? 16 : 32);
+  static constexpr int SLAB = NPL * KC * (KROW + VROW);
   static constexpr int KZ = 32;                  // blocks per zero-order chunk
-  static constexpr int HR = F32 ? 32 : DP;       // rows of Hbar staged at a time
-  static constexpr int Z_BYTES = KZ * (KROW + VROW);
+  static constexpr int HR = F32 || (SPLIT && DP == 96) ? 32 : (SPLIT ? 64 : DP);  // Hbar rows staged at a time
+  static constexpr int Z_BYTES = NPL * KZ * (KROW + VROW);
+  static constexpr int H_BYTES = NPL * HR * VROW;
   static constexpr int P1 = (4 / TEAM) * SLAB;
-  static constexpr int P2 = Z_BYTES + HR * VROW;
+  // SPLIT: Hbar takes the place of the zero-order rows, whose chunk is done by then.
+  static constexpr int P2 = SPLIT ? (Z_BYTES > H_BYTES ? Z_BYTES : H_BYTES) : Z_BYTES + H_BYTES;
   static constexpr int LDS = P1 > P2 ? P1 : P2;
   static constexpr int CH = DP * ES / 16;        // 16-byte chunks per row
   static constexpr int CHP = pow2_at_least(CH);  // lanes per staged row
@@ -115,29 +139,68 @@ __device__ __forceinline__ uint4 load_elems(const unsigned char* row, int c, int
   return make_uint4(w[0], w[1], w[2], w[3]);
 }
 
+// Four fp32 as three bf16 each, x = x1 + x2 + x3: x1 is x cut to its upper 16 bits (so that no
+// rounding overflows), x2 and x3 the rounded rests; together they hold all 24 bits of x.  The rest
+// of an infinity or NaN is NaN.
+__device__ __forceinline__ void split4(const float (&x)[4], uint2 (&pl)[3]) {
+  uint32_t u[4];
+  float r[4];
+#pragma unroll
+  for (int i = 0; i < 4; ++i) {
+    u[i] = __float_as_uint(x[i]);
+    r[i] = x[i] - __uint_as_float(u[i] & 0xffff0000u);
+  }
+  pl[0] = make_uint2(__builtin_amdgcn_perm(u[1], u[0], 0x07060302u), __builtin_amdgcn_perm(u[3], u[2], 0x07060302u));
+  pl[1] = make_uint2(Bf16::pack2(r[0], r[1]), Bf16::pack2(r[2], r[3]));
+  r[0] -= __uint_as_float(pl[1].x << 16);
+  r[1] -= __uint_as_float(pl[1].x & 0xffff0000u);
+  r[2] -= __uint_as_float(pl[1].y << 16);
+  r[3] -= __uint_as_float(pl[1].y & 0xffff0000u);
+  pl[2] = make_uint2(Bf16::pack2(r[0], r[1]), Bf16::pack2(r[2], r[3]));
+}
+
+// For j = 0, 1: hi[j] += a1 b1 and lo[j] += the five products of the next orders of a = a[j], smallest
+// first; what is left out is below 2^-24 of a b.  The two sums alternate, held in this order: an MFMA
+// that adds to the one before waits for it (480p shape above: 625 us with one after the other,
+// 615 in the compiler's order, 609 so).
+__device__ __forceinline__ void mfma_split(const bf16x8_t (&a)[2][3], const bf16x8_t (&b)[3], f32x4_t* const (&hi)[2],
+                                           f32x4_t* const (&lo)[2]) {
+  constexpr int PA[6] = {2, 0, 0, 1, 1, 0}, PB[6] = {0, 0, 2, 1, 0, 1};
+#pragma unroll
+  for (int i = 0; i < 6; ++i) {
+#pragma unroll
+    for (int j = 0; j < 2; ++j) {
+      f32x4_t& t = PA[i] + PB[i] == 0 ? *hi[j] : *lo[j];
+      t = Bf16::mfma16(a[j][PA[i]], b[PB[i]], t);
+    }
+    __builtin_amdgcn_sched_barrier(0);
+  }
+}
+
 constexpr uint32_t kOutside = 0x80000000u;  // a buffer offset past every chunk: the load gives zeros
 
-}  // namespace
-
+// One workgroup's tile of k4_any_mfma, in the workgroup's `lds`; false: the tile holds a NaN and
+// nothing has been stored (split fp32 only).
 // VEC: the rows of q, k, v, o, kc, vc and hgroup are whole aligned 16-byte chunks.  They are then
 // loaded through buffer resources over just the rows wanted, so rows past them read as zero with
 // no branch around any load (a branch per load makes the compiler wait for each by itself: the
 // bf16 call above took 0.67 ms, now 0.42, with a run-time test of the alignment in its load loop).
 // all: dense (every key of the segment, no selection, no correction; BT is then ROWS).
-// video: query blocks are computed (0: the text rows alone, where the blocks run with TEAM = 1).
+// nvt: the first nvt tiles are query blocks (0: the text rows alone, where the blocks run with
+// TEAM = 1), the rest up to ntiles text rows.
 template <typename E, int DP, int TEAM, int RW, bool VEC>
-__global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2))) void k4_any_mfma(
-    const unsigned char* __restrict__ q, const unsigned char* __restrict__ k, const unsigned char* __restrict__ v,
-    const float* __restrict__ kc, const float* __restrict__ vc, const float* __restrict__ hgroup,
-    const uint32_t* __restrict__ selmask, unsigned char* __restrict__ o, float scale, float c, int T, int text,
-    int text_valid, int D, int BT, int NT, int G, int NG, int NW, int gamma_literal, int all, int nvt,
-    int ntiles) {
+__device__ __forceinline__ bool any_tile(
+    unsigned char* lds, const unsigned char* __restrict__ q, const unsigned char* __restrict__ k,
+    const unsigned char* __restrict__ v, const float* __restrict__ kc, const float* __restrict__ vc,
+    const float* __restrict__ hgroup, const uint32_t* __restrict__ selmask, unsigned char* __restrict__ o, float scale,
+    float c, int T, int text, int text_valid, int D, int BT, int NT, int G, int NG, int NW, int gamma_literal, int all,
+    int nvt, int ntiles) {
   using C = AnyCfg<E, DP, TEAM, RW>;
   using frag = typename E::frag;
   constexpr int ES = C::ES, QT = C::QT, NF = C::NF, DT = C::DT, KC = C::KC;
   constexpr int KROW = C::KROW, VROW = C::VROW;
-  constexpr bool F32 = C::F32;
-  __shared__ __attribute__((aligned(16))) unsigned char lds[C::LDS];
+  constexpr bool F32 = C::F32, SPLIT = C::SPLIT;
+  constexpr int NPL = C::NPL;
 
   const int tid = threadIdx.x;
   const int lane = tid & 63;
@@ -147,7 +210,7 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2))) void k
   const int bh = blockIdx.y;
   // Consecutive workgroups go to consecutive XCDs; each takes a contiguous run of a slice's tiles.
   const int tile = (int)(blockIdx.x & 7) * (int)(gridDim.x >> 3) + (int)(blockIdx.x >> 3);
-  if (tile >= ntiles) return;
+  if (tile >= ntiles) return true;
 
   const int Ttot = T + text;
   const int seg = T + text_valid;
@@ -167,7 +230,7 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2))) void k
     I = tile / tpb;
     const int r0 = I * BT + (tile - I * tpb) * C::ROWS;
     row_end = min(T, min(r0 + C::ROWS, (I + 1) * BT));
-    if (r0 >= row_end) return;  // a tile past the last block's rows
+    if (r0 >= row_end) return true;  // a tile past the last block's rows
     row0 = r0 + wave * RW;
     cur = all ? 0 : T;
     cend = seg;
@@ -186,7 +249,7 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2))) void k
   const unsigned char* vsl = v + slice;
 
   // Q as B operands: fragment f of query tile qt holds the slots of feature step f.
-  frag qf[QT][NF];
+  frag qf[QT][NF][NPL];
   const rsrc_t qrs = make_rsrc(q + slice + (int64_t)row0 * row_bytes,
                                (uint32_t)(min(RW, max(0, row_end - row0)) * (int)row_bytes));
 #pragma unroll
@@ -196,6 +259,33 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2))) void k
 #pragma unroll
     for (int f = 0; f < NF; ++f) {
       u32x4_t w = {0u, 0u, 0u, 0u};
+      if constexpr (SPLIT) {
+        u32x4_t pw[3];
+#pragma unroll
+        for (int h = 0; h < 2; ++h) {
+          const int d = 32 * f + 16 * h + 4 * g4;
+          u32x4_t x4 = {0u, 0u, 0u, 0u};
+          if constexpr (VEC) {
+            x4 = __builtin_amdgcn_raw_buffer_load_b128(
+                qrs, d < D ? (uint32_t)(r * (int)row_bytes + d * 4) : kOutside, 0, 0);
+          } else if (row0 + r < row_end) {
+            const uint4 y = load_elems<4>(qrow, d / 4, D);
+            x4 = (u32x4_t){y.x, y.y, y.z, y.w};
+          }
+          const float x[4] = {__uint_as_float(x4[0]), __uint_as_float(x4[1]), __uint_as_float(x4[2]),
+                              __uint_as_float(x4[3])};
+          uint2 pl[3];
+          split4(x, pl);
+#pragma unroll
+          for (int i = 0; i < 3; ++i) {
+            pw[i][2 * h] = pl[i].x;
+            pw[i][2 * h + 1] = pl[i].y;
+          }
+        }
+#pragma unroll
+        for (int i = 0; i < NPL; ++i) qf[qt][f][i] = __builtin_bit_cast(frag, pw[i]);
+        continue;
+      }
       if constexpr (F32) {
         const int d = 16 * f + 4 * g4;
         if constexpr (VEC) {
@@ -221,7 +311,7 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2))) void k
           }
         }
       }
-      qf[qt][f] = __builtin_bit_cast(frag, w);
+      qf[qt][f][0] = __builtin_bit_cast(frag, w);
     }
   }
 
@@ -242,8 +332,27 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2))) void k
     const uint2 hi = lds_read_tr16(p, 16 * VROW);
     return __builtin_bit_cast(frag, (u32x4_t){lo.x, lo.y, hi.x, hi.y});
   };
+  // The three planes of a fragment: K rows of tile kt at step f (planes kp bytes apart), and the V
+  // form (planes vp bytes apart).
+  auto kfrag3 = [&](const unsigned char* rows, int kp, int f, int kt, frag (&a)[3]) {
+#pragma unroll
+    for (int i = 0; i < 3; ++i) a[i] = lds_ld<frag>(rows, i * kp + (kt * 16 + l16) * KROW + f * 64 + g4 * 16);
+  };
+  auto vfrag3 = [&](const unsigned char* rows, int vp, int s, int dt, frag (&a)[3]) {
+#pragma unroll
+    for (int i = 0; i < 3; ++i) a[i] = vt16(rows + i * vp, s, dt);
+  };
   auto vt32 = [&](const unsigned char* rows, int r, int dt) {
     return lds_ld<float>(rows, (r + 4 * g4) * VROW + dt * 64 + l16 * 4);
+  };
+
+  // Four fp32 as their three parts, one plane each.
+  auto st_split = [&](unsigned char* base, int plane, int off, const uint4& x) {
+    const float f[4] = {__uint_as_float(x.x), __uint_as_float(x.y), __uint_as_float(x.z), __uint_as_float(x.w)};
+    uint2 pl[3];
+    split4(f, pl);
+#pragma unroll
+    for (int i = 0; i < 3; ++i) lds_st(base, i * plane + off, pl[i]);
   };
 
   // One online-softmax step over the 16 KTN rows at Kb / Vb.  mask(s) drops scores (to -inf),
@@ -251,7 +360,37 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2))) void k
   auto step = [&](const unsigned char* Kb, const unsigned char* Vb, auto ktn, auto mask, auto on_rescale,
                   auto add) __attribute__((always_inline)) {
     constexpr int KTN = decltype(ktn)::value;
-    f32x4_t s[KTN][QT], sb[F32 ? KTN : 1][QT];
+    f32x4_t s[KTN][QT], sb[F32 || SPLIT ? KTN : 1][QT];
+    if constexpr (SPLIT) {
+      constexpr int KP = 16 * KTN * KROW;
+      // Feature steps per sum of first-order products, as in fp32: half of them (one of 96's three).
+      constexpr int HC = NF % 2 ? 1 : NF / 2;
+      f32x4_t hi[KTN][QT];
+#pragma unroll
+      for (int kt = 0; kt < KTN; ++kt)
+#pragma unroll
+        for (int qt = 0; qt < QT; ++qt) s[kt][qt] = sb[kt][qt] = (f32x4_t){0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+      for (int f = 0; f < NF; ++f)
+        for (int kt = 0; kt < KTN; kt += 2) {
+          frag a[2][3];
+          kfrag3(Kb, KP, f, kt, a[0]);
+          kfrag3(Kb, KP, f, kt + 1, a[1]);
+#pragma unroll
+          for (int qt = 0; qt < QT; ++qt) {
+            if (f % HC == 0) hi[kt][qt] = hi[kt + 1][qt] = (f32x4_t){0.f, 0.f, 0.f, 0.f};
+            mfma_split(a, qf[qt][f], {&hi[kt][qt], &hi[kt + 1][qt]}, {&sb[kt][qt], &sb[kt + 1][qt]});
+            if (f % HC == HC - 1) {
+              s[kt][qt] += hi[kt][qt];
+              s[kt + 1][qt] += hi[kt + 1][qt];
+            }
+          }
+        }
+#pragma unroll
+      for (int kt = 0; kt < KTN; ++kt)
+#pragma unroll
+        for (int qt = 0; qt < QT; ++qt) s[kt][qt] += sb[kt][qt];
+    } else
 #pragma unroll
     for (int f = 0; f < NF; ++f)
 #pragma unroll
@@ -263,11 +402,11 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2))) void k
             f32x4_t& t = f < NF / 2 ? s[kt][qt] : sb[kt][qt];
             if (f == 0 || f == NF / 2) t = (f32x4_t){0.f, 0.f, 0.f, 0.f};
 #pragma unroll
-            for (int i = 0; i < 4; ++i) t = __builtin_amdgcn_mfma_f32_16x16x4f32(a[i], qf[qt][f][i], t, 0, 0, 0);
+            for (int i = 0; i < 4; ++i) t = __builtin_amdgcn_mfma_f32_16x16x4f32(a[i], qf[qt][f][0][i], t, 0, 0, 0);
             if (f == NF - 1) s[kt][qt] += t;
           } else {
             if (f == 0) s[kt][qt] = (f32x4_t){0.f, 0.f, 0.f, 0.f};
-            s[kt][qt] = E::M::mfma16(a, qf[qt][f], s[kt][qt]);
+            s[kt][qt] = E::M::mfma16(a, qf[qt][f][0], s[kt][qt]);
           }
         }
       }
@@ -325,6 +464,41 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2))) void k
 #pragma unroll
           for (int qt = 0; qt < QT; ++qt) oacc[d2 + j][qt] += t[j][qt];
       }
+    } else if constexpr (SPLIT) {
+      constexpr int VP = 16 * KTN * VROW;
+      static_assert(KTN == 2, "one 32-key step");
+      frag pf[QT][3];
+#pragma unroll
+      for (int qt = 0; qt < QT; ++qt) {
+        u32x4_t pw[3];
+#pragma unroll
+        for (int h = 0; h < 2; ++h) {
+          const float x[4] = {s[h][qt][0], s[h][qt][1], s[h][qt][2], s[h][qt][3]};
+          uint2 pl[3];
+          split4(x, pl);
+#pragma unroll
+          for (int i = 0; i < 3; ++i) {
+            pw[i][2 * h] = pl[i].x;
+            pw[i][2 * h + 1] = pl[i].y;
+          }
+        }
+#pragma unroll
+        for (int i = 0; i < 3; ++i) pf[qt][i] = __builtin_bit_cast(frag, pw[i]);
+      }
+#pragma unroll
+      for (int dt = 0; dt < DT; dt += 2) {
+        frag a[2][3];
+        vfrag3(Vb, VP, 0, dt, a[0]);
+        vfrag3(Vb, VP, 0, dt + 1, a[1]);
+#pragma unroll
+        for (int qt = 0; qt < QT; ++qt) {
+          f32x4_t lo[2];  // the first-order products add to o itself: one addition per 32 keys
+          lo[0] = lo[1] = (f32x4_t){0.f, 0.f, 0.f, 0.f};
+          mfma_split(a, pf[qt], {&oacc[dt][qt], &oacc[dt + 1][qt]}, {&lo[0], &lo[1]});
+          oacc[dt][qt] += lo[0];
+          oacc[dt + 1][qt] += lo[1];
+        }
+      }
     } else {
 #pragma unroll
       for (int s2 = 0; s2 < KTN / 2; ++s2) {
@@ -350,7 +524,7 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2))) void k
   const const_u32_ptr mrow = (const_u32_ptr)(selmask + ((int64_t)bh * NT + (I < 0 ? 0 : I)) * NW);
   {
     unsigned char* Kb = lds + (TEAM == 1 ? wave : 0) * C::SLAB;
-    unsigned char* Vb = Kb + KC * KROW;
+    unsigned char* Vb = Kb + NPL * KC * KROW;
     const int tt = tid & (C::TT - 1);
     const int sc = tt % C::CHP;   // this thread's 16-byte chunk of a staged row
     const int sr = tt / C::CHP;   // its row in each pass
@@ -402,8 +576,8 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2))) void k
     // Rows r of a chunk: ra + r, and rb + r - 16 from row 16 on where each wave stages its own.
     const uint32_t lane_off = in_row ? (uint32_t)(sr * (int)row_bytes + sc * 16) : kOutside;
     auto fetch = [&](int ra, int rb, int n) {
-      constexpr int SPLIT = TEAM == 1 && KC == 32 && RW == 16 ? 16 : KC;  // 32-row blocks (RW 32) fill a chunk
-      const int na = min(n, SPLIT), nb = n - na;
+      constexpr int RUN = TEAM == 1 && KC == 32 && RW == 16 ? 16 : KC;  // 32-row blocks (RW 32) fill a chunk
+      const int na = min(n, RUN), nb = n - na;
       const unsigned char* base_k[2] = {ksl + (int64_t)ra * row_bytes, ksl + (int64_t)rb * row_bytes};
       const unsigned char* base_v[2] = {vsl + (int64_t)ra * row_bytes, vsl + (int64_t)rb * row_bytes};
       const rsrc_t rk[2] = {make_rsrc(base_k[0], (uint32_t)(na * (int)row_bytes)),
@@ -412,8 +586,8 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2))) void k
                             make_rsrc(base_v[1], (uint32_t)(nb * (int)row_bytes))};
 #pragma unroll
       for (int p = 0; p < C::PASSES; ++p) {
-        const int h = p * C::RPP >= SPLIT ? 1 : 0;
-        const int r0 = p * C::RPP - h * SPLIT;  // of the pass, within its run
+        const int h = p * C::RPP >= RUN ? 1 : 0;
+        const int r0 = p * C::RPP - h * RUN;  // of the pass, within its run
         if constexpr (VEC) {
           const uint32_t off = lane_off + (uint32_t)(r0 * (int)row_bytes);
           kreg[p] = buf_load16(rk[h], off);
@@ -432,6 +606,11 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2))) void k
 #pragma unroll
       for (int p = 0; p < C::PASSES; ++p) {
         const int r = p * C::RPP + sr;
+        if constexpr (SPLIT) {
+          st_split(Kb, KC * KROW, r * KROW + (sc >> 3) * 64 + (sc & 3) * 16 + ((sc >> 2) & 1) * 8, kreg[p]);
+          st_split(Vb, KC * VROW, r * VROW + sc * 8, vreg[p]);
+          continue;
+        }
         if constexpr (F32) {
           lds_st(Kb, r * KROW + sc * 16, kreg[p]);
         } else {  // features in slot order: 8 sc .. + 3 and + 4 .. + 7 are halves of two slots
@@ -475,8 +654,9 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2))) void k
     const float* kcb = kc + (int64_t)bh * NT * D;
     const float* vcb = vc + (int64_t)bh * NT * D;
     unsigned char* Kz = lds;
-    unsigned char* Vz = lds + C::KZ * KROW;
-    unsigned char* Hs = lds + C::Z_BYTES;
+    unsigned char* Vz = lds + NPL * C::KZ * KROW;
+    unsigned char* Hs = SPLIT ? lds : lds + C::Z_BYTES;
+    constexpr int H0 = SPLIT ? 1 : 0;  // the item that Hbar's first rows come with
     const int c4 = tid % C::C4P, r4 = tid / C::C4P;
     // Blocks [a, b) of one mask word that some wave of the workgroup does not select.
     auto word_unselected = [&](int wd) -> uint32_t {
@@ -503,9 +683,11 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2))) void k
       if (sh != 0 && wd + 1 < NW) sel |= mrow[wd + 1] << (32 - sh);
       return ~sel & (cn >= 32 ? 0xffffffffu : (1u << cn) - 1u);
     };
-    // Four floats to LDS as four elements of the input type.
-    auto st4 = [&](unsigned char* base, int off16, int off32, const float4& x) {
-      if constexpr (F32)
+    // Four floats to LDS as four elements of the input type (or their parts, `plane` bytes apart).
+    auto st4 = [&](unsigned char* base, int plane, int off16, int off32, const float4& x) {
+      if constexpr (SPLIT)
+        st_split(base, plane, off16, __builtin_bit_cast(uint4, x));
+      else if constexpr (F32)
         lds_st(base, off32, x);
       else
         lds_st(base, off16, make_uint2(E::M::pack2(x.x, x.y), E::M::pack2(x.z, x.w)));
@@ -524,9 +706,9 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2))) void k
       }
     };
     // Work items in order: a group's zero-order chunks of 32 blocks (the first one brings Hbar's
-    // first HR rows along), then the rest of its Hbar HR rows at a time.  In 16 bits the next item's
-    // rows load into registers while one is computed (430 -> 391 us at the bf16 shape above); fp32,
-    // bound by its MFMAs, is 2% slower with that.
+    // first HR rows along, but for the split ones), then the rest of its Hbar HR rows at a time.  The
+    // next item's rows load into registers while one is computed (430 -> 391 us at the bf16 shape
+    // above, split fp32 0.5%); with the fp32 MFMA that is 2% slower.
     int ig = -1, ijc = 0, ihs = 0;
     auto group_end = [&](int g) -> int { return (int)min((int64_t)NT, (int64_t)(g + 1) * G); };
     auto chunk_from = [&](int g, int jc) -> bool {  // the group's first chunk at or after jc with work
@@ -540,7 +722,7 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2))) void k
     auto next_item = [&]() -> bool {
       if (ig >= 0) {
         if (ihs == 0 && chunk_from(ig, ijc + C::KZ)) return true;
-        if ((ihs + 1) * C::HR < D) {
+        if ((ihs + 1 - H0) * C::HR < D) {
           ++ihs;
           return true;
         }
@@ -574,7 +756,7 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2))) void k
 #pragma unroll
       for (int p = 0; p < HP; ++p) {
         const int r = p * C::RPP4 + r4;
-        st4(Hs, r * VROW + c4 * 8, r * VROW + c4 * 16, hx[p]);
+        st4(Hs, C::HR * VROW, r * VROW + c4 * 8, r * VROW + c4 * 16, hx[p]);
       }
     };
     auto stash_z = [&]() {
@@ -582,8 +764,9 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2))) void k
 #pragma unroll
       for (int p = 0; p < ZP; ++p) {
         const int r = p * C::RPP4 + r4;
-        st4(Kz, r * KROW + (c4 >> 3) * 64 + (c4 & 3) * 16 + ((c4 >> 2) & 1) * 8, r * KROW + c4 * 16, zk[p]);
-        st4(Vz, r * VROW + c4 * 8, r * VROW + c4 * 16, zv[p]);
+        st4(Kz, C::KZ * KROW, r * KROW + (c4 >> 3) * 64 + (c4 & 3) * 16 + ((c4 >> 2) & 1) * 8, r * KROW + c4 * 16,
+            zk[p]);
+        st4(Vz, C::KZ * VROW, r * VROW + c4 * 8, r * VROW + c4 * 16, zv[p]);
       }
     };
     // Per row, of the current group: the sums of p and of p times the block's length, relative to
@@ -594,24 +777,25 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2))) void k
     bool more = next_item();
     if (more && !F32) {
       fetch_z(ijc, min(C::KZ, group_end(ig) - ijc));
-      fetch_h(ig, 0);
+      if (!SPLIT) fetch_h(ig, 0);
     }
     while (more) {
       const int g = ig, jc = ijc, hs = ihs;
       const bool first = g != pg;
       pg = g;
       __syncthreads();  // the previous item's rows have been read
+      const bool h_rows = hs > 0 || (first && !SPLIT);
       if (F32) {
         if (hs == 0) fetch_z(jc, min(C::KZ, group_end(g) - jc));
-        if (hs > 0 || first) fetch_h(g, hs);
+        if (h_rows) fetch_h(g, hs);
       }
       if (hs == 0) stash_z();
-      if (hs > 0 || first) stash_h();
+      if (h_rows) stash_h();
       __syncthreads();
       more = next_item();
       if (more && !F32) {
         if (ihs == 0) fetch_z(ijc, min(C::KZ, group_end(ig) - ijc));
-        if (ihs > 0 || ig != g) fetch_h(ig, ihs);
+        if (ihs > 0 || (ig != g && !SPLIT)) fetch_h(ig, ihs - H0);
       }
       if (hs == 0) {
         if (first) {
@@ -646,6 +830,7 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2))) void k
           g_run[qt] += gsum[qt];
           f[qt] = quad16_sum(psum[qt]) * scale;
         }
+        if (SPLIT) continue;  // Hbar comes with the next items
       }
       // First order: o += f (q . Hbar), over this item's rows of Hbar.
       if constexpr (F32) {
@@ -668,7 +853,7 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2))) void k
                   const float a = vt32(Hs, 16 * cc + i, d2 + j);
 #pragma unroll
                   for (int qt = 0; qt < QT; ++qt)
-                    r[j][qt] = __builtin_amdgcn_mfma_f32_16x16x4f32(a, qf[qt][h * (C::HR / 16) + cc][i], r[j][qt], 0,
+                    r[j][qt] = __builtin_amdgcn_mfma_f32_16x16x4f32(a, qf[qt][h * (C::HR / 16) + cc][0][i], r[j][qt], 0,
                                                                     0, 0);
                 }
 #pragma unroll
@@ -677,6 +862,35 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2))) void k
               for (int qt = 0; qt < QT; ++qt)
 #pragma unroll
                 for (int i = 0; i < 4; ++i) oacc[d2 + j][qt][i] = fmaf(r[j][qt][i], f[qt], oacc[d2 + j][qt][i]);
+          }
+        }
+      } else if constexpr (SPLIT) {
+#pragma unroll
+        for (int h = 0; h < DP / C::HR; ++h) {
+          if (h != hs - H0) continue;
+#pragma unroll
+          for (int dt = 0; dt < DT; dt += 2) {
+            f32x4_t hi[QT][2], lo[QT][2];
+#pragma unroll
+            for (int qt = 0; qt < QT; ++qt)
+#pragma unroll
+              for (int j = 0; j < 2; ++j) hi[qt][j] = lo[qt][j] = (f32x4_t){0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+            for (int s2 = 0; s2 < C::HR / 32; ++s2) {
+              frag a[2][3];
+              vfrag3(Hs, C::HR * VROW, s2, dt, a[0]);
+              vfrag3(Hs, C::HR * VROW, s2, dt + 1, a[1]);
+#pragma unroll
+              for (int qt = 0; qt < QT; ++qt)
+                mfma_split(a, qf[qt][h * (C::HR / 32) + s2], {&hi[qt][0], &hi[qt][1]}, {&lo[qt][0], &lo[qt][1]});
+            }
+#pragma unroll
+            for (int qt = 0; qt < QT; ++qt)
+#pragma unroll
+              for (int j = 0; j < 2; ++j)
+#pragma unroll
+                for (int i = 0; i < 4; ++i)
+                  oacc[dt + j][qt][i] = fmaf(hi[qt][j][i] + lo[qt][j][i], f[qt], oacc[dt + j][qt][i]);
           }
         }
       } else {
@@ -689,7 +903,7 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2))) void k
           for (int s2 = 0; s2 < NF; ++s2) {
             const frag a = vt16(Hs, s2, dt);
 #pragma unroll
-            for (int qt = 0; qt < QT; ++qt) r[qt] = E::M::mfma16(a, qf[qt][s2], r[qt]);
+            for (int qt = 0; qt < QT; ++qt) r[qt] = E::M::mfma16(a, qf[qt][s2][0], r[qt]);
           }
 #pragma unroll
           for (int qt = 0; qt < QT; ++qt)
@@ -698,6 +912,17 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2))) void k
         }
       }
     }
+  }
+
+  if constexpr (SPLIT) {
+    float t = 0.f;
+#pragma unroll
+    for (int qt = 0; qt < QT; ++qt) {
+      t += l_run[qt] + g_run[qt];
+#pragma unroll
+      for (int dt = 0; dt < DT; ++dt) t += (oacc[dt][qt][0] + oacc[dt][qt][1]) + (oacc[dt][qt][2] + oacc[dt][qt][3]);
+    }
+    if (__syncthreads_or(t != t)) return false;
   }
 
   // o = A / (L + Gamma) (:258-259), stored in the input type (:262).
@@ -713,7 +938,7 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2))) void k
         const float x[4] = {oacc[dt][qt][0] / den, oacc[dt][qt][1] / den, oacc[dt][qt][2] / den,
                             oacc[dt][qt][3] / den};
         if (VEC && e < D) {
-          if constexpr (F32)
+          if constexpr (ES == 4)
             *reinterpret_cast<float4*>(orow + e * 4) = make_float4(x[0], x[1], x[2], x[3]);
           else
             *reinterpret_cast<uint2*>(orow + e * 2) = make_uint2(E::M::pack2(x[0], x[1]), E::M::pack2(x[2], x[3]));
@@ -721,7 +946,7 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2))) void k
 #pragma unroll
           for (int i = 0; i < 4; ++i)
             if (e + i < D) {
-              if constexpr (F32)
+              if constexpr (ES == 4)
                 reinterpret_cast<float*>(orow)[e + i] = x[i];
               else
                 reinterpret_cast<uint16_t*>(orow)[e + i] = (uint16_t)E::M::bits(x[i]);
@@ -729,6 +954,34 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2))) void k
         }
       }
     }
+  }
+  return true;
+}
+
+}  // namespace
+
+template <typename E, int DP, int TEAM, int RW, bool VEC>
+__global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2))) void k4_any_mfma(
+    const unsigned char* __restrict__ q, const unsigned char* __restrict__ k, const unsigned char* __restrict__ v,
+    const float* __restrict__ kc, const float* __restrict__ vc, const float* __restrict__ hgroup,
+    const uint32_t* __restrict__ selmask, unsigned char* __restrict__ o, float scale, float c, int T, int text,
+    int text_valid, int D, int BT, int NT, int G, int NG, int NW, int gamma_literal, int all, int nvt,
+    int ntiles) {
+  using C = AnyCfg<E, DP, TEAM, RW>;
+  if constexpr (E::SPLIT) {
+    // An infinite operand meets the zero parts of another and gives NaN where an fp32 product would
+    // not: a tile with a NaN is done again in fp32.
+    using C32 = AnyCfg<Any32, DP, TEAM, RW>;
+    __shared__ __attribute__((aligned(16))) unsigned char lds[C::LDS > C32::LDS ? C::LDS : C32::LDS];
+    if (any_tile<E, DP, TEAM, RW, VEC>(lds, q, k, v, kc, vc, hgroup, selmask, o, scale, c, T, text, text_valid, D, BT,
+                                       NT, G, NG, NW, gamma_literal, all, nvt, ntiles))
+      return;
+    any_tile<Any32, DP, TEAM, RW, VEC>(lds, q, k, v, kc, vc, hgroup, selmask, o, scale, c, T, text, text_valid, D, BT,
+                                       NT, G, NG, NW, gamma_literal, all, nvt, ntiles);
+  } else {
+    __shared__ __attribute__((aligned(16))) unsigned char lds[C::LDS];
+    any_tile<E, DP, TEAM, RW, VEC>(lds, q, k, v, kc, vc, hgroup, selmask, o, scale, c, T, text, text_valid, D, BT, NT,
+                                   G, NG, NW, gamma_literal, all, nvt, ntiles);
   }
 }
 
@@ -771,8 +1024,8 @@ bool wide_tiles(const AnyCall& a, int BT) {
   return BT >= 128 && (int64_t)a.bh * ((a.T + 127) / 128) >= 256;
 }
 
-// WIDE: 32 rows per wave where the blocks are long enough (not in fp32: its MFMAs outlast their
-// LDS reads with 16 rows already, and 32 spill).
+// WIDE: 32 rows per wave where the blocks are long enough (not in fp32, whose planes or wider
+// fragments then spill).
 template <typename E, int DP, bool VEC, bool WIDE>
 hipError_t launch_dp(const AnyCall& a) {
   if (!a.all && a.BT < 64) {
@@ -786,15 +1039,15 @@ hipError_t launch_dp(const AnyCall& a) {
       e = launch_any<E, DP, 1, WIDE ? 32 : 16, VEC>(a, a.BT, ntiles, ntiles);
     }
     if (e != hipSuccess || a.text == 0) return e;
-    return launch_any<E, DP, 4, 16, VEC>(a, a.BT, 0, text_tiles(a, 64));  // the text rows
+    return launch_any<typename E::Team4, DP, 4, 16, VEC>(a, a.BT, 0, text_tiles(a, 64));  // the text rows
   }
   const bool wide = WIDE && wide_tiles(a, a.all ? 128 : a.BT);
   const int rows = wide ? 128 : 64;
   const int BT = a.all ? rows : a.BT;
   const int nvt = (a.T + BT - 1) / BT * ((BT + rows - 1) / rows);
   const int ntiles = nvt + text_tiles(a, rows);
-  return wide ? launch_any<E, DP, 4, WIDE ? 32 : 16, VEC>(a, BT, nvt, ntiles)
-              : launch_any<E, DP, 4, 16, VEC>(a, BT, nvt, ntiles);
+  return wide ? launch_any<typename E::Team4, DP, 4, WIDE ? 32 : 16, VEC>(a, BT, nvt, ntiles)
+              : launch_any<typename E::Team4, DP, 4, 16, VEC>(a, BT, nvt, ntiles);
 }
 
 template <typename E>

@@ -97,6 +97,40 @@ def test_dense_edges(device, T, D, dtype, text, valid, shift):
     assert err <= {F32: 4e-6, B16: 6e-3, F16: 1e-3}[dtype]
 
 
+@pytest.mark.parametrize("case", ["finite_range", "minus_inf_score", "inf_value", "nan_row"])
+@pytest.mark.parametrize("T,D", [(64, 64), (131, 37), (200, 128)])
+def test_dense_fp32_range(device, T, D, case):
+    """fp32 rows are multiplied as three bf16 parts each, and tiles that hold an infinity or NaN in
+    fp32: the ends of the range and the infinities come out as fp32 products give them."""
+    q, k, v = make(1, T, D, F32, 3 * T + D)
+    q[..., 0] = q[..., 0].abs() + 0.1
+    hot = T // 2  # the key, or the query row, that is special
+    if case == "finite_range":
+        v[..., 1] *= 2.0 ** 110      # sums of up to 200 weights <= 1 before they are normalised:
+        v[..., 2] = 2.0 ** 119       # below 2^127
+        v[..., 3] *= 2.0 ** -80      # and small ones
+        k[..., hot, 0] = -3.0e38     # a weight of exactly 0
+    elif case == "minus_inf_score":
+        k[..., hot, 0] = -torch.inf  # a score of -inf in every row: that key has no weight
+    elif case == "inf_value":
+        v[..., hot, 1], v[..., hot, 2] = torch.inf, -torch.inf
+    else:
+        q[..., hot, 1] = torch.nan   # one row of NaN, the others as they were
+    o = ops.dense_attention(*(to_dev(t, device, 0) for t in (q, k, v))).double().cpu()
+    es = O.effective_scale(D ** -0.5)
+    s = (q.double() @ k.double().transpose(-1, -2)) * es
+    ref = torch.softmax(s, -1) @ v.double()
+    if case == "finite_range":
+        assert float((torch.softmax(s, -1)[..., hot]).max()) == 0.0
+    assert torch.equal(torch.isnan(o), torch.isnan(ref)) and torch.equal(torch.isinf(o), torch.isinf(ref))
+    assert torch.equal(o.isposinf(), ref.isposinf())
+    ok = torch.isfinite(ref)
+    for col in range(D):  # per feature: their magnitudes differ
+        a, b = o[..., col][ok[..., col]], ref[..., col][ok[..., col]]
+        if a.numel():
+            assert float((a - b).norm() / b.norm()) <= 1e-5, col  # cancellation within one feature: 2.5x the bound above
+
+
 @pytest.mark.parametrize("heads,T,D,BT,G,dtype", [(2, 1024, 64, 64, 32, F32), (1, 777, 37, 16, 50, F16),
                                                   (3, 1000, 96, 32, 16, B16), (1, 300, 128, 256, 2, F32),
                                                   (2, 3001, 64, 64, 32, B16), (1, 4099, 64, 128, 32, B16)])
