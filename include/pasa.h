@@ -21,7 +21,7 @@
  * any group size, any power-of-two block size): fp32, bf16 or fp16 inputs, head_dim
  * 1 .. 128, block_size a power of two in [16, 256], group_size 1 .. 2^20, on the
  * any-shape kernels (the same mathematics; products on the MFMA of the input type, fp32
- * inputs in fp32).  The pack / packed / placed entry points take the tuned shapes only.
+ * inputs to fp32's precision).  The pack / packed / placed entry points take the tuned shapes only.
  *
  * Text segment (text_len > 0; head_dim 128 on the tuned kernels): the last text_len rows of each
  * slice are text tokens (HunyuanVideo appends its text last).  Blocks, statistics,

@@ -10,19 +10,13 @@
 //     rescaled "consistent" form).
 //   Finalize (:258-262): o = A / (L + Gamma).
 //
-// MI355X mapping.  One workgroup = one (slice, query block) of BT rows; one
-// wavefront per 32 query rows.  Everything is computed transposed so that the softmax
-// statistics of a query row stay in the lanes that hold it.  In the D = 64 kernel
-// (k4_sparse_attn) a lane owns one query (lane % 32):
-//   S^T[key][q]  = K  * Q^T   (v_mfma_f32_32x32x16_bf16, K from LDS, Q in VGPRs)
+// MI355X mapping.  One workgroup = one (slice, query block) of BT rows, or two blocks of 64
+// (PAIR); one wavefront per 32 query rows.  Everything is computed transposed so that the
+// softmax statistics of a query row stay in the lanes that hold it:
+//   S^T[key][q]  = K  * Q^T    (16x16x32 MFMA, K from LDS, Q in VGPRs)
 //   O^T[e][q]   += V^T * P^T   (V^T read from the row-major V tile with
 //                               ds_read_b64_tr_b16, P from the S^T accumulators)
-// The S^T accumulator of a lane holds, per 16-key step s, exactly the 8 keys
-// (16s + 8i' + 4h + j) its P^T B-operand slots need; two transposing LDS reads
-// fetch the matching V^T slots.  Keys of a block are consumed in halves of 64
-// (one online-softmax step each) to bound live accumulators.  The D = 128 kernel
-// (k4_sparse_attn_dma) runs the same transposed products on the 16x16x32 MFMA, a lane
-// owning two query rows (its lane layout is described at the kernel).
+// The lane layout is described at k4_body.
 //
 // Phase 1 walks the selected blocks in ascending block order (the selection
 // bitmask) instead of top-k order: exact online softmax is order-independent up
@@ -31,24 +25,22 @@
 // Workgroups are mapped XCD-aware: each XCD walks a contiguous run of query
 // blocks of the same head.
 //
-// Two kernels.  k4_sparse_attn_dma (D = 128) loads K/V tiles straight into LDS
-// (buffer_load ... lds, XOR-swizzled rows), double-buffered between the K and V
-// tiles, with an exact online softmax.  At BT = 64 it runs two query blocks per
-// four-wave workgroup (PAIR), each wave pair on its own selected tiles in lock
-// step: co-resident workgroups on a CU drift into start-time cohorts, each sweeping
-// a different region of key space, and pairing halves the number of cohorts (and so
-// the L2 working set), while each group's phase-2 operands are loaded once for both
-// blocks.  k4_sparse_attn (D = 64) stages tiles through registers; its online
-// softmax is the same exact one (rescale whenever a row's max rises).
+// One body, k4_body, for head dims 64 and 128 (kernels k4_sparse_attn, k4_sparse_attn_dma and
+// k4_cross_attn): K/V tiles go straight into LDS (buffer_load ... lds, XOR-swizzled rows),
+// double-buffered between the K and V tiles, with an exact online softmax (rescale whenever a
+// row's max rises).  At BT = 64 a four-wave workgroup runs two query blocks (PAIR), each wave
+// pair on its own selected tiles in lock step: co-resident workgroups on a CU drift into
+// start-time cohorts, each sweeping a different region of key space, and pairing halves the
+// number of cohorts (and so the L2 working set), while each group's phase-2 operands are loaded
+// once for both blocks.
 //
-// Both keep the row sum of P in fp32 (adds, not v_dot2c_f32_bf16: on gfx950 a dot
+// The row sum of P is kept in fp32 (adds, not v_dot2c_f32_bf16: on gfx950 a dot
 // instruction issues only between the MFMAs of the SIMD's other wave, so it stalls
 // its wave behind the partner's MFMA stream).
 //
 // Phase-2 operands (kbar, V^ transposed, Hbar transposed; in the input's 16-bit type) are
-// packed per (slice, group) by k4_pack / k4_pack_xor into the exact LDS image K4 copies in.
-// The D = 128 kernels and k4_pack_xor take that type as a template argument (Bf16 or
-// F16: the MFMA and the rounding of P, the pack and o); the D = 64 ones are bf16.
+// packed per (slice, group) by k4_pack_xor into the exact LDS image K4 copies in.  That type
+// is a template argument (Bf16, or F16 at D = 128).
 #include "common.h"
 #include "k4_layout.h"
 #include "kernels.h"
@@ -140,10 +132,9 @@ __global__ __launch_bounds__(256) void k4_pack_xor(const float* __restrict__ kc,
   }
 }
 
-// ---- D = 128: tiles loaded straight into LDS ----------------------------------
+// ---- tiles loaded straight into LDS -----------------------------------------
 //
-// Same computation as k4_sparse_attn, restructured for D = 128 so that the K/V
-// tiles never pass through VGPRs: buffer_load_dwordx4 ... lds writes each lane's
+// The K/V tiles never pass through VGPRs: buffer_load_dwordx4 ... lds writes each lane's
 // 16 bytes to LDS directly (zeros past the end of the slice), which frees the
 // staging registers for deeper LDS-operand prefetching while two workgroups
 // still share each CU.  Per block i, with one K and one V buffer, two barriers:
@@ -162,7 +153,7 @@ __global__ __launch_bounds__(256) void k4_pack_xor(const float* __restrict__ kc,
 // a 32-key step s a lane holds (tiles 2s and 2s + 1) are its B-operand k-slots as they
 // stand, and two transposing LDS reads fetch the V^T A-operand slots for the same keys.
 //
-// Tiles use 256-byte rows with XOR-swizzled 16-byte chunks: K chunk c of row r sits at
+// Tiles at D = 128 use 256-byte rows with XOR-swizzled 16-byte chunks: K chunk c of row r sits at
 // c ^ (r & 15) (the A-operand reads of 16 rows by one 16-lane group touch 16 distinct
 // chunks), V chunk c at c ^ 2 (r & 7) (the transposing reads of 32 lanes, rows 8 apart,
 // touch 16 distinct chunks).  The phase-2 pack image is loaded the same way.
