@@ -215,7 +215,7 @@ constexpr int kSchedDsRead = 0x100;
 // one the unpaired kernel computes.
 // CROSS (with ALL): the slices of q and o have q_len rows, those of k and v T; the query tiles
 // cover q's rows and each visits all of k's.
-// o_heads: 0, o is [slice, row, D] as q; else o is [batch, row, head, D] with o_heads heads, the
+// o_heads (ALL): 0, o is [slice, row, D] as q; else o is [batch, row, head, D] with o_heads heads, the
 // layout the projection after the attention reads.
 template <int D, int BT, bool ALL, bool PERM, bool PAIR, typename E, bool CROSS = false>
 __device__ __forceinline__ void k4_body(const uint16_t* __restrict__ q, const uint16_t* __restrict__ k,
@@ -757,8 +757,8 @@ __device__ __forceinline__ void k4_body(const uint16_t* __restrict__ q, const ui
     g = gn;
   }
 
-  const int ob = o_heads > 0 ? bh / o_heads : bh;  // o's rows are o_heads (or one) rows of D apart
-  const int on = o_heads > 0 ? o_heads : 1;
+  const int ob = ALL && o_heads > 0 ? bh / o_heads : bh;  // o's rows are o_heads (or one) rows of D apart
+  const int on = ALL && o_heads > 0 ? o_heads : 1;
   uint16_t* const oslice = o + ((int64_t)ob * q_rows * on + (bh - ob * on)) * D;
   const int ostride = on * D;
   // O = A / (L + Gamma): one correctly rounded reciprocal per row, then products.
