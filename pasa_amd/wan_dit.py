@@ -37,6 +37,7 @@ import torch.nn.functional as F
 from . import ops
 from .processors.qknorm import fusable, norm_eps
 from .processors.rope import apply_rotary_emb_complex
+from .processors.wan import Wan_PASA_Processor
 from .prologue import qkv_prologue
 
 
@@ -201,6 +202,13 @@ def _plain(module: nn.Module, cls) -> bool:
     return type(module) is cls and not (module._forward_hooks or module._forward_pre_hooks)
 
 
+def _reads_timestep_on_host(block) -> bool:
+    """Whether all that ``block`` does with the timestep is the PASA processor's comparison on the host.
+    Every other block, processor or hook is given the caller's tensor."""
+    return (_plain(block, WanBlock) and _plain(block.attn1, WanAttention)
+            and type(block.attn1.processor) is Wan_PASA_Processor)
+
+
 def _cross_fusable(attn, x: torch.Tensor, text: torch.Tensor) -> bool:
     """Whether ``_cross_attention_fused`` computes what ``attn``'s call does: the stock processor,
     torch RMSNorms with bf16 weights, bf16 text, head_dim 128, and nothing hooked in between."""
@@ -299,9 +307,7 @@ class WanDiT(nn.Module):
         b, _, f, h, w = hidden_states.shape
         pt, ph, pw = self.cfg.patch_size
         nf, nh, nw = f // pt, h // ph, w // pw
-        # The processors compare the timestep on the host: one copy here, not two per layer (each of
-        # which would wait for the layers before it).
-        host_timestep = timestep.tolist()
+        host_timestep = None
         rotary_emb = self.rope(hidden_states)
         x = self.patch_embedding(hidden_states).flatten(2).transpose(1, 2).contiguous()
 
@@ -312,7 +318,11 @@ class WanDiT(nn.Module):
         text = self.text_embedder(encoder_hidden_states)
 
         for block in self.blocks:
-            x = block(x, text, tproj, rotary_emb, timestep=host_timestep)
+            ts = timestep
+            if _reads_timestep_on_host(block):
+                # One copy for all layers, not two in each (which would wait for the layers before it).
+                ts = host_timestep = timestep.cpu() if host_timestep is None else host_timestep
+            x = block(x, text, tproj, rotary_emb, timestep=ts)
 
         shift, scale = (self.scale_shift_table + temb.unsqueeze(1)).chunk(2, dim=1)
         x = (self.norm_out(x.float()) * (1 + scale) + shift).type_as(x)

@@ -121,3 +121,35 @@ def test_fused_paths_leave_replaced_and_hooked_modules_alone():
     blk.ffn[1] = torch.nn.GELU()                             # the erf form has no fused counterpart
     with torch.no_grad():
         torch.testing.assert_close(blk._ffn_fused(x), blk.ffn(x))
+
+
+def test_only_the_pasa_processor_is_given_the_timestep_on_the_host(monkeypatch):
+    """The stock processor (whose forward may be captured in a graph) and any other one that takes a
+    timestep see the caller's own tensor, unread; the PASA processors share one host copy."""
+    from pasa_amd.processors.wan import Wan_PASA_Processor
+
+    class Takes(W.WanAttnProcessor):
+        def __call__(self, attn, hidden_states, timestep=None, **kw):
+            self.seen = timestep
+            return super().__call__(attn, hidden_states, **kw)
+
+    class Pasa(Wan_PASA_Processor):
+        pass
+
+    m = W.WanDiT(tiny_cfg(4))
+    m.blocks[1].attn1.set_processor(Takes())
+    m.blocks[2].attn1.set_processor(Wan_PASA_Processor(2))
+    m.blocks[3].attn1.set_processor(Pasa(3))
+    assert [W._reads_timestep_on_host(b) for b in m.blocks] == [False, False, True, False]
+    m.blocks[2].attn1.register_forward_pre_hook(lambda *a: None)
+    assert not W._reads_timestep_on_host(m.blocks[2])
+
+    m = W.WanDiT(tiny_cfg(2))
+    m.blocks[1].attn1.set_processor(Takes())
+    copies = []
+    for name in ("cpu", "tolist", "item"):
+        monkeypatch.setattr(torch.Tensor, name, lambda self, name=name: copies.append(name))
+    t = torch.tensor([500.0])
+    with torch.no_grad():
+        m(torch.randn(1, 16, 2, 4, 4), t, torch.randn(1, 5, m.cfg.text_dim))
+    assert m.blocks[1].attn1.processor.seen is t and not copies
