@@ -33,6 +33,7 @@ from typing import Optional, Tuple
 import torch
 import torch.nn as nn
 import torch.nn.functional as F
+from torch.nn.modules.module import _has_any_global_hook
 
 from . import ops
 from .processors.qknorm import fusable, norm_eps
@@ -190,16 +191,24 @@ class WanBlock(nn.Module):
         8960, 1110 with the GELU as a pass of its own over the 587 MB between them."""
         up, act, down = self.ffn
         if not (_plain(self.ffn, nn.Sequential) and _plain(up, nn.Linear) and _plain(act, nn.GELU)
-                and act.approximate == "tanh" and up.bias is not None):
+                and act.approximate == "tanh" and _in_type(x, up.weight, up.bias)):
             return self.ffn(x)
         h = torch._addmm_activation(up.bias, x.reshape(-1, x.shape[-1]), up.weight.t(), use_gelu=True)
         return down(h).view(*x.shape[:-1], -1)
 
 
 def _plain(module: nn.Module, cls) -> bool:
-    """``module`` is a ``cls`` itself whose call is its forward alone: no hooks of its own and not a
-    subclass or replacement (an adapter, a quantised layer) that a fused call would pass by."""
-    return type(module) is cls and not (module._forward_hooks or module._forward_pre_hooks)
+    """``module`` is a ``cls`` itself whose call is its forward alone: no hooks (its own or for all
+    modules), no forward set on the object (an offloading wrapper) and not a subclass or replacement
+    (an adapter, a quantised layer) that a fused call would pass by."""
+    return (type(module) is cls and "forward" not in vars(module) and not _has_any_global_hook()
+            and not (module._forward_hooks or module._forward_pre_hooks))
+
+
+def _in_type(x: torch.Tensor, *tensors) -> bool:
+    """All of x's type and device, with no autocast that would change either."""
+    return (not torch.is_autocast_enabled(x.device.type)
+            and all(t is not None and t.dtype == x.dtype and t.device == x.device for t in tensors))
 
 
 def _reads_timestep_on_host(block) -> bool:
@@ -211,10 +220,13 @@ def _reads_timestep_on_host(block) -> bool:
 
 def _cross_fusable(attn, x: torch.Tensor, text: torch.Tensor) -> bool:
     """Whether ``_cross_attention_fused`` computes what ``attn``'s call does: the stock processor,
-    torch RMSNorms with bf16 weights, bf16 text, head_dim 128, and nothing hooked in between."""
+    torch RMSNorms with bf16 weights, bf16 text (one row of it or more for each sample), head_dim
+    128, no autocast and nothing hooked in between."""
     C = x.shape[-1]
     return (_plain(attn, WanAttention) and type(attn.processor) is WanAttnProcessor
-            and text is not None and text.is_cuda and text.dtype == x.dtype == torch.bfloat16 and C == attn.heads * 128
+            and text is not None and x.dtype == torch.bfloat16 and C == attn.heads * 128
+            and text.dim() == 3 and text.shape[0] == x.shape[0] and text.numel() > 0
+            and _in_type(x, text, *(m.weight for m in (attn.to_q, attn.to_k, attn.to_v) if type(m) is nn.Linear))
             and all(_plain(m, nn.RMSNorm) for m in (attn.norm_q, attn.norm_k))
             and fusable(x, attn.heads, (attn.norm_q, attn.norm_k), C))
 

@@ -4,6 +4,7 @@ processor's dense branch against the harness's own dense processor."""
 import cmath
 import math
 
+import pytest
 import torch
 
 from pasa_amd import wan_dit as W
@@ -116,7 +117,17 @@ def test_fused_paths_leave_replaced_and_hooked_modules_alone():
     assert not W._plain(blk.attn2, W.WanAttention)
     handle.remove()
     assert W._plain(blk.attn2, W.WanAttention)
+    handle = torch.nn.modules.module.register_module_forward_hook(lambda m, a, o: o)
+    assert not W._plain(blk.attn2, W.WanAttention)
+    handle.remove()
+    blk.ffn[0].forward = lambda x: torch.nn.Linear.forward(blk.ffn[0], x) * 2
+    with torch.no_grad():                                    # a wrapper set on the object runs
+        torch.testing.assert_close(blk._ffn_fused(torch.ones(1, 3, 256)), blk.ffn(torch.ones(1, 3, 256)))
+    assert not W._plain(blk.ffn[0], torch.nn.Linear)
+    del blk.ffn[0].forward
     x, text = torch.randn(1, 3, 256), torch.randn(1, 5, 256)
+    with torch.no_grad(), torch.autocast("cpu", torch.bfloat16):
+        assert blk._ffn_fused(x).dtype == blk.ffn(x).dtype == torch.bfloat16
     assert not W._cross_fusable(blk.attn2, x, text)          # host tensors
     blk.ffn[1] = torch.nn.GELU()                             # the erf form has no fused counterpart
     with torch.no_grad():
@@ -126,8 +137,6 @@ def test_fused_paths_leave_replaced_and_hooked_modules_alone():
 def test_only_the_pasa_processor_is_given_the_timestep_on_the_host(monkeypatch):
     """The stock processor (whose forward may be captured in a graph) and any other one that takes a
     timestep see the caller's own tensor, unread; the PASA processors share one host copy."""
-    from pasa_amd.processors.wan import Wan_PASA_Processor
-
     class Takes(W.WanAttnProcessor):
         def __call__(self, attn, hidden_states, timestep=None, **kw):
             self.seen = timestep
@@ -153,3 +162,17 @@ def test_only_the_pasa_processor_is_given_the_timestep_on_the_host(monkeypatch):
     with torch.no_grad():
         m(torch.randn(1, 16, 2, 4, 4), t, torch.randn(1, 5, m.cfg.text_dim))
     assert m.blocks[1].attn1.processor.seen is t and not copies
+
+
+@pytest.mark.parametrize("text_shape, fused", [((2, 5, 256), True), ((1, 5, 256), False), ((2, 0, 256), False)])
+def test_fused_cross_attention_takes_one_text_per_sample(monkeypatch, text_shape, fused):
+    """A text that broadcasts over the samples, and an empty one, stay on the module's own route."""
+    cfg = W.WanDiTConfig(num_layers=1, num_attention_heads=2, ffn_dim=64, text_dim=32, freq_dim=16)
+    attn = W.WanBlock(cfg).to(torch.bfloat16).attn2
+    monkeypatch.setattr(W, "fusable", lambda *a: True)       # the device test, as on a GPU
+    x, text = torch.zeros(2, 3, 256, dtype=torch.bfloat16), torch.zeros(text_shape, dtype=torch.bfloat16)
+    assert W._cross_fusable(attn, x, text) is fused
+    with torch.autocast("cpu", torch.bfloat16):
+        assert not W._cross_fusable(attn, x, text)
+    attn.to_k.float()
+    assert not W._cross_fusable(attn, x, text)
