@@ -78,6 +78,15 @@ def fusable(x: torch.Tensor, heads: int, norms, weight_len: int) -> bool:
     return True
 
 
+def _transformed(x: torch.Tensor) -> bool:
+    """Whether something follows the operations on ``x`` that a kernel call would be invisible to:
+    reverse- or forward-mode differentiation, vmap, a tracer or compiler, a tensor subclass."""
+    return (type(x) not in (torch.Tensor, torch.nn.Parameter) or (torch.is_grad_enabled() and x.requires_grad)
+            or torch.jit.is_tracing() or torch.compiler.is_compiling()
+            or torch._C._functorch.is_functorch_wrapped_tensor(x)
+            or torch.autograd.forward_ad.unpack_dual(x).tangent is not None)
+
+
 def merge_heads(x: torch.Tensor) -> torch.Tensor:
     """[B, H, S, D] -> [B, S, H * D], the output projection's input.  A contiguous bf16 device tensor
     goes through the prologue kernel's layout pass, which moves whole rows (40 us at 12 heads x
@@ -85,7 +94,7 @@ def merge_heads(x: torch.Tensor) -> torch.Tensor:
     only viewed."""
     B, H, S, D = x.shape
     if (x.is_cuda and x.dtype == torch.bfloat16 and x.is_contiguous() and H > 1 and D in (64, 128)
-            and H * D <= MAX_ROW_CHANNELS and B <= 65535 and x.numel() > 0 and x.data_ptr() % 16 == 0
-            and not (torch.is_grad_enabled() and x.requires_grad)):
+            and H * D <= MAX_ROW_CHANNELS and B <= 65535 and x.numel() > 0 and not _transformed(x)
+            and x.data_ptr() % 16 == 0):
         return qkv_prologue(x, None, None, H, in_layout="bhsd", out_layout="bshd")[0]
     return x.transpose(1, 2).flatten(2, 3)

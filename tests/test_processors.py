@@ -360,3 +360,28 @@ def test_timestep_hook_exposes_forward_timestep():
     m.forward(1, timestep=torch.tensor([9]))
     assert [int(t) for t in seen] == [7, 9]
     assert timestep_hook.current_timestep() is None   # reset after the call
+
+
+def test_head_merge_stays_visible_to_transforms():
+    """A kernel call is invisible to autograd, forward mode, vmap and tracers: the head merge sees each."""
+    from pasa_amd.processors.qknorm import _transformed, merge_heads
+    x = torch.randn(2, 3, 4, 64)
+    seen = []
+
+    def f(t):
+        seen.append(_transformed(t))
+        return merge_heads(t)
+
+    f(x)
+    with torch.inference_mode():
+        f(torch.ones(1, 2, 3, 64))
+    torch.func.vmap(f)(x[None])
+    _, tangent = torch.func.jvp(f, (x,), (x,))
+    torch.testing.assert_close(tangent, merge_heads(x))
+    with torch.autograd.forward_ad.dual_level():
+        f(torch.autograd.forward_ad.make_dual(x, x))
+    torch.jit.trace(f, (x,), check_trace=False)
+    f(x.clone().requires_grad_())
+    with torch.no_grad():
+        f(x.clone().requires_grad_())
+    assert seen == [False, False, True, True, True, True, True, False]
