@@ -35,7 +35,8 @@ namespace pasa {
 // or half the head dim doubles that each.  D = 64 at block 64, 24 heads x 18,073 rows: 90 us with
 // tiles staged through registers and both operands gathered by 2-byte LDS reads, now 34 + 5 for the
 // reduction of split groups.
-template <int BT, bool PERM, typename E = Bf16, int D = 128>
+// AL: k and v are 16-byte aligned.
+template <int BT, bool PERM, typename E = Bf16, int D = 128, bool AL = true>
 __global__ __launch_bounds__(256, 128 / BT * (128 / D)) void k2_block_stats_dma(
     const uint16_t* __restrict__ q, const uint16_t* __restrict__ k,
     const uint16_t* __restrict__ v, float* __restrict__ qc, float* __restrict__ kc,
@@ -73,6 +74,12 @@ __global__ __launch_bounds__(256, 128 / BT * (128 / D)) void k2_block_stats_dma(
   const int64_t slice = (int64_t)bh * Tslice * D;
   const uint32_t slice_bytes = (uint32_t)T * D * 2u;  // rows >= T read as zero
   const rsrc_t qr = make_rsrc(q + slice, slice_bytes);
+  auto tile_load = [](u32x4_t rsrc, uint32_t lds, uint32_t off, uint32_t so) {
+    if constexpr (AL)
+      dma_load16_lds_nt(rsrc, lds, off, so);
+    else
+      staged_load16_lds(rsrc, lds, off, so);
+  };
   const u32x4_t kd = make_rsrc_words(k + slice, slice_bytes);
   const u32x4_t vd = make_rsrc_words(v + slice, slice_bytes);
   const uint32_t kb_lds = lds_addr(Kb);
@@ -102,8 +109,8 @@ __global__ __launch_bounds__(256, 128 / BT * (128 / D)) void k2_block_stats_dma(
       off = t_lane + SL * n * ROWB;
       soff = (uint32_t)j * BT * (uint32_t)ROWB;
     }
-    dma_load16_lds_nt(kd, kb_lds + buf * TILE + (SL * n + SL / 4 * wave) * ROWB, off, soff);
-    dma_load16_lds_nt(vd, vb_lds + buf * TILE + (SL * n + SL / 4 * wave) * ROWB, off, soff);
+    tile_load(kd, kb_lds + buf * TILE + (SL * n + SL / 4 * wave) * ROWB, off, soff);
+    tile_load(vd, vb_lds + buf * TILE + (SL * n + SL / 4 * wave) * ROWB, off, soff);
   };
   auto load_q = [&](int j, int n, uint4& qdst) {
     qdst = buf_load16_nt(qr, (st(j * BT + SL * n + prow) * D + pc * 8) * 2u);
@@ -409,6 +416,7 @@ hipError_t launch_block_stats(const void* q, const void* k, const void* v, float
     return hipErrorInvalidValue;
   if (f16 && D != 128) return hipErrorInvalidValue;  // fp16 inputs: the D = 128 kernels only
   dim3 grid(NG * split, bh);
+  const bool aligned = (((uintptr_t)k | (uintptr_t)v) & 15u) == 0;
   auto a = (const uint16_t*)q;
   auto b = (const uint16_t*)k;
   auto c = (const uint16_t*)v;
@@ -433,11 +441,17 @@ hipError_t launch_block_stats(const void* q, const void* k, const void* v, float
       dma(k2_block_stats_dma<64, false, F16>, RowMap{}, nullptr);
     else
       dma(k2_block_stats_dma<64, false, Bf16>, RowMap{}, nullptr);
-  } else if (D == 64 && BT == 128)
-    dma(k2_block_stats_dma<128, false, Bf16, 64>, RowMap{}, nullptr);
-  else if (D == 64 && BT == 64)
-    dma(k2_block_stats_dma<64, false, Bf16, 64>, RowMap{}, nullptr);
-  else
+  } else if (D == 64 && BT == 128) {
+    if (aligned)
+      dma(k2_block_stats_dma<128, false, Bf16, 64>, RowMap{}, nullptr);
+    else
+      dma(k2_block_stats_dma<128, false, Bf16, 64, false>, RowMap{}, nullptr);
+  } else if (D == 64 && BT == 64) {
+    if (aligned)
+      dma(k2_block_stats_dma<64, false, Bf16, 64>, RowMap{}, nullptr);
+    else
+      dma(k2_block_stats_dma<64, false, Bf16, 64, false>, RowMap{}, nullptr);
+  } else
     return hipErrorInvalidValue;
   if (split > 1) {
     const hipError_t e = hipGetLastError();

@@ -94,6 +94,18 @@ __device__ __forceinline__ void dma_load16_lds_nt(u32x4_t rsrc, uint32_t lds_add
                : "memory");
 }
 
+// dma_load16_lds for a base that is not 16-byte aligned, which the direct load is not issued for: the
+// rows pass through registers, and are in LDS on return (a direct load may land as early).
+__device__ __forceinline__ void staged_load16_lds(u32x4_t rsrc, uint32_t lds_addr, uint32_t byte_off, uint32_t soff) {
+  u32x4_t x;
+  asm volatile("buffer_load_dwordx4 %0, %1, %2, %3 offen\n\ts_waitcnt vmcnt(0)\n\t"
+               "ds_write_b128 %4, %0\n\ts_waitcnt lgkmcnt(0)"
+               : "=&v"(x)
+               : "v"(byte_off), "s"(rsrc), "s"(__builtin_amdgcn_readfirstlane(soff)),
+                 "v"(lds_addr + 16u * (threadIdx.x & 63u))
+               : "memory");
+}
+
 // buf_load16 with the nontemporal cache policy (cache-policy operand bit 1: nt on gfx950).
 __device__ __forceinline__ uint4 buf_load16_nt(rsrc_t r, uint32_t byte_off) {
   const u32x4_t v = __builtin_amdgcn_raw_buffer_load_b128(r, byte_off, 0, 2);

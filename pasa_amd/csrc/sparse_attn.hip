@@ -217,7 +217,8 @@ constexpr int kSchedDsRead = 0x100;
 // cover q's rows and each visits all of k's.
 // o_heads (ALL): 0, o is [slice, row, D] as q; else o is [batch, row, head, D] with o_heads heads, the
 // layout the projection after the attention reads.
-template <int D, int BT, bool ALL, bool PERM, bool PAIR, typename E, bool CROSS = false>
+// AL: k and v are 16-byte aligned.
+template <int D, int BT, bool ALL, bool PERM, bool PAIR, typename E, bool CROSS = false, bool AL = true>
 __device__ __forceinline__ void k4_body(const uint16_t* __restrict__ q, const uint16_t* __restrict__ k,
                                         const uint16_t* __restrict__ v, const unsigned char* __restrict__ pack,
                                         const uint32_t* __restrict__ selmask, uint16_t* __restrict__ o, float scale,
@@ -356,6 +357,12 @@ __device__ __forceinline__ void k4_body(const uint16_t* __restrict__ q, const ui
     v_lane[vw] = (uint32_t)(r * ROWB + ((lch ^ TL::vx(r)) << 4));
   }
 
+  auto tile_load = [](u32x4_t rsrc, uint32_t lds, uint32_t off, uint32_t so) {
+    if constexpr (AL)
+      dma_load16_lds(rsrc, lds, off, so);
+    else
+      staged_load16_lds(rsrc, lds, off, so);
+  };
   const u32x4_t kd = make_rsrc_words(k + slice, slice_bytes);
   const u32x4_t vd = make_rsrc_words(v + slice, slice_bytes);
   const uint32_t ks_lds = lds_addr(Ks);
@@ -371,7 +378,7 @@ __device__ __forceinline__ void k4_body(const uint16_t* __restrict__ q, const ui
     for (int vw = 0; vw < C::VW; ++vw)
 #pragma unroll
       for (int n = 0; n < BT / SPAN; ++n)
-        dma_load16_lds(kd, kt_lds + (SPAN * n + RPL * (qw + C::QWAVES * vw)) * ROWB, k_lane[vw] + SPAN * n * ROWB, soff);
+        tile_load(kd, kt_lds + (SPAN * n + RPL * (qw + C::QWAVES * vw)) * ROWB, k_lane[vw] + SPAN * n * ROWB, soff);
   };
   auto load_v = [&](int row0) {
     const uint32_t soff = (uint32_t)row0 * (uint32_t)ROWB;
@@ -379,7 +386,7 @@ __device__ __forceinline__ void k4_body(const uint16_t* __restrict__ q, const ui
     for (int vw = 0; vw < C::VW; ++vw)
 #pragma unroll
       for (int n = 0; n < BT / SPAN; ++n)
-        dma_load16_lds(vd, vt_lds + (SPAN * n + RPL * (qw + C::QWAVES * vw)) * ROWB, v_lane[vw] + SPAN * n * ROWB, soff);
+        tile_load(vd, vt_lds + (SPAN * n + RPL * (qw + C::QWAVES * vw)) * ROWB, v_lane[vw] + SPAN * n * ROWB, soff);
   };
 
   // MFMA A-operand offsets of K-layout tiles (K, Hbar^T, kbar): row l16 of a 16-row tile,
@@ -803,10 +810,10 @@ void k4_cross_attn(PASA_K4_PARAMS) {
 }
 
 // D = 64: half the accumulators, operands and tile bytes.
-template <int D, int BT>
+template <int D, int BT, bool AL>
 __global__ __attribute__((amdgpu_flat_work_group_size(1, 256), amdgpu_waves_per_eu(2)))
 void k4_sparse_attn(PASA_K4_PARAMS) {
-  k4_body<D, BT, false, false, BT == 64, Bf16>(PASA_K4_ARGS);
+  k4_body<D, BT, false, false, BT == 64, Bf16, false, AL>(PASA_K4_ARGS);
 }
 #undef PASA_K4_PARAMS
 #undef PASA_K4_ARGS
@@ -854,6 +861,7 @@ hipError_t launch_sparse_attn(const void* q, const void* k, const void* v, const
     hipLaunchKernelGGL(kern, g, dim3(256), 0, stream, a, b, cc, pk, selmask, oo, scale, c, T, NT, NG, NW, chunk,
                        gamma_literal, text, text_valid, n_text, bh, 0, 0, map);
   };
+  const bool aligned = (((uintptr_t)k | (uintptr_t)v) & 15u) == 0;
   static_assert(K4D<128, 128>::THREADS == 256 && K4D<128, 64, true>::THREADS == 256 &&
                     K4D<64, 128>::THREADS == 256 && K4D<64, 64, true>::THREADS == 256,
                 "four-wave workgroups");
@@ -879,9 +887,15 @@ hipError_t launch_sparse_attn(const void* q, const void* k, const void* v, const
     else
       dma(k4_sparse_attn_dma<64, false, false, true, Bf16>, grid_pairs, pair_chunk, n_text_pairs, RowMap{});
   } else if (D == 64 && BT == 128) {
-    dma(k4_sparse_attn<64, 128>, grid, xcd_chunk, 0, RowMap{});
+    if (aligned)
+      dma(k4_sparse_attn<64, 128, true>, grid, xcd_chunk, 0, RowMap{});
+    else
+      dma(k4_sparse_attn<64, 128, false>, grid, xcd_chunk, 0, RowMap{});
   } else if (D == 64 && BT == 64) {
-    dma(k4_sparse_attn<64, 64>, grid_pairs, pair_chunk, 0, RowMap{});
+    if (aligned)
+      dma(k4_sparse_attn<64, 64, true>, grid_pairs, pair_chunk, 0, RowMap{});
+    else
+      dma(k4_sparse_attn<64, 64, false>, grid_pairs, pair_chunk, 0, RowMap{});
   } else {
     return hipErrorInvalidValue;
   }

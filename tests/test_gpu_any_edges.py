@@ -178,3 +178,17 @@ def test_scores_any(device, heads, NT, D):
     assert bool(((sel.scores.cpu().double() - ref).abs() <= (D + 8) * 2.0 ** -24 * (mag + 1)).all())
     idx = O.topk_indices(sel.scores.cpu(), sel.ns)
     assert torch.equal(idx.reshape(sel.idx.shape), sel.idx.cpu())
+
+
+@pytest.mark.parametrize("T, BT, shift", [(64, 64, 1), (1000, 64, 3), (1000, 128, 4), (4500, 64, 5), (4500, 128, 1)])
+def test_head_dim_64_takes_misaligned_data(device, T, BT, shift):
+    """bf16 head dim 64 on data that is not 16-byte aligned: staged through registers, the same bits."""
+    q, k, v = make(2, T, 64, B16, T + BT)
+    outs = []
+    for n in (0, shift):
+        d = [to_dev(t, device, n) for t in (q, k, v)]
+        st = ops.block_stats(*d, BT)
+        sel = ops.select_blocks(st, 0.2, 64 ** -0.5)
+        outs.append((st.qc, st.kc, st.vc, st.hnorm, st.hgroup, ops.sparse_attn(*d, st, sel, 64 ** -0.5, BT)))
+    for a, b in zip(*outs):
+        assert torch.equal(a, b)
