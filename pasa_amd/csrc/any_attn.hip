@@ -38,8 +38,10 @@
 // and 2.1e-6 at 3,000 rows; with one sum over all 128 features 2.4e-6); K4 there 2.07 ms, 0.66 and
 // 0.45.
 // TEAM = 1 stays on the fp32 MFMA (Any32): a wave would split its own K/V rows for 16 queries.
-// Its fp32 sums are taken in short chains (half the features, a chunk of keys, 32 rows of Hbar) that
-// are then added; chains of 16 features round less and are 8% slower.
+// Its fp32 sums are taken in short chains (16 features, a chunk of keys, 32 rows of Hbar) that are
+// then added: where q and k have a common mean the scores' rounding is the error, and it grows with
+// the chain (2 heads x 1,000 rows, D 128, block 32, means 1 and 3: 1.6e-6 with one FMA per lane, 3.0e-6
+// with chains of 64 features, which are 1 to 3% faster, 1.4e-6 so).
 //
 // What bounds it: Split32, the MFMA pipe (75 GFLOP of fp32, so 450 of bf16, in 0.45 ms, where a
 // large bf16 product takes 0.34), with a third as many VALU instructions for the splits;
@@ -95,8 +97,9 @@ struct AnyCfg {
   static constexpr int ROWS = 4 * RW;            // query rows per workgroup (TEAM = 4)
   static constexpr int NF = DP * LE / 64;  // 64-byte feature steps per row: one fragment each
   static constexpr int DT = DP / 16;       // 16-feature tiles of O
-  // Keys per chunk: what two workgroups per CU leave room for (fp32 planes: 27 KB each of K and V).
-  static constexpr int KC = TEAM == 1 ? (F32 ? 16 : 32) : (SPLIT ? 32 : 64);
+  // Keys per chunk: what two workgroups per CU leave room for (fp32 planes: 27 KB each of K and V; the
+  // fp32 pass over a split tile keeps its count, whose registers the split pass needs too).
+  static constexpr int KC = TEAM == 1 ? (F32 ? 16 : 32) : (ES == 4 ? 32 : 64);
   // Row strides.  K: an odd number of 16-byte chunks, so that 16 rows read at one chunk touch 16
   // distinct bank groups.  V in 16 bits: twice an odd number of chunks, so that the 8 rows x 32
   // bytes half a wave transposes do; in fp32 4 rows x 64 bytes, four rows apart, already do.
@@ -360,12 +363,12 @@ __device__ __forceinline__ bool any_tile(
   auto step = [&](const unsigned char* Kb, const unsigned char* Vb, auto ktn, auto mask, auto on_rescale,
                   auto add) __attribute__((always_inline)) {
     constexpr int KTN = decltype(ktn)::value;
-    f32x4_t s[KTN][QT], sb[F32 || SPLIT ? KTN : 1][QT];
+    f32x4_t s[KTN][QT];
     if constexpr (SPLIT) {
       constexpr int KP = 16 * KTN * KROW;
-      // Feature steps per sum of first-order products, as in fp32: half of them (one of 96's three).
+      // Feature steps per sum of first-order products: half of them (one of 96's three).
       constexpr int HC = NF % 2 ? 1 : NF / 2;
-      f32x4_t hi[KTN][QT];
+      f32x4_t hi[KTN][QT], sb[KTN][QT];
 #pragma unroll
       for (int kt = 0; kt < KTN; ++kt)
 #pragma unroll
@@ -390,26 +393,46 @@ __device__ __forceinline__ bool any_tile(
       for (int kt = 0; kt < KTN; ++kt)
 #pragma unroll
         for (int qt = 0; qt < QT; ++qt) s[kt][qt] += sb[kt][qt];
-    } else
-#pragma unroll
-    for (int f = 0; f < NF; ++f)
+    } else if constexpr (F32) {
+      // Chains of 16 features (one f), added as a tree: longer chains round more (see above).  Two at
+      // a time, so that an MFMA does not wait for the one before it.
 #pragma unroll
       for (int kt = 0; kt < KTN; ++kt) {
-        const frag a = lds_ld<frag>(Kb, (kt * 16 + l16) * KROW + f * 64 + g4 * 16);
+        f32x4_t half[QT][3];  // [h]: the finished sum of 2^(h + 1) chains that waits for its pair
 #pragma unroll
-        for (int qt = 0; qt < QT; ++qt) {
-          if constexpr (F32) {  // chains of half the features, added: shorter fp32 chains round less
-            f32x4_t& t = f < NF / 2 ? s[kt][qt] : sb[kt][qt];
-            if (f == 0 || f == NF / 2) t = (f32x4_t){0.f, 0.f, 0.f, 0.f};
+        for (int f = 0; f < NF; f += 2) {
+          const frag a0 = lds_ld<frag>(Kb, (kt * 16 + l16) * KROW + f * 64 + g4 * 16);
+          const frag a1 = lds_ld<frag>(Kb, (kt * 16 + l16) * KROW + (f + 1) * 64 + g4 * 16);
 #pragma unroll
-            for (int i = 0; i < 4; ++i) t = __builtin_amdgcn_mfma_f32_16x16x4f32(a[i], qf[qt][f][0][i], t, 0, 0, 0);
-            if (f == NF - 1) s[kt][qt] += t;
-          } else {
+          for (int qt = 0; qt < QT; ++qt) {
+            f32x4_t t0 = {0.f, 0.f, 0.f, 0.f}, t1 = {0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+            for (int i = 0; i < 4; ++i) {
+              t0 = __builtin_amdgcn_mfma_f32_16x16x4f32(a0[i], qf[qt][f][0][i], t0, 0, 0, 0);
+              t1 = __builtin_amdgcn_mfma_f32_16x16x4f32(a1[i], qf[qt][f + 1][0][i], t1, 0, 0, 0);
+            }
+            t0 += t1;
+            int h = 0;
+#pragma unroll
+            for (int p = f / 2; p & 1; p >>= 1) t0 = half[qt][h++] + t0;
+            half[qt][h] = t0;
+            if (f == NF - 2) s[kt][qt] = NF == 6 ? half[qt][1] + t0 : t0;
+          }
+        }
+      }
+    } else {
+#pragma unroll
+      for (int f = 0; f < NF; ++f)
+#pragma unroll
+        for (int kt = 0; kt < KTN; ++kt) {
+          const frag a = lds_ld<frag>(Kb, (kt * 16 + l16) * KROW + f * 64 + g4 * 16);
+#pragma unroll
+          for (int qt = 0; qt < QT; ++qt) {
             if (f == 0) s[kt][qt] = (f32x4_t){0.f, 0.f, 0.f, 0.f};
             s[kt][qt] = E::M::mfma16(a, qf[qt][f][0], s[kt][qt]);
           }
         }
-      }
+    }
     mask(s);
 #pragma unroll
     for (int qt = 0; qt < QT; ++qt) {
@@ -960,8 +983,10 @@ __device__ __forceinline__ bool any_tile(
 
 }  // namespace
 
+// Three waves per SIMD for Any32 at DP 96: its scores' partial sums take it past 168 registers, and two
+// waves are slower than the 24 that then spill (12 heads x 7,800 rows, D 96, block 32: 850 and 779 us).
 template <typename E, int DP, int TEAM, int RW, bool VEC>
-__global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2))) void k4_any_mfma(
+__global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(AnyCfg<E, DP, TEAM, RW>::F32 && DP == 96 ? 3 : 2))) void k4_any_mfma(
     const unsigned char* __restrict__ q, const unsigned char* __restrict__ k, const unsigned char* __restrict__ v,
     const float* __restrict__ kc, const float* __restrict__ vc, const float* __restrict__ hgroup,
     const uint32_t* __restrict__ selmask, unsigned char* __restrict__ o, float scale, float c, int T, int text,

@@ -131,6 +131,42 @@ def test_dense_fp32_range(device, T, D, case):
             assert float((a - b).norm() / b.norm()) <= 1e-5, col  # cancellation within one feature: 2.5x the bound above
 
 
+def short_chain_scores(q, k):
+    """q k^T in fp32 with one FMA chain per 16 features, the chains added pairwise."""
+    x, y = q.double(), k.double()
+    parts = []
+    for f in range(0, q.shape[-1], 16):
+        acc = torch.zeros(*q.shape[:-1], k.shape[-2], dtype=torch.float64)
+        for d in range(f, min(f + 16, q.shape[-1])):
+            acc = (x[..., :, None, d] * y[..., None, :, d] + acc).float().double()
+        parts.append(acc)
+    while len(parts) > 1:
+        parts = [(sum(parts[i:i + 2])).float().double() for i in range(0, len(parts), 2)]
+    return parts[0]
+
+
+@pytest.mark.parametrize("BT", [16, 32])
+@pytest.mark.parametrize("D,mq,mk", [(128, 1.0, 3.0), (128, 3.0, 3.0), (96, 1.0, 3.0), (64, 3.0, 3.0), (37, 1.0, 3.0)])
+def test_fp32_scores_of_q_and_k_with_a_mean(device, BT, D, mq, mk):
+    """fp32 below block 64, every block selected (so plain attention): q and k with a common mean give
+    scores of about D mq mk / sqrt(D), whose rounding is then the whole error.  It is no larger than
+    with chains of 16 features in 64-bit arithmetic otherwise, but for a quarter (the order within a chain
+    is another) and what the exponentials and P V add (4e-7, as with no mean)."""
+    q, k, v = make(1, 512, D, F32, D + BT)
+    q, k = q + mq, k + mk
+    d = [t.to(device) for t in (q, k, v)]
+    scale = D ** -0.5
+    st = ops.block_stats(*d, BT, 8)
+    sel = ops.select_blocks(st, 1.0, scale)
+    o = ops.sparse_attn(*d, st, sel, scale, BT, group_size=8).double().cpu()
+    es = O.effective_scale(scale)
+    ref = torch.softmax(q.double() @ k.double().transpose(-1, -2) * es, -1) @ v.double()
+    short = torch.softmax(short_chain_scores(q, k) * es, -1) @ v.double()
+    err, bound = (float((x - ref).norm() / ref.norm()) for x in (o, short))
+    print(f"[edges] means {mq} {mk} BT={BT} D={D}: rel {err:.2e}, chains of 16 {bound:.2e}", flush=True)
+    assert err <= 1.25 * bound + 4e-7
+
+
 @pytest.mark.parametrize("heads,T,D,BT,G,dtype", [(2, 1024, 64, 64, 32, F32), (1, 777, 37, 16, 50, F16),
                                                   (3, 1000, 96, 32, 16, B16), (1, 300, 128, 256, 2, F32),
                                                   (2, 3001, 64, 64, 32, B16), (1, 4099, 64, 128, 32, B16)])
