@@ -142,28 +142,24 @@ __device__ __forceinline__ uint4 load_elems(const unsigned char* row, int c, int
   return make_uint4(w[0], w[1], w[2], w[3]);
 }
 
-// Four fp32 as three bf16 each, x = x1 + x2 + x3: x1 is x cut to its upper 16 bits (so that no
-// rounding overflows), x2 and x3 the rounded rests; together they hold all 24 bits of x.  The rest
-// of an infinity or NaN is NaN.
+// Four fp32 as three bf16 each, x = x1 + x2 + x3, each part the rounded rest of the ones before it;
+// together they hold all 24 bits of x (down to 2^-110, below which x3 is a bf16 subnormal).  The rest of
+// an infinity, of a NaN or of an x that rounds to infinity is NaN.
 __device__ __forceinline__ void split4(const float (&x)[4], uint2 (&pl)[3]) {
-  uint32_t u[4];
-  float r[4];
+  float r[4] = {x[0], x[1], x[2], x[3]};
 #pragma unroll
-  for (int i = 0; i < 4; ++i) {
-    u[i] = __float_as_uint(x[i]);
-    r[i] = x[i] - __uint_as_float(u[i] & 0xffff0000u);
+  for (int i = 0; i < 3; ++i) {
+    pl[i] = make_uint2(Bf16::pack2(r[0], r[1]), Bf16::pack2(r[2], r[3]));
+    r[0] -= __uint_as_float(pl[i].x << 16);
+    r[1] -= __uint_as_float(pl[i].x & 0xffff0000u);
+    r[2] -= __uint_as_float(pl[i].y << 16);
+    r[3] -= __uint_as_float(pl[i].y & 0xffff0000u);
   }
-  pl[0] = make_uint2(__builtin_amdgcn_perm(u[1], u[0], 0x07060302u), __builtin_amdgcn_perm(u[3], u[2], 0x07060302u));
-  pl[1] = make_uint2(Bf16::pack2(r[0], r[1]), Bf16::pack2(r[2], r[3]));
-  r[0] -= __uint_as_float(pl[1].x << 16);
-  r[1] -= __uint_as_float(pl[1].x & 0xffff0000u);
-  r[2] -= __uint_as_float(pl[1].y << 16);
-  r[3] -= __uint_as_float(pl[1].y & 0xffff0000u);
-  pl[2] = make_uint2(Bf16::pack2(r[0], r[1]), Bf16::pack2(r[2], r[3]));
 }
 
 // For j = 0, 1: hi[j] += a1 b1 and lo[j] += the five products of the next orders of a = a[j], smallest
-// first; what is left out is below 2^-24 of a b.  The two sums alternate, held in this order: an MFMA
+// first.  With |x2| <= 2^-8 |x| and |x3| <= 2^-17 |x| what is left out (x2 y3 + x3 y2 + x3 y3) is at most
+// 2^-24 (1 + 2^-10) of a b (5.4e-2 of 2^-24 on average; with x1 cut instead of rounded up to 3.9 of 2^-24).  The two sums alternate, held in this order: an MFMA
 // that adds to the one before waits for it (480p shape above: 625 us with one after the other,
 // 615 in the compiler's order, 609 so).
 __device__ __forceinline__ void mfma_split(const bf16x8_t (&a)[2][3], const bf16x8_t (&b)[3], f32x4_t* const (&hi)[2],

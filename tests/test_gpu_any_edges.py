@@ -167,6 +167,28 @@ def test_fp32_scores_of_q_and_k_with_a_mean(device, BT, D, mq, mk):
     assert err <= 1.25 * bound + 4e-7
 
 
+@pytest.mark.parametrize("D", [4, 5, 68, 100])
+def test_fp32_split_product(device, D):
+    """fp32 on the bf16 MFMA: one key of 64 has scores s = q a scale of -20 to -80, the others 0, so its
+    weight is exp(s) / (63 + exp(s)) and shows the relative error of a single product times |s|.  That
+    is at most 2^-24 for what the product leaves out, 2^-24 for its rounding and 2^-24 for that of
+    s log2(e); a part cut instead of rounded leaves out up to 3.9 of 2^-24.  The exponential, the sum and
+    the quotient round to 4 x 2^-23 more."""
+    heads, T = 512, 64
+    g = torch.Generator().manual_seed(D)
+    q, k, v = (torch.zeros(1, heads, T, D) for _ in range(3))
+    scale = 0.5
+    q[..., D - 1] = 8 + 8 * torch.rand(1, heads, T, generator=g)
+    k[..., T // 2, D - 1] = -5 - 5 * torch.rand(1, heads, generator=g)
+    v[..., T // 2, 0] = 1.0
+    o = ops.dense_attention(*(t.to(device) for t in (q, k, v)), scale=scale)[..., 0].double().cpu()
+    s = q[..., D - 1].double() * k[..., T // 2, D - 1, None].double() * O.effective_scale(scale)
+    ref = torch.exp(s) / (T - 1 + torch.exp(s))
+    err = ((o / ref - 1).abs() - 4 * 2.0 ** -23) / (s.abs() * 2.0 ** -24)
+    print(f"[edges] split product D={D}: {float(err.max()):.2f} of 2^-24 per unit of score", flush=True)
+    assert float(err.max()) <= 3.1
+
+
 @pytest.mark.parametrize("heads,T,D,BT,G,dtype", [(2, 1024, 64, 64, 32, F32), (1, 777, 37, 16, 50, F16),
                                                   (3, 1000, 96, 32, 16, B16), (1, 300, 128, 256, 2, F32),
                                                   (2, 3001, 64, 64, 32, B16), (1, 4099, 64, 128, 32, B16)])
