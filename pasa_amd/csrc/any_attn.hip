@@ -143,8 +143,9 @@ __device__ __forceinline__ uint4 load_elems(const unsigned char* row, int c, int
 }
 
 // Four fp32 as three bf16 each, x = x1 + x2 + x3, each part the rounded rest of the ones before it;
-// together they hold all 24 bits of x (down to 2^-110, below which x3 is a bf16 subnormal).  The rest of
-// an infinity, of a NaN or of an x that rounds to infinity is NaN.
+// together they hold all 24 bits of x down to 2^-110, below which x3 is a bf16 subnormal: operands are
+// split times a power of two (kUp below), which makes the parts of every fp32 exact.  The rest of an
+// infinity, of a NaN or of an x that rounds to infinity is NaN.
 __device__ __forceinline__ void split4(const float (&x)[4], uint2 (&pl)[3]) {
   float r[4] = {x[0], x[1], x[2], x[3]};
 #pragma unroll
@@ -176,9 +177,19 @@ __device__ __forceinline__ void mfma_split(const bf16x8_t (&a)[2][3], const bf16
   }
 }
 
+// Powers of two that Split32 multiplies operands by before their split (16 or more cover the subnormals,
+// whose last bit is 2^-149 where a bf16 part's is 2^-133).  The scores are then 2^40, O 2^56 times
+// their values, in P V^ as in q Hbar.  K stays as it is: with q below 2^88 (above, its parts are not
+// finite) a part below 2^-133 of it moves no exponent c s by more than 2^-28.
+// Without them v of 2^-118 comes out to 6.7e-6, of 2^-130 to 2.8e-2; with them as with fp32 products.
+// They cost 1 to 2% (12 heads x 7,800 rows, block 64: D 128 564 -> 571 us, D 64 276 -> 281).
+constexpr float kUpQ = 0x1p40f, kUpP = 0x1p16f, kUpV = 0x1p40f, kUpH = 0x1p16f;
+constexpr float kDownS = 0x1p-40f, kDownO = 0x1p-56f;
+constexpr float kMinSplitC = 0x1p-40f, kMaxSplitC = 0x1p12f;  // the c that this holds for
+
 constexpr uint32_t kOutside = 0x80000000u;  // a buffer offset past every chunk: the load gives zeros
 
-// One workgroup's tile of k4_any_mfma, in the workgroup's `lds`; false: the tile holds a NaN and
+// One workgroup's tile of k4_any_mfma, in the workgroup's `lds`; false: the tile is not finite and
 // nothing has been stored (split fp32 only).
 // VEC: the rows of q, k, v, o, kc, vc and hgroup are whole aligned 16-byte chunks.  They are then
 // loaded through buffer resources over just the rows wanted, so rows past them read as zero with
@@ -271,8 +282,8 @@ __device__ __forceinline__ bool any_tile(
             const uint4 y = load_elems<4>(qrow, d / 4, D);
             x4 = (u32x4_t){y.x, y.y, y.z, y.w};
           }
-          const float x[4] = {__uint_as_float(x4[0]), __uint_as_float(x4[1]), __uint_as_float(x4[2]),
-                              __uint_as_float(x4[3])};
+          const float x[4] = {__uint_as_float(x4[0]) * kUpQ, __uint_as_float(x4[1]) * kUpQ,
+                              __uint_as_float(x4[2]) * kUpQ, __uint_as_float(x4[3]) * kUpQ};
           uint2 pl[3];
           split4(x, pl);
 #pragma unroll
@@ -345,15 +356,17 @@ __device__ __forceinline__ bool any_tile(
     return lds_ld<float>(rows, (r + 4 * g4) * VROW + dt * 64 + l16 * 4);
   };
 
-  // Four fp32 as their three parts, one plane each.
-  auto st_split = [&](unsigned char* base, int plane, int off, const uint4& x) {
-    const float f[4] = {__uint_as_float(x.x), __uint_as_float(x.y), __uint_as_float(x.z), __uint_as_float(x.w)};
+  // Four fp32, times `up`, as their three parts, one plane each.
+  auto st_split = [&](unsigned char* base, int plane, int off, const uint4& x, float up) {
+    const float f[4] = {__uint_as_float(x.x) * up, __uint_as_float(x.y) * up, __uint_as_float(x.z) * up,
+                        __uint_as_float(x.w) * up};
     uint2 pl[3];
     split4(f, pl);
 #pragma unroll
     for (int i = 0; i < 3; ++i) lds_st(base, i * plane + off, pl[i]);
   };
 
+  const float cs = SPLIT ? c * kDownS : c;
   // One online-softmax step over the 16 KTN rows at Kb / Vb.  mask(s) drops scores (to -inf),
   // on_rescale(qt, alpha) sees a rise of the running max, add(qt, key, p) every weight.
   auto step = [&](const unsigned char* Kb, const unsigned char* Vb, auto ktn, auto mask, auto on_rescale,
@@ -437,7 +450,7 @@ __device__ __forceinline__ bool any_tile(
       for (int kt = 0; kt < KTN; ++kt)
 #pragma unroll
         for (int i = 0; i < 4; ++i) mx = fmaxf(mx, s[kt][qt][i]);
-      const float mxc = quad16_max(mx) * c;
+      const float mxc = quad16_max(mx) * cs;
       if (__any(mxc > m_run[qt])) {
         const float m_new = fmaxf(m_run[qt], mxc);
         const float alpha = fast_exp2(m_run[qt] - m_new);  // 0 on the first step
@@ -453,7 +466,7 @@ __device__ __forceinline__ bool any_tile(
       for (int kt = 0; kt < KTN; ++kt)
 #pragma unroll
         for (int i = 0; i < 4; ++i) {
-          const float p = fast_exp2(fmaf(s[kt][qt][i], c, -m_run[qt]));
+          const float p = fast_exp2(fmaf(s[kt][qt][i], cs, -m_run[qt]));
           add(qt, 16 * kt + i, p);
           s[kt][qt][i] = p;
         }
@@ -492,7 +505,7 @@ __device__ __forceinline__ bool any_tile(
         u32x4_t pw[3];
 #pragma unroll
         for (int h = 0; h < 2; ++h) {
-          const float x[4] = {s[h][qt][0], s[h][qt][1], s[h][qt][2], s[h][qt][3]};
+          const float x[4] = {s[h][qt][0] * kUpP, s[h][qt][1] * kUpP, s[h][qt][2] * kUpP, s[h][qt][3] * kUpP};
           uint2 pl[3];
           split4(x, pl);
 #pragma unroll
@@ -626,8 +639,8 @@ __device__ __forceinline__ bool any_tile(
       for (int p = 0; p < C::PASSES; ++p) {
         const int r = p * C::RPP + sr;
         if constexpr (SPLIT) {
-          st_split(Kb, KC * KROW, r * KROW + (sc >> 3) * 64 + (sc & 3) * 16 + ((sc >> 2) & 1) * 8, kreg[p]);
-          st_split(Vb, KC * VROW, r * VROW + sc * 8, vreg[p]);
+          st_split(Kb, KC * KROW, r * KROW + (sc >> 3) * 64 + (sc & 3) * 16 + ((sc >> 2) & 1) * 8, kreg[p], 1.f);
+          st_split(Vb, KC * VROW, r * VROW + sc * 8, vreg[p], kUpV);
           continue;
         }
         if constexpr (F32) {
@@ -703,9 +716,9 @@ __device__ __forceinline__ bool any_tile(
       return ~sel & (cn >= 32 ? 0xffffffffu : (1u << cn) - 1u);
     };
     // Four floats to LDS as four elements of the input type (or their parts, `plane` bytes apart).
-    auto st4 = [&](unsigned char* base, int plane, int off16, int off32, const float4& x) {
+    auto st4 = [&](unsigned char* base, int plane, int off16, int off32, const float4& x, float up) {
       if constexpr (SPLIT)
-        st_split(base, plane, off16, __builtin_bit_cast(uint4, x));
+        st_split(base, plane, off16, __builtin_bit_cast(uint4, x), up);
       else if constexpr (F32)
         lds_st(base, off32, x);
       else
@@ -775,7 +788,7 @@ __device__ __forceinline__ bool any_tile(
 #pragma unroll
       for (int p = 0; p < HP; ++p) {
         const int r = p * C::RPP4 + r4;
-        st4(Hs, C::HR * VROW, r * VROW + c4 * 8, r * VROW + c4 * 16, hx[p]);
+        st4(Hs, C::HR * VROW, r * VROW + c4 * 8, r * VROW + c4 * 16, hx[p], kUpH);
       }
     };
     auto stash_z = [&]() {
@@ -784,8 +797,8 @@ __device__ __forceinline__ bool any_tile(
       for (int p = 0; p < ZP; ++p) {
         const int r = p * C::RPP4 + r4;
         st4(Kz, C::KZ * KROW, r * KROW + (c4 >> 3) * 64 + (c4 & 3) * 16 + ((c4 >> 2) & 1) * 8, r * KROW + c4 * 16,
-            zk[p]);
-        st4(Vz, C::KZ * VROW, r * VROW + c4 * 8, r * VROW + c4 * 16, zv[p]);
+            zk[p], 1.f);
+        st4(Vz, C::KZ * VROW, r * VROW + c4 * 8, r * VROW + c4 * 16, zv[p], kUpV);
       }
     };
     // Per row, of the current group: the sums of p and of p times the block's length, relative to
@@ -941,7 +954,7 @@ __device__ __forceinline__ bool any_tile(
 #pragma unroll
       for (int dt = 0; dt < DT; ++dt) t += (oacc[dt][qt][0] + oacc[dt][qt][1]) + (oacc[dt][qt][2] + oacc[dt][qt][3]);
     }
-    if (__syncthreads_or(t != t)) return false;
+    if (__syncthreads_or(!(fabsf(t) < INFINITY))) return false;
   }
 
   // o = A / (L + Gamma) (:258-259), stored in the input type (:262).
@@ -954,8 +967,9 @@ __device__ __forceinline__ bool any_tile(
 #pragma unroll
       for (int dt = 0; dt < DT; ++dt) {
         const int e = 16 * dt + 4 * g4;
-        const float x[4] = {oacc[dt][qt][0] / den, oacc[dt][qt][1] / den, oacc[dt][qt][2] / den,
-                            oacc[dt][qt][3] / den};
+        float x[4];
+#pragma unroll
+        for (int i = 0; i < 4; ++i) x[i] = SPLIT ? oacc[dt][qt][i] / den * kDownO : oacc[dt][qt][i] / den;
         if (VEC && e < D) {
           if constexpr (ES == 4)
             *reinterpret_cast<float4*>(orow + e * 4) = make_float4(x[0], x[1], x[2], x[3]);
@@ -991,10 +1005,12 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(AnyCfg<E, D
   using C = AnyCfg<E, DP, TEAM, RW>;
   if constexpr (E::SPLIT) {
     // An infinite operand meets the zero parts of another and gives NaN where an fp32 product would
-    // not: a tile with a NaN is done again in fp32.
+    // not, and the scaled sums leave the range before the sums themselves: a tile that is not finite is
+    // done again in fp32.
     using C32 = AnyCfg<Any32, DP, TEAM, RW>;
     __shared__ __attribute__((aligned(16))) unsigned char lds[C::LDS > C32::LDS ? C::LDS : C32::LDS];
-    if (any_tile<E, DP, TEAM, RW, VEC>(lds, q, k, v, kc, vc, hgroup, selmask, o, scale, c, T, text, text_valid, D, BT,
+    if (c >= kMinSplitC && c <= kMaxSplitC &&
+        any_tile<E, DP, TEAM, RW, VEC>(lds, q, k, v, kc, vc, hgroup, selmask, o, scale, c, T, text, text_valid, D, BT,
                                        NT, G, NG, NW, gamma_literal, all, nvt, ntiles))
       return;
     any_tile<Any32, DP, TEAM, RW, VEC>(lds, q, k, v, kc, vc, hgroup, selmask, o, scale, c, T, text, text_valid, D, BT,

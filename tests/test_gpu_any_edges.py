@@ -189,6 +189,36 @@ def test_fp32_split_product(device, D):
     assert float(err.max()) <= 3.1
 
 
+@pytest.mark.parametrize("eq,ek,ev", [(0, 0, -112), (0, 0, -121), (-121, 121, 0), (121, -121, 0), (85, -85, -118),
+                                      (-118, 90, 30), (0, 0, 100), (0, 0, -130), (0, 0, -140)])
+@pytest.mark.parametrize("D,BT", [(64, 64), (37, 128), (128, 64)])
+def test_fp32_range(device, D, BT, eq, ek, ev):
+    """fp32 down to the subnormals and up to where the split sums leave the range: q, k and v times 2^eq,
+    2^ek and 2^ev, with the scores' magnitude kept.  Relative error as for ordinary values, and for
+    subnormal results half of 2^-149 each besides.  (Where v or the block
+    moments k v are below 2^-121 only the dense call: the statistics' own sums are subnormal there.)"""
+    T = 300
+    q, k, v = make(1, T, D, F32, T + D)
+    d = [(t * 2.0 ** e) for t, e in zip((q, k, v), (eq, ek, ev))]
+    c = [t.to(device) for t in d]
+    scale = D ** -0.5 * 2.0 ** -(eq + ek)
+
+    def check(o, ref):
+        err, n = float((o - ref).norm()), float(ref.norm())
+        print(f"[edges] fp32 range D={D} BT={BT} 2^{eq} 2^{ek} 2^{ev}: rel {err / n:.2e}", flush=True)
+        assert err <= 4e-6 * n + 2.0 ** -150 * o.numel() ** 0.5
+
+    es = O.effective_scale(scale)
+    ref = torch.softmax(d[0].double() @ d[1].double().transpose(-1, -2) * es, -1) @ d[2].double()
+    check(ops.dense_attention(*c, scale=scale).double().cpu(), ref)
+    if min(ev, ek + ev) < -121:
+        return
+    st = ops.block_stats(*c, BT, 2)
+    sel = ops.select_blocks(st, 0.4, scale)
+    o = ops.sparse_attn(*c, st, sel, scale, BT, group_size=2).double().cpu()
+    check(o, O.pisa_pg_attention(*d, 0.4, BT, 2, scale, dtype=torch.float64, indices=sel.idx.cpu()))
+
+
 @pytest.mark.parametrize("heads,T,D,BT,G,dtype", [(2, 1024, 64, 64, 32, F32), (1, 777, 37, 16, 50, F16),
                                                   (3, 1000, 96, 32, 16, B16), (1, 300, 128, 256, 2, F32),
                                                   (2, 3001, 64, 64, 32, B16), (1, 4099, 64, 128, 32, B16)])
