@@ -368,9 +368,10 @@ __device__ __forceinline__ bool any_tile(
 
   const float cs = SPLIT ? c * kDownS : c;
   // One online-softmax step over the 16 KTN rows at Kb / Vb.  mask(s) drops scores (to -inf),
-  // on_rescale(qt, alpha) sees a rise of the running max, add(qt, key, p) every weight.
-  auto step = [&](const unsigned char* Kb, const unsigned char* Vb, auto ktn, auto mask, auto on_rescale,
-                  auto add) __attribute__((always_inline)) {
+  // on_rescale(qt, alpha) sees a rise of the running max, add(qt, key, p) every weight; rows_v(a, key)
+  // sees every operand of V: key 16 kt + i of this lane in fp32, the eight of a 32-key step in 16 bits.
+  auto step = [&](const unsigned char* Kb, const unsigned char* Vb, auto ktn, auto mask, auto on_rescale, auto add,
+                  auto rows_v) __attribute__((always_inline)) {
     constexpr int KTN = decltype(ktn)::value;
     f32x4_t s[KTN][QT];
     if constexpr (SPLIT) {
@@ -486,7 +487,7 @@ __device__ __forceinline__ bool any_tile(
           for (int i = 0; i < 4; ++i)
 #pragma unroll
             for (int j = 0; j < 2; ++j) {
-              const float a = vt32(Vb, 16 * kt + i, d2 + j);
+              const float a = rows_v(vt32(Vb, 16 * kt + i, d2 + j), 16 * kt + i);
 #pragma unroll
               for (int qt = 0; qt < QT; ++qt)
                 t[j][qt] = __builtin_amdgcn_mfma_f32_16x16x4f32(a, s[kt][qt][i], t[j][qt], 0, 0, 0);
@@ -543,7 +544,7 @@ __device__ __forceinline__ bool any_tile(
         }
 #pragma unroll
         for (int dt = 0; dt < DT; ++dt) {
-          const frag a = vt16(Vb, s2, dt);
+          const frag a = rows_v(vt16(Vb, s2, dt), 32 * s2);
 #pragma unroll
           for (int qt = 0; qt < QT; ++qt) oacc[dt][qt] = E::M::mfma16(a, pf[qt], oacc[dt][qt]);
         }
@@ -675,7 +676,7 @@ __device__ __forceinline__ bool any_tile(
                      if (16 * kt + i >= lim) s[kt][qt][i] = -INFINITY;
              }
            },
-           [](int, float) {}, [&](int qt, int, float p) { l_run[qt] += p; });
+           [](int, float) {}, [&](int qt, int, float p) { l_run[qt] += p; }, [](auto a, int) { return a; });
       n = n2;
     }
   }
@@ -726,14 +727,14 @@ __device__ __forceinline__ bool any_tile(
     };
     const bool in4 = 4 * c4 < D;
     const uint32_t off4 = in4 ? (uint32_t)(r4 * D + 4 * c4) * 4u : kOutside;
-    // Piece c4 of row r0 + r4 of the statistics rows at base, of which n are wanted.
-    auto load4 = [&](const float* base, const rsrc_t& rs, int r0, int n) -> float4 {
+    // Piece c4 of row r0 + r4 of the statistics rows at base, of which n are wanted; zero without `want`.
+    auto load4 = [&](const float* base, const rsrc_t& rs, int r0, int n, bool want = true) -> float4 {
       if constexpr (VEC) {
-        const uint4 x = buf_load16(rs, off4 + (uint32_t)(r0 * D) * 4u);
+        const uint4 x = buf_load16(rs, want ? off4 + (uint32_t)(r0 * D) * 4u : kOutside);
         return make_float4(__uint_as_float(x.x), __uint_as_float(x.y), __uint_as_float(x.z), __uint_as_float(x.w));
       } else {
         uint4 x = make_uint4(0u, 0u, 0u, 0u);
-        if (r0 + r4 < n) x = load_elems<4>((const unsigned char*)(base + (int64_t)(r0 + r4) * D), c4, D);
+        if (want && r0 + r4 < n) x = load_elems<4>((const unsigned char*)(base + (int64_t)(r0 + r4) * D), c4, D);
         return make_float4(__uint_as_float(x.x), __uint_as_float(x.y), __uint_as_float(x.z), __uint_as_float(x.w));
       }
     };
@@ -773,14 +774,17 @@ __device__ __forceinline__ bool any_tile(
 #pragma unroll
       for (int p = 0; p < HP; ++p) hx[p] = load4(hb, rh, p * C::RPP4, n);
     };
+    // V^ of a selected block is taken as zero: its weight is, but 0 times a sum that left the type's
+    // range is NaN.  TEAM = 1: each wave selects its own, and clears them from its operands (below).
     auto fetch_z = [&](int jc, int cn) {
+      const uint32_t approx = TEAM == 1 ? 0xffffffffu : approx_bits(jc, cn);
       const float* kb = kcb + (int64_t)jc * D;
       const float* vb = vcb + (int64_t)jc * D;
       const rsrc_t rk = make_rsrc(kb, (uint32_t)(cn * D * 4)), rv = make_rsrc(vb, (uint32_t)(cn * D * 4));
 #pragma unroll
       for (int p = 0; p < ZP; ++p) {
         zk[p] = load4(kb, rk, p * C::RPP4, cn);
-        zv[p] = load4(vb, rv, p * C::RPP4, cn);
+        zv[p] = load4(vb, rv, p * C::RPP4, cn, (approx >> (p * C::RPP4 + r4)) & 1u);
       }
     };
     auto stash_h = [&]() {
@@ -806,6 +810,7 @@ __device__ __forceinline__ bool any_tile(
     // :231-235), then f = scale * (sum of p).
     float psum[QT], gsum[QT], f[QT];
     int pg = -1;  // the group of the previous item
+    bool mine = true;  // this wave approximates some block of the group (TEAM = 1: another wave may instead)
     bool more = next_item();
     if (more && !F32) {
       fetch_z(ijc, min(C::KZ, group_end(ig) - ijc));
@@ -833,29 +838,48 @@ __device__ __forceinline__ bool any_tile(
         if (first) {
 #pragma unroll
           for (int qt = 0; qt < QT; ++qt) psum[qt] = gsum[qt] = 0.f;
+          mine = false;
         }
         // Zero order: o += p V^.
-        const uint32_t ub = approx_bits(jc, min(C::KZ, group_end(g) - jc)) >> (4 * g4);
+        const uint32_t approx = approx_bits(jc, min(C::KZ, group_end(g) - jc));
+        const bool visit = TEAM != 1 || approx != 0u;
+        if (visit) mine = true;
+        const uint32_t ub = approx >> (4 * g4);
+        u32x4_t keep;  // 16 bits: keys 4 g4 .. + 3 and 16 + 4 g4 .. + 3 of the step, two to a word
+#pragma unroll
+        for (int i = 0; i < 4; ++i) {
+          const uint32_t two = ub >> (2 * (i & 1) + 16 * (i >> 1));
+          keep[i] = ((two & 1u) ? 0xffffu : 0u) | ((two & 2u) ? 0xffff0000u : 0u);
+        }
         const int last = NT - 1 - jc - 4 * g4;  // this lane's key index of the last block
-        step(Kz, Vz, std::integral_constant<int, C::KZ / 16>{},
-             [&](auto& s) {
+        if (visit)
+          step(Kz, Vz, std::integral_constant<int, C::KZ / 16>{},
+               [&](auto& s) {
 #pragma unroll
-               for (int kt = 0; kt < C::KZ / 16; ++kt)
+                 for (int kt = 0; kt < C::KZ / 16; ++kt)
 #pragma unroll
-                 for (int qt = 0; qt < QT; ++qt)
+                   for (int qt = 0; qt < QT; ++qt)
 #pragma unroll
-                   for (int i = 0; i < 4; ++i)
-                     if (!((ub >> (16 * kt + i)) & 1u)) s[kt][qt][i] = -INFINITY;
-             },
-             [&](int qt, float alpha) {
-               psum[qt] *= alpha;
-               gsum[qt] *= alpha;
-               if (!gamma_literal) g_run[qt] *= alpha;
-             },
-             [&](int qt, int key, float p) {
-               psum[qt] += p;
-               gsum[qt] += p * (float)(key == last ? last_len : BT);
-             });
+                     for (int i = 0; i < 4; ++i)
+                       if (!((ub >> (16 * kt + i)) & 1u)) s[kt][qt][i] = -INFINITY;
+               },
+               [&](int qt, float alpha) {
+                 psum[qt] *= alpha;
+                 gsum[qt] *= alpha;
+                 if (!gamma_literal) g_run[qt] *= alpha;
+               },
+               [&](int qt, int key, float p) {
+                 psum[qt] += p;
+                 gsum[qt] += p * (float)(key == last ? last_len : BT);
+               },
+               [&](auto a, int key) {
+                 if constexpr (TEAM != 1)
+                   return a;
+                 else if constexpr (F32)
+                   return (ub >> key) & 1u ? a : 0.f;
+                 else
+                   return __builtin_bit_cast(frag, __builtin_bit_cast(u32x4_t, a) & keep);
+               });
         if (more && ig == g && ihs == 0) continue;  // another chunk of this group
 #pragma unroll
         for (int qt = 0; qt < QT; ++qt) {
@@ -864,7 +888,9 @@ __device__ __forceinline__ bool any_tile(
         }
         if (SPLIT) continue;  // Hbar comes with the next items
       }
-      // First order: o += f (q . Hbar), over this item's rows of Hbar.
+      // First order: o += f (q . Hbar), over this item's rows of Hbar.  A wave that selects the whole
+      // group has f = 0 and leaves Hbar, which may not be finite, alone.
+      if (TEAM == 1 && !mine) continue;
       if constexpr (F32) {
 #pragma unroll
         for (int h = 0; h < DP / C::HR; ++h) {

@@ -219,6 +219,67 @@ def test_fp32_range(device, D, BT, eq, ek, ev):
     check(o, O.pisa_pg_attention(*d, 0.4, BT, 2, scale, dtype=torch.float64, indices=sel.idx.cpu()))
 
 
+def selection(rows, device):
+    """The selection of one slice whose query block I selects the key blocks rows[I]."""
+    NT = len(rows)
+    m = torch.zeros(NT, (NT + 31) // 32, dtype=torch.int64)
+    for i, js in enumerate(rows):
+        for j in js:
+            m[i, j // 32] |= 1 << (j % 32)
+    idx = torch.tensor([sorted(js) for js in rows], dtype=torch.int32)[None, None]
+    mask = torch.where(m >= 2 ** 31, m - 2 ** 32, m).to(torch.int32)[None, None].to(device)
+    return ops.Selection(None, mask, None, idx.shape[-1]), idx
+
+
+@pytest.mark.parametrize("BT,D,dtype", [(16, 72, F32), (16, 72, B16), (32, 40, F16), (32, 128, F32), (64, 72, F32),
+                                        (64, 72, B16), (128, 37, F16), (128, 128, B16), (128, 64, B16)])
+def test_infinity_in_a_selected_group_stays_there(device, BT, D, dtype):
+    """Two value rows of one group hold an infinity.  Query blocks that select the whole group do not
+    approximate it: their output is infinite in those two features and what it was in all others, whatever
+    other query blocks of their workgroup approximate."""
+    G = 32 if ops.tuned_shape(dtype, D, BT) else 2
+    NT = 2 * G + 6
+    T = NT * BT - 3
+    q, k, v = make(1, T, D, dtype, T + D)
+    whole = set(range(G))                                   # the first group
+    rows = [whole | {NT - 1, NT - 2} if i % 2 == 0 else set(range(NT - 1, NT - 1 - G - 2, -1)) for i in range(NT)]
+    sel, idx = selection(rows, device)
+    bad = v.clone()
+    bad[0, 0, 3, 7], bad[0, 0, (G - 1) * BT + 5, 30] = torch.inf, -torch.inf
+    scale = D ** -0.5
+    d = [t.to(device) for t in (q, k, bad)]
+    st = ops.block_stats(*d, BT, G)
+    o = ops.sparse_attn(*d, st, sel, scale, BT, group_size=G).double().cpu()
+    ref = O.pisa_pg_attention(q, k, v, 0.5, BT, G, scale, dtype=torch.float64, indices=idx)
+    even = (torch.arange(T) // BT) % 2 == 0
+    fine = [c for c in range(D) if c not in (7, 30)]
+    assert bool((o[..., even, 7] == torch.inf).all()) and bool((o[..., even, 30] == -torch.inf).all())
+    a, b = o[..., fine], ref[..., fine]
+    err = float((a - b).norm() / b.norm())
+    print(f"[edges] infinity BT={BT} D={D} {dtype}: rel {err:.2e}", flush=True)
+    assert err <= {F32: 4e-6, B16: 1e-2, F16: 2e-3}[dtype]    # 16 bits: kc, vc, Hbar, P and o rounded once each
+
+
+@pytest.mark.parametrize("BT,D", [(16, 72), (32, 128), (64, 72), (128, 40), (256, 96)])
+def test_a_selected_block_whose_value_sum_leaves_fp16(device, BT, D):
+    """Every query block selects block 4, whose values add up to more than fp16 holds; the other blocks of
+    its group are approximated, and that sum, whose weight there is 0, does not show."""
+    NT = 9
+    T = NT * BT - 3
+    q, k, v = make(1, T, D, F16, T + D)
+    v[..., 4 * BT:5 * BT, :] += 8192.0
+    sel, idx = selection([{4, i if i != 4 else 0} for i in range(NT)], device)
+    scale = D ** -0.5
+    d = [t.to(device) for t in (q, k, v)]
+    st = ops.block_stats(*d, BT, 4)
+    assert bool((st.vc[0, 0, 4] > 65520).all()) and bool((st.hgroup.abs() < 65504).all())
+    o = ops.sparse_attn(*d, st, sel, scale, BT, group_size=4).double().cpu()
+    ref = O.pisa_pg_attention(q, k, v, 0.5, BT, 4, scale, dtype=torch.float64, indices=idx)
+    err = float((o - ref).norm() / ref.norm())
+    print(f"[edges] fp16 value sum BT={BT} D={D}: rel {err:.2e}", flush=True)
+    assert err <= 2e-3
+
+
 @pytest.mark.parametrize("heads,T,D,BT,G,dtype", [(2, 1024, 64, 64, 32, F32), (1, 777, 37, 16, 50, F16),
                                                   (3, 1000, 96, 32, 16, B16), (1, 300, 128, 256, 2, F32),
                                                   (2, 3001, 64, 64, 32, B16), (1, 4099, 64, 128, 32, B16)])
