@@ -232,7 +232,8 @@ def selection(rows, device):
 
 
 @pytest.mark.parametrize("BT,D,dtype", [(16, 72, F32), (16, 72, B16), (32, 40, F16), (32, 128, F32), (64, 72, F32),
-                                        (64, 72, B16), (128, 37, F16), (128, 128, B16), (128, 64, B16)])
+                                        (64, 72, B16), (128, 37, F16), (64, 64, B16), (64, 128, B16), (64, 128, F16),
+                                        (128, 128, B16), (128, 64, B16)])
 def test_infinity_in_a_selected_group_stays_there(device, BT, D, dtype):
     """Two value rows of one group hold an infinity.  Query blocks that select the whole group do not
     approximate it: their output is infinite in those two features and what it was in all others, whatever
