@@ -11,7 +11,9 @@
  * No atomics on global memory: identical inputs give bitwise-identical outputs.
  *
  * Tensor layout: q, k, v, o are [B, H, T, D] contiguous, passed as BH = B*H
- * slices of [T, D].  Reference interface cited per entry point; paths are
+ * slices of [T, D].  They may start at any element: the tuned kernels load k and v
+ * straight into LDS where both are 16-byte aligned, else through registers (slower,
+ * the same bits).  Reference interface cited per entry point; paths are
  * relative to the reference tree (ZHANGWENTAI/PASA).
  *
  * Shapes.  The tuned gfx950 kernels take bf16 q, k, v (fp16 at head_dim 128), head_dim

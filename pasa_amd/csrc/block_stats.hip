@@ -420,37 +420,32 @@ hipError_t launch_block_stats(const void* q, const void* k, const void* v, float
   auto a = (const uint16_t*)q;
   auto b = (const uint16_t*)k;
   auto c = (const uint16_t*)v;
-  auto dma = [&](auto kern, const RowMap& map, void* const* cp) {
-    hipLaunchKernelGGL(kern, grid, dim3(256), 0, stream, a, b, c, qc, kc, vc, hnorm, hgroup, T, Tslice, NT, G, map,
+  auto dma = [&](auto direct, auto staged, const RowMap& map, void* const* cp) {
+    hipLaunchKernelGGL((aligned ? direct : staged), grid, dim3(256), 0, stream, a, b, c, qc, kc, vc, hnorm, hgroup, T, Tslice, NT, G, map,
                        split, partials, cp ? (uint16_t*)cp[0] : nullptr, cp ? (uint16_t*)cp[1] : nullptr,
                        cp ? (uint16_t*)cp[2] : nullptr);
   };
   if (rm != nullptr) {  // token-major view of frame-major slices: D = 128, BT = 128 only
     if (D != 128 || BT != 128 || tm_copies == nullptr) return hipErrorInvalidValue;
     if (f16)
-      dma(k2_block_stats_dma<128, true, F16>, *rm, tm_copies);
+      dma(k2_block_stats_dma<128, true, F16>, k2_block_stats_dma<128, true, F16, 128, false>, *rm, tm_copies);
     else
-      dma(k2_block_stats_dma<128, true, Bf16>, *rm, tm_copies);
+      dma(k2_block_stats_dma<128, true, Bf16>, k2_block_stats_dma<128, true, Bf16, 128, false>, *rm, tm_copies);
   } else if (D == 128 && BT == 128) {
     if (f16)
-      dma(k2_block_stats_dma<128, false, F16>, RowMap{}, nullptr);
+      dma(k2_block_stats_dma<128, false, F16>, k2_block_stats_dma<128, false, F16, 128, false>, RowMap{}, nullptr);
     else
-      dma(k2_block_stats_dma<128, false, Bf16>, RowMap{}, nullptr);
+      dma(k2_block_stats_dma<128, false, Bf16>, k2_block_stats_dma<128, false, Bf16, 128, false>, RowMap{}, nullptr);
   } else if (D == 128 && BT == 64) {
     if (f16)
-      dma(k2_block_stats_dma<64, false, F16>, RowMap{}, nullptr);
+      dma(k2_block_stats_dma<64, false, F16>, k2_block_stats_dma<64, false, F16, 128, false>, RowMap{}, nullptr);
     else
-      dma(k2_block_stats_dma<64, false, Bf16>, RowMap{}, nullptr);
+      dma(k2_block_stats_dma<64, false, Bf16>, k2_block_stats_dma<64, false, Bf16, 128, false>, RowMap{}, nullptr);
   } else if (D == 64 && BT == 128) {
-    if (aligned)
-      dma(k2_block_stats_dma<128, false, Bf16, 64>, RowMap{}, nullptr);
-    else
-      dma(k2_block_stats_dma<128, false, Bf16, 64, false>, RowMap{}, nullptr);
+    dma(k2_block_stats_dma<128, false, Bf16, 64>, k2_block_stats_dma<128, false, Bf16, 64, false>, RowMap{},
+        nullptr);
   } else if (D == 64 && BT == 64) {
-    if (aligned)
-      dma(k2_block_stats_dma<64, false, Bf16, 64>, RowMap{}, nullptr);
-    else
-      dma(k2_block_stats_dma<64, false, Bf16, 64, false>, RowMap{}, nullptr);
+    dma(k2_block_stats_dma<64, false, Bf16, 64>, k2_block_stats_dma<64, false, Bf16, 64, false>, RowMap{}, nullptr);
   } else
     return hipErrorInvalidValue;
   if (split > 1) {

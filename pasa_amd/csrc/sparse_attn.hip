@@ -821,8 +821,19 @@ __global__ __attribute__((amdgpu_flat_work_group_size(1, 256), amdgpu_waves_per_
 void k4_sparse_attn(PASA_K4_PARAMS) {
   k4_body<D, BT, false, false, BT == 64, Bf16, false, AL>(PASA_K4_ARGS);
 }
+
+// The D = 128 kernels where k or v is not 16-byte aligned: tiles staged through registers (a few of
+// which spill at block 128).
+template <int BT, bool ALL, bool PERM, bool PAIR, typename E, bool CROSS = false>
+__global__ __attribute__((amdgpu_flat_work_group_size(1, 256), amdgpu_waves_per_eu(2, 2)))
+void k4_staged(PASA_K4_PARAMS) {
+  k4_body<128, BT, ALL, PERM, PAIR, E, CROSS, false>(PASA_K4_ARGS);
+}
 #undef PASA_K4_PARAMS
 #undef PASA_K4_ARGS
+
+// Whether K and V tiles can load straight into LDS.
+static bool aligned16(const void* k, const void* v) { return (((uintptr_t)k | (uintptr_t)v) & 15u) == 0; }
 
 size_t k4_pack_bytes(int D, int BT) {
   if (BT != 64 && BT != 128) return 0;
@@ -863,11 +874,11 @@ hipError_t launch_sparse_attn(const void* q, const void* k, const void* v, const
   auto cc = (const uint16_t*)v;
   auto pk = (const unsigned char*)pack;
   auto oo = (uint16_t*)o;
-  auto dma = [&](auto kern, dim3 g, int chunk, int n_text, const RowMap& map) {
-    hipLaunchKernelGGL(kern, g, dim3(256), 0, stream, a, b, cc, pk, selmask, oo, scale, c, T, NT, NG, NW, chunk,
-                       gamma_literal, text, text_valid, n_text, bh, 0, 0, map);
+  const bool aligned = aligned16(k, v);
+  auto dma = [&](auto direct, auto staged, dim3 g, int chunk, int n_text, const RowMap& map) {
+    hipLaunchKernelGGL((aligned ? direct : staged), g, dim3(256), 0, stream, a, b, cc, pk, selmask, oo, scale, c, T, NT,
+                       NG, NW, chunk, gamma_literal, text, text_valid, n_text, bh, 0, 0, map);
   };
-  const bool aligned = (((uintptr_t)k | (uintptr_t)v) & 15u) == 0;
   static_assert(K4D<128, 128>::THREADS == 256 && K4D<128, 64, true>::THREADS == 256 &&
                     K4D<64, 128>::THREADS == 256 && K4D<64, 64, true>::THREADS == 256,
                 "four-wave workgroups");
@@ -879,29 +890,29 @@ hipError_t launch_sparse_attn(const void* q, const void* k, const void* v, const
   if (rm != nullptr) {  // token-major view of frame-major slices: D = 128, BT = 128 only
     if (D != 128 || BT != 128) return hipErrorInvalidValue;
     if (f16)
-      dma(k4_sparse_attn_dma<128, false, true, false, F16>, grid, xcd_chunk, n_text_wg, *rm);
+      dma(k4_sparse_attn_dma<128, false, true, false, F16>, k4_staged<128, false, true, false, F16>, grid, xcd_chunk,
+          n_text_wg, *rm);
     else
-      dma(k4_sparse_attn_dma<128, false, true, false, Bf16>, grid, xcd_chunk, n_text_wg, *rm);
+      dma(k4_sparse_attn_dma<128, false, true, false, Bf16>, k4_staged<128, false, true, false, Bf16>, grid, xcd_chunk,
+          n_text_wg, *rm);
   } else if (D == 128 && BT == 128) {
     if (f16)
-      dma(k4_sparse_attn_dma<128, false, false, false, F16>, grid, xcd_chunk, n_text_wg, RowMap{});
+      dma(k4_sparse_attn_dma<128, false, false, false, F16>, k4_staged<128, false, false, false, F16>, grid, xcd_chunk,
+          n_text_wg, RowMap{});
     else
-      dma(k4_sparse_attn_dma<128, false, false, false, Bf16>, grid, xcd_chunk, n_text_wg, RowMap{});
+      dma(k4_sparse_attn_dma<128, false, false, false, Bf16>, k4_staged<128, false, false, false, Bf16>, grid, xcd_chunk,
+          n_text_wg, RowMap{});
   } else if (D == 128 && BT == 64) {
     if (f16)
-      dma(k4_sparse_attn_dma<64, false, false, true, F16>, grid_pairs, pair_chunk, n_text_pairs, RowMap{});
+      dma(k4_sparse_attn_dma<64, false, false, true, F16>, k4_staged<64, false, false, true, F16>, grid_pairs, pair_chunk,
+          n_text_pairs, RowMap{});
     else
-      dma(k4_sparse_attn_dma<64, false, false, true, Bf16>, grid_pairs, pair_chunk, n_text_pairs, RowMap{});
+      dma(k4_sparse_attn_dma<64, false, false, true, Bf16>, k4_staged<64, false, false, true, Bf16>, grid_pairs,
+          pair_chunk, n_text_pairs, RowMap{});
   } else if (D == 64 && BT == 128) {
-    if (aligned)
-      dma(k4_sparse_attn<64, 128, true>, grid, xcd_chunk, 0, RowMap{});
-    else
-      dma(k4_sparse_attn<64, 128, false>, grid, xcd_chunk, 0, RowMap{});
+    dma(k4_sparse_attn<64, 128, true>, k4_sparse_attn<64, 128, false>, grid, xcd_chunk, 0, RowMap{});
   } else if (D == 64 && BT == 64) {
-    if (aligned)
-      dma(k4_sparse_attn<64, 64, true>, grid_pairs, pair_chunk, 0, RowMap{});
-    else
-      dma(k4_sparse_attn<64, 64, false>, grid_pairs, pair_chunk, 0, RowMap{});
+    dma(k4_sparse_attn<64, 64, true>, k4_sparse_attn<64, 64, false>, grid_pairs, pair_chunk, 0, RowMap{});
   } else {
     return hipErrorInvalidValue;
   }
@@ -917,15 +928,15 @@ hipError_t launch_dense_attn(const void* q, const void* k, const void* v, void* 
   const int text_qtiles = (text_valid + BT - 1) / BT + (text - text_valid + BT - 1) / BT;
   const int n_text_wg = (bh * text_qtiles + 7) / 8 * 8;
   dim3 grid(n_text_wg + 8 * bh * xcd_chunk);
-  auto launch = [&](auto kern) {
-    hipLaunchKernelGGL(kern, grid, dim3(K4D<128, BT>::THREADS), 0, stream, (const uint16_t*)q, (const uint16_t*)k,
+  auto launch = [&](auto direct, auto staged) {
+    hipLaunchKernelGGL((aligned16(k, v) ? direct : staged), grid, dim3(K4D<128, BT>::THREADS), 0, stream, (const uint16_t*)q, (const uint16_t*)k,
                        (const uint16_t*)v, nullptr, nullptr, (uint16_t*)o, scale, scale * kLog2e, T, NT, 0, 0,
                        xcd_chunk, 1, text, text_valid, n_text_wg, bh, o_heads, 0, RowMap{});
   };
   if (f16)
-    launch(k4_sparse_attn_dma<BT, true, false, false, F16>);
+    launch(k4_sparse_attn_dma<BT, true, false, false, F16>, k4_staged<BT, true, false, false, F16>);
   else
-    launch(k4_sparse_attn_dma<BT, true, false, false, Bf16>);
+    launch(k4_sparse_attn_dma<BT, true, false, false, Bf16>, k4_staged<BT, true, false, false, Bf16>);
   return hipGetLastError();
 }
 
@@ -934,15 +945,15 @@ hipError_t launch_cross_attn(const void* q, const void* k, const void* v, void* 
   constexpr int BT = 128;
   if (q_len < 1 || kv_len < 1) return hipErrorInvalidValue;
   const int xcd_chunk = ((q_len + BT - 1) / BT + 7) / 8;
-  auto launch = [&](auto kern) {
-    hipLaunchKernelGGL(kern, dim3(8 * bh * xcd_chunk), dim3(K4D<128, BT>::THREADS), 0, stream, (const uint16_t*)q,
+  auto launch = [&](auto direct, auto staged) {
+    hipLaunchKernelGGL((aligned16(k, v) ? direct : staged), dim3(8 * bh * xcd_chunk), dim3(K4D<128, BT>::THREADS), 0, stream, (const uint16_t*)q,
                        (const uint16_t*)k, (const uint16_t*)v, nullptr, nullptr, (uint16_t*)o, scale, scale * kLog2e,
                        kv_len, (kv_len + BT - 1) / BT, 0, 0, xcd_chunk, 1, 0, 0, 0, bh, o_heads, q_len, RowMap{});
   };
   if (f16)
-    launch(k4_cross_attn<F16>);
+    launch(k4_cross_attn<F16>, k4_staged<BT, true, false, false, F16, true>);
   else
-    launch(k4_cross_attn<Bf16>);
+    launch(k4_cross_attn<Bf16>, k4_staged<BT, true, false, false, Bf16, true>);
   return hipGetLastError();
 }
 

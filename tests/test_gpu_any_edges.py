@@ -342,3 +342,41 @@ def test_head_dim_64_takes_misaligned_data(device, T, BT, shift):
         outs.append((st.qc, st.kc, st.vc, st.hnorm, st.hgroup, ops.sparse_attn(*d, st, sel, 64 ** -0.5, BT)))
     for a, b in zip(*outs):
         assert torch.equal(a, b)
+
+
+@pytest.mark.parametrize("T, BT, text, valid, dtype, shift", [(128, 128, 0, 0, B16, 1), (1000, 128, 0, 0, F16, 4),
+                                                              (1000, 64, 0, 0, B16, 3), (4500, 64, 70, 9, F16, 5),
+                                                              (4500, 128, 200, 130, B16, 2), (5000, 128, 0, 0, B16, 7)])
+def test_head_dim_128_takes_misaligned_data(device, T, BT, text, valid, dtype, shift):
+    """16-bit head dim 128 on data that is not 16-byte aligned: staged through registers, the same bits."""
+    q, k, v = make(2, T, 128, dtype, T + BT)
+    outs = []
+    for n in (0, shift):
+        d = [to_dev(t, device, n) for t in (q, k, v)]
+        st = ops.block_stats(*d, BT, text_tokens=text)
+        sel = ops.select_blocks(st, 0.2, 128 ** -0.5)
+        kw = dict(text_tokens=text, text_valid=valid)
+        outs.append((st.qc, st.kc, st.vc, st.hnorm, st.hgroup, ops.sparse_attn(*d, st, sel, 128 ** -0.5, BT, **kw),
+                     ops.dense_attention(*d, **kw), ops.dense_attention(*d, token_major_out=True, **kw),
+                     ops.cross_attention(d[0], *(to_dev(t[:, :, :77].contiguous(), device, n) for t in (k, v)))))
+    for a, b in zip(*outs):
+        assert torch.equal(a, b)
+
+
+@pytest.mark.parametrize("dtype, shift", [(B16, 1), (F16, 6)])
+def test_placed_call_takes_misaligned_data(device, dtype, shift):
+    """The same for the frame-major call: its inputs, and the token-major k and v its second half reads."""
+    frames, size, text = 5, 210, 40
+    q, k, v = make(2, frames * size + text, 128, dtype, 5)
+    pl = ops.Placement(frames, size)
+    outs = []
+    for n in (0, shift):
+        d = [to_dev(t, device, n) for t in (q, k, v)]
+        st = ops.block_stats(*d, 128, text_tokens=text, placement=pl)
+        sel = ops.select_blocks(st, 0.3, 128 ** -0.5)
+        pack = ops.pack_phase2(d[0], st, 128, text)
+        tm = [to_dev(t, device, n) for t in (st.k_tm, st.v_tm)]
+        o = ops.sparse_attn_packed(d[0], *tm, pack, sel, 128 ** -0.5, 128, text_tokens=text, placement=pl)
+        outs.append((st.qc, st.kc, st.vc, st.hnorm, st.hgroup, st.k_tm, st.v_tm, o))
+    for a, b in zip(*outs):
+        assert torch.equal(a, b)
