@@ -94,7 +94,7 @@ __device__ __forceinline__ void dma_load16_lds_nt(u32x4_t rsrc, uint32_t lds_add
                : "memory");
 }
 
-// dma_load16_lds for k or v that are not 16-byte aligned, which the direct load is not issued for: the
+// dma_load16_lds for a base that is not 16-byte aligned, which the direct load is not issued for: the
 // rows pass through registers, and are in LDS on return (a direct load may land as early).
 __device__ __forceinline__ void staged_load16_lds(u32x4_t rsrc, uint32_t lds_addr, uint32_t byte_off, uint32_t soff) {
   u32x4_t x;

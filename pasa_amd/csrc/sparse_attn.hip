@@ -216,7 +216,7 @@ constexpr int kSchedDsRead = 0x100;
 // cover q's rows and each visits all of k's.
 // o_heads (ALL): 0, o is [slice, row, D] as q; else o is [batch, row, head, D] with o_heads heads, the
 // layout the projection after the attention reads.
-// AL: k and v are 16-byte aligned.
+// AL: k, v and pack are 16-byte aligned.
 template <int D, int BT, bool ALL, bool PERM, bool PAIR, typename E, bool CROSS = false, bool AL = true>
 __device__ __forceinline__ void k4_body(const uint16_t* __restrict__ q, const uint16_t* __restrict__ k,
                                         const uint16_t* __restrict__ v, const unsigned char* __restrict__ pack,
@@ -617,7 +617,7 @@ __device__ __forceinline__ void k4_body(const uint16_t* __restrict__ q, const ui
 #pragma unroll
     for (int n = 0; n < P2_LOADS; ++n) {
       const int kb = n * C::WAVES + wave;
-      dma_load16_lds(pd, vs_lds + kb * 1024, (uint32_t)(PK::HT_BYTES + kb * 1024 + lane * 16), gsoff);
+      tile_load(pd, vs_lds + kb * 1024, (uint32_t)(PK::HT_BYTES + kb * 1024 + lane * 16), gsoff);
     }
   };
   auto load_ht = [&](int g) {
@@ -625,7 +625,7 @@ __device__ __forceinline__ void k4_body(const uint16_t* __restrict__ q, const ui
 #pragma unroll
     for (int n = 0; n < HT_LOADS; ++n) {
       const int kb = n * C::WAVES + wave;  // 1 KB piece of Hbar^T
-      dma_load16_lds(pd, ks_lds + kb * 1024, (uint32_t)(kb * 1024 + lane * 16), gsoff);
+      tile_load(pd, ks_lds + kb * 1024, (uint32_t)(kb * 1024 + lane * 16), gsoff);
     }
   };
   int g = next_group(-1);
@@ -822,7 +822,7 @@ void k4_sparse_attn(PASA_K4_PARAMS) {
   k4_body<D, BT, false, false, BT == 64, Bf16, false, AL>(PASA_K4_ARGS);
 }
 
-// The D = 128 kernels where k or v is not 16-byte aligned: tiles staged through registers (a few of
+// The D = 128 kernels where k, v or pack is not 16-byte aligned: tiles staged through registers (a few of
 // which spill at block 128).
 template <int BT, bool ALL, bool PERM, bool PAIR, typename E, bool CROSS = false>
 __global__ __attribute__((amdgpu_flat_work_group_size(1, 256), amdgpu_waves_per_eu(2, 2)))
@@ -832,8 +832,10 @@ void k4_staged(PASA_K4_PARAMS) {
 #undef PASA_K4_PARAMS
 #undef PASA_K4_ARGS
 
-// Whether K and V tiles can load straight into LDS.
-static bool aligned16(const void* k, const void* v) { return (((uintptr_t)k | (uintptr_t)v) & 15u) == 0; }
+// Whether K and V tiles (and the pack) can load straight into LDS.
+static bool aligned16(const void* k, const void* v, const void* pack = nullptr) {
+  return (((uintptr_t)k | (uintptr_t)v | (uintptr_t)pack) & 15u) == 0;
+}
 
 size_t k4_pack_bytes(int D, int BT) {
   if (BT != 64 && BT != 128) return 0;
@@ -874,7 +876,7 @@ hipError_t launch_sparse_attn(const void* q, const void* k, const void* v, const
   auto cc = (const uint16_t*)v;
   auto pk = (const unsigned char*)pack;
   auto oo = (uint16_t*)o;
-  const bool aligned = aligned16(k, v);
+  const bool aligned = aligned16(k, v, pack);
   auto dma = [&](auto direct, auto staged, dim3 g, int chunk, int n_text, const RowMap& map) {
     hipLaunchKernelGGL((aligned ? direct : staged), g, dim3(256), 0, stream, a, b, cc, pk, selmask, oo, scale, c, T, NT,
                        NG, NW, chunk, gamma_literal, text, text_valid, n_text, bh, 0, 0, map);

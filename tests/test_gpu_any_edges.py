@@ -380,3 +380,18 @@ def test_placed_call_takes_misaligned_data(device, dtype, shift):
         outs.append((st.qc, st.kc, st.vc, st.hnorm, st.hgroup, st.k_tm, st.v_tm, o))
     for a, b in zip(*outs):
         assert torch.equal(a, b)
+
+
+@pytest.mark.parametrize("T, D, BT, dtype, shift", [(700, 64, 64, B16, 8), (700, 64, 128, B16, 2), (700, 128, 64, F16, 4),
+                                                    (4500, 128, 128, B16, 12)])
+def test_pack_takes_any_address(device, T, D, BT, dtype, shift):
+    """A phase-2 pack (or workspace) that is not 16-byte aligned: the same bits."""
+    q, k, v = (t.to(device) for t in make(2, T, D, dtype, T + BT))
+    st = ops.block_stats(q, k, v, BT)
+    sel = ops.select_blocks(st, 0.2, D ** -0.5)
+    pack = ops.pack_phase2(q, st, BT)
+    moved = torch.empty(pack.numel() + shift, dtype=torch.uint8, device=device)[shift:]
+    ops._lib.call("pasa_pack_phase2", st.kc.data_ptr(), st.vc.data_ptr(), st.hgroup.data_ptr(), moved.data_ptr(),
+                  moved.numel(), 2, T, 0, D, BT, 32, ops._DTYPES[dtype], ops._stream(q))
+    a, b = (ops.sparse_attn_packed(q, k, v, p, sel, D ** -0.5, BT) for p in (pack, moved))
+    assert torch.equal(a, b)
