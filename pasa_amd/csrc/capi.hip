@@ -397,7 +397,9 @@ int pasa_select(const float* qc, const float* kc, const float* hnorm, const floa
     scores = (float*)workspace;
   }
   hipStream_t s = (hipStream_t)stream;
-  if (head_dim == 64 || head_dim == 128)
+  // The tuned score kernel loads its rows straight into LDS, 16 bytes at 16-byte addresses.
+  const bool aligned = (((uintptr_t)qc | (uintptr_t)kc) & 15u) == 0;
+  if ((head_dim == 64 || head_dim == 128) && aligned)
     rc = launch_status(pasa::launch_scores(qc, kc, hnorm, noise, (float)scale, use_cov_bias, scores, (int)bh,
                                            (int)num_blocks, (int)head_dim, s),
                        "pasa_select(scores)");

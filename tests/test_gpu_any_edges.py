@@ -395,3 +395,18 @@ def test_pack_takes_any_address(device, T, D, BT, dtype, shift):
                   moved.numel(), 2, T, 0, D, BT, 32, ops._DTYPES[dtype], ops._stream(q))
     a, b = (ops.sparse_attn_packed(q, k, v, p, sel, D ** -0.5, BT) for p in (pack, moved))
     assert torch.equal(a, b)
+
+
+@pytest.mark.parametrize("D, shift", [(64, 1), (128, 2), (128, 3)])
+def test_scores_take_any_address(device, D, shift):
+    """Block means that are not 16-byte aligned, at the head dims of the tuned score kernel: the bound of
+    test_scores_any against 64 bits."""
+    g = torch.Generator().manual_seed(D + shift)
+    qc, kc = (torch.randn(1, 2, 130, D, generator=g) for _ in range(2))
+    hn = torch.rand(1, 2, 130, generator=g) + 0.5
+    st = ops.BlockStats(to_dev(qc, device, shift), to_dev(kc, device, shift), torch.empty(0), to_dev(hn, device, shift),
+                        torch.empty(0))
+    sel = ops.select_blocks(st, 0.3, 0.37, return_scores=True)
+    ref = O.select_scores(qc.double(), kc.double(), hn.double(), 0.37)
+    mag = O.select_scores(qc.double().abs(), kc.double().abs(), hn.double(), 0.37, use_cov_bias=False)
+    assert bool(((sel.scores.cpu().double() - ref).abs() <= (D + 8) * 2.0 ** -24 * (mag + 1)).all())
