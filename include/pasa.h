@@ -50,7 +50,7 @@
 extern "C" {
 #endif
 
-#define PASA_ABI_VERSION 11
+#define PASA_ABI_VERSION 12
 
 typedef enum {
   PASA_OK = 0,

@@ -86,7 +86,7 @@ SIGNATURES = {
                             _i64, _i64, _i64, _i64, _dbl, _vp]),
 }
 
-ABI_VERSION = 11
+ABI_VERSION = 12
 
 # Size of the static device array behind pasa_sparse_attn_noalloc (PASA_NOALLOC_SCRATCH_BYTES).
 NOALLOC_SCRATCH_BYTES = 64 << 20
@@ -115,13 +115,14 @@ def load() -> ctypes.CDLL:
             f"{LIB_PATH} is missing: build it with `python -m pasa_amd.build` "
             "(there is no CPU fallback for the PISA kernels)")
     lib = ctypes.CDLL(str(LIB_PATH))
+    # The version first: a library of another one may lack some of the entry points.
+    ver = lib.pasa_abi_version()
+    if ver != ABI_VERSION:
+        raise RuntimeError(f"{LIB_PATH}: ABI version {ver}, expected {ABI_VERSION}")
     for name, (res, args) in SIGNATURES.items():
         fn = getattr(lib, name)
         fn.restype = res
         fn.argtypes = args
-    ver = lib.pasa_abi_version()
-    if ver != ABI_VERSION:
-        raise RuntimeError(f"{LIB_PATH}: ABI version {ver}, expected {ABI_VERSION}")
     _LIB = lib
     return lib
 

@@ -44,6 +44,19 @@ def test_version_and_status_strings(lib):
     assert lib.pasa_status_string(12345) == b"unknown status"
 
 
+@pytest.mark.parametrize("version", [11, 99])
+def test_library_of_another_version_is_named_as_such(version, tmp_path, monkeypatch):
+    """Version 11 had neither pasa_dense_attn_bshd nor pasa_block_stats_workspace_bytes_dtype: a library
+    without them is refused for its version, not for a missing symbol."""
+    src, so = tmp_path / "old.c", tmp_path / "old.so"
+    src.write_text("int pasa_abi_version(void) { return %d; }\n" % version)
+    subprocess.run(["gcc", "-shared", "-fPIC", str(src), "-o", str(so)], check=True)
+    monkeypatch.setattr(_lib, "LIB_PATH", so)
+    monkeypatch.setattr(_lib, "_LIB", None)
+    with pytest.raises(RuntimeError, match=f"ABI version {version}, expected"):
+        _lib.load()
+
+
 @pytest.mark.parametrize("density,nt,expect", [
     (0.1, 591, 59), (0.15, 256, 38), (0.25, 16, 4), (0.10, 929, 92), (1.0, 10, 10),
     (0.0, 10, 1), (2.0, 10, 10), (0.29, 100, 28), (-0.5, 8, 1), (0.999999, 3, 2)])
