@@ -206,9 +206,11 @@ def _plain(module: nn.Module, cls) -> bool:
 
 
 def _in_type(x: torch.Tensor, *tensors) -> bool:
-    """All of x's type and device, with no autocast that would change either."""
+    """All of x's type and device, with no autocast that would change either, and tensors of torch itself
+    (a subclass, a quantised or distributed weight, may only be known to F.linear)."""
     return (not torch.is_autocast_enabled(x.device.type)
-            and all(t is not None and t.dtype == x.dtype and t.device == x.device for t in tensors))
+            and all(type(t) in (torch.Tensor, nn.Parameter) and t.dtype == x.dtype and t.device == x.device
+                    for t in tensors))
 
 
 def _reads_timestep_on_host(block) -> bool:

@@ -176,3 +176,29 @@ def test_fused_cross_attention_takes_one_text_per_sample(monkeypatch, text_shape
         assert not W._cross_fusable(attn, x, text)
     attn.to_k.float()
     assert not W._cross_fusable(attn, x, text)
+
+
+class QuantisedLike(torch.Tensor):
+    """A weight that reports bf16 and is only ever multiplied through F.linear."""
+
+    @classmethod
+    def __torch_function__(cls, func, types, args=(), kwargs=None):
+        plain = [a.as_subclass(torch.Tensor) if isinstance(a, cls) else a for a in args]
+        if func is torch.nn.functional.linear or func.__name__ in ("__get__", "dim", "size"):
+            return func(*plain, **(kwargs or {}))
+        raise NotImplementedError(str(func))
+
+
+@pytest.mark.parametrize("name", ["weight", "bias"])
+def test_fused_feed_forward_leaves_other_kinds_of_weights_to_the_module(name):
+    """A plain Linear whose weight or bias is a tensor subclass (weight-only quantisation, distributed
+    tensors) multiplies through F.linear alone."""
+    cfg = W.WanDiTConfig(num_layers=1, num_attention_heads=2, ffn_dim=64, text_dim=32, freq_dim=16)
+    blk = W.WanBlock(cfg).to(torch.bfloat16)
+    up = blk.ffn[0]
+    w = getattr(up, name).detach().as_subclass(QuantisedLike)
+    del up._parameters[name]
+    object.__setattr__(up, name, w)
+    x = torch.randn(1, 3, 256, dtype=torch.bfloat16)
+    with torch.no_grad():
+        assert torch.equal(blk._ffn_fused(x), blk.ffn(x))
