@@ -194,7 +194,7 @@ class WanBlock(nn.Module):
                 and act.approximate == "tanh" and _in_type(x, up.weight, up.bias)):
             return self.ffn(x)
         h = torch._addmm_activation(up.bias, x.reshape(-1, x.shape[-1]), up.weight.t(), use_gelu=True)
-        return down(h).view(*x.shape[:-1], -1)
+        return down(h.view(*x.shape[:-1], h.shape[-1]))
 
 
 def _plain(module: nn.Module, cls) -> bool:

@@ -202,3 +202,18 @@ def test_fused_feed_forward_leaves_other_kinds_of_weights_to_the_module(name):
     x = torch.randn(1, 3, 256, dtype=torch.bfloat16)
     with torch.no_grad():
         assert torch.equal(blk._ffn_fused(x), blk.ffn(x))
+
+
+def test_fused_feed_forward_keeps_the_shapes_that_modules_see():
+    """The down projection (a hook on it, an adapter in its place) is called with the module path's shape,
+    and a batch without rows passes through."""
+    cfg = W.WanDiTConfig(num_layers=1, num_attention_heads=2, ffn_dim=64, text_dim=32, freq_dim=16)
+    blk = W.WanBlock(cfg)
+    seen = []
+    blk.ffn[2].register_forward_pre_hook(lambda m, args: seen.append(tuple(args[0].shape)))
+    with torch.no_grad():
+        for shape in ((1, 3, 256), (2, 0, 256)):
+            x = torch.randn(shape)
+            a, b = blk._ffn_fused(x), blk.ffn(x)
+            assert seen[-2] == seen[-1] == (*shape[:2], 64)
+            torch.testing.assert_close(a, b)
