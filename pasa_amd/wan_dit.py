@@ -222,14 +222,15 @@ def _reads_timestep_on_host(block) -> bool:
 
 def _cross_fusable(attn, x: torch.Tensor, text: torch.Tensor) -> bool:
     """Whether ``_cross_attention_fused`` computes what ``attn``'s call does: the stock processor,
-    torch RMSNorms with bf16 weights, bf16 text (one row of it or more for each sample), head_dim
+    plain projections to the full width, torch RMSNorms with bf16 weights, bf16 text (one row of it or more for each sample), head_dim
     128, no autocast and nothing hooked in between."""
     C = x.shape[-1]
     return (_plain(attn, WanAttention) and type(attn.processor) is WanAttnProcessor
             and text is not None and x.dtype == torch.bfloat16 and C == attn.heads * 128
             and text.dim() == 3 and text.shape[0] == x.shape[0] and text.numel() > 0
-            and _in_type(x, text, *(m.weight for m in (attn.to_q, attn.to_k, attn.to_v) if type(m) is nn.Linear))
+            and all(_plain(m, nn.Linear) and m.out_features == C for m in (attn.to_q, attn.to_k, attn.to_v))
             and all(_plain(m, nn.RMSNorm) for m in (attn.norm_q, attn.norm_k))
+            and _in_type(x, text, *(m.weight for m in (attn.to_q, attn.to_k, attn.to_v, attn.norm_q, attn.norm_k)))
             and fusable(x, attn.heads, (attn.norm_q, attn.norm_k), C))
 
 

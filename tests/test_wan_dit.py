@@ -217,3 +217,29 @@ def test_fused_feed_forward_keeps_the_shapes_that_modules_see():
             a, b = blk._ffn_fused(x), blk.ffn(x)
             assert seen[-2] == seen[-1] == (*shape[:2], 64)
             torch.testing.assert_close(a, b)
+
+
+def test_fused_cross_attention_wants_plain_projections(monkeypatch):
+    """A projection that is not nn.Linear itself may return another type or width than the kernels take."""
+    class Widening(torch.nn.Module):
+        def __init__(self, lin):
+            super().__init__()
+            self.lin = lin
+
+        def forward(self, x):
+            return self.lin(x).float()
+
+    cfg = W.WanDiTConfig(num_layers=1, num_attention_heads=2, ffn_dim=64, text_dim=32, freq_dim=16)
+    monkeypatch.setattr(W, "fusable", lambda *a: True)       # the device test, as on a GPU
+    x, text = torch.zeros(2, 3, 256, dtype=torch.bfloat16), torch.zeros(2, 5, 256, dtype=torch.bfloat16)
+    for name in ("to_q", "to_k", "to_v"):
+        attn = W.WanBlock(cfg).to(torch.bfloat16).attn2
+        assert W._cross_fusable(attn, x, text)
+        lin = getattr(attn, name)
+        setattr(attn, name, Widening(lin))
+        assert not W._cross_fusable(attn, x, text)
+        setattr(attn, name, torch.nn.Linear(256, 512, dtype=torch.bfloat16))
+        assert not W._cross_fusable(attn, x, text)
+        setattr(attn, name, lin)
+        lin.register_forward_hook(lambda m, i, o: o.float())
+        assert not W._cross_fusable(attn, x, text)
