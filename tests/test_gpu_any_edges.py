@@ -410,3 +410,39 @@ def test_scores_take_any_address(device, D, shift):
     ref = O.select_scores(qc.double(), kc.double(), hn.double(), 0.37)
     mag = O.select_scores(qc.double().abs(), kc.double().abs(), hn.double(), 0.37, use_cov_bias=False)
     assert bool(((sel.scores.cpu().double() - ref).abs() <= (D + 8) * 2.0 ** -24 * (mag + 1)).all())
+
+
+@pytest.mark.parametrize("case", ["nan_row", "infinite_unselected", "infinite_selected", "out_of_scaled_range"])
+@pytest.mark.parametrize("BT,D,G", [(64, 64, 3), (64, 128, 32), (128, 100, 2), (256, 37, 1)])
+def test_fp32_tiles_done_again(device, BT, D, G, case):
+    """Sparse fp32 calls whose tiles are not finite in the split form and are computed again in fp32, after
+    phase 2 has used their LDS for the sums and moments: the rows and features that are finite come out as
+    the oracle's, the others are not finite."""
+    NT = 9
+    T = NT * BT - 5
+    q, k, v = make(1, T, D, F32, T + D)
+    rows = [{3, *[j % NT for j in (i, i + 2, i + 5, i + 4) if j % NT not in (3, 6)][:2]} for i in range(NT)]
+    sel, idx = selection(rows, device)
+    bad_rows = torch.zeros(T, dtype=torch.bool)
+    bad_cols = torch.zeros(D, dtype=torch.bool)
+    qb, vb = q.clone(), v.clone()
+    if case == "nan_row":
+        qb[0, 0, 2 * BT + 1, 0] = torch.nan
+        bad_rows[2 * BT + 1] = True
+    elif case == "out_of_scaled_range":
+        vb = v = v * 2.0 ** 95                               # finite, but not times 2^56
+    else:
+        vb[0, 0, (6 if case == "infinite_unselected" else 3) * BT + 7, 11] = torch.inf
+        bad_cols[11] = True
+    scale = D ** -0.5
+    d = [t.to(device) for t in (qb, k, vb)]
+    st = ops.block_stats(*d, BT, G)
+    o = ops.sparse_attn(*d, st, sel, scale, BT, group_size=G).double().cpu()[0, 0]
+    ref = O.pisa_pg_attention(q, k, v, 0.5, BT, G, scale, dtype=torch.float64, indices=idx)[0, 0]
+    assert bool(torch.isnan(o[bad_rows]).all())
+    a, b = o[~bad_rows][:, ~bad_cols], ref[~bad_rows][:, ~bad_cols]
+    err = float((a - b).norm() / b.norm())
+    print(f"[edges] fp32 again BT={BT} D={D} G={G} {case}: rel {err:.2e}", flush=True)
+    assert err <= 4e-6
+    if bad_cols.any():
+        assert not bool(torch.isfinite(o[:, bad_cols]).any())
