@@ -1087,8 +1087,10 @@ bool wide_tiles(const AnyCall& a, int BT) {
   return BT >= 128 && (int64_t)a.bh * ((a.T + 127) / 128) >= 256;
 }
 
-// WIDE: 32 rows per wave where the blocks are long enough (not in fp32, whose planes or wider
-// fragments then spill).
+// WIDE: 32 rows per wave where the blocks are long enough, measured at D 96.  Not in fp32, whose planes
+// or wider fragments then spill (283 registers).  At DP 128 the 16-bit ones spill too, 60 VGPRs below
+// block 64 and 45 from block 128 on, which every group of phase 2 reloads (16 rows would not; not
+// measured there: 12 heads x 16,380 rows, D 128, bf16, block 32 620-640 us, block 128, groups of 16 440).
 template <typename E, int DP, bool VEC, bool WIDE>
 hipError_t launch_dp(const AnyCall& a) {
   if (!a.all && a.BT < 64) {
