@@ -210,8 +210,8 @@ constexpr int kSchedDsRead = 0x100;
 // (a shorter selection row, or a text pair spanning the prompt and the padding
 // segment, idles through its partner's extra tiles); a pair past the last block
 // repeats it and stores nothing.  Phase 2 visits the groups
-// either block approximates; a wave whose block selects the whole group only loads its
-// share of the operands, so each block's result is the one the unpaired kernel computes.
+// either block approximates; a wave whose block selects the whole group adds nothing
+// there, so each block's result is the one the unpaired kernel computes.
 // CROSS (with ALL): the slices of q and o have q_len rows, those of k and v T; the query tiles
 // cover q's rows and each visits all of k's.
 // o_heads (ALL): 0, o is [slice, row, D] as q; else o is [batch, row, head, D] with o_heads heads, the
@@ -639,94 +639,96 @@ __device__ __forceinline__ void k4_body(const uint16_t* __restrict__ q, const ui
     const int gn = next_group(g);
     const uint32_t approx = approx_of(g);
 
-    // PAIR: a wave whose block selects the whole group leaves it alone (its weights are 0, and 0 times a
-    // sum that is not finite would be NaN).
+    // PAIR: a wave whose block selects the whole group adds nothing to o (its weights are 0, and 0 times a
+    // sum that is not finite would be NaN).  The branches enclose just the two sums: around the scores and
+    // q Hbar as well they cost 1 to 2% (24 heads x 119 k rows: 28.19-28.53 ms against 27.54-27.83 without
+    // any; so 27.65-28.31 against 27.93-28.44 on another box).
     const bool mine = !PAIR || approx != 0u;
-    float psum[2];
-    if (mine) {
-      // s-bar^T = kbar Q^T: sb[bt][qt] element i = block 16 bt + 4 g4 + i of the group.
-      f32x4_t sb[2][2];
+    // s-bar^T = kbar Q^T: sb[bt][qt] element i = block 16 bt + 4 g4 + i of the group.
+    f32x4_t sb[2][2];
+#pragma unroll
+    for (int bt = 0; bt < 2; ++bt)
+#pragma unroll
+      for (int qt = 0; qt < 2; ++qt)
+#pragma unroll
+        for (int i = 0; i < 4; ++i) sb[bt][qt][i] = 0.f;
+#pragma unroll
+    for (int ks = 0; ks < KS; ++ks)
+#pragma unroll
+      for (int bt = 0; bt < 2; ++bt) {
+        const vec8 a = as_vec8<E>(lds_ld<uint4>(Vs, PK::KB_OFF + kofs[ks] + bt * 16 * ROWB));
+#pragma unroll
+        for (int qt = 0; qt < 2; ++qt) sb[bt][qt] = E::mfma16(a, qf[qt][ks], sb[bt][qt]);
+      }
+    // Blocks of the group that are selected (or past NT) drop out: element i of sb[bt]
+    // is block 16 bt + 4 g4 + i, so its keep mask is one sign-extended bit of approx >> 4 g4.
+    const uint32_t ah = approx >> (4 * g4);
+    float m_new[2], alpha[2];
+#pragma unroll
+    for (int qt = 0; qt < 2; ++qt) {
+      float gmx = -INFINITY;
 #pragma unroll
       for (int bt = 0; bt < 2; ++bt)
 #pragma unroll
-        for (int qt = 0; qt < 2; ++qt)
-#pragma unroll
-          for (int i = 0; i < 4; ++i) sb[bt][qt][i] = 0.f;
-#pragma unroll
-      for (int ks = 0; ks < KS; ++ks)
-#pragma unroll
-        for (int bt = 0; bt < 2; ++bt) {
-          const vec8 a = as_vec8<E>(lds_ld<uint4>(Vs, PK::KB_OFF + kofs[ks] + bt * 16 * ROWB));
-#pragma unroll
-          for (int qt = 0; qt < 2; ++qt) sb[bt][qt] = E::mfma16(a, qf[qt][ks], sb[bt][qt]);
+        for (int i = 0; i < 4; ++i) {
+          const uint32_t keep = (uint32_t)__builtin_amdgcn_sbfe((int)ah, 16 * bt + i, 1);
+          sb[bt][qt][i] = __uint_as_float((__float_as_uint(sb[bt][qt][i]) & keep) | (~keep & 0xff800000u));  // -inf if dropped
+          gmx = fmaxf(gmx, sb[bt][qt][i]);
         }
-      // Blocks of the group that are selected (or past NT) drop out: element i of sb[bt]
-      // is block 16 bt + 4 g4 + i, so its keep mask is one sign-extended bit of approx >> 4 g4.
-      const uint32_t ah = approx >> (4 * g4);
-      float m_new[2], alpha[2];
+      m_new[qt] = fmaxf(m_run[qt], quad16_max(gmx) * c);
+      alpha[qt] = fast_exp2(m_run[qt] - m_new[qt]);
+      m_run[qt] = m_new[qt];
+      l_run[qt] *= alpha[qt];
+      if (!gamma_literal) g_run[qt] *= alpha[qt];
+    }
 #pragma unroll
-      for (int qt = 0; qt < 2; ++qt) {
-        float gmx = -INFINITY;
+    for (int qt = 0; qt < 2; ++qt)
+      if (__any(alpha[qt] != 1.f)) {
 #pragma unroll
-        for (int bt = 0; bt < 2; ++bt)
+        for (int dt = 0; dt < DT; ++dt)
 #pragma unroll
-          for (int i = 0; i < 4; ++i) {
-            const uint32_t keep = (uint32_t)__builtin_amdgcn_sbfe((int)ah, 16 * bt + i, 1);
-            sb[bt][qt][i] = __uint_as_float((__float_as_uint(sb[bt][qt][i]) & keep) | (~keep & 0xff800000u));  // -inf if dropped
-            gmx = fmaxf(gmx, sb[bt][qt][i]);
-          }
-        m_new[qt] = fmaxf(m_run[qt], quad16_max(gmx) * c);
-        alpha[qt] = fast_exp2(m_run[qt] - m_new[qt]);
-        m_run[qt] = m_new[qt];
-        l_run[qt] *= alpha[qt];
-        if (!gamma_literal) g_run[qt] *= alpha[qt];
+          for (int i = 0; i < 4; ++i) oacc[dt][qt][i] *= alpha[qt];
       }
+    float psum[2];
+    vec8 pbf[2];
 #pragma unroll
-      for (int qt = 0; qt < 2; ++qt)
-        if (__any(alpha[qt] != 1.f)) {
+    for (int qt = 0; qt < 2; ++qt) {
+      uint32_t w[4];
 #pragma unroll
-          for (int dt = 0; dt < DT; ++dt)
-#pragma unroll
-            for (int i = 0; i < 4; ++i) oacc[dt][qt][i] *= alpha[qt];
-        }
-      vec8 pbf[2];
-#pragma unroll
-      for (int qt = 0; qt < 2; ++qt) {
-        uint32_t w[4];
-#pragma unroll
-        for (int j = 0; j < 4; ++j) {
-          const f32x4_t& src = sb[j >> 1][qt];
-          const float p0 = fast_exp2(fmaf(src[2 * (j & 1)], c, -m_new[qt]));
-          const float p1 = fast_exp2(fmaf(src[2 * (j & 1) + 1], c, -m_new[qt]));
-          psum[qt] = j == 0 ? p0 + p1 : psum[qt] + (p0 + p1);  // no 0 + x: x may be -0
-          w[j] = E::pack2(p0, p1);
-        }
-        pbf[qt] = as_vec8<E>((u32x4_t){w[0], w[1], w[2], w[3]});
+      for (int j = 0; j < 4; ++j) {
+        const f32x4_t& src = sb[j >> 1][qt];
+        const float p0 = fast_exp2(fmaf(src[2 * (j & 1)], c, -m_new[qt]));
+        const float p1 = fast_exp2(fmaf(src[2 * (j & 1) + 1], c, -m_new[qt]));
+        psum[qt] = j == 0 ? p0 + p1 : psum[qt] + (p0 + p1);  // no 0 + x: x may be -0
+        w[j] = E::pack2(p0, p1);
       }
-      // Gamma += sum_j p_j * n_j.  Every block holds BT rows except the last one, NT - 1,
-      // which holds last_len: BT * sum(p) (exact, BT being a power of two), corrected for
-      // that block in the one group holding it.
-      float gsum[2] = {psum[0] * (float)BT, psum[1] * (float)BT};
-      if (g == NG - 1 && last_len != BT) {
-        const int mm_last = (NT - 1) - g * kGroup;  // block 16 bt + 4 g4 + i of the group
-        if (g4 == ((mm_last >> 2) & 3)) {
+      pbf[qt] = as_vec8<E>((u32x4_t){w[0], w[1], w[2], w[3]});
+    }
+    // Gamma += sum_j p_j * n_j.  Every block holds BT rows except the last one, NT - 1,
+    // which holds last_len: BT * sum(p) (exact, BT being a power of two), corrected for
+    // that block in the one group holding it.
+    float gsum[2] = {psum[0] * (float)BT, psum[1] * (float)BT};
+    if (g == NG - 1 && last_len != BT) {
+      const int mm_last = (NT - 1) - g * kGroup;  // block 16 bt + 4 g4 + i of the group
+      if (g4 == ((mm_last >> 2) & 3)) {
 #pragma unroll
-          for (int qt = 0; qt < 2; ++qt) {
-            float sl = sb[0][qt][0];
+        for (int qt = 0; qt < 2; ++qt) {
+          float sl = sb[0][qt][0];
 #pragma unroll
-            for (int bt = 0; bt < 2; ++bt)
+          for (int bt = 0; bt < 2; ++bt)
 #pragma unroll
-              for (int i = 0; i < 4; ++i)
-                if (16 * bt + i == (mm_last & 16) + (mm_last & 3)) sl = sb[bt][qt][i];
-            gsum[qt] += fast_exp2(fmaf(sl, c, -m_new[qt])) * (float)(last_len - BT);
-          }
+            for (int i = 0; i < 4; ++i)
+              if (16 * bt + i == (mm_last & 16) + (mm_last & 3)) sl = sb[bt][qt][i];
+          gsum[qt] += fast_exp2(fmaf(sl, c, -m_new[qt])) * (float)(last_len - BT);
         }
       }
+    }
 #pragma unroll
-      for (int qt = 0; qt < 2; ++qt) {
-        g_run[qt] += gsum[qt];
-        psum[qt] = quad16_sum(psum[qt]);
-      }
+    for (int qt = 0; qt < 2; ++qt) {
+      g_run[qt] += gsum[qt];
+      psum[qt] = quad16_sum(psum[qt]);
+    }
+    if (mine) {
 #pragma unroll
       for (int dt = 0; dt < DT; ++dt) {
         const vec8 a = as_vec8<E>(lds_ld<uint4>(Vs, pv_base + dt * 16 * kVtRow));
@@ -738,23 +740,23 @@ __device__ __forceinline__ void k4_body(const uint16_t* __restrict__ q, const ui
     barrier_lds_reads_done();  // every wave is done reading part 2 of group g; Hbar^T of g is in place
     if (gn >= 0) load_part2(gn);
 
+    // r^T = Hbar^T Q^T: racc[dt][qt] element i = feature 16 dt + 4 g4 + i of q.Hbar.
+    f32x4_t racc[DT][2];
+#pragma unroll
+    for (int dt = 0; dt < DT; ++dt)
+#pragma unroll
+      for (int qt = 0; qt < 2; ++qt)
+#pragma unroll
+        for (int i = 0; i < 4; ++i) racc[dt][qt][i] = 0.f;
+#pragma unroll
+    for (int ks = 0; ks < KS; ++ks)
+#pragma unroll
+      for (int dt = 0; dt < DT; ++dt) {
+        const vec8 a = as_vec8<E>(lds_ld<uint4>(Ks, kofs[ks] + dt * 16 * ROWB));
+#pragma unroll
+        for (int qt = 0; qt < 2; ++qt) racc[dt][qt] = E::mfma16(a, qf[qt][ks], racc[dt][qt]);
+      }
     if (mine) {
-      // r^T = Hbar^T Q^T: racc[dt][qt] element i = feature 16 dt + 4 g4 + i of q.Hbar.
-      f32x4_t racc[DT][2];
-#pragma unroll
-      for (int dt = 0; dt < DT; ++dt)
-#pragma unroll
-        for (int qt = 0; qt < 2; ++qt)
-#pragma unroll
-          for (int i = 0; i < 4; ++i) racc[dt][qt][i] = 0.f;
-#pragma unroll
-      for (int ks = 0; ks < KS; ++ks)
-#pragma unroll
-        for (int dt = 0; dt < DT; ++dt) {
-          const vec8 a = as_vec8<E>(lds_ld<uint4>(Ks, kofs[ks] + dt * 16 * ROWB));
-#pragma unroll
-          for (int qt = 0; qt < 2; ++qt) racc[dt][qt] = E::mfma16(a, qf[qt][ks], racc[dt][qt]);
-        }
 #pragma unroll
       for (int qt = 0; qt < 2; ++qt) {
         const float f = psum[qt] * scale;
