@@ -691,9 +691,8 @@ __device__ __forceinline__ bool any_tile(
     unsigned char* Hs = SPLIT ? lds : lds + C::Z_BYTES;
     constexpr int H0 = SPLIT ? 1 : 0;  // the item that Hbar's first rows come with
     const int c4 = tid % C::C4P, r4 = tid / C::C4P;
-    // Blocks [a, b) of one mask word that some wave of the workgroup does not select.
+    // TEAM = 1: blocks of one mask word that some wave of the workgroup does not select.
     auto word_unselected = [&](int wd) -> uint32_t {
-      if (TEAM != 1) return ~mrow[wd];
       uint32_t m = 0xffffffffu;
 #pragma unroll
       for (int i = 0; i < 4; ++i)
@@ -744,12 +743,16 @@ __device__ __forceinline__ bool any_tile(
     // above, split fp32 0.5%); with the fp32 MFMA that is 2% slower.
     int ig = -1, ijc = 0, ihs = 0;
     auto group_end = [&](int g) -> int { return (int)min((int64_t)NT, (int64_t)(g + 1) * G); };
+    uint32_t iap = 0u;  // TEAM = 4: the item's approximated blocks
     auto chunk_from = [&](int g, int jc) -> bool {  // the group's first chunk at or after jc with work
-      for (const int jb = group_end(g); jc < jb; jc += C::KZ)
-        if (any_unselected(jc, min(jc + C::KZ, jb))) {
+      for (const int jb = group_end(g); jc < jb; jc += C::KZ) {
+        const int cn = min(C::KZ, jb - jc);
+        if (TEAM != 1) iap = approx_bits(jc, cn);
+        if (TEAM == 1 ? any_unselected(jc, jc + cn) : iap != 0u) {
           ijc = jc;
           return true;
         }
+      }
       return false;
     };
     auto next_item = [&]() -> bool {
@@ -777,7 +780,7 @@ __device__ __forceinline__ bool any_tile(
     // V^ of a selected block is taken as zero: its weight is, but 0 times a sum that left the type's
     // range is NaN.  TEAM = 1: each wave selects its own, and clears them from its operands (below).
     auto fetch_z = [&](int jc, int cn) {
-      const uint32_t approx = TEAM == 1 ? 0xffffffffu : approx_bits(jc, cn);
+      const uint32_t approx = TEAM == 1 ? 0xffffffffu : iap;
       const float* kb = kcb + (int64_t)jc * D;
       const float* vb = vcb + (int64_t)jc * D;
       const rsrc_t rk = make_rsrc(kb, (uint32_t)(cn * D * 4)), rv = make_rsrc(vb, (uint32_t)(cn * D * 4));
@@ -818,6 +821,7 @@ __device__ __forceinline__ bool any_tile(
     }
     while (more) {
       const int g = ig, jc = ijc, hs = ihs;
+      const uint32_t ap = iap;
       const bool first = g != pg;
       pg = g;
       __syncthreads();  // the previous item's rows have been read
@@ -841,7 +845,7 @@ __device__ __forceinline__ bool any_tile(
           mine = false;
         }
         // Zero order: o += p V^.
-        const uint32_t approx = approx_bits(jc, min(C::KZ, group_end(g) - jc));
+        const uint32_t approx = TEAM == 1 ? approx_bits(jc, min(C::KZ, group_end(g) - jc)) : ap;
         const bool visit = TEAM != 1 || approx != 0u;
         if (visit) mine = true;
         const uint32_t ub = approx >> (4 * g4);
@@ -1089,8 +1093,8 @@ bool wide_tiles(const AnyCall& a, int BT) {
 
 // WIDE: 32 rows per wave where the blocks are long enough, measured at D 96.  Not in fp32, whose planes
 // or wider fragments then spill (283 registers).  At DP 128 the 16-bit ones spill too, 60 VGPRs below
-// block 64 and 45 from block 128 on, which every group of phase 2 reloads (16 rows would not; not
-// measured there: 12 heads x 16,380 rows, D 128, bf16, block 32 620-640 us, block 128, groups of 16 440).
+// block 64 and 33 from block 128 on, which every group of phase 2 reloads (16 rows would not; not
+// measured there: 12 heads x 16,380 rows, D 128, bf16, block 32 637 us, block 128, groups of 16 400).
 template <typename E, int DP, bool VEC, bool WIDE>
 hipError_t launch_dp(const AnyCall& a) {
   if (!a.all && a.BT < 64) {
