@@ -33,17 +33,17 @@
 // exponential), and a product is six MFMAs: x1 y1 into one sum, the smaller five into another, so
 // that they round at their own size.  Six bf16 MFMAs take 3/8 of the fp32 MFMA's time for the same
 // product, and round less: one addition per 32 terms where the fp32 MFMA rounds after every product.
-// Error against 64 bits at 12 heads x 7,800 rows, D 128, block 64: 7.3e-7 with one FMA per lane,
-// 5.0e-7 on the fp32 MFMA, 4.0e-7 so (with q and k of mean 1 and 3, where the scores cancel, 2.3e-6
-// and 2.1e-6 at 3,000 rows; with one sum over all 128 features 2.4e-6); K4 there 2.07 ms, 0.66 and
-// 0.45.
+// Error against 64 bits at 12 heads x 7,800 rows, D 128, block 64: 7.2e-7 with one FMA per lane,
+// 5.0e-7 on the fp32 MFMA, 3.8e-7 so (with q and k of mean 1 and 3, where the scores cancel, 1.8e-6
+// and 1.7e-6 at 2 heads x 3,000 rows; one sum over all 128 features rounds 8% more than one FMA per
+// lane); K4 there 2.07 ms, 0.66 and 0.46.
 // TEAM = 1 stays on the fp32 MFMA (Any32): a wave would split its own K/V rows for 16 queries.
 // Its fp32 sums are taken in short chains (16 features, a chunk of keys, 32 rows of Hbar) that are
 // then added: where q and k have a common mean the scores' rounding is the error, and it grows with
 // the chain (2 heads x 1,000 rows, D 128, block 32, means 1 and 3: 1.6e-6 with one FMA per lane, 3.0e-6
 // with chains of 64 features, which are 1 to 3% faster, 1.4e-6 so).
 //
-// What bounds it: Split32, the MFMA pipe (75 GFLOP of fp32, so 450 of bf16, in 0.45 ms, where a
+// What bounds it: Split32, the MFMA pipe (75 GFLOP of fp32, so 450 of bf16, in 0.46 ms, where a
 // large bf16 product takes 0.34), with a third as many VALU instructions for the splits;
 // Any32, the fp32 MFMA (153 TFLOP/s in a large product); 16 bits, the latency of the staged loads
 // and, in phase 2, of Hbar (16 heads x 8,610 rows, D 96, block 32, groups of 16: 149 GFLOP in
@@ -161,8 +161,8 @@ __device__ __forceinline__ void split4(const float (&x)[4], uint2 (&pl)[3]) {
 // For j = 0, 1: hi[j] += a1 b1 and lo[j] += the five products of the next orders of a = a[j], smallest
 // first.  With |x2| <= 2^-8 |x| and |x3| <= 2^-17 |x| what is left out (x2 y3 + x3 y2 + x3 y3) is at most
 // 2^-24 (1 + 2^-10) of a b (5.4e-2 of 2^-24 on average; with x1 cut instead of rounded up to 3.9 of 2^-24).  The two sums alternate, held in this order: an MFMA
-// that adds to the one before waits for it (480p shape above: 625 us with one after the other,
-// 615 in the compiler's order, 609 so).
+// that adds to the one before waits for it (the call above, when K2 and the loads were
+// slower: 625 us with one after the other, 615 in the compiler's order, 609 so).
 __device__ __forceinline__ void mfma_split(const bf16x8_t (&a)[2][3], const bf16x8_t (&b)[3], f32x4_t* const (&hi)[2],
                                            f32x4_t* const (&lo)[2]) {
   constexpr int PA[6] = {2, 0, 0, 1, 1, 0}, PB[6] = {0, 0, 2, 1, 0, 1};

@@ -60,8 +60,8 @@ constexpr int kAnyChunk = 32;  // rows of a staged K/V chunk
 //
 // Bound: the fp32 MFMA (2 D^2 FLOP per row) against three rows read; a block of 64 rows at D 128 is
 // 3.4 us of MFMA issue.  One workgroup per group left most of the 256 CUs idle and its FMAs waited
-// on four LDS reads per row: 12 heads x 7,800 fp32 rows of D 128 took 847 us (now 73 + 12 for the
-// reduction), 2 heads x 1,024 of D 64 291 us (now 11 + 6), 16 x 8,610 bf16 of D 96 248 us (65 + 7).
+// on four LDS reads per row: 12 heads x 7,800 fp32 rows of D 128 took 847 us (now 66 + 12 for the
+// reduction), 2 heads x 1,024 of D 64 291 us (now 8 + 6), 16 x 8,610 bf16 of D 96 248 us (66 + 7).
 template <typename EL, int DP>
 struct StatsCfg {
   static constexpr int CH = kAnyChunk;
@@ -299,7 +299,7 @@ __global__ __launch_bounds__(256) void k2_any_reduce(const float* __restrict__ p
 // times an odd number: 16 rows x 4 features fall into 64 distinct banks.
 //
 // One thread per score instead, each reading both of its rows from L2, took 420 us at 16 heads x
-// 270 blocks of D 96 (now 10).
+// 270 blocks of D 96 (now 11).
 constexpr int kScoreTile = 64;
 
 __global__ __launch_bounds__(256) void k3_scores_any(const float* __restrict__ qc, const float* __restrict__ kc,

@@ -80,7 +80,8 @@ hipError_t launch_sparse_attn_any(const void* q, const void* k, const void* v, c
                                   const float* hgroup, const uint32_t* selmask, void* o, float scale, int bh, int T,
                                   int text, int text_valid, int D, int BT, int G, int gamma_literal, int all,
                                   int dtype, hipStream_t stream);
-int64_t sparse_attn_any_tiles(int T, int text, int text_valid, int BT);  // grid.x of launch_sparse_attn_any
+// 64-row tiles of a slice: at least as many as any launch of launch_sparse_attn_any has along grid x.
+int64_t sparse_attn_any_tiles(int T, int text, int text_valid, int BT);
 
 // ---- K5: processor prologue (RMSNorm + rotary embedding + head-major layout) ----
 constexpr int kNormHead = 1;       // RMSNorm over each head's D channels, weight [D]

@@ -641,8 +641,8 @@ __device__ __forceinline__ void k4_body(const uint16_t* __restrict__ q, const ui
 
     // PAIR: a wave whose block selects the whole group adds nothing to o (its weights are 0, and 0 times a
     // sum that is not finite would be NaN).  The branches enclose just the two sums: around the scores and
-    // q Hbar as well they cost 1 to 2% (24 heads x 119 k rows: 28.19-28.53 ms against 27.54-27.83 without
-    // any; so 27.65-28.31 against 27.93-28.44 on another box).
+    // q Hbar as well they cost 1 to 2%, so 0 to 0.5% (24 heads x 119 k rows, three comparisons with neither:
+    // 28.3 ms against 28.2, 27.7 against 27.6, 27.9 against 28.3).
     const bool mine = !PAIR || approx != 0u;
     // s-bar^T = kbar Q^T: sb[bt][qt] element i = block 16 bt + 4 g4 + i of the group.
     f32x4_t sb[2][2];
