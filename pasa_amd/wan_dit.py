@@ -189,9 +189,11 @@ class WanBlock(nn.Module):
     def _ffn_fused(self, x):
         """The feed-forward with its GELU in the first product's epilogue: 782 us at 32,760 x 1536 x
         8960, 1110 with the GELU as a pass of its own over the 587 MB between them."""
+        if not _plain(self.ffn, nn.Sequential) or len(self.ffn) != 3:
+            return self.ffn(x)
         up, act, down = self.ffn
-        if not (_plain(self.ffn, nn.Sequential) and _plain(up, nn.Linear) and _plain(act, nn.GELU)
-                and act.approximate == "tanh" and _in_type(x, up.weight, up.bias)):
+        if not (_plain(up, nn.Linear) and _plain(act, nn.GELU) and act.approximate == "tanh"
+                and _in_type(x, up.weight, up.bias)):
             return self.ffn(x)
         h = torch._addmm_activation(up.bias, x.reshape(-1, x.shape[-1]), up.weight.t(), use_gelu=True)
         return down(h.view(*x.shape[:-1], h.shape[-1]))

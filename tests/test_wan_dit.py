@@ -245,3 +245,20 @@ def test_fused_cross_attention_wants_plain_projections(monkeypatch):
         setattr(attn, name, lin)
         lin.register_forward_hook(lambda m, i, o: o.float())
         assert not W._cross_fusable(attn, x, text)
+
+
+def test_feed_forward_of_another_make():
+    """A feed-forward that is not the block's own three modules is called as it is."""
+    class Mlp(torch.nn.Module):
+        def forward(self, x):
+            return x * 3
+
+    cfg = W.WanDiTConfig(num_layers=1, num_attention_heads=2, ffn_dim=64, text_dim=32, freq_dim=16)
+    x = torch.randn(1, 3, 256)
+    lin = lambda a, b: torch.nn.Linear(a, b)
+    for ffn in (Mlp(), torch.nn.Sequential(lin(256, 256)), torch.nn.Sequential(),
+                torch.nn.Sequential(lin(256, 64), torch.nn.GELU(approximate="tanh"), torch.nn.Dropout(0.0), lin(64, 256))):
+        blk = W.WanBlock(cfg)
+        blk.ffn = ffn
+        with torch.no_grad():
+            assert torch.equal(blk._ffn_fused(x), ffn(x))
