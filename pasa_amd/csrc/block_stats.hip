@@ -396,11 +396,14 @@ __global__ __launch_bounds__(256) void k2_group_reduce(const float* __restrict__
 }
 
 // Parts per group: enough workgroups for about two per CU (256 CUs) when the grid of
-// groups alone is small, at least 4 blocks per part.
-int block_stats_split(int bh, int T, int BT, int G) {
+// groups alone is small, at least 4 blocks per part.  At head dim 64 groups of fewer than 16 blocks stay
+// whole: two parts of 4 save 2.6 us there (2 heads x 1,024 rows, block 128: 12.2 and 9.6 us; 16 blocks of
+// 64 17.8 and 9.0), and the second launch and the workspace cost the host 5 (a call 49 and 54 us).
+int block_stats_split(int bh, int T, int D, int BT, int G) {
   const int NT = (T + BT - 1) / BT;
   const int64_t groups = (int64_t)((NT + G - 1) / G) * bh;
   const int nblk = min(G, NT);
+  if (D == 64 && nblk < 16) return 1;
   int split = 1;
   while (split < 8 && groups * split < 512 && nblk / (2 * split) >= 4) split *= 2;
   return split;

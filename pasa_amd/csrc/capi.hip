@@ -240,7 +240,8 @@ static int block_stats_impl(const void* q, const void* k, const void* v, float* 
   if (group_size <= 0 || group_size > 1 << 20) return fail(PASA_ERR_GROUP_SIZE, "group_size %lld must be in [1, 2^20]", (long long)group_size);
   int split = 1;
   if (workspace != nullptr) {
-    split = pasa::block_stats_split((int)bh, (int)(seq_len - text_len), (int)block_size, (int)group_size);
+    split = pasa::block_stats_split((int)bh, (int)(seq_len - text_len), (int)head_dim, (int)block_size,
+                                            (int)group_size);
     const size_t need = pasa_block_stats_workspace_bytes(bh, seq_len, text_len, head_dim, block_size, group_size);
     if (workspace_bytes < need)
       return fail(PASA_ERR_WORKSPACE, "pasa_block_stats_ws: workspace %zu bytes < %zu", workspace_bytes, need);
@@ -266,7 +267,8 @@ size_t pasa_block_stats_workspace_bytes(int64_t bh, int64_t seq_len, int64_t tex
       group_size > 1 << 20)
     return 0;
   if (head_dim != 128) return 0;
-  const int split = pasa::block_stats_split((int)bh, (int)(seq_len - text_len), (int)block_size, (int)group_size);
+  const int split = pasa::block_stats_split((int)bh, (int)(seq_len - text_len), (int)head_dim, (int)block_size,
+                                            (int)group_size);
   if (split == 1) return 0;
   const int64_t ng = cdiv(cdiv(seq_len - text_len, block_size), group_size);
   return (size_t)bh * (size_t)ng * (size_t)split * (size_t)(head_dim * head_dim) * sizeof(float);
@@ -280,7 +282,8 @@ size_t pasa_block_stats_workspace_bytes_dtype(int64_t bh, int64_t seq_len, int64
   if (check_any_dtype(dtype, "pasa_block_stats") ||
       check_any_shape(bh, seq_len, text_len, head_dim, block_size, group_size, "pasa_block_stats"))
     return 0;
-  const int split = tuned ? pasa::block_stats_split((int)bh, (int)(seq_len - text_len), (int)block_size, (int)group_size)
+  const int split = tuned ? pasa::block_stats_split((int)bh, (int)(seq_len - text_len), (int)head_dim, (int)block_size,
+                                                    (int)group_size)
                           : pasa::block_stats_any_split((int)bh, (int)(seq_len - text_len), (int)block_size,
                                                         (int)group_size);
   if (split == 1) return 0;

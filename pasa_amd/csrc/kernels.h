@@ -27,7 +27,7 @@ hipError_t launch_block_stats(const void* q, const void* k, const void* v, float
                               float* vc, float* hnorm, float* hgroup, int bh, int T, int Tslice, int D,
                               int BT, int G, const RowMap* rm, void* const* tm_copies, float* partials, int split,
                               bool f16, hipStream_t stream);
-int block_stats_split(int bh, int T, int BT, int G);  // the split the launcher is given by the C ABI
+int block_stats_split(int bh, int T, int D, int BT, int G);  // the split the launcher is given by the C ABI
 
 hipError_t launch_scores(const float* qc, const float* kc, const float* hnorm, const float* noise,
                          float scale, int use_cov_bias, float* scores, int bh, int NT, int D,

@@ -11,6 +11,9 @@ def test_workspace_bytes_dtype():
     assert f(12, 32760, 0, 128, 128, 32, _lib.DTYPE_F16) == old(12, 32760, 0, 128, 128, 32)
     # head_dim 64: at least four blocks to a part (eight groups of 32 blocks per slice here)
     assert f(12, 32760, 0, 64, 128, 32, _lib.DTYPE_BF16) == 12 * 8 * 8 * 64 * 64 * 4
+    # and groups of 16 or more: a smaller one is done before a second launch pays
+    assert f(2, 1024, 0, 64, 128, 32, _lib.DTYPE_BF16) == f(2, 959, 0, 64, 64, 32, _lib.DTYPE_BF16) == 0
+    assert f(2, 1024, 0, 64, 64, 32, _lib.DTYPE_BF16) == 2 * 4 * 64 * 64 * 4
     # the any-shape kernels: a power-of-two number of parts of D x D floats per group, at most one per block
     per_group = 64 * 64 * 4
     assert f(2, 1024, 0, 64, 64, 32, _lib.DTYPE_F32) == 2 * 16 * per_group
