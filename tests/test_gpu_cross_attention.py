@@ -54,6 +54,21 @@ def test_merge_heads(device, B, H, S, D):
     assert torch.equal(merge_heads(view), want) and merge_heads(view).data_ptr() == view.data_ptr()
 
 
+@pytest.mark.parametrize("B,H,S,D", [(1, 12, 1000, 128), (2, 3, 5, 64), (1, 64, 9, 128), (1, 12, 4200, 128)])
+def test_merge_heads_on_the_kernel(device, monkeypatch, B, H, S, D):
+    """The layout pass itself at the sizes that the rule leaves to PyTorch, and one that it takes."""
+    from pasa_amd.processors import qknorm
+    calls = []
+    prologue = qknorm.qkv_prologue
+    monkeypatch.setattr(qknorm, "qkv_prologue", lambda *a, **k: calls.append(1) or prologue(*a, **k))
+    x = torch.randn(B, H, S, D, device=device, dtype=torch.bfloat16)
+    want = x.transpose(1, 2).flatten(2, 3)
+    assert torch.equal(merge_heads(x), want)
+    assert len(calls) == (x.numel() >= qknorm.MERGE_KERNEL_MIN)
+    monkeypatch.setattr(qknorm, "MERGE_KERNEL_MIN", 0)
+    assert torch.equal(merge_heads(x), want) and calls
+
+
 def test_rejected_arguments(device):
     q, k, v = (t.to(device) for t in make(1, 2, 16, 8, torch.bfloat16, 0))
     with pytest.raises(ValueError):
