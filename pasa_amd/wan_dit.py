@@ -134,6 +134,10 @@ class WanBlock(nn.Module):
     run as four fused row-ops calls (``pasa_amd.modulate``) instead of PyTorch
     elementwise passes; off, the block is diffusers' PyTorch forward."""
     fast_kernels = True
+    # Rows (of all samples) from which the fused cross-attention and feed-forward are taken: below, the
+    # host bounds the block, and their checks and calls cost it 12 and 5 us (dim 1536: 64 to 1,560 rows
+    # 460-466 us with both, 441-448 without; 2,048 464 and 464; 3,120 735 and 774).
+    fused_min_rows = 2048
 
     def __init__(self, cfg: WanDiTConfig):
         super().__init__()
@@ -178,12 +182,13 @@ class WanBlock(nn.Module):
         norm = torch.empty_like(hidden_states)
         M.row_ops(attn_out.contiguous(), residual=hidden_states.contiguous(), gate=gate_msa, h_out=h,
                   layernorm=True, weight=self.norm2.weight, bias=self.norm2.bias, y=norm, eps=self.norm2.eps)
-        if _cross_fusable(self.attn2, norm, encoder_hidden_states):
+        many = h.shape[0] * h.shape[1] >= self.fused_min_rows
+        if many and _cross_fusable(self.attn2, norm, encoder_hidden_states):
             attn_out = _cross_attention_fused(self.attn2, norm, encoder_hidden_states)
         else:
             attn_out = self.attn2(norm, encoder_hidden_states=encoder_hidden_states)
         norm = M.residual_ln_modulate(h, attn_out.contiguous(), c_scale_msa, c_shift_msa, self.norm3.eps)
-        M.gate_residual(h, self._ffn_fused(norm), c_gate_msa)
+        M.gate_residual(h, self._ffn_fused(norm) if many else self.ffn(norm), c_gate_msa)
         return h
 
     def _ffn_fused(self, x):

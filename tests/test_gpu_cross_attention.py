@@ -87,6 +87,7 @@ def test_block_with_and_without_the_fused_cross_attention(device):
     torch.manual_seed(0)
     cfg = W.WanDiTConfig(num_layers=1, num_attention_heads=2, ffn_dim=512, text_dim=64, freq_dim=16)
     blk = W.WanBlock(cfg).to(device, torch.bfloat16).eval()
+    blk.fused_min_rows = 0
     x = torch.randn(1, 300, 256, device=device, dtype=torch.bfloat16)
     text = torch.randn(1, 37, 256, device=device, dtype=torch.bfloat16)
     temb = torch.randn(1, 6, 256, device=device, dtype=torch.bfloat16)
@@ -101,3 +102,28 @@ def test_block_with_and_without_the_fused_cross_attention(device):
     err = float((a.double() - b.double()).norm() / b.double().norm())
     print(f"[cross] block fused against modules: rel {err:.2e}", flush=True)
     assert err <= 2.0 ** -7
+
+
+@pytest.mark.parametrize("B,S,least,fused", [(1, 300, 0, True), (2, 1025, 2048, True), (1, 300, 2048, False)])
+def test_block_fuses_from_a_number_of_rows_on(device, monkeypatch, B, S, least, fused):
+    """The routes of the same block by its rows, with the bound of the test above between the two."""
+    from pasa_amd import wan_dit as W
+    torch.manual_seed(0)
+    cfg = W.WanDiTConfig(num_layers=1, num_attention_heads=2, ffn_dim=512, text_dim=64, freq_dim=16)
+    blk = W.WanBlock(cfg).to(device, torch.bfloat16).eval()
+    x = torch.randn(B, S, 256, device=device, dtype=torch.bfloat16)
+    text = torch.randn(B, 37, 256, device=device, dtype=torch.bfloat16)
+    temb = torch.randn(B, 6, 256, device=device, dtype=torch.bfloat16)
+    calls = []
+    cross = W._cross_attention_fused
+    monkeypatch.setattr(W, "_cross_attention_fused", lambda *a: calls.append(1) or cross(*a))
+    ffn = W.WanBlock._ffn_fused
+    monkeypatch.setattr(W.WanBlock, "_ffn_fused", lambda self, x: calls.append(2) or ffn(self, x))
+    with torch.no_grad():
+        blk.fused_min_rows = B * S + 1
+        b = blk(x, text, temb, None)
+        assert not calls
+        blk.fused_min_rows = least
+        a = blk(x, text, temb, None)
+    assert calls == ([1, 2] if fused else [])
+    assert float((a.double() - b.double()).norm() / b.double().norm()) <= (2.0 ** -7 if fused else 0.0)
