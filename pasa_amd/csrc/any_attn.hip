@@ -160,9 +160,9 @@ __device__ __forceinline__ void split4(const float (&x)[4], uint2 (&pl)[3]) {
 
 // For j = 0, 1: hi[j] += a1 b1 and lo[j] += the five products of the next orders of a = a[j], smallest
 // first.  With |x2| <= 2^-8 |x| and |x3| <= 2^-17 |x| what is left out (x2 y3 + x3 y2 + x3 y3) is at most
-// 2^-24 (1 + 2^-10) of a b (5.4e-2 of 2^-24 on average; with x1 cut instead of rounded up to 3.9 of 2^-24).  The two sums alternate, held in this order: an MFMA
-// that adds to the one before waits for it (the call above, when K2 and the loads were
-// slower: 625 us with one after the other, 615 in the compiler's order, 609 so).
+// 2^-24 (1 + 2^-10) of a b, 0.054 of 2^-24 on average (up to 3.9 with x1 cut instead of rounded).  The two
+// sums alternate, held in this order: an MFMA that adds to the one before waits for it (the call above,
+// when its loads were slower: 625 us with one after the other, 615 in the compiler's order, 609 so).
 __device__ __forceinline__ void mfma_split(const bf16x8_t (&a)[2][3], const bf16x8_t (&b)[3], f32x4_t* const (&hi)[2],
                                            f32x4_t* const (&lo)[2]) {
   constexpr int PA[6] = {2, 0, 0, 1, 1, 0}, PB[6] = {0, 0, 2, 1, 0, 1};
@@ -180,7 +180,7 @@ __device__ __forceinline__ void mfma_split(const bf16x8_t (&a)[2][3], const bf16
 // Powers of two that Split32 multiplies operands by before their split (16 or more cover the subnormals,
 // whose last bit is 2^-149 where a bf16 part's is 2^-133).  The scores are then 2^40, O 2^56 times
 // their values, in P V^ as in q Hbar.  K stays as it is: with q below 2^88 (above, its parts are not
-// finite) a part below 2^-133 of it moves no exponent c s by more than 2^-28.
+// finite) a part below 2^-133 of it moves no exponent c s by more than 2^-27.
 // Without them v of 2^-118 comes out to 6.7e-6, of 2^-130 to 2.8e-2; with them as with fp32 products.
 // They cost 1 to 2% (12 heads x 7,800 rows, block 64: D 128 564 -> 571 us, D 64 276 -> 281).
 constexpr float kUpQ = 0x1p40f, kUpP = 0x1p16f, kUpV = 0x1p40f, kUpH = 0x1p16f;
@@ -1024,9 +1024,10 @@ __device__ __forceinline__ bool any_tile(
 }  // namespace
 
 // Three waves per SIMD for Any32 at DP 96: its scores' partial sums take it past 168 registers, and two
-// waves are slower than the 24 that then spill (12 heads x 7,800 rows, D 96, block 32: 850 and 779 us).
+// waves are slower than the 20 that then spill (12 heads x 7,800 rows, D 96, block 32: 850 and 779 us).
 template <typename E, int DP, int TEAM, int RW, bool VEC>
-__global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(AnyCfg<E, DP, TEAM, RW>::F32 && DP == 96 ? 3 : 2))) void k4_any_mfma(
+__global__ __launch_bounds__(256)
+__attribute__((amdgpu_waves_per_eu(AnyCfg<E, DP, TEAM, RW>::F32 && DP == 96 ? 3 : 2))) void k4_any_mfma(
     const unsigned char* __restrict__ q, const unsigned char* __restrict__ k, const unsigned char* __restrict__ v,
     const float* __restrict__ kc, const float* __restrict__ vc, const float* __restrict__ hgroup,
     const uint32_t* __restrict__ selmask, unsigned char* __restrict__ o, float scale, float c, int T, int text,
